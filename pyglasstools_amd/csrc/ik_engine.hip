@@ -176,11 +176,21 @@ int gl_rule(int n, std::vector<double> &s, std::vector<double> &w)
 // the box faces (as numpy.linspace makes them) maps onto the indices 0..n-1
 // exactly, so for n a power of two every run of 4^k (2D) or 8^k (3D) points
 // is a square (cube) block.
-std::vector<int> morton_order(int64_t G, const double *grid, bool use_z)
+// `tiles` gets where the tile gather's tiles start in the order (and G at the
+// end): a tile is the points of one block of 8 x 8 (2D) or 4 x 4 x 4 lattice
+// sites, at most kTilePoints of them.  Runs of kTilePoints points regardless
+// of the blocks would straddle two of them wherever the grid's side is not a
+// multiple of the block's, and two blocks that follow each other can lie far
+// apart, which would make the tile's window of particles large.
+std::vector<int> morton_order(int64_t G, const double *grid, bool use_z, std::vector<int> &tiles)
 {
     std::vector<int> perm((size_t)G);
     std::iota(perm.begin(), perm.end(), 0);
-    if (G < 2) return perm;
+    tiles.assign(1, 0);
+    if (G < 2) {
+        if (G == 1) tiles.push_back(1);
+        return perm;
+    }
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (int64_t i = 0; i < G; ++i)
         for (int a = 0; a < 3; ++a) {
@@ -204,6 +214,10 @@ std::vector<int> morton_order(int64_t G, const double *grid, bool use_z)
         key[(size_t)i] = k;
     }
     std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return key[(size_t)x] < key[(size_t)y]; });
+    for (int64_t t = 1; t < G; ++t)
+        if (t - tiles.back() == kTilePoints || key[(size_t)perm[t]] >> 6 != key[(size_t)perm[t - 1]] >> 6)
+            tiles.push_back((int)t);
+    tiles.push_back((int)G);
     return perm;
 }
 
@@ -253,6 +267,8 @@ struct pgt_ik_engine {
     DBuf<double> d_pos, d_diam, d_mass, d_vel, d_disp;  // single-frame host uploads
     DBuf<double> d_grid;
     DBuf<int> d_perm;
+    DBuf<int> d_tiles;  // tile starts in d_perm (morton_order), ntiles + 1
+    int ntiles = 0;
     // work arrays of a batch (see WorkArray), as raw bytes
     DBuf<unsigned char> d_keys0, d_vals0, d_keys1, d_vals1, d_hist, d_cstart, d_bcount;
     DBuf<unsigned char> d_spos, d_sdiam, d_skin, d_sdisp;
@@ -415,6 +431,7 @@ Geom make_geom(const pgt_ik_engine *e, int D)
         g.cs[a] = e->L[a] / nc;
         g.ncell *= nc;
     }
+    g.rc = e->prm.cg_rcut;
     g.rc2 = e->prm.cg_rcut * e->prm.cg_rcut;
     g.inv_rc = 1.0 / e->prm.cg_rcut;
     g.inv_rc2 = 1.0 / g.rc2;
@@ -489,7 +506,8 @@ struct JobShape {
     int npass, nbits, radix;
     size_t ebytes;
     int block, pl;
-    bool tile;       // the item-balanced tile gather (kTilePoints points per workgroup of kTileThreads lanes)
+    bool tile;       // the item-balanced tile gather
+    int tp;          // its grid points per workgroup of kTileThreads lanes
     int64_t gwaves;  // gather wavefronts per frame
     bool qag_global; // adaptive rule: interval tables of the caller's limit in e->d_qag
 };
@@ -527,7 +545,8 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     if (j.tile) {
         j.block = kTileThreads;
         j.pl = 1;
-        j.gwaves = (e->G + kTilePoints - 1) / kTilePoints * (kTileThreads / 64);
+        j.tp = kTilePoints;
+        j.gwaves = (int64_t)e->ntiles * (kTilePoints / j.tp);
     } else {
         // the adaptive gather deals each point's integrals to several lanes
         const int64_t lanes = j.adaptive ? e->G * adaptive_lanes(e->G) : (e->G + j.pl - 1) / j.pl;
@@ -692,6 +711,9 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     c.block = j.block;
     c.grid = e->d_grid.p;
     c.perm = e->d_perm.p;
+    c.tiles = e->d_tiles.p;
+    c.ntiles = e->ntiles;
+    c.tp = j.tp;
     c.R.n = (int)e->gl_s.size();
     for (int k = 0; k < c.R.n && k < kMaxQArg; ++k) {
         c.R.s[k] = e->gl_s[k];
@@ -1068,7 +1090,7 @@ void pgt_ik_destroy(pgt_ik_engine *e)
     DBuf<double> *dbufs[] = {&e->d_pos, &e->d_diam, &e->d_mass, &e->d_vel, &e->d_disp, &e->d_grid,
                              &e->d_out, &e->d_gl};
     for (auto *b : dbufs) b->release();
-    DBuf<int> *ibufs[] = {&e->d_perm, &e->d_maxcount};
+    DBuf<int> *ibufs[] = {&e->d_perm, &e->d_tiles, &e->d_maxcount};
     for (auto *b : ibufs) b->release();
     DBuf<unsigned char> *wbufs[] = {&e->d_keys0, &e->d_vals0, &e->d_keys1, &e->d_vals1, &e->d_hist, &e->d_cstart,
                                     &e->d_bcount, &e->d_spos, &e->d_sdiam, &e->d_skin, &e->d_sdisp, &e->d_bonds,
@@ -1161,17 +1183,22 @@ int pgt_ik_set_grid(pgt_ik_engine *e, int64_t g, const double *grid)
         for (int a = 0; a < 3; ++a) amax = std::max(amax, std::fabs(grid[3 * i + a]));
     }
     if (!(amax < INFINITY)) amax = INFINITY;  // NaN coordinates: no FP32 pre-test
-    const std::vector<int> perm = morton_order(g, grid, !flat || e->prm.dim == 3);
+    std::vector<int> tiles;
+    const std::vector<int> perm = morton_order(g, grid, !flat || e->prm.dim == 3, tiles);
     int rc;
-    if ((rc = e->d_grid.ensure((size_t)g * 3)) || (rc = e->d_perm.ensure((size_t)g))) return rc;
+    if ((rc = e->d_grid.ensure((size_t)g * 3)) || (rc = e->d_perm.ensure((size_t)g)) ||
+        (rc = e->d_tiles.ensure(tiles.size())))
+        return rc;
     if (g > 0) {
         HIPCHK(hipMemcpyAsync(e->d_grid.p, grid, sizeof(double) * g * 3, hipMemcpyHostToDevice, e->stream));
         HIPCHK(hipMemcpyAsync(e->d_perm.p, perm.data(), sizeof(int) * g, hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->d_tiles.p, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice, e->stream));
     }
     HIPCHK(hipStreamSynchronize(e->stream));
     e->h_grid.assign(grid, grid + 3 * g);
     e->grid_z_flat = flat;
     e->grid_absmax = amax;
+    e->ntiles = (int)tiles.size() - 1;
     e->G = g;
     e->have_grid = true;
     return PGT_OK;
@@ -1786,7 +1813,8 @@ struct pgt_ik_sweep {
     bool held = false;     // enqueued launches a captured graph may replay
     DBuf<SweepSys> d_tab;
     DBuf<double> d_grid;   // the systems' grids, back to back
-    DBuf<int> d_perm;      // and their Morton orders
+    DBuf<int> d_perm;      // their Morton orders
+    DBuf<int> d_tiles;     // and tile starts
     DBuf<unsigned char> d_keys0, d_vals0, d_keys1, d_vals1, d_hist, d_cstart, d_spos, d_sdiam, d_bcount, d_skin;
     DBuf<unsigned char> d_bonds, d_wcounts, d_wmax, d_rec;
     DBuf<int> d_maxcount;                // [0] largest bond count, [1] tile overflow bits
@@ -1900,7 +1928,6 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
     c.skin = s->kin ? skin : nullptr;
     c.cap = s->cap;
     c.bcount = s->vir ? bcount : nullptr;
-    c.rec = rec;
     c.bonds = s->vir ? (const void *)s->d_bonds.p : nullptr;
     c.wave_counts = (unsigned long long *)s->d_wcounts.p;
     c.flags = s->d_maxcount.p + 1;
@@ -1990,7 +2017,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
                          : sizeof(double) * BondLayout<3, 3, false, double>::ES;
     s->tab.resize((size_t)nsys);
     int maxcell = 1, cap = 0;
-    int64_t gtotal = 0;
+    int64_t gtotal = 0, ttotal = 0;
     for (int k = 0; k < nsys; ++k) {
         const pgt_ik_engine *e = systems[k].engine;
         SweepSys &S = s->tab[(size_t)k];
@@ -2005,6 +2032,8 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         maxcell = std::max(maxcell, S.g.ncell);
         cap = std::max(cap, e->cap);
         gtotal += e->G;
+        ttotal += e->ntiles + 1;
+        S.tp = kTilePoints;
     }
     int kbits = 0;
     while ((1 << kbits) < maxcell) ++kbits;
@@ -2028,7 +2057,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         S.bpf[SW_SORT] = S.nchunk;
         S.bpf[SW_FINISH] = (S.n + 255) / 256;
         S.bpf[SW_BONDS] = (S.n + bond_block(D) - 1) / bond_block(D);
-        S.bpf[SW_GATHER] = (S.G + kTilePoints - 1) / kTilePoints;
+        S.bpf[SW_GATHER] = systems[k].engine->ntiles * (kTilePoints / S.tp);
         for (int st = 0; st < SW_NSTAGE; ++st) {
             const int64_t nb = (st == SW_SORT || st == SW_FINISH)
                                    ? (int64_t)frame_rows(S.nf) * S.bpf[st]
@@ -2051,19 +2080,23 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         return bail(fail(PGT_ERR_RANGE, "the sweep holds more than 2^31 - 1 particles over all frames: split it"));
     int rc;
     if ((rc = s->d_grid.ensure((size_t)gtotal * 3)) || (rc = s->d_perm.ensure((size_t)gtotal)) ||
-        (rc = s->d_tab.ensure((size_t)nsys)))
+        (rc = s->d_tiles.ensure((size_t)ttotal)) || (rc = s->d_tab.ensure((size_t)nsys)))
         return bail(rc);
-    int64_t goff = 0;
+    int64_t goff = 0, toff = 0;
     for (int k = 0; k < nsys; ++k) {
         const pgt_ik_engine *e = systems[k].engine;
         SweepSys &S = s->tab[(size_t)k];
         S.grid = s->d_grid.p + goff * 3;
         S.perm = s->d_perm.p + goff;
+        S.tiles = s->d_tiles.p + toff;
         if (hipMemcpy((void *)S.grid, e->d_grid.p, sizeof(double) * 3 * (size_t)e->G, hipMemcpyDeviceToDevice) !=
                 hipSuccess ||
-            hipMemcpy((void *)S.perm, e->d_perm.p, sizeof(int) * (size_t)e->G, hipMemcpyDeviceToDevice) != hipSuccess)
+            hipMemcpy((void *)S.perm, e->d_perm.p, sizeof(int) * (size_t)e->G, hipMemcpyDeviceToDevice) != hipSuccess ||
+            hipMemcpy((void *)S.tiles, e->d_tiles.p, sizeof(int) * (size_t)(e->ntiles + 1), hipMemcpyDeviceToDevice) !=
+                hipSuccess)
             return bail(fail(PGT_ERR_HIP, "copying a system's grid"));
         goff += e->G;
+        toff += e->ntiles + 1;
     }
     if (hipMemcpy(s->d_tab.p, s->tab.data(), sizeof(SweepSys) * (size_t)nsys, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(PGT_ERR_HIP, "uploading the sweep's table"));
@@ -2086,6 +2119,7 @@ void pgt_ik_sweep_destroy(pgt_ik_sweep *s)
     s->d_tab.release();
     s->d_grid.release();
     s->d_perm.release();
+    s->d_tiles.release();
     s->d_maxcount.release();
     s->d_stats.release();
     for (hipEvent_t v : s->ev)

@@ -1,31 +1,40 @@
 // ik_gather_tile.hpp -- the item-balanced field gather ("tile" gather) of
 // the IK stress-field engine.  Included by ik_gather_launch.hpp.
 //
-// A workgroup is one wavefront and takes 64 consecutive grid points in Morton
-// order (a compact tile of the grid), one per lane.  Work items are the
-// (grid point, particle) pairs with the particle inside the point's ball;
-// an item integrates the particle's bonds for the point.
+// A workgroup is one wavefront and takes a tile: up to 64 neighbouring grid
+// points (a block of the grid's Morton order).  Work items are the (grid
+// point, particle) pairs with the particle inside the point's ball; an item
+// integrates the particle's bonds for the point.
 //
-// 1. Scan: each lane walks the cells around its point, as the lane gather
-//    does, in steps of NB candidates that every lane takes together, and
-//    tests them exactly (FP64 minimum image, |a|^2 < r_cg^2; in 3D with
-//    bonds an FP32 test on the bond kernel's records first, with the FP64
-//    test for the band where FP32 rounding could decide).  The items found
-//    go to a list shared by the wavefront (ballot, prefix count).  A 2D
-//    scan reads candidate positions only; the bond counts of the items found
-//    are loaded before the sort, a batch per lane (in 3D the record holds
-//    the count).
-// 2. When the list could overflow, and at the end: the list is sorted by
-//    the particle's bond count, largest first (stable counting sort), and
-//    lane l takes items l, l + 64, ...: the 64 items of a step have nearly
-//    equal bond counts, so the bond loop wastes few lanes whatever the
-//    spread of the counts between points.  The next step's particle data and
-//    first bond entries are loaded while the current step integrates.  A lane
-//    sums its item in registers and adds it to the point's FP64 accumulators
-//    in LDS.
+// 1. Window: the particles within r_cg of the tile's bounding box, read from
+//    the rows of cells that cover it, one particle per lane, into a list in
+//    LDS.
+// 2. Masks: a lane holds one window particle and tests it against every point
+//    of the tile (FP64, |a|^2 < r_cg^2; the points are broadcast from LDS),
+//    which gives the particle's mask of points.
+// 3. Items: the particles are ordered by bond count, largest first, and their
+//    items written to a list in that order, a particle's items side by side.
+// 4. Integration: lane l takes items l, l + 64, ...: the 64 items of a step
+//    have nearly equal bond counts, so the bond loop wastes few lanes
+//    whatever the spread of the counts, and neighbouring lanes mostly share
+//    their particle, so that a load of bond entries touches the entries of
+//    about nine particles instead of 64.  A lane sums its item in registers
+//    and adds it to the point's FP64 accumulators in LDS.
 //
 // The wavefront runs alone in its workgroup and every step is in a fixed
 // order, so the sums are the same from run to run.
+//
+// Why particles, not points, are spread over the lanes in the scan: scattered
+// loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
+// when the lanes' lines differ).  With a point per lane, each lane walked its
+// own cells and every item fetched its particle from memory: 216 loads a
+// wavefront on the 2D N = 65,536 job with a 256^2 grid.  Here a window
+// particle is loaded once per tile, and an item's entries are shared by its
+// neighbours.  Measured against that scan (one launch): 100 such frames
+// 1.68 -> 1.38 ms, 3D N = 131,072 with a 64^3 grid, FP32 form, 20 frames
+// 4.30 -> 3.72 ms, 3D FP64 with the kinetic field, N = 20,011, 5 frames
+// 0.43 -> 0.37 ms, a sweep of eight systems whose grids are up to 2.4 r_cg / 2
+// apart 0.80 -> 0.65 ms.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -43,13 +52,13 @@ namespace pgt {
 // Capacities of the tile gather.
 struct TileCaps {
     static constexpr int BLK = kTileThreads;  // one wavefront
-    static constexpr int TP = kTilePoints;    // grid points per tile, one per lane
-    static constexpr int MAXI = 768;          // items in the list
-    static constexpr int NB = 4;              // candidates per lane per scan step
-    static constexpr int PBITS = 26;          // item word: particle index | point << PBITS
-    static constexpr int MAXNB = 255;         // bond count of an item (one byte); more: overflow
-    static_assert(TP == 64 && BLK == 64, "one wavefront of 64 points");
-    static_assert(MAXI >= 2 * 64 * NB, "the list holds two scan steps");
+    static constexpr int TP = kTilePoints;    // most grid points of a tile
+    static constexpr int MAXW = 128;          // window particles listed at a time
+    static constexpr int MAXI = 1024;         // items listed at a time
+    static constexpr int SBITS = 8;           // item word: window slot | point << SBITS
+    static constexpr int MAXNB = 255;         // bond count of a particle (one byte); more: overflow
+    static_assert(TP == 64 && BLK == 64, "one wavefront, masks of 64 points");
+    static_assert(MAXW <= (1 << SBITS) && MAXW % 64 == 0, "window slots of an item word");
 };
 
 template <typename T>
@@ -57,6 +66,14 @@ __device__ __forceinline__ T wave_max(T v)
 {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
+    return v;
+}
+
+template <typename T>
+__device__ __forceinline__ T wave_min(T v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
     return v;
 }
 
@@ -72,23 +89,41 @@ struct TileWaves {
     static constexpr int value = ((D == 2 && !ELA) || (D == 3 && F32 && !ELA && !KIN)) ? 4 : 1;
 };
 
+// Cells of one axis that hold every particle within r of [lo, hi]: w0 (in
+// [0, nc)) and wn cells from it, taken periodically; the whole axis when
+// they would reach around it.  The margin covers the rounding of the cell
+// coordinates, and bounds that are not finite give the whole axis.
+__device__ __forceinline__ void axis_cells(const Geom &g, int a, double lo, double hi, double r, int &w0, int &wn)
+{
+    const int nc = g.nc[a];
+    w0 = 0;
+    wn = nc;
+    if (nc == 1) return;
+    const double m = r + 1e-10 * (fabs(lo) + fabs(hi) + g.L[a]);
+    const double f0 = floor((lo - m - g.lo[a]) / g.cs[a]), f1 = floor((hi + m - g.lo[a]) / g.cs[a]);
+    if (!(f1 - f0 + 1.0 < (double)nc)) return;
+    const int k = (int)(f0 - (double)nc * floor(f0 / (double)nc));
+    w0 = k < 0 ? 0 : (k >= nc ? nc - 1 : k);
+    wn = (int)(f1 - f0) + 1;
+}
+
 // The body works on one frame's arrays (cell starts st, sorted positions
-// sp, kinetic terms sk, bond counts bc, FP32 records rf, entries bd; out's
-// field pointers at the frame's first value) for the tile-th 64 points of
-// the Morton order perm, and stores its counts at out.wave_counts[2 wi ..].
+// sp, kinetic terms sk, bond counts bc, entries bd; out's field pointers at
+// the frame's first value) for the cnt points from t0 on of the Morton order
+// perm (cnt <= 0: none), and stores its counts at out.wave_counts[2 wi ..].
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
-__device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, const double *__restrict__ grid,
+__device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const double *__restrict__ grid,
                                                  const int *__restrict__ perm, const GLRule &R,
                                                  const double *__restrict__ gld, double cgnorm,
                                                  const int *__restrict__ st, const double *__restrict__ sp,
                                                  const double *__restrict__ sk, int cap,
-                                                 const int *__restrict__ bc, const float4 *__restrict__ rf,
-                                                 const ER *__restrict__ bd, const GatherOut &out, size_t wi, int tile,
+                                                 const int *__restrict__ bc, const ER *__restrict__ bd,
+                                                 const GatherOut &out, size_t wi, int t0, int cnt,
                                                  int *__restrict__ overflow)
 {
     using CP = TileCaps;
     using LY = BondLayout<D, OD, ELA, ER>;
-    constexpr int MAXI = CP::MAXI, NB = CP::NB, PBITS = CP::PBITS;
+    constexpr int MAXW = CP::MAXW, MAXI = CP::MAXI, SBITS = CP::SBITS;
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
     constexpr bool PAIRS = VIR || ELA;
@@ -99,131 +134,91 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, co
     constexpr int ES = LY::ES;    // values per entry
     constexpr int GRP = LY::GRP;  // entries per read group
     constexpr int GV = LY::GV;    // values per read group
-    constexpr unsigned PMASK = (1u << PBITS) - 1u;
-    static_assert(((int64_t)1 << PBITS) == kTileMaxParticles, "item word: particle bits");
 
-    __shared__ double s_pt[64][D];            // the tile's points
-    __shared__ double s_acc[64][KTA];         // their accumulators
-    __shared__ unsigned s_item[MAXI];         // items in scan order
-    __shared__ unsigned char s_inb[MAXI];     // their bond counts
-    __shared__ unsigned short s_perm[MAXI];   // the items in bond-count order
-    __shared__ int s_bucket[64];
+    __shared__ double s_pt[64][PS];              // the tile's points (NaN beyond them)
+    __shared__ double s_acc[64][KTA];            // their accumulators
+    __shared__ double s_wp[MAXW][D];             // window: positions,
+    __shared__ int s_wid[MAXW];                  // particles,
+    __shared__ unsigned long long s_wm[MAXW];    // point masks,
+    __shared__ unsigned char s_wnb[MAXW];        // bond counts,
+    __shared__ unsigned short s_wof[MAXW];       // first items
+    __shared__ unsigned short s_item[MAXI];      // items in order
+    __shared__ int s_bucket[64];                 // items per bond count, then their offsets
+    __shared__ int s_seg[64], s_segb[64];        // segments of cells: first candidate, first particle
 
     const int l = threadIdx.x;
-    const int t0 = tile * 64;
-    const int t = t0 + l;
-    const bool live = t < G;
-    // 3D with bonds: the scan reads the bond kernel's 16-byte records (FP32
-    // position, bond count) and tests in FP32 first, as the lane gather does
-    constexpr bool RECS = PAIRS && D == 3;
-
-    const int gp = perm[live ? t : t0];
-    double xg[3];
-    xg[0] = grid[(size_t)gp * 3];
-    xg[1] = grid[(size_t)gp * 3 + 1];
-    xg[2] = (D == 3) ? grid[(size_t)gp * 3 + 2] : 0.0;
+    if (cnt <= 0) {
+        if (l == 0) {
+            out.wave_counts[2 * wi] = 0;
+            out.wave_counts[2 * wi + 1] = 0;
+        }
+        return;
+    }
+    const bool live = l < cnt;
+    const int gp = perm[t0 + (live ? l : 0)];
+    double xg[D];
 #pragma unroll
-    for (int a = 0; a < D; ++a) s_pt[l][a] = xg[a];
+    for (int a = 0; a < D; ++a) xg[a] = grid[(size_t)gp * 3 + a];
+#pragma unroll
+    for (int a = 0; a < D; ++a) s_pt[l][a] = live ? xg[a] : __builtin_nan("");
 #pragma unroll
     for (int k = 0; k < KTA; ++k) s_acc[l][k] = 0.0;
 
-    unsigned long long nball = 0;  // items listed (the same in every lane)
+    // bounding box of the points: centre xc, half lengths xh.  When the box
+    // and its ball fit in less than a period (near), a particle has one image
+    // that can be inside any of the balls, the one nearest to xc.
+    double xc[D], xh[D];
+    int w0[3] = {0, 0, 0}, wn[3] = {1, 1, 1};
+    bool near = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const double lo = wave_min(xg[a]), hi = wave_max(xg[a]);
+        axis_cells(g, a, lo, hi, g.rc, w0[a], wn[a]);
+        w0[a] = __builtin_amdgcn_readfirstlane(w0[a]);
+        wn[a] = __builtin_amdgcn_readfirstlane(wn[a]);
+        xc[a] = 0.5 * (lo + hi);
+        xh[a] = 0.5 * (hi - lo);
+        near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh[a] + g.rc) < 0.999 * g.L[a]);
+    }
+
+    unsigned long long nball = 0;     // items, per lane
     unsigned long long ncontrib = 0;  // bond counts of the items, per lane
-    bool over = false;  // an item's bond count exceeds MAXNB
+    bool over = false;                // an item's bond count exceeds MAXNB
     const double s2 = 2.0 * g.inv_rc;
 
-    // ---- sort the first ni items of the list by bond count and integrate --
-    auto flush = [&](int ni) {
-        // counting sort by bond count, largest first: bucket sizes, their
-        // offsets, then each item takes the next slot of its bucket (an LDS
-        // atomic; the lanes of one instruction are served in a fixed order)
-        s_bucket[l] = 0;
-        __syncthreads();
-        nball += (unsigned long long)ni;
-        if constexpr (PAIRS && !RECS) {
-            // the items' bond counts, loaded here U at a time rather than
-            // with every scanned candidate (2D scans read positions only)
-            constexpr int U = 8;
-            for (int k0 = l; k0 < ni; k0 += 64 * U) {
-                int nbv[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int k = k0 + 64 * u;
-                    nbv[u] = k < ni ? bc[s_item[k] & PMASK] : 0;
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int k = k0 + 64 * u;
-                    if (k < ni) {
-                        const int nbc = min(nbv[u], cap);
-                        if (nbc > CP::MAXNB) over = true;
-                        const int nbk = min(nbc, CP::MAXNB);
-                        s_inb[k] = (unsigned char)nbk;
-                        ncontrib += (unsigned long long)nbk;
-                        atomicAdd(&s_bucket[63 - min(nbk, 63)], 1);
-                    }
-                }
-            }
-        } else {
-            for (int k = l; k < ni; k += 64) {
-                const int nbk = s_inb[k];
-                ncontrib += (unsigned long long)nbk;
-                atomicAdd(&s_bucket[63 - min(nbk, 63)], 1);
-            }
-        }
-        __syncthreads();
-        {
-            const int c = s_bucket[l];
-            int v = c;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int u = __shfl_up(v, off, 64);
-                if (l >= off) v += u;
-            }
-            __syncthreads();
-            s_bucket[l] = v - c;  // first slot of the bucket
-        }
-        __syncthreads();
-        for (int k = l; k < ni; k += 64) {
-            const int slot = atomicAdd(&s_bucket[63 - min((int)s_inb[k], 63)], 1);
-            s_perm[slot] = (unsigned short)k;
-        }
-        __syncthreads();
-
-        // lane l takes sorted items l, l + 64, ...; the data of the next one
-        // is loaded before the current one is integrated
-        auto fetch = [&](int k, int &p, int &ip, int &nb, double (&pos)[3], double (&kk)[KNA], ER (&E)[GV]) {
+    // ---- integrate items 0 .. ni - 1 of the list --------------------------
+    auto integrate = [&](int ni) {
+        // the next item's first bond entries and kinetic term are loaded
+        // before the current one is integrated
+        auto fetch = [&](int k, int &slot, int &ip, int &nb, double (&kk)[KNA], ER (&E)[GV]) {
             const bool valid = k < ni;
-            const int ix = s_perm[valid ? k : 0];
-            const unsigned it = s_item[ix];
-            p = (int)(it & PMASK);
-            ip = (int)(it >> PBITS);
-            nb = (PAIRS && valid) ? (int)s_inb[ix] : 0;
-            pos[0] = sp[(size_t)p * PS];
-            pos[1] = sp[(size_t)p * PS + 1];
-            pos[2] = (D == 3) ? sp[(size_t)p * PS + 2] : 0.0;
+            const unsigned it = s_item[valid ? k : 0];
+            slot = (int)(it & ((1u << SBITS) - 1u));
+            ip = (int)(it >> SBITS);
+            const int p = s_wid[slot];
+            nb = (PAIRS && valid) ? (int)s_wnb[slot] : 0;
             if constexpr (KIN)
 #pragma unroll
                 for (int q = 0; q < KN; ++q) kk[q] = sk[(size_t)p * KN + q];
             if constexpr (PAIRS)
                 if (nb > 0) load_entry<ER, GV>(bd + (size_t)p * cap * ES, E);
         };
-        int p, ip, nb;
-        double pos[3], kk[KNA];
+        int slot, ip, nb;
+        double kk[KNA];
         ER E0[GV];
-        fetch(l, p, ip, nb, pos, kk, E0);
+        fetch(l, slot, ip, nb, kk, E0);
         for (int k0 = 0; k0 < ni; k0 += 64) {
             const int k = k0 + l;
-            int np_, nip, nnb;
-            double npos[3], nkk[KNA];
+            int nslot, nip, nnb;
+            double nkk[KNA];
             ER nE0[GV];
-            fetch(k + 64, np_, nip, nnb, npos, nkk, nE0);
+            fetch(k + 64, nslot, nip, nnb, nkk, nE0);
             if (k < ni) {
                 double a[3];
-                a[0] = minimg(pos[0] - s_pt[ip][0], g.L[0], g.pinvL[0]);
-                a[1] = minimg(pos[1] - s_pt[ip][1], g.L[1], g.pinvL[1]);
+                a[0] = minimg(s_wp[slot][0] - s_pt[ip][0], g.L[0], g.pinvL[0]);
+                a[1] = minimg(s_wp[slot][1] - s_pt[ip][1], g.L[1], g.pinvL[1]);
                 a[2] = 0.0;
-                if constexpr (D == 3) a[2] = minimg(pos[2] - s_pt[ip][D - 1], g.L[2], g.pinvL[2]);
+                if constexpr (D == 3) a[2] = minimg(s_wp[slot][D - 1] - s_pt[ip][D - 1], g.L[2], g.pinvL[2]);
                 const double A = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * g.inv_rc2;
                 double acc[KTA];
 #pragma unroll
@@ -303,7 +298,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, co
                         if constexpr (GRP >= 4)
                             if (GRP * kk2 + 3 < nb) one(Gv, std::integral_constant<int, 3 * ES>());
                     };
-                    const ER *ptr = bd + (size_t)p * cap * ES;
+                    const ER *ptr = bd + (size_t)s_wid[slot] * cap * ES;
                     const int ng = (nb + GRP - 1) / GRP;
                     ER E1[GV];
                     int kk2 = 0;
@@ -319,11 +314,9 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, co
                 for (int q = 0; q < KT; ++q)
                     __hip_atomic_fetch_add(&s_acc[ip][q], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             }
-            p = np_;
+            slot = nslot;
             ip = nip;
             nb = nnb;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) pos[a] = npos[a];
             if constexpr (KIN)
 #pragma unroll
                 for (int q = 0; q < KN; ++q) kk[q] = nkk[q];
@@ -334,166 +327,174 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, co
         __syncthreads();
     };
 
-    // ---- scan: the cells around each lane's point ---------------------------
-    // per axis the window is cells c - reach .. c + reach, or the whole axis
-    // when that would reach around it (the same count for every lane)
-    int wlo[3], wn[3];
-    for (int a = 0; a < 3; ++a) {
-        const int nc = g.nc[a];
-        const int c = cell_coord(g, a, xg[a]);
-        if (nc == 1 || 2 * g.reach + 1 >= nc) {
-            wlo[a] = 0;
-            wn[a] = nc;
-        } else {
-            wn[a] = 2 * g.reach + 1;
-            int lo = c - g.reach;
-            if (lo < 0) lo += nc;
-            wlo[a] = lo;
+    // ---- the items of window particles 0 .. nw - 1 --------------------------
+    auto process = [&](int nw) {
+        s_bucket[l] = 0;
+        __syncthreads();
+        for (int r = 0; r < nw; r += 64) {
+            const int slot = r + l;
+            const bool valid = slot < nw;
+            const int ws = valid ? slot : 0;
+            int nbc = 0;
+            if constexpr (PAIRS) nbc = min(bc[s_wid[ws]], cap);
+            double x[D];
+#pragma unroll
+            for (int a = 0; a < D; ++a) x[a] = s_wp[ws][a];
+            bool shift = !near;
+#pragma unroll
+            for (int a = 0; a < D; ++a) shift = shift || !(rint((x[a] - xc[a]) * g.pinvL[a]) == 0.0);
+            // bit j of the mask: the particle is in point j's ball.  Bits
+            // enter at the low end (m = 2 m + bit, one add with carry).
+            unsigned m[2] = {0u, 0u};
+            auto test = [&](auto image) {
+                constexpr bool IMAGE = decltype(image)::value;
+#pragma unroll
+                for (int h = 1; h >= 0; --h) {
+                    if (32 * h >= cnt) continue;
+                    unsigned mm = 0u;
+#pragma unroll 4
+                    for (int j = 31; j >= 0; --j) {
+                        double d[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            d[a] = x[a] - s_pt[32 * h + j][a];
+                            if constexpr (IMAGE) d[a] = minimg(d[a], g.L[a], g.pinvL[a]);
+                        }
+                        const bool in = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] < g.rc2;
+                        mm = mm + mm + (in ? 1u : 0u);
+                    }
+                    m[h] = mm;
+                }
+            };
+            // no lane's particle needs another image: the plain difference is
+            // the minimum image of every pair that can be inside a ball
+            if (__builtin_amdgcn_ballot_w64(shift) == 0ull) test(std::false_type());
+            else test(std::true_type());
+            if (!valid) m[0] = m[1] = 0u;
+            const int pc = __popc(m[0]) + __popc(m[1]);
+            if (nbc > CP::MAXNB && pc > 0) over = true;
+            const int nb = min(nbc, CP::MAXNB);
+            nball += (unsigned long long)pc;
+            ncontrib += (unsigned long long)pc * (unsigned long long)nb;
+            if (valid) {
+                s_wnb[slot] = (unsigned char)nb;
+                s_wm[slot] = (unsigned long long)m[1] << 32 | m[0];
+                atomicAdd(&s_bucket[63 - min(nb, 63)], pc);
+            }
         }
-    }
+        __syncthreads();
+        int total;
+        {
+            const int c = s_bucket[l];
+            int v = c;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int u = __shfl_up(v, off, 64);
+                if (l >= off) v += u;
+            }
+            total = __builtin_amdgcn_readlane(v, 63);
+            __syncthreads();
+            s_bucket[l] = v - c;  // first item of the bond count
+        }
+        __syncthreads();
+        for (int base = 0; base < total; base += MAXI) {
+            for (int r = 0; r < nw; r += 64) {
+                const int slot = r + l;
+                if (slot < nw) {
+                    const unsigned long long mk = s_wm[slot];
+                    unsigned m0 = (unsigned)mk, m1 = (unsigned)(mk >> 32);
+                    int k;
+                    if (base == 0) {
+                        // an LDS atomic; the lanes of one instruction are
+                        // served in a fixed order
+                        k = atomicAdd(&s_bucket[63 - min((int)s_wnb[slot], 63)], __popc(m0) + __popc(m1));
+                        s_wof[slot] = (unsigned short)k;
+                    } else {
+                        k = s_wof[slot] - base;
+                    }
+                    while (m0 | m1) {
+                        const bool low = m0 != 0u;
+                        const unsigned mm = low ? m0 : m1;
+                        const int j = __ffs(mm) - 1 + (low ? 0 : 32);
+                        const unsigned rest = mm & (mm - 1u);
+                        m0 = low ? rest : 0u;
+                        m1 = low ? m1 : rest;
+                        if ((unsigned)k < (unsigned)MAXI) s_item[k] = (unsigned short)(slot | (j << SBITS));
+                        ++k;
+                    }
+                }
+            }
+            __syncthreads();
+            integrate(min(total - base, MAXI));
+        }
+    };
+
+    // ---- window: candidates of the cell rows, in segments of one row --------
     const int nx = g.nc[0], ny = g.nc[1], nz = g.nc[2];
-    const int nrows = wn[1] * wn[2];
-    // row r of the window: cells wlo[0] .. wlo[0] + wn[0] - 1, as one or two
-    // particle ranges read as one run [b0, b0 + len0) + [b1, b1 + len - len0)
-    auto row = [&](int r, int &b0, int &len0, int &b1, int &len) {
-        const int iz = r / wn[1], iy = r - iz * wn[1];
-        const int z = wlo[2] + iz < nz ? wlo[2] + iz : wlo[2] + iz - nz;
-        const int y = wlo[1] + iy < ny ? wlo[1] + iy : wlo[1] + iy - ny;
-        const int rowbase = (z * ny + y) * nx;
-        const int xe = wlo[0] + wn[0];
-        b0 = st[rowbase + wlo[0]];
-        int e0, e1 = 0;
-        b1 = 0;
-        if (xe <= nx) {
-            e0 = st[rowbase + xe];
-        } else {
-            e0 = st[rowbase + nx];
-            b1 = st[rowbase];
-            e1 = st[rowbase + xe - nx];
+    const int parts = w0[0] + wn[0] > nx ? 2 : 1;  // a row that wraps is two segments
+    const int nseg = wn[1] * wn[2] * parts;
+    const double rr = g.rc2 * (1.0 + 1e-9);
+    int nw = 0;
+    for (int s0 = 0; s0 < nseg; s0 += 64) {
+        int b = 0, len = 0;
+        if (s0 + l < nseg) {
+            const int r = (s0 + l) / parts, part = (s0 + l) - r * parts;
+            const int iz = r / wn[1], iy = r - iz * wn[1];
+            const int z = w0[2] + iz < nz ? w0[2] + iz : w0[2] + iz - nz;
+            const int y = w0[1] + iy < ny ? w0[1] + iy : w0[1] + iy - ny;
+            const int row = (z * ny + y) * nx;
+            b = st[part ? row : row + w0[0]];
+            len = st[part ? row + w0[0] + wn[0] - nx : row + min(w0[0] + wn[0], nx)] - b;
         }
-        len0 = e0 - b0;
-        len = live ? len0 + (e1 - b1) : 0;
-    };
-    // candidates c0 .. c0 + NB - 1 of a row (clamped into it; a lane with an
-    // empty row reads particle 0, and every lane has one when any reads)
-    struct Cand {
-        int p[NB], nb[RECS ? NB : 1];
-        double q[RECS ? 1 : NB][3];
-        float r[RECS ? NB : 1][3];
-    };
-    auto load = [&](int c0, int b0, int len0, int b1, int len, Cand &C) {
+        int v = len;
 #pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int c = min(c0 + u, len - 1);
-            C.p[u] = len == 0 ? 0 : (c < len0 ? b0 + c : b1 + (c - len0));
-            if constexpr (RECS) {
-                const float4 r4 = rf[C.p[u]];
-                C.r[u][0] = r4.x;
-                C.r[u][1] = r4.y;
-                C.r[u][2] = r4.z;
-                C.nb[u] = __float_as_int(r4.w);
-            } else {
-                C.q[u][0] = sp[(size_t)C.p[u] * PS];
-                C.q[u][1] = sp[(size_t)C.p[u] * PS + 1];
-                C.q[u][2] = (D == 3) ? sp[(size_t)C.p[u] * PS + 2] : 0.0;
-            }
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(v, off, 64);
+            if (l >= off) v += u;
         }
-    };
-    float xg32[3];
+        const int total = __builtin_amdgcn_readlane(v, 63);
+        __syncthreads();
+        s_seg[l] = v - len;
+        s_segb[l] = b;
+        __syncthreads();
+        const int ns = min(nseg - s0, 64);
+        for (int c0 = 0; c0 < total; c0 += 64) {
+            const int c = min(c0 + l, total - 1);
+            // the last segment that starts at or before candidate c
+            int lo = 0;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) xg32[a] = (float)xg[a];
-    // the exact test: FP64 minimum image and |a|^2 against r_cg^2
-    auto exact_in = [&](const double *q) {
-        const double a0 = minimg(q[0] - xg[0], g.L[0], g.pinvL[0]);
-        const double a1 = minimg(q[1] - xg[1], g.L[1], g.pinvL[1]);
-        const double a2 = (D == 3) ? minimg(q[2] - xg[2], g.L[2], g.pinvL[2]) : 0.0;
-        return a0 * a0 + a1 * a1 + a2 * a2 < g.rc2;
-    };
-    // the scan visits rows r = 0 .. nrows - 1, each in steps of NB candidates
-    // per lane (one step for a row that is empty in every lane)
-    auto test_append = [&](const Cand &C, int c0, int len, int &ni) {
+            for (int h = 32; h > 0; h >>= 1)
+                if (lo + h < ns && s_seg[lo + h] <= c) lo += h;
+            const int id = s_segb[lo] + c - s_seg[lo];
+            double x[D], d2 = 0.0;
 #pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            bool in;
-            if constexpr (RECS) {
-                // FP32 pre-test against bounds of the FP64 rounding; a
-                // candidate in the band between them (or any, when the
-                // geometry gives no bound) is decided by the exact test
-                float d0 = C.r[u][0] - xg32[0], d1 = C.r[u][1] - xg32[1], d2 = C.r[u][2] - xg32[2];
-                d0 = fmaf(-g.L32[0], rintf(d0 * g.pinvL32[0]), d0);
-                d1 = fmaf(-g.L32[1], rintf(d1 * g.pinvL32[1]), d1);
-                d2 = fmaf(-g.L32[2], rintf(d2 * g.pinvL32[2]), d2);
-                const float a2f = d0 * d0 + d1 * d1 + d2 * d2;
-                in = a2f < g.in32;
-                if (!in && !(a2f > g.out32) && c0 + u < len) {
-                    double q[3];
+            for (int a = 0; a < D; ++a) x[a] = sp[(size_t)id * PS + a];
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) q[a] = sp[(size_t)C.p[u] * PS + a];
-                    in = exact_in(q);
-                }
-                in = in && c0 + u < len;
-            } else {
-                in = c0 + u < len && exact_in(C.q[u]);
+            for (int a = 0; a < D; ++a) {
+                const double d = fmax(fabs(minimg(x[a] - xc[a], g.L[a], g.pinvL[a])) - xh[a], 0.0);
+                d2 = fma(d, d, d2);
             }
+            // not near: any image may matter, so every candidate is kept
+            const bool in = c0 + l < total && (!near || d2 < rr);
             const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
-            if (in) {
-                const int k = ni + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
-                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
-                s_item[k] = (unsigned)C.p[u] | ((unsigned)l << PBITS);
-                if constexpr (RECS) {
-                    const int nbc = min(C.nb[u], cap);
-                    if (nbc > CP::MAXNB) over = true;
-                    s_inb[k] = (unsigned char)min(nbc, CP::MAXNB);
-                } else if constexpr (!PAIRS) {
-                    s_inb[k] = 0;
-                }
+            const int k = __popcll(bm);
+            if (nw + k > MAXW) {
+                __syncthreads();
+                process(nw);
+                nw = 0;
             }
-            ni += __popcll(bm);
+            if (in) {
+                const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
+                s_wid[w] = id;
+#pragma unroll
+                for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
+            }
+            nw += k;
         }
-    };
-    int ni = 0;  // items in the list (the same in every lane)
-    int r = 0, c0 = 0;
-    int b0, len0, b1, len, nb0 = 0, nlen0 = 0, nb1 = 0, nlen = 0;
-    row(0, b0, len0, b1, len);
-    int maxlen = wave_max(len);
-    if (nrows > 1) row(1, nb0, nlen0, nb1, nlen);  // the next row's ranges load ahead
-    auto advance = [&](bool same) {
-        if (same) {
-            c0 += NB;
-            return;
-        }
-        ++r;
-        c0 = 0;
-        b0 = nb0;
-        len0 = nlen0;
-        b1 = nb1;
-        len = nlen;
-        maxlen = wave_max(len);
-        if (r + 1 < nrows) row(r + 1, nb0, nlen0, nb1, nlen);
-    };
-    Cand C0;
-    if (n > 0) load(0, b0, len0, b1, len, C0);
-    for (; n > 0;) {
-        const bool same = c0 + NB < maxlen;
-        const bool last = !same && r + 1 >= nrows;
-        // the next step's candidates load while these are tested (loaded
-        // again after a flush, which needs the registers)
-        Cand C1;
-        if (!last) {
-            if (same) load(c0 + NB, b0, len0, b1, len, C1);
-            else load(0, nb0, nlen0, nb1, nlen, C1);
-        }
-        test_append(C0, c0, len, ni);
-        if (last) break;
-        advance(same);
-        if (ni > MAXI - 64 * NB) {
-            flush(ni);
-            ni = 0;
-            load(c0, b0, len0, b1, len, C1);
-        }
-        C0 = C1;
     }
-    if (ni > 0) flush(ni);
+    __syncthreads();
+    if (nw > 0) process(nw);
     __syncthreads();
 
     if (live) {
@@ -520,37 +521,50 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, int G, co
         if (ELA) store(out.ela, ae, 1.0);
         if (KIN) store(out.kin, ak, cgnorm);
     }
+    nball = wave_sum(nball);
     ncontrib = wave_sum(ncontrib);
     if (l == 0) {
-        out.wave_counts[2 * wi] = nball;  // uniform: not summed over lanes
+        out.wave_counts[2 * wi] = nball;
         out.wave_counts[2 * wi + 1] = ncontrib;
     }
     if (over) atomicOr(overflow, 2);
 }
 
-// One frame per y row; block x takes the tile xcd_tile(x, gridDim.x), so
-// each XCD works through a contiguous eighth of the frame's points.
+// The points of workgroup b of a frame: tile b / (64 / tp), its tp points
+// from b mod (64 / tp) times tp on (tp 64: the whole tile).  tiles[k] is
+// where tile k starts in the Morton order.
+__device__ __forceinline__ void tile_points(const int *__restrict__ tiles, int b, int tp, int &t0, int &cnt)
+{
+    const int sub = kTilePoints / tp, k = b / sub;
+    t0 = tiles[k] + (b - k * sub) * tp;
+    cnt = min(tiles[k + 1] - t0, tp);
+}
+
+// One frame per y row; block x takes the points of tile_points(xcd_tile(x,
+// gridDim.x)), so each XCD works through a contiguous eighth of the frame's
+// points.
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
 __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gather_tile(
-    Geom g, int n, int G, const double *__restrict__ grid, const int *__restrict__ perm, GLRule R,
-    const double *__restrict__ gld, double cgnorm, const int *__restrict__ cstart, const double *__restrict__ spos,
-    const double *__restrict__ skin, int cap, const int *__restrict__ bcount, const float4 *__restrict__ rec,
-    const ER *__restrict__ bonds, GatherOut out, int *__restrict__ overflow)
+    Geom g, int n, int G, const double *__restrict__ grid, const int *__restrict__ perm,
+    const int *__restrict__ tiles, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
+    const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap,
+    const int *__restrict__ bcount, const ER *__restrict__ bonds, GatherOut out, int *__restrict__ overflow)
 {
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
     constexpr int ES = BondLayout<D, OD, ELA, ER>::ES;
-    constexpr bool RECS = (VIR || ELA) && D == 3;
     const int f = blockIdx.y;
     const size_t fo = (size_t)f * n, oo = (size_t)f * G * OD * OD;
     GatherOut of = out;
     if (VIR) of.vir = out.vir + oo;
     if (ELA) of.ela = out.ela + oo;
     if (KIN) of.kin = out.kin + oo;
+    int t0, cnt;
+    tile_points(tiles, xcd_tile(blockIdx.x, gridDim.x), tp, t0, cnt);
     gather_tile_body<D, OD, CG, NQ, VIR, ELA, KIN, ER>(
-        g, n, G, grid, perm, R, gld, cgnorm, cstart + (size_t)f * (g.ncell + 1), spos + fo * PS,
-        KIN ? skin + fo * KN : nullptr, cap, bcount + fo, RECS ? rec + fo : nullptr, bonds + fo * (size_t)cap * ES, of,
-        (size_t)blockIdx.y * gridDim.x + blockIdx.x, xcd_tile(blockIdx.x, gridDim.x), overflow);
+        g, n, grid, perm, R, gld, cgnorm, cstart + (size_t)f * (g.ncell + 1), spos + fo * PS,
+        KIN ? skin + fo * KN : nullptr, cap, bcount + fo, bonds + fo * (size_t)cap * ES, of,
+        (size_t)blockIdx.y * gridDim.x + blockIdx.x, t0, cnt, overflow);
 }
 
 // The sweep's field gather (2D or 3D, virial and/or kinetic): each
@@ -568,16 +582,15 @@ template <int D, int OD, bool VIR, bool KIN, typename ER>
 __global__ __launch_bounds__(64, kSweepGatherWaves) void k_sweep_gather(
     const SweepSys *__restrict__ T, int ns, GLRule R, const int *__restrict__ cstart,
     const double *__restrict__ spos, const double *__restrict__ skin, int cap, const int *__restrict__ bcount,
-    const float4 *__restrict__ rec, const ER *__restrict__ bonds, unsigned long long *__restrict__ wave_counts,
+    const ER *__restrict__ bonds, unsigned long long *__restrict__ wave_counts,
     int *__restrict__ overflow)
 {
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
     constexpr int ES = BondLayout<D, OD, false, ER>::ES;
-    constexpr bool RECS = VIR && D == 3;
     const SweepSys &S = T[sweep_system(T, ns, SW_GATHER, blockIdx.x)];
-    int f, tile;
-    if (!sweep_frame_tile(S, SW_GATHER, blockIdx.x, f, tile)) {
+    int f, b;
+    if (!sweep_frame_tile(S, SW_GATHER, blockIdx.x, f, b)) {
         if (threadIdx.x == 0) {
             wave_counts[2 * (size_t)blockIdx.x] = 0;
             wave_counts[2 * (size_t)blockIdx.x + 1] = 0;
@@ -591,10 +604,12 @@ __global__ __launch_bounds__(64, kSweepGatherWaves) void k_sweep_gather(
     of.vir = VIR ? S.vir + oo : nullptr;
     of.kin = KIN ? S.kin + oo : nullptr;
     of.wave_counts = wave_counts;
+    int t0, cnt;
+    tile_points(S.tiles, b, S.tp, t0, cnt);
     gather_tile_body<D, OD, 0, 5, VIR, false, KIN, ER>(
-        g, n, G, S.grid, S.perm, R, nullptr, S.cgnorm, cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1),
-        spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, VIR ? bcount + fo : nullptr, RECS ? rec + fo : nullptr,
-        VIR ? bonds + fo * (size_t)cap * ES : nullptr, of, blockIdx.x, tile, overflow);
+        g, n, S.grid, S.perm, R, nullptr, S.cgnorm, cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1),
+        spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, VIR ? bcount + fo : nullptr,
+        VIR ? bonds + fo * (size_t)cap * ES : nullptr, of, blockIdx.x, t0, cnt, overflow);
 }
 
 }  // namespace pgt

@@ -17,6 +17,7 @@ struct Geom {
     double cs[3];  // cell edge, at least (search radius) / reach
     int ncell;
     int reach;     // cells on each side of a cell that a search covers
+    double rc;       // cg_rcut
     double rc2;      // cg_rcut^2
     double inv_rc;   // 1/cg_rcut
     double inv_rc2;  // 1/cg_rcut^2

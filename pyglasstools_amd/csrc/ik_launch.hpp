@@ -20,6 +20,9 @@ struct LaunchCtx {
     mutable int pl_launched;  // points per lane of the gather actually launched
     const double *grid;
     const int *perm;
+    const int *tiles;  // starts of the tile gather's tiles in perm, ntiles + 1 of them
+    int ntiles;
+    int tp;            // tile gather: grid points per workgroup (a divisor of kTilePoints)
     GLRule R;
     const double *gld;
     double cgnorm;
@@ -44,10 +47,11 @@ inline int gather_pl(int tuned, int cg, int nq, int D, int OD)
 // Whether the tile gather serves this form (the Octic 5-node rule).
 inline bool tile_form(int cg, int nq, int D, int OD) { return cg == 0 && nq == 5 && !(D == 3 && OD == 2); }
 
-// The tile gather's launch shape: kTilePoints grid points per workgroup of
-// kTileThreads lanes (one wavefront, one point per lane), in every form.
+// The tile gather's launch shape: a tile holds at most kTilePoints grid
+// points; a workgroup of kTileThreads lanes (one wavefront) takes a tile or
+// an equal part of it.
 constexpr int kTilePoints = 64, kTileThreads = 64;
-// Particles per frame the tile gather can index (26 bits of an item word).
+// Most particles per frame of a tile gather.
 constexpr int64_t kTileMaxParticles = (int64_t)1 << 26;
 
 // Field gather of one batch (fixed-order rule), one function per form and
@@ -90,7 +94,6 @@ struct SweepGatherCtx {
     const double *spos, *skin;
     int cap;
     const int *bcount;
-    const float4 *rec;  // 3D: FP32 position and bond count per sorted particle
     const void *bonds;
     unsigned long long *wave_counts;
     int *flags;
