@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 namespace pgt {
 
 constexpr double kPi = 3.14159265358979323846;
@@ -134,7 +136,25 @@ struct GLRule {
     int n;
     double s[kMaxQArg];
     double w[kMaxQArg];
+    // Octic kernel with 5 nodes (bond_octic5), with q_k = w_k^(1/4): q of
+    // nodes 0, 1, 2 (3 and 4 mirror 1 and 0), s_k q_k, s_k^2 q_k, q_k^2
+    double oct_a[3], oct_b[5], oct_c[5], oct_r[3];
 };
+
+// Fills the oct_ terms of a 5-node rule.
+inline void fold_octic5(GLRule &R)
+{
+    if (R.n != 5) return;
+    for (int k = 0; k < 5; ++k) {
+        const long double q = sqrtl(sqrtl((long double)R.w[k]));
+        R.oct_b[k] = (double)(R.s[k] * q);
+        R.oct_c[k] = (double)(R.s[k] * R.s[k] * q);
+        if (k < 3) {
+            R.oct_a[k] = (double)q;
+            R.oct_r[k] = (double)(q * q);
+        }
+    }
+}
 
 // sum_k w_k shape(t(s_k)), t(s) = A + s B + s^2 C: the bond integral of the
 // unnormalised kernel along the segment, in units of the kernel width.
@@ -155,6 +175,22 @@ __device__ __forceinline__ ER bond_quad(const GLRule &R, const double *__restric
             const ER t = fma(s, fma(s, C, B), A);
             acc = fma((ER)gld[nq + k], shape<CG, ER>(t), acc);
         }
+    }
+    return acc;
+}
+
+// bond_quad of the Octic kernel's 5-node rule with the weights folded into
+// the nodes: w (1 - t^2)_+^2 = (q^2 - (q t)^2)_+^2, q = w^(1/4), and q t is as
+// many operations as t when q A is at hand (Aq, for nodes 0, 1 and 2).
+__device__ __forceinline__ double bond_octic5(const GLRule &R, const double (&Aq)[3], double B, double C)
+{
+    double acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const int h = k < 3 ? k : 4 - k;
+        const double t = fma(R.oct_b[k], B, fma(R.oct_c[k], C, Aq[h]));
+        const double u = fmax(fma(-t, t, R.oct_r[h]), 0.0);
+        acc = fma(u, u, acc);
     }
     return acc;
 }

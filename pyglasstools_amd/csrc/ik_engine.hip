@@ -176,21 +176,24 @@ int gl_rule(int n, std::vector<double> &s, std::vector<double> &w)
 // the box faces (as numpy.linspace makes them) maps onto the indices 0..n-1
 // exactly, so for n a power of two every run of 4^k (2D) or 8^k (3D) points
 // is a square (cube) block.
-// `tiles` gets where the tile gather's tiles start in the order (and G at the
-// end): a tile is the points of one block of 8 x 8 (2D) or 4 x 4 x 4 lattice
-// sites, at most kTilePoints of them.  Runs of kTilePoints points regardless
-// of the blocks would straddle two of them wherever the grid's side is not a
-// multiple of the block's, and two blocks that follow each other can lie far
-// apart, which would make the tile's window of particles large.
-std::vector<int> morton_order(int64_t G, const double *grid, bool use_z, std::vector<int> &tiles)
+// The same blocks make the tile gather's tiles (TileRec): runs of kTilePoints
+// points regardless of the blocks would straddle two of them wherever the
+// grid's side is not a multiple of the block's, and blocks that follow each
+// other can lie far apart, which would make the tile's window of particles
+// large.
+struct GridOrder {
+    std::vector<int> perm;
+    std::vector<TileRec> tiles;
+    std::vector<int> tperm;  // kTilePoints per tile
+};
+
+GridOrder order_grid(int64_t G, const double *grid, bool use_z)
 {
-    std::vector<int> perm((size_t)G);
+    GridOrder o;
+    std::vector<int> &perm = o.perm;
+    perm.resize((size_t)G);
     std::iota(perm.begin(), perm.end(), 0);
-    tiles.assign(1, 0);
-    if (G < 2) {
-        if (G == 1) tiles.push_back(1);
-        return perm;
-    }
+    if (G < 1) return o;
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (int64_t i = 0; i < G; ++i)
         for (int a = 0; a < 3; ++a) {
@@ -214,11 +217,48 @@ std::vector<int> morton_order(int64_t G, const double *grid, bool use_z, std::ve
         key[(size_t)i] = k;
     }
     std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return key[(size_t)x] < key[(size_t)y]; });
-    for (int64_t t = 1; t < G; ++t)
-        if (t - tiles.back() == kTilePoints || key[(size_t)perm[t]] >> 6 != key[(size_t)perm[t - 1]] >> 6)
-            tiles.push_back((int)t);
-    tiles.push_back((int)G);
-    return perm;
+    const int side = use_z ? 4 : 8;  // sites of a block along an axis
+    for (int64_t t0 = 0, t1; t0 < G; t0 = t1) {
+        for (t1 = t0 + 1; t1 < G && t1 - t0 < kTilePoints && key[(size_t)perm[t1]] >> 6 == key[(size_t)perm[t0]] >> 6;)
+            ++t1;
+        TileRec rec{};
+        double line[3][8];
+        bool have[3][8] = {};
+        int slot[kTilePoints];
+        uint64_t used = 0;
+        bool product = true;
+        for (int64_t t = t0; t < t1 && product; ++t) {
+            const uint64_t k = key[(size_t)perm[t]];
+            int at[3] = {0, 0, 0};  // the site in its block: the key's low 6 bits, de-interleaved
+            for (int b = 0; b < 6; ++b) at[b % d] |= (int)((k >> b) & 1u) << (b / d);
+            const int j = use_z ? ((at[2] >> 1) * 2 + (at[1] >> 1)) * 16 + (at[2] & 1) * 8 + (at[1] & 1) * 4 + at[0]
+                                : ((at[1] >> 2) * 2 + (at[0] >> 2)) * 16 + (at[1] & 3) * 4 + (at[0] & 3);
+            product = !((used >> j) & 1u);
+            used |= (uint64_t)1 << j;
+            slot[t - t0] = j;
+            for (int a = 0; a < d; ++a) {
+                const double x = grid[3 * (int64_t)perm[t] + a];
+                if (!have[a][at[a]]) {
+                    have[a][at[a]] = true;
+                    line[a][at[a]] = x;
+                }
+                product = product && line[a][at[a]] == x;
+            }
+        }
+        rec.product = product ? 1 : 0;
+        for (int a = 0; a < d; ++a)
+            for (int k = 0; k < side; ++k)
+                if (!have[a][k]) line[a][k] = NAN;
+        for (int q = 0; q < 4; ++q)
+            for (int k = 0; k < 8; ++k)
+                rec.ax[q][k] = use_z ? (k < 4 ? line[0][k] : k < 6 ? line[1][(q & 1) * 2 + k - 4] : line[2][(q >> 1) * 2 + k - 6])
+                                     : (k < 4 ? line[0][(q & 1) * 4 + k] : line[1][(q >> 1) * 4 + k - 4]);
+        o.tiles.push_back(rec);
+        o.tperm.resize(o.tperm.size() + kTilePoints, -1);
+        int *tp = o.tperm.data() + o.tperm.size() - kTilePoints;
+        for (int64_t t = t0; t < t1; ++t) tp[product ? slot[t - t0] : (int)(t - t0)] = perm[t];
+    }
+    return o;
 }
 
 template <typename T>
@@ -267,7 +307,8 @@ struct pgt_ik_engine {
     DBuf<double> d_pos, d_diam, d_mass, d_vel, d_disp;  // single-frame host uploads
     DBuf<double> d_grid;
     DBuf<int> d_perm;
-    DBuf<int> d_tiles;  // tile starts in d_perm (morton_order), ntiles + 1
+    DBuf<TileRec> d_tiles;  // the tile gather's tiles (order_grid)
+    DBuf<int> d_tperm;      // and their points
     int ntiles = 0;
     // work arrays of a batch (see WorkArray), as raw bytes
     DBuf<unsigned char> d_keys0, d_vals0, d_keys1, d_vals1, d_hist, d_cstart, d_bcount;
@@ -712,6 +753,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     c.grid = e->d_grid.p;
     c.perm = e->d_perm.p;
     c.tiles = e->d_tiles.p;
+    c.tperm = e->d_tperm.p;
     c.ntiles = e->ntiles;
     c.tp = j.tp;
     c.R.n = (int)e->gl_s.size();
@@ -719,6 +761,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         c.R.s[k] = e->gl_s[k];
         c.R.w[k] = e->gl_w[k];
     }
+    fold_octic5(c.R);
     c.gld = e->d_gl.p;
     c.cgnorm = cg_norm(e->prm.cg_kind, e->prm.cg_rcut);
     c.cstart = cstart;
@@ -940,6 +983,7 @@ GLRule engine_rule(const pgt_ik_engine *e)
         R.s[k] = e->gl_s[k];
         R.w[k] = e->gl_w[k];
     }
+    fold_octic5(R);
     return R;
 }
 
@@ -1090,8 +1134,9 @@ void pgt_ik_destroy(pgt_ik_engine *e)
     DBuf<double> *dbufs[] = {&e->d_pos, &e->d_diam, &e->d_mass, &e->d_vel, &e->d_disp, &e->d_grid,
                              &e->d_out, &e->d_gl};
     for (auto *b : dbufs) b->release();
-    DBuf<int> *ibufs[] = {&e->d_perm, &e->d_tiles, &e->d_maxcount};
+    DBuf<int> *ibufs[] = {&e->d_perm, &e->d_tperm, &e->d_maxcount};
     for (auto *b : ibufs) b->release();
+    e->d_tiles.release();
     DBuf<unsigned char> *wbufs[] = {&e->d_keys0, &e->d_vals0, &e->d_keys1, &e->d_vals1, &e->d_hist, &e->d_cstart,
                                     &e->d_bcount, &e->d_spos, &e->d_sdiam, &e->d_skin, &e->d_sdisp, &e->d_bonds,
                                     &e->d_wcounts, &e->d_wmax, &e->d_rec};
@@ -1183,22 +1228,24 @@ int pgt_ik_set_grid(pgt_ik_engine *e, int64_t g, const double *grid)
         for (int a = 0; a < 3; ++a) amax = std::max(amax, std::fabs(grid[3 * i + a]));
     }
     if (!(amax < INFINITY)) amax = INFINITY;  // NaN coordinates: no FP32 pre-test
-    std::vector<int> tiles;
-    const std::vector<int> perm = morton_order(g, grid, !flat || e->prm.dim == 3, tiles);
+    const GridOrder o = order_grid(g, grid, !flat || e->prm.dim == 3);
     int rc;
     if ((rc = e->d_grid.ensure((size_t)g * 3)) || (rc = e->d_perm.ensure((size_t)g)) ||
-        (rc = e->d_tiles.ensure(tiles.size())))
+        (rc = e->d_tiles.ensure(o.tiles.size())) || (rc = e->d_tperm.ensure(o.tperm.size())))
         return rc;
     if (g > 0) {
         HIPCHK(hipMemcpyAsync(e->d_grid.p, grid, sizeof(double) * g * 3, hipMemcpyHostToDevice, e->stream));
-        HIPCHK(hipMemcpyAsync(e->d_perm.p, perm.data(), sizeof(int) * g, hipMemcpyHostToDevice, e->stream));
-        HIPCHK(hipMemcpyAsync(e->d_tiles.p, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->d_perm.p, o.perm.data(), sizeof(int) * g, hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->d_tiles.p, o.tiles.data(), sizeof(TileRec) * o.tiles.size(), hipMemcpyHostToDevice,
+                              e->stream));
+        HIPCHK(hipMemcpyAsync(e->d_tperm.p, o.tperm.data(), sizeof(int) * o.tperm.size(), hipMemcpyHostToDevice,
+                              e->stream));
     }
     HIPCHK(hipStreamSynchronize(e->stream));
     e->h_grid.assign(grid, grid + 3 * g);
     e->grid_z_flat = flat;
     e->grid_absmax = amax;
-    e->ntiles = (int)tiles.size() - 1;
+    e->ntiles = (int)o.tiles.size();
     e->G = g;
     e->have_grid = true;
     return PGT_OK;
@@ -1813,8 +1860,8 @@ struct pgt_ik_sweep {
     bool held = false;     // enqueued launches a captured graph may replay
     DBuf<SweepSys> d_tab;
     DBuf<double> d_grid;   // the systems' grids, back to back
-    DBuf<int> d_perm;      // their Morton orders
-    DBuf<int> d_tiles;     // and tile starts
+    DBuf<TileRec> d_tiles; // their tiles
+    DBuf<int> d_tperm;     // and the tiles' points
     DBuf<unsigned char> d_keys0, d_vals0, d_keys1, d_vals1, d_hist, d_cstart, d_spos, d_sdiam, d_bcount, d_skin;
     DBuf<unsigned char> d_bonds, d_wcounts, d_wmax, d_rec;
     DBuf<int> d_maxcount;                // [0] largest bond count, [1] tile overflow bits
@@ -1922,6 +1969,8 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
     c.tab = T;
     c.ns = ns;
     c.blocks = s->blocks[SW_GATHER];
+    c.tiles = s->d_tiles.p;
+    c.tperm = s->d_tperm.p;
     c.R = s->R;
     c.cstart = cstart;
     c.spos = spos;
@@ -2032,7 +2081,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         maxcell = std::max(maxcell, S.g.ncell);
         cap = std::max(cap, e->cap);
         gtotal += e->G;
-        ttotal += e->ntiles + 1;
+        ttotal += e->ntiles;
         S.tp = kTilePoints;
     }
     int kbits = 0;
@@ -2079,24 +2128,24 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
     if (s->np > ((int64_t)1 << 31) - 1)
         return bail(fail(PGT_ERR_RANGE, "the sweep holds more than 2^31 - 1 particles over all frames: split it"));
     int rc;
-    if ((rc = s->d_grid.ensure((size_t)gtotal * 3)) || (rc = s->d_perm.ensure((size_t)gtotal)) ||
-        (rc = s->d_tiles.ensure((size_t)ttotal)) || (rc = s->d_tab.ensure((size_t)nsys)))
+    if ((rc = s->d_grid.ensure((size_t)gtotal * 3)) || (rc = s->d_tiles.ensure((size_t)ttotal)) ||
+        (rc = s->d_tperm.ensure((size_t)ttotal * kTilePoints)) || (rc = s->d_tab.ensure((size_t)nsys)))
         return bail(rc);
     int64_t goff = 0, toff = 0;
     for (int k = 0; k < nsys; ++k) {
         const pgt_ik_engine *e = systems[k].engine;
         SweepSys &S = s->tab[(size_t)k];
         S.grid = s->d_grid.p + goff * 3;
-        S.perm = s->d_perm.p + goff;
-        S.tiles = s->d_tiles.p + toff;
+        S.tile0 = (int)toff;
         if (hipMemcpy((void *)S.grid, e->d_grid.p, sizeof(double) * 3 * (size_t)e->G, hipMemcpyDeviceToDevice) !=
                 hipSuccess ||
-            hipMemcpy((void *)S.perm, e->d_perm.p, sizeof(int) * (size_t)e->G, hipMemcpyDeviceToDevice) != hipSuccess ||
-            hipMemcpy((void *)S.tiles, e->d_tiles.p, sizeof(int) * (size_t)(e->ntiles + 1), hipMemcpyDeviceToDevice) !=
-                hipSuccess)
+            hipMemcpy(s->d_tiles.p + toff, e->d_tiles.p, sizeof(TileRec) * (size_t)e->ntiles, hipMemcpyDeviceToDevice) !=
+                hipSuccess ||
+            hipMemcpy(s->d_tperm.p + toff * kTilePoints, e->d_tperm.p, sizeof(int) * (size_t)e->ntiles * kTilePoints,
+                      hipMemcpyDeviceToDevice) != hipSuccess)
             return bail(fail(PGT_ERR_HIP, "copying a system's grid"));
         goff += e->G;
-        toff += e->ntiles + 1;
+        toff += e->ntiles;
     }
     if (hipMemcpy(s->d_tab.p, s->tab.data(), sizeof(SweepSys) * (size_t)nsys, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(PGT_ERR_HIP, "uploading the sweep's table"));
@@ -2118,8 +2167,8 @@ void pgt_ik_sweep_destroy(pgt_ik_sweep *s)
     for (auto *b : bufs) b->release();
     s->d_tab.release();
     s->d_grid.release();
-    s->d_perm.release();
     s->d_tiles.release();
+    s->d_tperm.release();
     s->d_maxcount.release();
     s->d_stats.release();
     for (hipEvent_t v : s->ev)

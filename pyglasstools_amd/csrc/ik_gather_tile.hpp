@@ -1,17 +1,20 @@
 // ik_gather_tile.hpp -- the item-balanced field gather ("tile" gather) of
 // the IK stress-field engine.  Included by ik_gather_launch.hpp.
 //
-// A workgroup is one wavefront and takes a tile: up to 64 neighbouring grid
-// points (a block of the grid's Morton order).  Work items are the (grid
-// point, particle) pairs with the particle inside the point's ball; an item
-// integrates the particle's bonds for the point.
+// A workgroup is one wavefront and takes a tile of the grid (a block of 8 x 8
+// or 4 x 4 x 4 of its sites, 64 slots, see TileRec) or a part of one.  Work
+// items are the (grid point, particle) pairs with the particle inside the
+// point's ball; an item integrates the particle's bonds for the point.
 //
-// 1. Window: the particles within r_cg of the tile's bounding box, read from
+// 1. Window: the particles within r_cg of the points' bounding box, read from
 //    the rows of cells that cover it, one particle per lane, into a list in
 //    LDS.
 // 2. Masks: a lane holds one window particle and tests it against every point
-//    of the tile (FP64, |a|^2 < r_cg^2; the points are broadcast from LDS),
-//    which gives the particle's mask of points.
+//    (FP64, |a|^2 < r_cg^2), which gives the particle's mask of points.  Where
+//    the tile's points are the product of their axes' coordinates (any
+//    regular grid), the squares of the differences along x are shared by a
+//    column of points, and those along x and y in 3D: 3 operations a pair
+//    and the axes' instead of 7 (2D) or 9 (3D).
 // 3. Items: the particles are ordered by bond count, largest first, and their
 //    items written to a list in that order, a particle's items side by side.
 // 4. Integration: lane l takes items l, l + 64, ...: the 64 items of a step
@@ -28,13 +31,17 @@
 // loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
 // when the lanes' lines differ).  With a point per lane, each lane walked its
 // own cells and every item fetched its particle from memory: 216 loads a
-// wavefront on the 2D N = 65,536 job with a 256^2 grid.  Here a window
-// particle is loaded once per tile, and an item's entries are shared by its
-// neighbours.  Measured against that scan (one launch): 100 such frames
-// 1.68 -> 1.38 ms, 3D N = 131,072 with a 64^3 grid, FP32 form, 20 frames
-// 4.30 -> 3.72 ms, 3D FP64 with the kinetic field, N = 20,011, 5 frames
-// 0.43 -> 0.37 ms, a sweep of eight systems whose grids are up to 2.4 r_cg / 2
-// apart 0.80 -> 0.65 ms.
+// wavefront on the 2D N = 65,536 job with a 256^2 grid, 5,814 VALU
+// instructions.  Here a window particle is loaded once per tile, and an
+// item's entries are shared by its neighbours: 126 loads, 4,501 VALU
+// instructions (5,360 before the product tiles' masks, the folded 5-node rule
+// and the two register sets of the item loop).  Measured (one launch, point
+// per lane / particle per lane / with those three): 100 such frames 1.68 /
+// 1.38 / 1.17 ms; 3D N = 131,072 with a 64^3 grid, FP32 form, 20 frames 4.30 /
+// 3.72 / 3.23 ms; 3D FP64 with the kinetic field, N = 20,011, 5 frames 0.43 /
+// 0.37 / 0.34 ms; 2D FP32 form, N = 30,011, 117^2 grid, 33 frames 0.152 /
+// 0.132 / 0.107 ms; a sweep of eight systems whose grid points are up to 2.4
+// apart (r_cg = 2) 0.80 / 0.65 / 0.58 ms.  VALU issue is now 72% of the time.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -49,7 +56,8 @@
 
 namespace pgt {
 
-// Capacities of the tile gather.
+// Capacities of the tile gather.  LDS in the 2D virial + kinetic form: 9.9 KB,
+// 16 wavefronts per CU, the four per SIMD that its registers allow.
 struct TileCaps {
     static constexpr int BLK = kTileThreads;  // one wavefront
     static constexpr int TP = kTilePoints;    // most grid points of a tile
@@ -107,23 +115,33 @@ __device__ __forceinline__ void axis_cells(const Geom &g, int a, double lo, doub
     wn = (int)(f1 - f0) + 1;
 }
 
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ double uniform(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
 // The body works on one frame's arrays (cell starts st, sorted positions
 // sp, kinetic terms sk, bond counts bc, entries bd; out's field pointers at
-// the frame's first value) for the cnt points from t0 on of the Morton order
-// perm (cnt <= 0: none), and stores its counts at out.wave_counts[2 wi ..].
+// the frame's first value) for slots j0 .. j0 + tp - 1 of tile record tr (tp:
+// 64, 16 or 4, j0 a multiple of it), whose grid points are tperm[0 .. 63],
+// and stores its counts at out.wave_counts[2 wi ..].
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
-__device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const double *__restrict__ grid,
-                                                 const int *__restrict__ perm, const GLRule &R,
-                                                 const double *__restrict__ gld, double cgnorm,
+__device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__restrict__ grid,
+                                                 const TileRec &tr, const int *__restrict__ tperm, int j0, int tp,
+                                                 const GLRule &R, const double *__restrict__ gld, double cgnorm,
                                                  const int *__restrict__ st, const double *__restrict__ sp,
                                                  const double *__restrict__ sk, int cap,
                                                  const int *__restrict__ bc, const ER *__restrict__ bd,
-                                                 const GatherOut &out, size_t wi, int t0, int cnt,
-                                                 int *__restrict__ overflow)
+                                                 const GatherOut &out, size_t wi, int *__restrict__ overflow)
 {
     using CP = TileCaps;
     using LY = BondLayout<D, OD, ELA, ER>;
     constexpr int MAXW = CP::MAXW, MAXI = CP::MAXI, SBITS = CP::SBITS;
+    constexpr int NR = MAXW / 64;  // window particles per lane
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
     constexpr bool PAIRS = VIR || ELA;
@@ -135,34 +153,34 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
     constexpr int GRP = LY::GRP;  // entries per read group
     constexpr int GV = LY::GV;    // values per read group
 
-    __shared__ double s_pt[64][PS];              // the tile's points (NaN beyond them)
+    __shared__ double s_pt[64][D];               // the points
     __shared__ double s_acc[64][KTA];            // their accumulators
     __shared__ double s_wp[MAXW][D];             // window: positions,
     __shared__ int s_wid[MAXW];                  // particles,
-    __shared__ unsigned long long s_wm[MAXW];    // point masks,
     __shared__ unsigned char s_wnb[MAXW];        // bond counts,
     __shared__ unsigned short s_wof[MAXW];       // first items
-    __shared__ unsigned short s_item[MAXI];      // items in order
     __shared__ int s_bucket[64];                 // items per bond count, then their offsets
-    __shared__ int s_seg[64], s_segb[64];        // segments of cells: first candidate, first particle
+    // items in order, and one past the list for those of another piece;
+    // while the window is filled, the segments' first candidates and particles
+    __shared__ union {
+        unsigned short item[MAXI + 2];
+        struct {
+            int first[64], particle[64];
+        } seg;
+    } s_u;
 
     const int l = threadIdx.x;
-    if (cnt <= 0) {
+    const int gp = tperm[l];
+    const bool live = gp >= 0 && l >= j0 && l < j0 + tp;
+    const unsigned long long points = __builtin_amdgcn_ballot_w64(live);
+    if (points == 0ull) {
         if (l == 0) {
             out.wave_counts[2 * wi] = 0;
             out.wave_counts[2 * wi + 1] = 0;
         }
         return;
     }
-    const bool live = l < cnt;
-    const int gp = perm[t0 + (live ? l : 0)];
-    double xg[D];
-#pragma unroll
-    for (int a = 0; a < D; ++a) xg[a] = grid[(size_t)gp * 3 + a];
-#pragma unroll
-    for (int a = 0; a < D; ++a) s_pt[l][a] = live ? xg[a] : __builtin_nan("");
-#pragma unroll
-    for (int k = 0; k < KTA; ++k) s_acc[l][k] = 0.0;
+    const bool product = tr.product != 0;
 
     // bounding box of the points: centre xc, half lengths xh.  When the box
     // and its ball fit in less than a period (near), a particle has one image
@@ -170,18 +188,62 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
     double xc[D], xh[D];
     int w0[3] = {0, 0, 0}, wn[3] = {1, 1, 1};
     bool near = true;
+    {
+        double xg[D], lo[D], hi[D];
 #pragma unroll
-    for (int a = 0; a < D; ++a) {
-        const double lo = wave_min(xg[a]), hi = wave_max(xg[a]);
-        axis_cells(g, a, lo, hi, g.rc, w0[a], wn[a]);
-        w0[a] = __builtin_amdgcn_readfirstlane(w0[a]);
-        wn[a] = __builtin_amdgcn_readfirstlane(wn[a]);
-        xc[a] = 0.5 * (lo + hi);
-        xh[a] = 0.5 * (hi - lo);
-        near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh[a] + g.rc) < 0.999 * g.L[a]);
+        for (int a = 0; a < D; ++a) {
+            xg[a] = live ? grid[(size_t)gp * 3 + a] : 0.0;
+            s_pt[l][a] = live ? xg[a] : __builtin_nan("");
+        }
+#pragma unroll
+        for (int k = 0; k < KTA; ++k) s_acc[l][k] = 0.0;
+        if (product) {
+            // over the axes' coordinates (lines without points are NaN,
+            // which the minimum and the maximum pass over)
+#pragma unroll
+            for (int a = 0; a < D; ++a) lo[a] = __builtin_huge_val(), hi[a] = -__builtin_huge_val();
+            const int q0 = j0 >> 4, q1 = (j0 + tp - 1) >> 4;
+            for (int q = q0; q <= q1; ++q) {
+                const double *ax = tr.ax[q];
+                // a row of four points (tp 4) has one y and one z
+                const int r = tp == 4 ? (j0 >> 2) & 3 : -1;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int a = k < 4 ? 0 : ((D == 2 || k < 6) ? 1 : D - 1);
+                    if (r >= 0 && k >= 4 && (D == 2 ? k - 4 != r : a == 1 ? k - 4 != (r & 1) : k - 6 != r >> 1))
+                        continue;
+                    lo[a] = fmin(lo[a], ax[k]);
+                    hi[a] = fmax(hi[a], ax[k]);
+                }
+            }
+        } else {
+            const int first = __ffsll(points) - 1;
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                const double v = live ? xg[a] : __shfl(xg[a], first, 64);
+                lo[a] = wave_min(v);
+                hi[a] = wave_max(v);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            axis_cells(g, a, lo[a], hi[a], g.rc, w0[a], wn[a]);
+            w0[a] = __builtin_amdgcn_readfirstlane(w0[a]);
+            wn[a] = __builtin_amdgcn_readfirstlane(wn[a]);
+            xc[a] = uniform(0.5 * (lo[a] + hi[a]));
+            xh[a] = uniform(0.5 * (hi[a] - lo[a]));
+            near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh[a] + g.rc) < 0.999 * g.L[a]);
+        }
+        near = __builtin_amdgcn_ballot_w64(near) != 0ull;  // the same in every lane: a scalar
     }
 
-    unsigned long long nball = 0;     // items, per lane
+    // whether a window particle's image nearest to xc is not the particle
+    // itself (or may not be): pairs then take the minimum image, which is the
+    // plain difference otherwise
+    bool images = !near;
+    auto nearest = [&](double v, int a) { return fma(-g.L[a], rint((v - xc[a]) * g.pinvL[a]), v); };
+
+    unsigned long long nball = 0;     // items (the same in every lane)
     unsigned long long ncontrib = 0;  // bond counts of the items, per lane
     bool over = false;                // an item's bond count exceeds MAXNB
     const double s2 = 2.0 * g.inv_rc;
@@ -192,7 +254,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
         // before the current one is integrated
         auto fetch = [&](int k, int &slot, int &ip, int &nb, double (&kk)[KNA], ER (&E)[GV]) {
             const bool valid = k < ni;
-            const unsigned it = s_item[valid ? k : 0];
+            const unsigned it = s_u.item[valid ? k : 0];
             slot = (int)(it & ((1u << SBITS) - 1u));
             ip = (int)(it >> SBITS);
             const int p = s_wid[slot];
@@ -203,22 +265,16 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
             if constexpr (PAIRS)
                 if (nb > 0) load_entry<ER, GV>(bd + (size_t)p * cap * ES, E);
         };
-        int slot, ip, nb;
-        double kk[KNA];
-        ER E0[GV];
-        fetch(l, slot, ip, nb, kk, E0);
-        for (int k0 = 0; k0 < ni; k0 += 64) {
-            const int k = k0 + l;
-            int nslot, nip, nnb;
-            double nkk[KNA];
-            ER nE0[GV];
-            fetch(k + 64, nslot, nip, nnb, nkk, nE0);
-            if (k < ni) {
+        auto item = [&](int slot, int ip, int nb, const double (&kk)[KNA], ER (&E0)[GV]) {
                 double a[3];
-                a[0] = minimg(s_wp[slot][0] - s_pt[ip][0], g.L[0], g.pinvL[0]);
-                a[1] = minimg(s_wp[slot][1] - s_pt[ip][1], g.L[1], g.pinvL[1]);
+                a[0] = s_wp[slot][0] - s_pt[ip][0];
+                a[1] = s_wp[slot][1] - s_pt[ip][1];
                 a[2] = 0.0;
-                if constexpr (D == 3) a[2] = minimg(s_wp[slot][D - 1] - s_pt[ip][D - 1], g.L[2], g.pinvL[2]);
+                if constexpr (D == 3) a[2] = s_wp[slot][D - 1] - s_pt[ip][D - 1];
+                if (images) {
+#pragma unroll
+                    for (int q = 0; q < D; ++q) a[q] = minimg(a[q], g.L[q], g.pinvL[q]);
+                }
                 const double A = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * g.inv_rc2;
                 double acc[KTA];
 #pragma unroll
@@ -233,16 +289,34 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
                     ta[0] = (ER)(a[0] * s2);
                     ta[1] = (ER)(a[1] * s2);
                     ta[2] = (ER)(a[2] * s2);
+                    // FP64 with the 5-node Octic rule: nodes with the weights
+                    // folded in (bond_octic5), 35 operations a bond instead
+                    // of 40; the FP32 form keeps its rounding
+                    constexpr bool FOLD = CG == 0 && NQ == 5 && std::is_same<ER, double>::value;
                     const ER Aj = (ER)A;
-                    auto one = [&](const ER (&Gv)[GV], auto O) {
+                    double Aq[3] = {0.0, 0.0, 0.0};
+                    if constexpr (FOLD)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) Aq[q] = A * R.oct_a[q];
+                    auto one = [&](const ER (&Gv)[GV], auto O, auto odd) {
                         constexpr int o = decltype(O)::value;
                         const ER *e = Gv + o;
                         ER C = e[0] * e[0];
                         C = fma(e[1], e[1], C);
                         if (D == 3) C = fma(e[2], e[2], C);
-                        ER B = ta[0] * e[0] + ta[1] * e[1];
-                        if (D == 3) B = fma(ta[2], e[2], B);
-                        const ER wq = bond_quad<CG, NQ, ER>(R, gld, R.n, Aj, B, C);
+                        // Written as fused operations, so that the FP32
+                        // form's rounding does not hang on how the compiler
+                        // contracts each copy: results of earlier builds
+                        // repeat bit for bit with y's product rounded first
+                        // in the odd groups and in 3D without elastic terms,
+                        // x's elsewhere.
+                        ER B;
+                        if constexpr ((D == 3 && !ELA) || decltype(odd)::value) B = fma(ta[0], e[0], ta[1] * e[1]);
+                        else B = fma(ta[1], e[1], ta[0] * e[0]);
+                        if constexpr (D == 3) B = fma(ta[2], e[2], B);
+                        ER wq;
+                        if constexpr (FOLD) wq = bond_octic5(R, Aq, B, C);
+                        else wq = bond_quad<CG, NQ, ER>(R, gld, R.n, Aj, B, C);
                         if constexpr (VIR) {
                             const ER c = wq * e[LY::OC];
                             const ER cb0 = c * e[0], cb1 = c * e[1];
@@ -289,14 +363,14 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
                             }
                         }
                     };
-                    auto group = [&](const ER (&Gv)[GV], int kk2) {
-                        one(Gv, std::integral_constant<int, 0>());
+                    auto group = [&](const ER (&Gv)[GV], int kk2, auto odd) {
+                        one(Gv, std::integral_constant<int, 0>(), odd);
                         if constexpr (GRP >= 2)
-                            if (GRP * kk2 + 1 < nb) one(Gv, std::integral_constant<int, ES>());
+                            if (GRP * kk2 + 1 < nb) one(Gv, std::integral_constant<int, ES>(), odd);
                         if constexpr (GRP >= 3)
-                            if (GRP * kk2 + 2 < nb) one(Gv, std::integral_constant<int, 2 * ES>());
+                            if (GRP * kk2 + 2 < nb) one(Gv, std::integral_constant<int, 2 * ES>(), odd);
                         if constexpr (GRP >= 4)
-                            if (GRP * kk2 + 3 < nb) one(Gv, std::integral_constant<int, 3 * ES>());
+                            if (GRP * kk2 + 3 < nb) one(Gv, std::integral_constant<int, 3 * ES>(), odd);
                     };
                     const ER *ptr = bd + (size_t)s_wid[slot] * cap * ES;
                     const int ng = (nb + GRP - 1) / GRP;
@@ -304,35 +378,104 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
                     int kk2 = 0;
                     for (; kk2 + 1 < ng; kk2 += 2) {
                         load_entry<ER, GV>(ptr + (size_t)(kk2 + 1) * GV, E1);
-                        group(E0, kk2);
+                        group(E0, kk2, std::false_type());
                         if (kk2 + 2 < ng) load_entry<ER, GV>(ptr + (size_t)(kk2 + 2) * GV, E0);
-                        group(E1, kk2 + 1);
+                        group(E1, kk2 + 1, std::true_type());
                     }
-                    if (kk2 < ng) group(E0, kk2);
+                    if (kk2 < ng) group(E0, kk2, std::false_type());
                 }
 #pragma unroll
                 for (int q = 0; q < KT; ++q)
                     __hip_atomic_fetch_add(&s_acc[ip][q], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            }
-            slot = nslot;
-            ip = nip;
-            nb = nnb;
-            if constexpr (KIN)
-#pragma unroll
-                for (int q = 0; q < KN; ++q) kk[q] = nkk[q];
-            if constexpr (PAIRS)
-#pragma unroll
-                for (int q = 0; q < GV; ++q) E0[q] = nE0[q];
+        };
+        // two sets of registers in turn, so that nothing is copied between steps
+        int slot, ip, nb, nslot, nip, nnb;
+        double kk[KNA], nkk[KNA];
+        ER E0[GV], nE0[GV];
+        fetch(l, slot, ip, nb, kk, E0);
+        for (int k0 = 0; k0 < ni; k0 += 128) {
+            fetch(k0 + 64 + l, nslot, nip, nnb, nkk, nE0);
+            if (k0 + l < ni) item(slot, ip, nb, kk, E0);
+            if (k0 + 64 >= ni) break;
+            fetch(k0 + 128 + l, slot, ip, nb, kk, E0);
+            if (k0 + 64 + l < ni) item(nslot, nip, nnb, nkk, nE0);
         }
         __syncthreads();
+    };
+
+    // m = 2 m + (d2 < r_cg^2) for a d2 that is a number: the sign of the
+    // difference, which rounding keeps, moved in by one instruction (a compare
+    // and the selects of its result would be three)
+    auto push = [&](unsigned &m, double d2) {
+        m = __builtin_amdgcn_alignbit(m, (unsigned)((unsigned long long)__double_as_longlong(d2 - g.rc2) >> 32), 31);
+    };
+    // Mask of the points whose balls hold x: bit j for slot j (bits enter at
+    // the low end, the last slot first).  Slots without a point are masked
+    // off: their coordinates are NaN.
+    auto point_mask = [&](const double (&x)[D], unsigned (&m)[2]) {
+        m[0] = m[1] = 0u;
+        if (near && product) {
+            for (int q = (j0 + tp - 1) >> 4; q >= j0 >> 4; --q) {
+                const double *ax = tr.ax[q];
+                double dx2[4], d1[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const double d = x[0] - ax[k];
+                    dx2[k] = d * d;
+                    d1[k] = D == 2 || k < 2 ? x[1] - ax[4 + k] : x[D - 1] - ax[4 + k];  // 3D: 2 along y, 2 along z
+                }
+                unsigned mm = (q & 2) ? m[1] : m[0];
+                if constexpr (D == 2) {
+#pragma unroll
+                    for (int r = 15; r >= 0; --r) push(mm, fma(d1[r >> 2], d1[r >> 2], dx2[r & 3]));
+                } else {
+                    double dxy2[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) dxy2[k] = fma(d1[k >> 2], d1[k >> 2], dx2[k & 3]);
+#pragma unroll
+                    for (int r = 15; r >= 0; --r) push(mm, fma(d1[2 + (r >> 3)], d1[2 + (r >> 3)], dxy2[r & 7]));
+                }
+                if (tp < 32) mm <<= (q & 1) * 16;
+                if (q & 2) m[1] = mm;
+                else m[0] = mm;
+            }
+        } else {
+#pragma unroll
+            for (int h = 1; h >= 0; --h) {
+                unsigned mm = 0u;
+                if ((unsigned)(points >> (32 * h)) != 0u) {
+#pragma unroll 4
+                    for (int j = 31; j >= 0; --j) {
+                        double d[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int a = 0; a < D; ++a) d[a] = x[a] - s_pt[32 * h + j][a];
+                        if (!near) {
+#pragma unroll
+                            for (int a = 0; a < D; ++a) d[a] = minimg(d[a], g.L[a], g.pinvL[a]);
+                        }
+                        const bool in = fma(d[2], d[2], fma(d[1], d[1], d[0] * d[0])) < g.rc2;
+                        mm = mm + mm + (in ? 1u : 0u);
+                    }
+                }
+                m[h] = mm;
+            }
+        }
+        m[0] &= (unsigned)points;
+        m[1] &= (unsigned)(points >> 32);
     };
 
     // ---- the items of window particles 0 .. nw - 1 --------------------------
     auto process = [&](int nw) {
         s_bucket[l] = 0;
         __syncthreads();
-        for (int r = 0; r < nw; r += 64) {
-            const int slot = r + l;
+        unsigned m[NR][2];
+        int nbs[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int slot = r * 64 + l;
+            m[r][0] = m[r][1] = 0u;
+            nbs[r] = 0;
+            if (r * 64 >= nw) continue;
             const bool valid = slot < nw;
             const int ws = valid ? slot : 0;
             int nbc = 0;
@@ -340,46 +483,20 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
             double x[D];
 #pragma unroll
             for (int a = 0; a < D; ++a) x[a] = s_wp[ws][a];
-            bool shift = !near;
+            if (images && near) {
 #pragma unroll
-            for (int a = 0; a < D; ++a) shift = shift || !(rint((x[a] - xc[a]) * g.pinvL[a]) == 0.0);
-            // bit j of the mask: the particle is in point j's ball.  Bits
-            // enter at the low end (m = 2 m + bit, one add with carry).
-            unsigned m[2] = {0u, 0u};
-            auto test = [&](auto image) {
-                constexpr bool IMAGE = decltype(image)::value;
-#pragma unroll
-                for (int h = 1; h >= 0; --h) {
-                    if (32 * h >= cnt) continue;
-                    unsigned mm = 0u;
-#pragma unroll 4
-                    for (int j = 31; j >= 0; --j) {
-                        double d[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-                        for (int a = 0; a < D; ++a) {
-                            d[a] = x[a] - s_pt[32 * h + j][a];
-                            if constexpr (IMAGE) d[a] = minimg(d[a], g.L[a], g.pinvL[a]);
-                        }
-                        const bool in = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] < g.rc2;
-                        mm = mm + mm + (in ? 1u : 0u);
-                    }
-                    m[h] = mm;
-                }
-            };
-            // no lane's particle needs another image: the plain difference is
-            // the minimum image of every pair that can be inside a ball
-            if (__builtin_amdgcn_ballot_w64(shift) == 0ull) test(std::false_type());
-            else test(std::true_type());
-            if (!valid) m[0] = m[1] = 0u;
-            const int pc = __popc(m[0]) + __popc(m[1]);
+                for (int a = 0; a < D; ++a) x[a] = nearest(x[a], a);
+            }
+            point_mask(x, m[r]);
+            if (!valid) m[r][0] = m[r][1] = 0u;
+            const int pc = __popc(m[r][0]) + __popc(m[r][1]);
             if (nbc > CP::MAXNB && pc > 0) over = true;
             const int nb = min(nbc, CP::MAXNB);
-            nball += (unsigned long long)pc;
             ncontrib += (unsigned long long)pc * (unsigned long long)nb;
+            nbs[r] = 63 - min(nb, 63);
             if (valid) {
                 s_wnb[slot] = (unsigned char)nb;
-                s_wm[slot] = (unsigned long long)m[1] << 32 | m[0];
-                atomicAdd(&s_bucket[63 - min(nb, 63)], pc);
+                atomicAdd(&s_bucket[nbs[r]], pc);
             }
         }
         __syncthreads();
@@ -393,34 +510,51 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
                 if (l >= off) v += u;
             }
             total = __builtin_amdgcn_readlane(v, 63);
+            nball += (unsigned long long)total;
             __syncthreads();
             s_bucket[l] = v - c;  // first item of the bond count
         }
         __syncthreads();
         for (int base = 0; base < total; base += MAXI) {
-            for (int r = 0; r < nw; r += 64) {
-                const int slot = r + l;
-                if (slot < nw) {
-                    const unsigned long long mk = s_wm[slot];
-                    unsigned m0 = (unsigned)mk, m1 = (unsigned)(mk >> 32);
-                    int k;
-                    if (base == 0) {
-                        // an LDS atomic; the lanes of one instruction are
-                        // served in a fixed order
-                        k = atomicAdd(&s_bucket[63 - min((int)s_wnb[slot], 63)], __popc(m0) + __popc(m1));
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const int slot = r * 64 + l;
+                if (r * 64 >= nw) continue;
+                int k = 0;
+                if (base == 0) {
+                    // an LDS atomic; the lanes of one instruction are served
+                    // in a fixed order
+                    if (slot < nw) {
+                        k = atomicAdd(&s_bucket[nbs[r]], __popc(m[r][0]) + __popc(m[r][1]));
                         s_wof[slot] = (unsigned short)k;
-                    } else {
-                        k = s_wof[slot] - base;
                     }
-                    while (m0 | m1) {
-                        const bool low = m0 != 0u;
-                        const unsigned mm = low ? m0 : m1;
-                        const int j = __ffs(mm) - 1 + (low ? 0 : 32);
-                        const unsigned rest = mm & (mm - 1u);
-                        m0 = low ? rest : 0u;
-                        m1 = low ? m1 : rest;
-                        if ((unsigned)k < (unsigned)MAXI) s_item[k] = (unsigned short)(slot | (j << SBITS));
-                        ++k;
+                } else {
+                    // a further piece of a long list: the masks again, rather
+                    // than registers held through the integration
+                    double x[D];
+#pragma unroll
+                    for (int a = 0; a < D; ++a) x[a] = s_wp[slot < nw ? slot : 0][a];
+                    if (images && near) {
+#pragma unroll
+                        for (int a = 0; a < D; ++a) x[a] = nearest(x[a], a);
+                    }
+                    point_mask(x, m[r]);
+                    if (slot < nw) k = s_wof[slot] - base;
+                    else m[r][0] = m[r][1] = 0u;
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    unsigned mm = m[r][h];
+                    const int word = slot | (32 * h) << SBITS;
+                    if (total <= MAXI) {
+                        unsigned short *q = s_u.item + k;
+                        k += __popc(mm);
+                        for (; mm; mm &= mm - 1u) *q++ = (unsigned short)(word + (__builtin_ctz(mm) << SBITS));
+                    } else {
+                        // items of other pieces go to the slot past the list
+                        for (; mm; mm &= mm - 1u, ++k)
+                            s_u.item[min((unsigned)k, (unsigned)MAXI)] =
+                                (unsigned short)(word + (__builtin_ctz(mm) << SBITS));
                     }
                 }
             }
@@ -431,71 +565,84 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
 
     // ---- window: candidates of the cell rows, in segments of one row --------
     const int nx = g.nc[0], ny = g.nc[1], nz = g.nc[2];
-    const int parts = w0[0] + wn[0] > nx ? 2 : 1;  // a row that wraps is two segments
-    const int nseg = wn[1] * wn[2] * parts;
+    const int wrap = w0[0] + wn[0] > nx ? 1 : 0;  // a row that wraps is two segments
+    const int nseg = (wn[1] * wn[2]) << wrap;
     const double rr = g.rc2 * (1.0 + 1e-9);
-    int nw = 0;
-    for (int s0 = 0; s0 < nseg; s0 += 64) {
-        int b = 0, len = 0;
-        if (s0 + l < nseg) {
-            const int r = (s0 + l) / parts, part = (s0 + l) - r * parts;
-            const int iz = r / wn[1], iy = r - iz * wn[1];
-            const int z = w0[2] + iz < nz ? w0[2] + iz : w0[2] + iz - nz;
-            const int y = w0[1] + iy < ny ? w0[1] + iy : w0[1] + iy - ny;
-            const int row = (z * ny + y) * nx;
-            b = st[part ? row : row + w0[0]];
-            len = st[part ? row + w0[0] + wn[0] - nx : row + min(w0[0] + wn[0], nx)] - b;
-        }
-        int v = len;
+    int s0 = 0, c0 = 0;  // the next candidate: c0 of the segments from s0 on
+    bool more = true;
+    while (more) {
+        int nw = 0;
+        bool full = false;
+        for (more = false; s0 < nseg && !full;) {
+            int b = 0, len = 0;
+            if (s0 + l < nseg) {
+                const int r = (s0 + l) >> wrap, part = (s0 + l) & wrap;
+                const int iz = D == 2 ? 0 : r / wn[1], iy = r - iz * wn[1];
+                const int z = w0[2] + iz < nz ? w0[2] + iz : w0[2] + iz - nz;
+                const int y = w0[1] + iy < ny ? w0[1] + iy : w0[1] + iy - ny;
+                const int row = (z * ny + y) * nx;
+                b = st[part ? row : row + w0[0]];
+                len = st[part ? row + w0[0] + wn[0] - nx : row + min(w0[0] + wn[0], nx)] - b;
+            }
+            int v = len;
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int u = __shfl_up(v, off, 64);
-            if (l >= off) v += u;
+            for (int off = 1; off < 64; off <<= 1) {
+                const int u = __shfl_up(v, off, 64);
+                if (l >= off) v += u;
+            }
+            const int total = __builtin_amdgcn_readlane(v, 63);
+            const int ns = min(nseg - s0, 64);
+            __syncthreads();
+            s_u.seg.first[l] = v - len;
+            s_u.seg.particle[l] = b;
+            __syncthreads();
+            for (; c0 < total; c0 += 64) {
+                const int c = min(c0 + l, total - 1);
+                // the last segment that starts at or before candidate c
+                int lo = 0;
+                for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1)
+                    if (lo + h < ns && s_u.seg.first[lo + h] <= c) lo += h;
+                const int id = s_u.seg.particle[lo] + c - s_u.seg.first[lo];
+                double x[D], d2 = 0.0;
+#pragma unroll
+                for (int a = 0; a < D; ++a) x[a] = sp[(size_t)id * PS + a];
+                bool shift = false;
+                if (near) {
+#pragma unroll
+                    for (int a = 0; a < D; ++a) {
+                        const double y = nearest(x[a], a);
+                        shift = shift || y != x[a];
+                        const double d = fabs(y - xc[a]) - xh[a];
+                        d2 = fma(d > 0.0 ? d : d - d, d > 0.0 ? d : d - d, d2);
+                    }
+                }
+                // not near: any image may matter, so every candidate is kept
+                const bool in = c0 + l < total && d2 < rr;
+                const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
+                const int k = __popcll(bm);
+                full = nw + k > MAXW;
+                if (full) break;  // these candidates again with the next window
+                images = images || __builtin_amdgcn_ballot_w64(in && shift) != 0ull;
+                if (in) {
+                    const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
+                    s_wid[w] = id;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
+                }
+                nw += k;
+            }
+            if (full) {
+                more = true;
+            } else {
+                c0 = 0;
+                s0 += 64;
+            }
         }
-        const int total = __builtin_amdgcn_readlane(v, 63);
         __syncthreads();
-        s_seg[l] = v - len;
-        s_segb[l] = b;
+        if (nw > 0) process(nw);
         __syncthreads();
-        const int ns = min(nseg - s0, 64);
-        for (int c0 = 0; c0 < total; c0 += 64) {
-            const int c = min(c0 + l, total - 1);
-            // the last segment that starts at or before candidate c
-            int lo = 0;
-#pragma unroll
-            for (int h = 32; h > 0; h >>= 1)
-                if (lo + h < ns && s_seg[lo + h] <= c) lo += h;
-            const int id = s_segb[lo] + c - s_seg[lo];
-            double x[D], d2 = 0.0;
-#pragma unroll
-            for (int a = 0; a < D; ++a) x[a] = sp[(size_t)id * PS + a];
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                const double d = fmax(fabs(minimg(x[a] - xc[a], g.L[a], g.pinvL[a])) - xh[a], 0.0);
-                d2 = fma(d, d, d2);
-            }
-            // not near: any image may matter, so every candidate is kept
-            const bool in = c0 + l < total && (!near || d2 < rr);
-            const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
-            const int k = __popcll(bm);
-            if (nw + k > MAXW) {
-                __syncthreads();
-                process(nw);
-                nw = 0;
-            }
-            if (in) {
-                const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
-                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
-                s_wid[w] = id;
-#pragma unroll
-                for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
-            }
-            nw += k;
-        }
     }
-    __syncthreads();
-    if (nw > 0) process(nw);
-    __syncthreads();
 
     if (live) {
         const size_t ob = (size_t)gp * OD * OD;
@@ -521,7 +668,6 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
         if (ELA) store(out.ela, ae, 1.0);
         if (KIN) store(out.kin, ak, cgnorm);
     }
-    nball = wave_sum(nball);
     ncontrib = wave_sum(ncontrib);
     if (l == 0) {
         out.wave_counts[2 * wi] = nball;
@@ -530,23 +676,13 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, int n, const dou
     if (over) atomicOr(overflow, 2);
 }
 
-// The points of workgroup b of a frame: tile b / (64 / tp), its tp points
-// from b mod (64 / tp) times tp on (tp 64: the whole tile).  tiles[k] is
-// where tile k starts in the Morton order.
-__device__ __forceinline__ void tile_points(const int *__restrict__ tiles, int b, int tp, int &t0, int &cnt)
-{
-    const int sub = kTilePoints / tp, k = b / sub;
-    t0 = tiles[k] + (b - k * sub) * tp;
-    cnt = min(tiles[k + 1] - t0, tp);
-}
-
-// One frame per y row; block x takes the points of tile_points(xcd_tile(x,
-// gridDim.x)), so each XCD works through a contiguous eighth of the frame's
-// points.
+// One frame per y row; block x takes part b mod (64 / tp) of tile b / (64 /
+// tp), b = xcd_tile(x, gridDim.x), so each XCD works through a contiguous
+// eighth of the frame's tiles.
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
 __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gather_tile(
-    Geom g, int n, int G, const double *__restrict__ grid, const int *__restrict__ perm,
-    const int *__restrict__ tiles, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
+    Geom g, int n, int G, const double *__restrict__ grid, const TileRec *__restrict__ tiles,
+    const int *__restrict__ tperm, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
     const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap,
     const int *__restrict__ bcount, const ER *__restrict__ bonds, GatherOut out, int *__restrict__ overflow)
 {
@@ -559,12 +695,11 @@ __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gat
     if (VIR) of.vir = out.vir + oo;
     if (ELA) of.ela = out.ela + oo;
     if (KIN) of.kin = out.kin + oo;
-    int t0, cnt;
-    tile_points(tiles, xcd_tile(blockIdx.x, gridDim.x), tp, t0, cnt);
+    const int b = xcd_tile(blockIdx.x, gridDim.x), sub = kTilePoints / tp, k = b / sub;
     gather_tile_body<D, OD, CG, NQ, VIR, ELA, KIN, ER>(
-        g, n, grid, perm, R, gld, cgnorm, cstart + (size_t)f * (g.ncell + 1), spos + fo * PS,
-        KIN ? skin + fo * KN : nullptr, cap, bcount + fo, bonds + fo * (size_t)cap * ES, of,
-        (size_t)blockIdx.y * gridDim.x + blockIdx.x, t0, cnt, overflow);
+        g, grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - k * sub) * tp, tp, R, gld, cgnorm,
+        cstart + (size_t)f * (g.ncell + 1), spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, bcount + fo,
+        bonds + fo * (size_t)cap * ES, of, (size_t)blockIdx.y * gridDim.x + blockIdx.x, overflow);
 }
 
 // The sweep's field gather (2D or 3D, virial and/or kinetic): each
@@ -580,8 +715,8 @@ constexpr int kSweepGatherWaves = 3;
 
 template <int D, int OD, bool VIR, bool KIN, typename ER>
 __global__ __launch_bounds__(64, kSweepGatherWaves) void k_sweep_gather(
-    const SweepSys *__restrict__ T, int ns, GLRule R, const int *__restrict__ cstart,
-    const double *__restrict__ spos, const double *__restrict__ skin, int cap, const int *__restrict__ bcount,
+    const SweepSys *__restrict__ T, int ns, const TileRec *__restrict__ tiles, const int *__restrict__ tperm,
+    GLRule R, const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap, const int *__restrict__ bcount,
     const ER *__restrict__ bonds, unsigned long long *__restrict__ wave_counts,
     int *__restrict__ overflow)
 {
@@ -604,12 +739,11 @@ __global__ __launch_bounds__(64, kSweepGatherWaves) void k_sweep_gather(
     of.vir = VIR ? S.vir + oo : nullptr;
     of.kin = KIN ? S.kin + oo : nullptr;
     of.wave_counts = wave_counts;
-    int t0, cnt;
-    tile_points(S.tiles, b, S.tp, t0, cnt);
+    const int sub = kTilePoints / S.tp, q = b / sub, k = S.tile0 + q;
     gather_tile_body<D, OD, 0, 5, VIR, false, KIN, ER>(
-        g, n, S.grid, S.perm, R, nullptr, S.cgnorm, cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1),
-        spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, VIR ? bcount + fo : nullptr,
-        VIR ? bonds + fo * (size_t)cap * ES : nullptr, of, blockIdx.x, t0, cnt, overflow);
+        g, S.grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - q * sub) * S.tp, S.tp, R, nullptr, S.cgnorm,
+        cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1), spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap,
+        VIR ? bcount + fo : nullptr, VIR ? bonds + fo * (size_t)cap * ES : nullptr, of, blockIdx.x, overflow);
 }
 
 }  // namespace pgt

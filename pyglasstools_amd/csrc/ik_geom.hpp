@@ -138,6 +138,21 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+// A tile of the tile gather: the grid points of one block of 8 x 8 (2D) or
+// 4 x 4 x 4 (3D) sites of the grid's lattice, in 64 slots (a slot may be
+// empty).  Slots are numbered in four quads of 16 sites, so that a quad is a
+// compact part of the tile: 2D quads of 4 x 4 (slot 16 q + 4 y + x), 3D quads
+// of 4 x 2 x 2 (16 q + 8 z + 4 y + x).  product: every point's coordinates are
+// those of its site's lines, ax[q] = the quad's four x, then four y (2D) or
+// two y and two z (3D), NaN for a line without points.  Other tiles (points
+// off a lattice, several on one site) list their points in the slots in
+// order and have no lines.
+struct TileRec {
+    double ax[4][8];
+    int product;
+    int pad;
+};
+
 // Outputs of a field gather.
 struct GatherOut {
     double *vir;

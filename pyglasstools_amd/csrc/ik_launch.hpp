@@ -20,7 +20,8 @@ struct LaunchCtx {
     mutable int pl_launched;  // points per lane of the gather actually launched
     const double *grid;
     const int *perm;
-    const int *tiles;  // starts of the tile gather's tiles in perm, ntiles + 1 of them
+    const TileRec *tiles;  // the tile gather's tiles
+    const int *tperm;      // grid point of each slot, kTilePoints per tile, -1: none
     int ntiles;
     int tp;            // tile gather: grid points per workgroup (a divisor of kTilePoints)
     GLRule R;
@@ -89,6 +90,8 @@ struct SweepGatherCtx {
     const SweepSys *tab;  // device copy of the sweep's table
     int ns;
     int blocks;
+    const TileRec *tiles;  // every system's tiles, and their points
+    const int *tperm;
     GLRule R;
     const int *cstart;
     const double *spos, *skin;

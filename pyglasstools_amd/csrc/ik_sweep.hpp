@@ -37,8 +37,7 @@ struct SweepSys {
     long long p0, c0, h0;
     int blk0[SW_NSTAGE], nblk[SW_NSTAGE], bpf[SW_NSTAGE];
     const double *grid;  // the sweep's copy of the system's grid (x, y, z per point)
-    const int *perm;     // of its Morton order
-    const int *tiles;    // and of its tile starts
+    int tile0;           // its first tile in the sweep's copy of the tiles
     int tp;              // grid points per gather workgroup
     const double *pos, *diam, *mass, *vel;  // caller's frame-stacked inputs
     double *vir, *kin;                      // caller's frame-stacked outputs

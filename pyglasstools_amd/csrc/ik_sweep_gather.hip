@@ -12,7 +12,7 @@ template <int D, bool VIR, bool KIN, typename ER>
 void launch_t(const SweepGatherCtx &c)
 {
     hipLaunchKernelGGL((k_sweep_gather<D, D, VIR, KIN, ER>), dim3((unsigned)c.blocks), dim3(kTileThreads), 0,
-                       c.stream, c.tab, c.ns, c.R, c.cstart, c.spos, c.skin, c.cap, c.bcount,
+                       c.stream, c.tab, c.ns, c.tiles, c.tperm, c.R, c.cstart, c.spos, c.skin, c.cap, c.bcount,
                        (const ER *)c.bonds, c.wave_counts, c.flags);
 }
 
