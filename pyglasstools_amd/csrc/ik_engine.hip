@@ -502,33 +502,21 @@ Geom make_geom(const pgt_ik_engine *e, int D)
 // ------------------------------------------------------------------------
 // launch dispatch
 // ------------------------------------------------------------------------
-// k_bonds threads per workgroup and LDS candidate-list length per lane (a
-// full list is processed early: the length must stay well above the ~11.5
-// (2D) or ~33 (3D) neighbours within max_rcut at unit density, or most
-// particles process their list twice).  Measured per step: 2D, 256 lanes and
-// 32 entries (32 KB of LDS) 1% faster than 128 lanes on the N = 65,536 job,
-// 24 entries equal, 16 entries 17% slower; 3D, 64 lanes and 48 entries
-// (12 KB) 9% faster on the N = 131,072 FP32 job than 128 lanes and 64
-// entries, 40 entries 12% slower.
-constexpr int bond_block(int D) { return D == 2 ? 256 : 64; }
-constexpr int bond_list(int D) { return D == 2 ? 32 : 48; }
-
 template <int D, int OD, typename ER>
-void launch_bonds_t(const LaunchCtx &c, unsigned fields, const PotParams &P, const double *sdiam, const double *sdisp,
-                    int *bcount, void *bonds, int *wave_max, float4 *rec)
+void launch_bonds_t(const LaunchCtx &c, unsigned fields, const PotParams &P, const int *keys, const double *sdiam,
+                    const double *sdisp, int *bcount, void *bonds, int *wave_max, float4 *rec)
 {
     const bool V = fields & PGT_FIELD_VIRIAL, E = fields & PGT_FIELD_ELASTIC;
-    constexpr int BLK = bond_block(D), MAXC = bond_list(D);
-    dim3 grid((unsigned)((c.n + BLK - 1) / BLK), (unsigned)c.nf);
+    dim3 grid((unsigned)((c.n + kBondBlock - 1) / kBondBlock), (unsigned)c.nf);
     if (V && E)
-        hipLaunchKernelGGL((k_bonds<D, OD, true, true, ER, BLK, MAXC>), grid, dim3(BLK), 0, c.stream, c.g, c.n, P,
-                           c.cgnorm, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
+        hipLaunchKernelGGL((k_bonds<D, OD, true, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+                           c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
     else if (E)
-        hipLaunchKernelGGL((k_bonds<D, OD, false, true, ER, BLK, MAXC>), grid, dim3(BLK), 0, c.stream, c.g, c.n, P,
-                           c.cgnorm, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
+        hipLaunchKernelGGL((k_bonds<D, OD, false, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+                           c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
     else
-        hipLaunchKernelGGL((k_bonds<D, OD, true, false, ER, BLK, MAXC>), grid, dim3(BLK), 0, c.stream, c.g, c.n, P,
-                           c.cgnorm, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
+        hipLaunchKernelGGL((k_bonds<D, OD, true, false, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+                           c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
 }
 
 template <int D, int OD, typename ER>
@@ -617,8 +605,7 @@ void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, size_t
     const size_t fn = (size_t)nf * (size_t)n;
     const size_t nchunk = (size_t)((n + kSortChunk - 1) / kSortChunk);
     const size_t nw_gather_max = (size_t)std::max<int64_t>(j.gwaves, (G + j.block - 1) / j.block * (j.block / 64)) * nf;
-    const int bb = bond_block(j.D);
-    const size_t nw_bonds = j.pairs ? (size_t)((n + bb - 1) / bb) * nf * (bb / 64) : 0;
+    const size_t nw_bonds = j.pairs ? (size_t)((n + kBondBlock - 1) / kBondBlock) * nf : 0;
     for (int k = 0; k < W_NARRAYS; ++k) out[k] = 0;
     out[W_KEYS0] = out[W_VALS0] = out[W_KEYS1] = out[W_VALS1] = fn * sizeof(int);
     out[W_HIST] = (size_t)nf * j.radix * std::max<size_t>(nchunk, 1) * sizeof(int);
@@ -708,6 +695,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     int *bcount = w.get<int>(W_BCOUNT);
     hipStream_t s = e->stream;
     if (ev_begin) HIPCHK(hipEventRecord(ev_begin, s));
+    const int *keys = nullptr;  // sorted cell keys
     // cell list: per pass a histogram, a scan and a scatter of one digit of
     // the cell keys; frames are dealt to XCDs whole (frame_block)
     {
@@ -730,7 +718,8 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
                                    vin, hist, kout, vout);
             }
         }
-        const int *keys = kb[j.npass & 1], *vals = vb[j.npass & 1];
+        keys = kb[j.npass & 1];
+        const int *vals = vb[j.npass & 1];
         const dim3 pgrid((unsigned)((n + 255) / 256), (unsigned)frame_rows(nf));
         if (D == 2)
             hipLaunchKernelGGL((k_sort_finish<2, 2>), pgrid, dim3(256), 0, s, g, n, nf, g.ncell, keys, vals, pos, diam,
@@ -777,8 +766,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     // per-wavefront statistics of this batch (see k_reduce_stats)
     c.pl = j.pl;
     const int nw_gather = (int)(j.gwaves * nf);
-    const int bb = bond_block(D);
-    const int nw_bonds = j.pairs ? (int)(((size_t)n + bb - 1) / bb) * nf * (bb / 64) : 0;
+    const int nw_bonds = j.pairs ? (int)(((size_t)n + kBondBlock - 1) / kBondBlock) * nf : 0;
     c.out.wave_counts = w.get<unsigned long long>(W_WCOUNTS);
     int *wmax = w.get<int>(W_WMAX);
     void *bonds = w.p[W_BONDS];
@@ -788,13 +776,13 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         c.cap = cap;
         const PotParams P = make_pot(e->prm);
         if (D == 2) {
-            if (j.fp32) launch_bonds_t<2, 2, float>(c, fields, P, sdiam, sdisp, bcount, bonds, wmax, rec);
-            else launch_bonds_t<2, 2, double>(c, fields, P, sdiam, sdisp, bcount, bonds, wmax, rec);
+            if (j.fp32) launch_bonds_t<2, 2, float>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            else launch_bonds_t<2, 2, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         } else if (OD == 2) {
-            launch_bonds_t<3, 2, double>(c, fields, P, sdiam, sdisp, bcount, bonds, wmax, rec);
+            launch_bonds_t<3, 2, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         } else {
-            if (j.fp32) launch_bonds_t<3, 3, float>(c, fields, P, sdiam, sdisp, bcount, bonds, wmax, rec);
-            else launch_bonds_t<3, 3, double>(c, fields, P, sdiam, sdisp, bcount, bonds, wmax, rec);
+            if (j.fp32) launch_bonds_t<3, 3, float>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            else launch_bonds_t<3, 3, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         }
         HIPCHK(hipGetLastError());
     } else {
@@ -1895,7 +1883,7 @@ int sweep_buffers(pgt_ik_sweep *s)
                              np * sizeof(double), s->vir ? np * sizeof(int) : 0, s->kin ? np * KN * sizeof(double) : 0,
                              s->vir ? np * (size_t)s->cap * s->ebytes : 0,
                              (size_t)s->blocks[SW_GATHER] * 2 * sizeof(unsigned long long),
-                             s->vir ? (size_t)s->blocks[SW_BONDS] * (bond_block(s->D) / 64) * sizeof(int) : 0,
+                             s->vir ? (size_t)s->blocks[SW_BONDS] * sizeof(int) : 0,
                              (s->vir && s->D == 3) ? np * sizeof(float4) : 0};
     DBuf<unsigned char> *bufs[14] = {&s->d_keys0, &s->d_vals0, &s->d_keys1, &s->d_vals1, &s->d_hist,
                                      &s->d_cstart, &s->d_spos, &s->d_sdiam, &s->d_bcount, &s->d_skin,
@@ -1949,18 +1937,17 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
     int *wmax = (int *)s->d_wmax.p;
     if (s->vir) {
         const dim3 bg((unsigned)s->blocks[SW_BONDS]);
-        constexpr int B2 = bond_block(2), M2 = bond_list(2), B3 = bond_block(3), M3 = bond_list(3);
         if (s->D == 2 && s->fp32)
-            hipLaunchKernelGGL((k_sweep_bonds<2, 2, float, B2, M2>), bg, dim3(B2), 0, st, T, ns, s->cap, cstart, spos,
+            hipLaunchKernelGGL((k_sweep_bonds<2, 2, float>), bg, dim3(kBondBlock), 0, st, T, ns, s->cap, keys, cstart, spos,
                                sdiam, bcount, (float *)s->d_bonds.p, wmax, rec);
         else if (s->D == 2)
-            hipLaunchKernelGGL((k_sweep_bonds<2, 2, double, B2, M2>), bg, dim3(B2), 0, st, T, ns, s->cap, cstart, spos,
+            hipLaunchKernelGGL((k_sweep_bonds<2, 2, double>), bg, dim3(kBondBlock), 0, st, T, ns, s->cap, keys, cstart, spos,
                                sdiam, bcount, (double *)s->d_bonds.p, wmax, rec);
         else if (s->fp32)
-            hipLaunchKernelGGL((k_sweep_bonds<3, 3, float, B3, M3>), bg, dim3(B3), 0, st, T, ns, s->cap, cstart, spos,
+            hipLaunchKernelGGL((k_sweep_bonds<3, 3, float>), bg, dim3(kBondBlock), 0, st, T, ns, s->cap, keys, cstart, spos,
                                sdiam, bcount, (float *)s->d_bonds.p, wmax, rec);
         else
-            hipLaunchKernelGGL((k_sweep_bonds<3, 3, double, B3, M3>), bg, dim3(B3), 0, st, T, ns, s->cap, cstart, spos,
+            hipLaunchKernelGGL((k_sweep_bonds<3, 3, double>), bg, dim3(kBondBlock), 0, st, T, ns, s->cap, keys, cstart, spos,
                                sdiam, bcount, (double *)s->d_bonds.p, wmax, rec);
         HIPCHK(hipGetLastError());
     }
@@ -1984,7 +1971,7 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
     launch_sweep_gather(c, s->D, s->fp32, s->fields);
     HIPCHK(hipGetLastError());
     if (timed) HIPCHK(hipEventRecord(s->ev[2], st));
-    const int nwg = s->blocks[SW_GATHER], nwb = s->vir ? s->blocks[SW_BONDS] * (bond_block(s->D) / 64) : 0;
+    const int nwg = s->blocks[SW_GATHER], nwb = s->vir ? s->blocks[SW_BONDS] : 0;
     const int nrb = std::max(1, std::min(256, (std::max(nwg, nwb) + 4095) / 4096));
     hipLaunchKernelGGL(k_reduce_stats, dim3(nrb), dim3(1024), 0, st, nwg, c.wave_counts, nwb, wmax, s->d_stats.p,
                        s->d_maxcount.p);
@@ -2105,7 +2092,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         s->nh += (int64_t)S.nf * s->radix * S.nchunk;
         S.bpf[SW_SORT] = S.nchunk;
         S.bpf[SW_FINISH] = (S.n + 255) / 256;
-        S.bpf[SW_BONDS] = (S.n + bond_block(D) - 1) / bond_block(D);
+        S.bpf[SW_BONDS] = (S.n + kBondBlock - 1) / kBondBlock;
         S.bpf[SW_GATHER] = systems[k].engine->ntiles * (kTilePoints / S.tp);
         for (int st = 0; st < SW_NSTAGE; ++st) {
             const int64_t nb = (st == SW_SORT || st == SW_FINISH)

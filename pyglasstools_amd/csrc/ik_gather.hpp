@@ -182,14 +182,9 @@ __global__ __launch_bounds__(BLK) void k_gather(Geom g, int n, int G, const doub
         auto integrate = [&](const ER (&Gv)[GV], auto O, int m, const ER (&ta)[PL][3], const ER (&Aj)[PL]) {
             constexpr int o = decltype(O)::value;
             const ER *e = Gv + o;
-            ER C;
-            if constexpr (LY::HAS_C2) {
-                C = e[D];
-            } else {
-                C = e[0] * e[0];
-                C = fma(e[1], e[1], C);
-                if (D == 3) C = fma(e[2], e[2], C);
-            }
+            ER C = e[0] * e[0];
+            C = fma(e[1], e[1], C);
+            if (D == 3) C = fma(e[2], e[2], C);
 #pragma unroll
             for (int j = 0; j < PL; ++j) {
                 if (PL > 1 && !((m >> j) & 1)) continue;

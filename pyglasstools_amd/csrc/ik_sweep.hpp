@@ -16,8 +16,8 @@ constexpr int kSweepMaxSystems = 16;
 
 // The stages with per-system workgroup ranges: radix-sort histogram and
 // scatter (one chunk of kSortChunk particles per workgroup), the sorted
-// arrays (256 particles), the bond list (256 particles) and the field
-// gather (kTilePoints grid points).
+// arrays (256 particles), the bond list (kBondBlock particles) and the field
+// gather (a tile of grid points, or an equal part of one).
 enum SweepStage { SW_SORT = 0, SW_FINISH = 1, SW_BONDS = 2, SW_GATHER = 3, SW_NSTAGE = 4 };
 
 // One system of a sweep.  The work arrays stack the systems' frames: frame f

@@ -77,9 +77,9 @@ __global__ __launch_bounds__(256) void k_sweep_finish(const SweepSys *__restrict
 
 // Virial bond entries.  Padding workgroups store zero maxima for their
 // wavefronts, so k_reduce_stats can read every slot.
-template <int D, int OD, typename ER, int BLK, int MAXC>
-__global__ __launch_bounds__(BLK) void k_sweep_bonds(const SweepSys *__restrict__ T, int ns, int cap,
-                                                     const int *__restrict__ cstart, const double *__restrict__ spos,
+template <int D, int OD, typename ER>
+__global__ __launch_bounds__(kBondBlock, bond_waves(D, false)) void k_sweep_bonds(const SweepSys *__restrict__ T, int ns, int cap,
+                                                     const int *__restrict__ keys, const int *__restrict__ cstart, const double *__restrict__ spos,
                                                      const double *__restrict__ sdiam, int *__restrict__ bcount,
                                                      ER *__restrict__ bonds, int *__restrict__ wave_max,
                                                      float4 *__restrict__ rec)
@@ -87,19 +87,20 @@ __global__ __launch_bounds__(BLK) void k_sweep_bonds(const SweepSys *__restrict_
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int ES = BondLayout<D, OD, false, ER>::ES;
     const SweepSys &S = T[sweep_system(T, ns, SW_BONDS, blockIdx.x)];
-    int *wm = wave_max + (size_t)blockIdx.x * (BLK / 64);
+    int *wm = wave_max + blockIdx.x;
     int f, pb;
     if (!sweep_frame_tile(S, SW_BONDS, blockIdx.x, f, pb)) {
-        if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = 0;
+        if (threadIdx.x == 0) *wm = 0;
         return;
     }
     const Geom g = S.g;
     const PotParams P = S.P;
     const int n = S.n;
     const size_t fo = (size_t)S.p0 + (size_t)f * n;
-    bonds_body<D, OD, true, false, ER, BLK, MAXC>(g, n, P, S.cgnorm, cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1),
-                                                  spos + fo * PS, sdiam + fo, nullptr, cap, bcount + fo,
-                                                  bonds + fo * (size_t)cap * ES, wm, D == 3 ? rec + fo : nullptr, pb);
+    bonds_body<D, OD, true, false, ER>(g, n, P, S.cgnorm, keys + fo,
+                                       cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1), spos + fo * PS, sdiam + fo,
+                                       nullptr, cap, bcount + fo, bonds + fo * (size_t)cap * ES, wm,
+                                       D == 3 ? rec + fo : nullptr, pb);
 }
 
 }  // namespace pgt
