@@ -291,19 +291,24 @@ int pgt_ik_sweep_get_stats(pgt_ik_sweep *s, pgt_ik_stats *out);
  * points that share one read of each particle and bond entry), and cell
  * reach (1: cells of at least the search radius, searched one cell to each
  * side; 2: cells of at least half of it, two to each side); 0 keeps the
- * current choice.  Used by the autotuner.  No counterpart in the reference. */
+ * current choice.  Frames per launch not set: as many as make about two
+ * million particles (or grid points), at least eight.  Used by the autotuner.  No counterpart in the reference. */
 int pgt_ik_set_tuning(pgt_ik_engine *e, int threads_per_block, int frames_per_launch, int points_per_lane,
                       int cell_reach);
 
-/* Field-gather kernel for the Octic 5-node rule (the driver scripts' rule):
- * 1, the tile gather (one wavefront per 64 grid points lists the (point,
- * particle) pairs of its balls, sorts them by bond count and integrates
- * them round-robin, so every lane has about the same number of bonds);
+/* Field-gather kernel: 1, the tile gather (one wavefront per tile of up to 64
+ * grid points lists the (point, particle) pairs of its balls, sorts them by
+ * bond count and integrates them round-robin, so every lane has about the
+ * same number of bonds);
  * 0, the lane gather (each lane walks the balls of its own one, two or four
- * points).  Same results to rounding; other rules always use the lane
- * gather, as do frames of more than 2^26 particles, and a particle with more
- * than 255 bonds makes the job run again with the lane gather.  No
- * counterpart in the reference. */
+ * points).  Same results to rounding.  The tile gather also serves the other
+ * fixed rules with FP64 entries; the FP32 form's other orders and frames of
+ * more than 2^26 particles always use the lane gather, and a particle with
+ * more than 255 bonds makes the job run again with the lane gather.  An
+ * engine on which neither this nor the lane gather's settings
+ * (pgt_ik_set_tuning's threads_per_block, points_per_lane) were chosen takes
+ * the tile gather for FP64 entries with at most 255 bond slots a particle,
+ * the lane gather otherwise.  No counterpart in the reference. */
 int pgt_ik_set_gather_mode(pgt_ik_engine *e, int mode);
 
 int pgt_ik_get_stats(pgt_ik_engine *e, pgt_ik_stats *out);

@@ -185,6 +185,7 @@ struct GridOrder {
     std::vector<int> perm;
     std::vector<TileRec> tiles;
     std::vector<int> tperm;  // kTilePoints per tile
+    double step[3] = {0.0, 0.0, 0.0};  // of the lattice
 };
 
 GridOrder order_grid(int64_t G, const double *grid, bool use_z)
@@ -203,7 +204,7 @@ GridOrder order_grid(int64_t G, const double *grid, bool use_z)
     const int d = use_z ? 3 : 2;
     const double nside = std::max(2.0, std::round(std::pow((double)G, 1.0 / d)));
     double h[3];
-    for (int a = 0; a < 3; ++a) h[a] = std::max(hi[a] - lo[a], 1e-300) / (nside - 1.0);
+    for (int a = 0; a < 3; ++a) o.step[a] = h[a] = std::max(hi[a] - lo[a], 1e-300) / (nside - 1.0);
     const int bits = use_z ? 10 : 16;
     const double qmax = (double)((1u << bits) - 1);
     std::vector<uint64_t> key((size_t)G);
@@ -310,6 +311,7 @@ struct pgt_ik_engine {
     DBuf<TileRec> d_tiles;  // the tile gather's tiles (order_grid)
     DBuf<int> d_tperm;      // and their points
     int ntiles = 0;
+    double grid_step[3] = {0, 0, 0};  // steps of the grid's lattice
     // work arrays of a batch (see WorkArray), as raw bytes
     DBuf<unsigned char> d_keys0, d_vals0, d_keys1, d_vals1, d_hist, d_cstart, d_bcount;
     DBuf<unsigned char> d_spos, d_sdiam, d_skin, d_sdisp;
@@ -331,10 +333,11 @@ struct pgt_ik_engine {
     std::vector<double> gl_s, gl_w;
     int cap = 0;
     int block = 256;
-    int frames_per_launch = 8;
+    int frames_per_launch = 0;  // 0: launch_frames
     int points_per_lane = 2;  // grid points per gather lane (Octic 5-node rule; 1 elsewhere)
     int cell_reach = 1;       // cells searched on each side (cell edge >= search radius / reach)
-    int gather_mode = 0;      // 1: item-balanced tile gather where the form has one, 0: one lane per point
+    int gather_mode = -1;     // 1: item-balanced tile gather where the form has one, 0: one lane per point, -1: not chosen
+    bool lane_knobs = false;  // threads per workgroup or points per lane were set
     // set by pgt_ik_enqueue_frames: launches that a captured graph may replay
     // hold the current device buffers, so nothing may free or move them (or
     // change the bond capacity the launches were built with) until
@@ -541,9 +544,66 @@ struct JobShape {
     bool qag_global; // adaptive rule: interval tables of the caller's limit in e->d_qag
 };
 
-// n: particles per frame.  allow_tile false: the lane gather even where the
-// tile gather is selected (the fallback when a tile reports an overflow)
-JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, bool allow_tile = true)
+// Whether an engine whose gather was not chosen takes the tile gather: where
+// it has the form, with FP64 entries (the two gathers round the FP32 form's
+// terms differently) and at most 255 bond slots a particle (the lane gather
+// holds more), unless the caller set one of the lane gather's knobs.  It is
+// the faster one from the smallest jobs to the largest: gather of one frame
+// of N = 2,000, 32^2 grid 77 -> 8 us, N = 1,024, 128^2 grid 54 -> 12 us, N = 65,536,
+// 256^2 grid 74 -> 25 us, a 10-node Mollifier rule on N = 4,000, 97^2 grid
+// 202 -> 41 us, 24 frames with elastic terms, N = 16,384, 128^2 grid 252 -> 95 us.
+bool default_tile(const pgt_ik_engine *e, const JobShape &j)
+{
+    return !e->lane_knobs && !j.fp32 && e->cap <= 255 &&
+           tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32);
+}
+
+// Grid points per workgroup of the tile gather: whole tiles (64), or parts of
+// them.  Two things ask for parts.  `tiles` (of all frames of a launch) must
+// fill the GPU's 4,096 wavefront slots or the launch is as long as one
+// wavefront: gather of one frame, parts of 64 / 32 / 16 / 4 points: 2D N = 2,000,
+// 16 tiles 30 / - / 14 / 8 us; N = 16,384, 256 tiles 28 / 20 / 16 / 16; N = 65,536,
+// 1,024 tiles 34 / 27 / 26 / 52; 2,048 tiles 40 / 37 / 45 / 96; 3,072 tiles
+// 48 / 54 / 63 / 138.  And on a coarse grid a whole tile's window holds many
+// particles that are near only a few of its points: with n particles per
+// frame, a part's window should hold at most about 600: N = 98,304, grid
+// spacing 2.4 (447 particles in a whole tile's window) 127 / 131 / 137 / 224 us,
+// 3.5 (812, 413 in half of it) 269 / 229 / 223 / 279, 4.9 (349 in a quarter)
+// 197 / 145 / 149 / 158, 7.8 (110 in a row of four) 391 / 334 / 270 / 223; 3D N = 131,072,
+// spacing 1.6 (708, 447) 360 / 328 / 340 / 548, 2.7 (534 in a quarter)
+// 381 / 372 / 360 / 476, 4.6 (285 in a row of four) 669 / 375 / 333 / 276.
+int tile_part(const pgt_ik_engine *e, const Geom &g, int D, int64_t n, int64_t tiles)
+{
+    int tp = tiles < 192 ? 4 : tiles < 1536 ? 16 : tiles < 3072 ? 32 : 64;
+    double density = (double)n;
+    for (int a = 0; a < D; ++a) density /= g.L[a];
+    for (; tp > 4; tp = tp == 16 ? 4 : tp / 2) {
+        // steps of the lattice that a part spans along each axis
+        const double span[3] = {D == 2 && tp >= 32 ? 7.0 : 3.0, D == 2 ? (tp == 64 ? 7.0 : 3.0) : (tp >= 32 ? 3.0 : 1.0),
+                                tp == 64 ? 3.0 : 1.0};
+        double window = density;
+        for (int a = 0; a < D; ++a) window *= std::min(g.L[a], span[a] * e->grid_step[a] + 2.0 * g.rc);
+        if (window <= 600.0) break;
+    }
+    return tp;
+}
+
+// Frames per launch of a job where the caller set none: all of them up to
+// about 2 M particles (or grid points) a launch, whose bond entries take
+// 0.8 GB in 2D and 2.1 GB in 3D; at least eight.  24 frames of N = 16,384 with
+// elastic terms took 518 us in three launches of eight with the lane gather,
+// 253 us in one launch with the tile gather.
+int launch_frames(const pgt_ik_engine *e, int64_t n, int nframes)
+{
+    if (e->frames_per_launch > 0) return e->frames_per_launch;
+    const int64_t per_frame = std::max<int64_t>(1, std::max(n, e->G));
+    return (int)std::min<int64_t>(nframes, std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
+}
+
+// n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
+// gather even where the tile gather is selected (the fallback when a tile
+// reports an overflow)
+JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nf, bool allow_tile = true)
 {
     JobShape j{};
     j.OD = e->prm.dim;
@@ -569,12 +629,13 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     else j.ebytes = j.fp32 ? bond_entry_bytes<3, 3, float>(fields) : bond_entry_bytes<3, 3, double>(fields);
     j.block = j.adaptive ? 128 : e->block;  // k_gather_adaptive runs 128-thread workgroups
     j.pl = j.adaptive ? 1 : gather_pl(e->points_per_lane, e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD);
-    j.tile = allow_tile && !j.adaptive && e->gather_mode == 1 && n <= kTileMaxParticles &&
-             tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD);
+    j.tile = allow_tile && !j.adaptive && n <= kTileMaxParticles && e->ntiles > 0 &&
+             (e->gather_mode == 1 ? tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32)
+                                  : e->gather_mode == -1 && default_tile(e, j));
     if (j.tile) {
         j.block = kTileThreads;
         j.pl = 1;
-        j.tp = kTilePoints;
+        j.tp = tile_part(e, j.g, j.D, n, (int64_t)e->ntiles * nf);
         j.gwaves = (int64_t)e->ntiles * (kTilePoints / j.tp);
     } else {
         // the adaptive gather deals each point's integrals to several lanes
@@ -806,6 +867,9 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         } else {
             launch_gather_adaptive(c, fields, cg, D, OD, Q, c.flags, nullptr, 0);
         }
+    } else if (j.tile && !(cg == PGT_CG_OCTIC && c.R.n == 5)) {
+        if (D == 2) launch_tile_rules_2d(c, fields, cg);
+        else launch_tile_rules_3d(c, fields, cg);
     } else if (D == 2) {
         if (j.fp32) launch_gather_2d32(c, fields, cg);
         else launch_gather_2d64(c, fields, cg);
@@ -852,9 +916,9 @@ int run_batch(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, const
 // capacity once; on overflow grow it and run the whole job again.
 int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 {
-    int fpl = std::max(1, e->frames_per_launch);
+    int fpl = launch_frames(e, fs.n, fs.nframes);
     int nb = (fs.nframes + fpl - 1) / fpl;
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n);
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes));
     int rc;
     if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
     if ((rc = e->d_maxcount.ensure(2)) || (rc = e->d_stats.ensure(2))) return rc;
@@ -907,7 +971,7 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
             // a tile item had more bonds than its one-byte count holds:
             // run the job again with the lane gather
             if (!j.tile) return fail(PGT_ERR_STATE, "tile overflow reported by a lane gather");
-            j = job_shape(e, fields, fs.z_flat, fs.n, false);
+            j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes), false);
         } else if (!grow) {
             break;
         }
@@ -940,11 +1004,11 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 // enqueued work shows up in pgt_ik_finish.
 int enqueue_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 {
-    const int fpl = std::max(1, e->frames_per_launch);
+    const int fpl = launch_frames(e, fs.n, fs.nframes);
     const int nb = (fs.nframes + fpl - 1) / fpl;
     if (e->cap < 1 || !e->d_maxcount.p || e->d_maxcount.n < 2 || !e->d_stats.p)
         return fail(PGT_ERR_STATE, "run pgt_ik_compute_frames of the same shape before enqueueing");
-    const JobShape j = job_shape(e, fields, fs.z_flat, fs.n);
+    const JobShape j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes));
     Work w{};
     if (int rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, true, w)) return rc;
     for (int b = 0; b < nb; ++b) {
@@ -1234,6 +1298,7 @@ int pgt_ik_set_grid(pgt_ik_engine *e, int64_t g, const double *grid)
     e->grid_z_flat = flat;
     e->grid_absmax = amax;
     e->ntiles = (int)o.tiles.size();
+    std::copy(o.step, o.step + 3, e->grid_step);
     e->G = g;
     e->have_grid = true;
     return PGT_OK;
@@ -1334,6 +1399,7 @@ int pgt_ik_set_tuning(pgt_ik_engine *e, int threads_per_block, int frames_per_la
         if (threads_per_block != 128 && threads_per_block != 256)
             return fail(PGT_ERR_ARG, "threads per block must be 128 or 256");
         e->block = threads_per_block;
+        e->lane_knobs = true;
     }
     if (frames_per_launch) {
         if (frames_per_launch < 1 || frames_per_launch > 65535) return fail(PGT_ERR_ARG, "bad frames per launch");
@@ -1343,6 +1409,7 @@ int pgt_ik_set_tuning(pgt_ik_engine *e, int threads_per_block, int frames_per_la
         if (points_per_lane != 1 && points_per_lane != 2 && points_per_lane != 4)
             return fail(PGT_ERR_ARG, "grid points per lane must be 1, 2 or 4");
         e->points_per_lane = points_per_lane;
+        e->lane_knobs = true;
     }
     if (cell_reach) {
         if (cell_reach != 1 && cell_reach != 2) return fail(PGT_ERR_ARG, "cell reach must be 1 or 2");
@@ -1494,7 +1561,8 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
     fs.kin = (fields & PGT_FIELD_KINETIC) ? d_out_kinetic : nullptr;
     fs.ela = (fields & PGT_FIELD_ELASTIC) ? d_out_elastic : nullptr;
     fs.z_flat = e->grid_z_flat;
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n);
+    const int fpl = std::min(launch_frames(e, n, nframes), nframes);
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
     int cap = e->scratch_cap;
     if (j.pairs && cap < 1) cap = j.D == 3 ? 32 : 16;
     if (!j.pairs) cap = 1;
@@ -1502,7 +1570,7 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
     unsigned long long h[2] = {0, 0};
     for (int attempt = 0; attempt < 3; ++attempt) {
         // the most frames per launch whose work arrays fit the scratch array
-        int nf = std::min(std::max(1, e->frames_per_launch), nframes);
+        int nf = fpl;
         while (nf > 0 && work_carve(j, nf, n, e->G, cap, nullptr, nullptr) > kScratchBytes) nf = nf / 2;
         if (nf < 1)
             return fail(PGT_ERR_RANGE, "one frame of this job needs " +
@@ -1530,7 +1598,7 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
         if (grow && mx > 65535) return fail(PGT_ERR_RANGE, "a particle has more than 65535 interacting neighbours");
         if (flags[1] & 6) {
             if (!j.tile) return fail(PGT_ERR_STATE, "tile overflow reported by a lane gather");
-            j = job_shape(e, fields, fs.z_flat, fs.n, false);
+            j = job_shape(e, fields, fs.z_flat, fs.n, fpl, false);
         } else if (!grow) {
             break;
         }
@@ -2053,7 +2121,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
                          : sizeof(double) * BondLayout<3, 3, false, double>::ES;
     s->tab.resize((size_t)nsys);
     int maxcell = 1, cap = 0;
-    int64_t gtotal = 0, ttotal = 0;
+    int64_t gtotal = 0, ttotal = 0, tiles = 0;
     for (int k = 0; k < nsys; ++k) {
         const pgt_ik_engine *e = systems[k].engine;
         SweepSys &S = s->tab[(size_t)k];
@@ -2069,7 +2137,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         cap = std::max(cap, e->cap);
         gtotal += e->G;
         ttotal += e->ntiles;
-        S.tp = kTilePoints;
+        tiles += (int64_t)e->ntiles * S.nf;
     }
     int kbits = 0;
     while ((1 << kbits) < maxcell) ++kbits;
@@ -2093,6 +2161,7 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         S.bpf[SW_SORT] = S.nchunk;
         S.bpf[SW_FINISH] = (S.n + 255) / 256;
         S.bpf[SW_BONDS] = (S.n + kBondBlock - 1) / kBondBlock;
+        S.tp = tile_part(systems[k].engine, S.g, D, S.n, tiles);
         S.bpf[SW_GATHER] = systems[k].engine->ntiles * (kTilePoints / S.tp);
         for (int st = 0; st < SW_NSTAGE; ++st) {
             const int64_t nb = (st == SW_SORT || st == SW_FINISH)

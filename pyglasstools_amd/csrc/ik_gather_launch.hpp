@@ -58,32 +58,41 @@ void launch_gather_f(const LaunchCtx &c, unsigned fields)
     else launch_gather_b<D, OD, CG, NQ, false, false, ER>(c);
 }
 
-template <int D, int OD, bool VIR, bool ELA, bool KIN, typename ER>
+template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
 void launch_tile_t(const LaunchCtx &c)
 {
     using CP = TileCaps;
     const dim3 grid((unsigned)(c.ntiles * (CP::TP / c.tp)), (unsigned)c.nf);
     c.pl_launched = 1;
-    hipLaunchKernelGGL((k_gather_tile<D, OD, 0, 5, VIR, ELA, KIN, ER>), grid, dim3(CP::BLK), 0, c.stream, c.g, c.n, c.G,
+    hipLaunchKernelGGL((k_gather_tile<D, OD, CG, NQ, VIR, ELA, KIN, ER>), grid, dim3(CP::BLK), 0, c.stream, c.g, c.n, c.G,
                        c.grid, c.tiles, c.tperm, c.tp, c.R, c.gld, c.cgnorm, c.cstart, c.spos, c.skin, c.cap,
                        c.bcount, (const ER *)c.bonds, c.out, c.flags);
 }
 
-template <int D, int OD, bool VIR, bool ELA, typename ER>
+template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, typename ER>
 void launch_tile_k(const LaunchCtx &c)
 {
-    if (c.skin) launch_tile_t<D, OD, VIR, ELA, true, ER>(c);
-    else launch_tile_t<D, OD, VIR, ELA, false, ER>(c);
+    if (c.skin) launch_tile_t<D, OD, CG, NQ, VIR, ELA, true, ER>(c);
+    else launch_tile_t<D, OD, CG, NQ, VIR, ELA, false, ER>(c);
 }
 
-template <int D, int OD, typename ER>
+template <int D, int OD, int CG, int NQ, typename ER>
 void launch_tile_f(const LaunchCtx &c, unsigned fields)
 {
     const bool V = fields & PGT_FIELD_VIRIAL, E = fields & PGT_FIELD_ELASTIC;
-    if (V && E) launch_tile_k<D, OD, true, true, ER>(c);
-    else if (V) launch_tile_k<D, OD, true, false, ER>(c);
-    else if (E) launch_tile_k<D, OD, false, true, ER>(c);
-    else launch_tile_k<D, OD, false, false, ER>(c);
+    if (V && E) launch_tile_k<D, OD, CG, NQ, true, true, ER>(c);
+    else if (V) launch_tile_k<D, OD, CG, NQ, true, false, ER>(c);
+    else if (E) launch_tile_k<D, OD, CG, NQ, false, true, ER>(c);
+    else launch_tile_k<D, OD, CG, NQ, false, false, ER>(c);
+}
+
+// The tile gather with any other fixed rule (FP64 entries).
+template <int D>
+void launch_tile_rules(const LaunchCtx &c, unsigned fields, int cg)
+{
+    if (cg == 0) launch_tile_f<D, D, 0, 0, double>(c, fields);
+    else if (cg == 1) launch_tile_f<D, D, 1, 0, double>(c, fields);
+    else launch_tile_f<D, D, 2, 0, double>(c, fields);
 }
 
 // The Octic kernel gets the unrolled 5-node rule (the driver scripts' order)
@@ -93,7 +102,7 @@ template <int D, int OD, typename ER>
 void launch_gather_c(const LaunchCtx &c, unsigned fields, int cg)
 {
     if constexpr (!(D == 3 && OD == 2)) {
-        if (c.tile && cg == 0 && c.R.n == 5) return launch_tile_f<D, OD, ER>(c, fields);
+        if (c.tile && cg == 0 && c.R.n == 5) return launch_tile_f<D, OD, 0, 5, ER>(c, fields);
     }
     if (cg == 0) {
         if (c.R.n == 5 && !(D == 3 && OD == 2)) launch_gather_f<D, OD, 0, 5, ER>(c, fields);

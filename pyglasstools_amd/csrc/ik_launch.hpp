@@ -45,8 +45,12 @@ inline int gather_pl(int tuned, int cg, int nq, int D, int OD)
     return (cg == 0 && nq == 5 && !(D == 3 && OD == 2)) ? tuned : 1;
 }
 
-// Whether the tile gather serves this form (the Octic 5-node rule).
-inline bool tile_form(int cg, int nq, int D, int OD) { return cg == 0 && nq == 5 && !(D == 3 && OD == 2); }
+// Whether the tile gather serves this form: the Octic 5-node rule, and every
+// fixed rule with FP64 entries.
+inline bool tile_form(int cg, int nq, int D, int OD, bool fp32)
+{
+    return ((cg == 0 && nq == 5) || !fp32) && !(D == 3 && OD == 2);
+}
 
 // The tile gather's launch shape: a tile holds at most kTilePoints grid
 // points; a workgroup of kTileThreads lanes (one wavefront) takes a tile or
@@ -64,6 +68,9 @@ void launch_gather_2d32(const LaunchCtx &c, unsigned fields, int cg);  // ik_gat
 void launch_gather_3d2(const LaunchCtx &c, unsigned fields, int cg);   // ik_gather_3d2.hip
 void launch_gather_3d64(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_3d64.hip
 void launch_gather_3d32(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_3d32.hip
+// The tile gather with rules other than the Octic 5-node one, FP64 entries.
+void launch_tile_rules_2d(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_rules_2d.hip
+void launch_tile_rules_3d(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_rules_3d.hip
 // Lanes per grid point of the adaptive gather: the point's bond integrals
 // are dealt to them, so that a small grid still fills the GPU (about 64K
 // lanes per frame; a power of two from 1 to 32).  Measured on a 1,024-point

@@ -388,8 +388,8 @@ class Engine(object):
 
     def set_gather_mode(self, mode):
         """'tile' (one wavefront per 64-point tile, work items balanced by
-        bond count) or 'lane' (one lane per grid point or group of points)
-        for the Octic 5-node rule; other rules always run the lane gather."""
+        bond count) or 'lane' (one lane per grid point or group of points).
+        Not called: the engine's own choice (see pgt_ik_set_gather_mode)."""
         _check(lib().pgt_ik_set_gather_mode(self.h, {"lane": 0, "tile": 1}[mode]), "pgt_ik_set_gather_mode")
 
     def stats(self):

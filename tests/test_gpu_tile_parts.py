@@ -1,0 +1,156 @@
+"""The tile gather's parts (whole tiles, halves, quarters, rows of four
+points, chosen by the number of tiles of a launch), the forms an engine takes
+it for by default, and the bond kernel's windows, at the sizes where they can
+go wrong.
+
+Default against lane gather: the same terms summed in another order (and the
+5-node rule's weights folded into its nodes), so a difference of a few
+rounding errors of the sum of |terms|.  The sums have up to ~4,000 terms and
+the sum of |terms| is below ~20 times the field's largest value, so the bound
+is 4,000 x 2.2e-16 x 20 = 2e-11 of the largest value."""
+import numpy as np
+import pytest
+
+import oracle
+from pyglasstools_amd import engine, workload
+
+from conftest import scaled_error
+
+pytestmark = pytest.mark.gpu
+REL = 2e-11
+
+
+def _frames(e, frames, fields):
+    import torch
+
+    dev = torch.device("cuda:0")
+    t = lambda k: torch.tensor(np.stack([f[k] for f in frames]), dtype=torch.float64, device=dev)
+    out = {k: torch.full((len(frames), e.G, e.dim, e.dim), np.nan, dtype=torch.float64, device=dev) for k in fields}
+    e.compute_frames(len(frames), len(frames[0]["diam"]), t("pos"), t("diam"), t("mass"), t("vel"),
+                     t("disp") if "elastic" in fields else None, fields=fields,
+                     **{"d_" + k: v for k, v in out.items()})
+    torch.cuda.synchronize()
+    return {k: v.cpu().numpy() for k, v in out.items()}, e.stats()
+
+
+def _system(N, dim, seed):
+    s = workload.make_system(N, dim, seed)
+    s["disp"] = np.random.default_rng(seed).normal(0.0, 0.02, (N, 3)) * np.array([1, 1, 1 if dim == 3 else 0])
+    return s
+
+
+def _both(frames, grid, dim, fields, lengths=None, periodic=None, reach=1, **kw):
+    res = []
+    for mode in (None, "lane"):
+        e = engine.Engine(dim=dim, max_rcut=1.25 * 1.62, **kw)
+        if mode:
+            e.set_gather_mode(mode)
+        e.set_tuning(frames_per_launch=len(frames), cell_reach=reach)
+        e.set_box(frames[0]["L"] if lengths is None else lengths,
+                  frames[0]["periodic"] if periodic is None else periodic)
+        e.set_grid(grid)
+        res.append(_frames(e, frames, fields))
+    (a, sa), (b, sb) = res
+    for k in fields:
+        assert np.isfinite(a[k]).all(), k
+        top = np.abs(b[k]).max()
+        assert top > 0
+        err = np.abs(a[k] - b[k]).max() / top
+        print("  %s: max |default - lane| / max %.2e" % (k, err), flush=True)
+        assert err <= REL, (k, err)
+    assert sa["n_ball"] == sb["n_ball"] and sa["n_contrib"] == sb["n_contrib"]
+
+
+@pytest.mark.parametrize("dim,side,N,nf", [(2, 57, 400, 1), (2, 57, 400, 4), (2, 57, 400, 28), (2, 57, 400, 50),
+                                           (3, 9, 300, 1), (3, 9, 300, 8), (3, 9, 300, 60), (3, 9, 300, 120),
+                                           (2, 5, 4000, 1), (2, 11, 9000, 30)])
+def test_parts_match_the_lane_gather(gpu, dim, side, N, nf):
+    """64 tiles (2D, the last row and column partly filled) or 27 (3D) per
+    frame: rows of four, quarters, halves and whole tiles as the launch has 64
+    to 3,200 of them; grids so coarse that a tile's window would be large."""
+    print("parts %dD grid %d N=%d frames %d" % (dim, side, N, nf), flush=True)
+    frames = [_system(N, dim, 9100 + f) for f in range(nf)]
+    L = frames[0]["L"][0]
+    grid = workload.cartesian_grid_2d(L, side) if dim == 2 else workload.cartesian_grid_3d(L, side)
+    _both(frames, grid, dim, ("virial", "kinetic"))
+
+
+def _grid(kind, L, dim, rng):
+    z = 1.0 if dim == 3 else 0.0
+    if kind == "scattered":  # several points on one lattice site, others empty, some outside the box
+        return rng.uniform(-0.8 * L, 0.8 * L, (150, 3)) * np.array([1, 1, z])
+    if kind == "polar":
+        r, t = np.meshgrid(np.linspace(0.1, 0.45 * L, 12), np.linspace(0, 2 * np.pi, 17), indexing="ij")
+        return np.stack([r.ravel() * np.cos(t.ravel()), r.ravel() * np.sin(t.ravel()), 0.2 * z * r.ravel()], axis=1)
+    if kind == "line":
+        return np.linspace(-0.5, 0.5, 70)[:, None] * np.array([L, 0.3 * L, 0.2 * z * L])
+    if kind == "point":
+        return np.array([[0.3, -0.2, 0.1 * z]])
+    g = workload.cartesian_grid_2d(L, 13) if dim == 2 else workload.cartesian_grid_3d(L, 6)
+    return np.delete(g, [3, 17, 18, 90], axis=0)  # "holes"
+
+
+@pytest.mark.parametrize("kind", ["scattered", "polar", "line", "point", "holes"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_grids_off_a_lattice(gpu, dim, kind):
+    N = 900 if dim == 2 else 1200
+    frames = [_system(N, dim, 9300)]
+    print("grid %s %dD" % (kind, dim), flush=True)
+    _both(frames, _grid(kind, frames[0]["L"][0], dim, np.random.default_rng(4)), dim, ("virial", "kinetic"))
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("fields", [("virial",), ("kinetic",), ("elastic",), ("virial", "elastic"),
+                                    ("kinetic", "elastic"), ("virial", "kinetic", "elastic")])
+@pytest.mark.parametrize("cg,order", [("octic", 5), ("octic", 3), ("rect", 5), ("mollifier", 10)])
+def test_default_forms_match_the_lane_gather(gpu, dim, fields, cg, order):
+    frames = [_system(700, dim, 9400)]
+    L = frames[0]["L"][0]
+    grid = workload.cartesian_grid_2d(L, 11) if dim == 2 else workload.cartesian_grid_3d(L, 5)
+    print("default %dD %s %s order %d" % (dim, fields, cg, order), flush=True)
+    _both(frames, grid, dim, fields, cg=cg, order=order)
+
+
+@pytest.mark.parametrize("dim,lengths,periodic,reach", [
+    (2, None, (0, 1, 0), 1), (2, None, (0, 0, 0), 2), (3, None, (1, 0, 1), 1), (3, None, (1, 1, 0), 2),
+    (2, (4.2, 90.0, 1.0), (1, 1, 0), 1), (2, (90.0, 4.2, 1.0), (1, 1, 0), 2), (2, (8.2, 8.2, 1.0), (1, 1, 0), 1),
+    (3, (6.2, 30.0, 4.1), (1, 1, 1), 1), (3, (6.2, 6.2, 40.0), (1, 1, 1), 1)])
+def test_boxes_match_the_lane_gather(gpu, dim, lengths, periodic, reach):
+    """Open axes; boxes of one to four cells along an axis, whose windows
+    reach around it."""
+    N = 380 if dim == 2 else 800
+    s = _system(N, dim, 9500)
+    if lengths is not None:
+        s["pos"][:, :dim] *= np.array(lengths[:dim]) / s["L"][0]
+    L = s["L"] if lengths is None else np.array(lengths)
+    g = [np.linspace(-0.5 * L[a], 0.5 * L[a], 9 if dim == 2 else 5) for a in range(dim)] + [np.zeros(1)] * (3 - dim)
+    grid = np.stack([x.ravel() for x in np.meshgrid(*g, indexing="ij")], axis=1)
+    print("box %s periodic %s reach %d" % (L, periodic, reach), flush=True)
+    _both([s], grid, dim, ("virial", "kinetic"), L, periodic, reach)
+
+
+@pytest.mark.parametrize("dim,N,keep,reach,rc", [
+    (2, 1, 1.0, 1, 1.25), (2, 63, 1.0, 1, 1.25), (2, 64, 1.0, 1, 1.25), (2, 65, 1.0, 2, 1.25), (2, 129, 1.0, 1, 1.25),
+    (2, 9000, 0.02, 1, 1.25), (2, 9000, 0.02, 2, 1.25), (3, 8000, 0.03, 1, 1.25), (3, 8000, 0.03, 2, 1.25),
+    (2, 2000, 1.0, 1, 2.6), (3, 1500, 1.0, 1, 1.9), (3, 1500, 1.0, 2, 1.25)])
+def test_bond_windows_match_the_oracle(gpu, dim, N, keep, reach, rc):
+    """Blocks of 64 particles cut at either end; dilute systems, whose blocks
+    fall into up to 64 pieces; pair cutoffs with more candidates than a lane's
+    list (16) and a window (256) hold.  FP64 drop-in bar."""
+    print("bonds %dD N=%d keep %.2f reach %d cutoff %.2f" % (dim, N, keep, reach, rc), flush=True)
+    s = workload.make_system(max(N, 30 if dim == 2 else 120), dim, 9600 + N)
+    n = max(1, int(N * keep))
+    s = dict(s, **{k: s[k][:n] for k in ("pos", "diam", "mass", "vel")})
+    L = s["L"][0]
+    grid = workload.cartesian_grid_2d(L, 9) if dim == 2 else workload.cartesian_grid_3d(L, 5)
+    mr = min(rc * 1.62, 0.49 * L)
+    params = oracle.poly12_params(rcut=rc)
+    e = engine.Engine(dim=dim, max_rcut=mr, params=params, scaled_rcut=rc)
+    e.set_tuning(cell_reach=reach)
+    e.set_system(s, grid)
+    got = e.compute(fields=("virial",))
+    ref = oracle.ik_compute(s, grid, fields=("virial",), max_rcut=mr, params=params, scaled_rcut=rc, with_abs=True)
+    err = scaled_error(got["virial"], ref["virial"], ref["virial_abs"]).max()
+    print("  max scaled err %.2e" % err, flush=True)
+    assert err <= 1e-10
+    assert e.stats()["n_contrib"] == ref["n_nonzero"] and e.stats()["n_ball"] == ref["n_ball"]
