@@ -213,10 +213,35 @@ constexpr int kQagMax = 128;
 struct QagPrivate {
     double v[4][kQagMax];
     __device__ int size() const { return kQagMax; }
-    __device__ double &a(int k) { return v[0][k]; }
-    __device__ double &b(int k) { return v[1][k]; }
-    __device__ double &r(int k) { return v[2][k]; }
-    __device__ double &e(int k) { return v[3][k]; }
+    __device__ double a(int k) const { return v[0][k]; }
+    __device__ double b(int k) const { return v[1][k]; }
+    __device__ double r(int k) const { return v[2][k]; }
+    __device__ double e(int k) const { return v[3][k]; }
+    __device__ void set_a(int k, double x) { v[0][k] = x; }
+    __device__ void set_b(int k, double x) { v[1][k] = x; }
+    __device__ void set_r(int k, double x) { v[2][k] = x; }
+    __device__ void set_e(int k, double x) { v[3][k] = x; }
+};
+
+// The same with the error estimates of the first kQagLds intervals, which
+// every bisection searches for the largest, in LDS: el[k * 64] for a lane.
+constexpr int kQagLds = 32;
+struct QagLds {
+    double v[3][kQagMax], more[kQagMax - kQagLds];
+    double *el;
+    __device__ int size() const { return kQagMax; }
+    __device__ double a(int k) const { return v[0][k]; }
+    __device__ double b(int k) const { return v[1][k]; }
+    __device__ double r(int k) const { return v[2][k]; }
+    __device__ double e(int k) const { return k < kQagLds ? el[k * 64] : more[k - kQagLds]; }
+    __device__ void set_a(int k, double x) { v[0][k] = x; }
+    __device__ void set_b(int k, double x) { v[1][k] = x; }
+    __device__ void set_r(int k, double x) { v[2][k] = x; }
+    __device__ void set_e(int k, double x)
+    {
+        if (k < kQagLds) el[k * 64] = x;
+        else more[k - kQagLds] = x;
+    }
 };
 
 // Interval table of n entries in global memory, lane-interleaved: entry k's
@@ -226,10 +251,16 @@ struct QagGlobal {
     size_t stride;
     int n;
     __device__ int size() const { return n; }
-    __device__ double &a(int k) { return p[(size_t)(4 * k) * stride]; }
-    __device__ double &b(int k) { return p[(size_t)(4 * k + 1) * stride]; }
-    __device__ double &r(int k) { return p[(size_t)(4 * k + 2) * stride]; }
-    __device__ double &e(int k) { return p[(size_t)(4 * k + 3) * stride]; }
+    __device__ double get(int q, int k) const { return p[(size_t)(4 * k + q) * stride]; }
+    __device__ void set(int q, int k, double x) { p[(size_t)(4 * k + q) * stride] = x; }
+    __device__ double a(int k) const { return get(0, k); }
+    __device__ double b(int k) const { return get(1, k); }
+    __device__ double r(int k) const { return get(2, k); }
+    __device__ double e(int k) const { return get(3, k); }
+    __device__ void set_a(int k, double x) { set(0, k, x); }
+    __device__ void set_b(int k, double x) { set(1, k, x); }
+    __device__ void set_r(int k, double x) { set(2, k, x); }
+    __device__ void set_e(int k, double x) { set(3, k, x); }
 };
 
 struct AdaptQ {
@@ -300,7 +331,8 @@ __device__ void gk15_dev(const F &f, double a, double b, double &result, double 
     rasc *= abs_half;
     ra *= abs_half;
     if (rasc != 0.0 && err != 0.0) {
-        const double scale = pow(200.0 * err / rasc, 1.5);
+        const double x = 200.0 * err / rasc;
+        const double scale = x * sqrt(x);  // x^1.5
         err = (scale < 1.0) ? rasc * scale : rasc;
     }
     if (ra > 2.2250738585072014e-308 / (50 * 2.2204460492503131e-16)) {
@@ -313,22 +345,38 @@ __device__ void gk15_dev(const F &f, double a, double b, double &result, double 
     resasc = rasc;
 }
 
-template <typename F, typename W>
-__device__ double qag_dev(const F &f, const AdaptQ &Q, bool &capped, W &w)
+// The rule on the whole segment, which QAG starts from.
+struct QagStart {
+    double result, abserr;
+    bool done;  // converged, or at the rounding floor, or no more intervals allowed
+};
+
+template <typename F>
+__device__ __forceinline__ QagStart qag_start(const F &f, const AdaptQ &Q)
+{
+    QagStart s;
+    double resabs, resasc;
+    gk15_dev(f, 0.0, 1.0, s.result, s.abserr, resabs, resasc);
+    const double tol = fmax(Q.epsabs, Q.epsrel * fabs(s.result));
+    const double round_off = 50 * 2.2204460492503131e-16 * resabs;
+    s.done = (s.abserr <= round_off && s.abserr > tol) || s.abserr <= tol || Q.limit <= 1;
+    return s;
+}
+
+// QAG from a start that is not done.  PAIR: lanes 2k and 2k + 1 hold the same
+// integral and each takes one half of a bisection; both follow every step
+// and return the same value.
+template <bool PAIR, typename F, typename W>
+__device__ __forceinline__ double qag_refine(const F &f, const AdaptQ &Q, const QagStart &s, bool &capped, W &w)
 {
     const int limit = Q.limit < 1 ? 1 : Q.limit;
     const int lim = limit < w.size() ? limit : w.size();
-    double result, abserr, resabs, resasc;
-    gk15_dev(f, 0.0, 1.0, result, abserr, resabs, resasc);
-    w.a(0) = 0.0;
-    w.b(0) = 1.0;
-    w.r(0) = result;
-    w.e(0) = abserr;
+    w.set_a(0, 0.0);
+    w.set_b(0, 1.0);
+    w.set_r(0, s.result);
+    w.set_e(0, s.abserr);
     int n = 1;
-    double tol = fmax(Q.epsabs, Q.epsrel * fabs(result));
-    const double round_off = 50 * 2.2204460492503131e-16 * resabs;
-    if ((abserr <= round_off && abserr > tol) || abserr <= tol || limit == 1) return result;
-    double area = result, errsum = abserr;
+    double area = s.result, errsum = s.abserr, tol = fmax(Q.epsabs, Q.epsrel * fabs(area));
     while (n < lim) {
         int imax = 0;
         double emax = w.e(0);
@@ -339,21 +387,41 @@ __device__ double qag_dev(const F &f, const AdaptQ &Q, bool &capped, W &w)
                 imax = k;
             }
         }
-        const double a1 = w.a(imax), b2 = w.b(imax);
-        const double a2 = 0.5 * (a1 + b2), b1 = a2;
-        double r1, e1, ra1, rs1, r2, e2, ra2, rs2;
-        gk15_dev(f, a1, b1, r1, e1, ra1, rs1);
-        gk15_dev(f, a2, b2, r2, e2, ra2, rs2);
-        area += r1 + r2 - w.r(imax);
-        errsum += e1 + e2 - w.e(imax);
-        w.a(imax) = a1;
-        w.b(imax) = b1;
-        w.r(imax) = r1;
-        w.e(imax) = e1;
-        w.a(n) = a2;
-        w.b(n) = b2;
-        w.r(n) = r2;
-        w.e(n) = e2;
+        const double a1 = w.a(imax), b2 = w.b(imax), old = w.r(imax);
+        const double mid = 0.5 * (a1 + b2);
+        double r[2], e[2];
+        if constexpr (PAIR) {
+            const bool upper = threadIdx.x & 1;
+            double ra, rs, rh, eh;
+            gk15_dev(f, upper ? mid : a1, upper ? b2 : mid, rh, eh, ra, rs);
+            const double ro = __shfl_xor(rh, 1, 64), eo = __shfl_xor(eh, 1, 64);
+            r[0] = upper ? ro : rh;
+            r[1] = upper ? rh : ro;
+            e[0] = upper ? eo : eh;
+            e[1] = upper ? eh : eo;
+        } else {
+#pragma unroll 1
+            for (int h = 0; h < 2; ++h) {  // one copy of the rule's code for both halves
+                double ra, rs, rh, eh;
+                gk15_dev(f, h ? mid : a1, h ? b2 : mid, rh, eh, ra, rs);
+                if (h) {
+                    r[1] = rh;
+                    e[1] = eh;
+                } else {
+                    r[0] = rh;
+                    e[0] = eh;
+                }
+            }
+        }
+        area += r[0] + r[1] - old;
+        errsum += e[0] + e[1] - emax;
+        w.set_b(imax, mid);
+        w.set_r(imax, r[0]);
+        w.set_e(imax, e[0]);
+        w.set_a(n, mid);
+        w.set_b(n, b2);
+        w.set_r(n, r[1]);
+        w.set_e(n, e[1]);
         ++n;
         tol = fmax(Q.epsabs, Q.epsrel * fabs(area));
         if (errsum <= tol) break;
@@ -362,6 +430,13 @@ __device__ double qag_dev(const F &f, const AdaptQ &Q, bool &capped, W &w)
     double sum = 0.0;
     for (int k = 0; k < n; ++k) sum += w.r(k);
     return sum;
+}
+
+template <typename F, typename W>
+__device__ double qag_dev(const F &f, const AdaptQ &Q, bool &capped, W &w)
+{
+    const QagStart s = qag_start(f, Q);
+    return s.done ? s.result : qag_refine<false>(f, Q, s, capped, w);
 }
 
 // The kernel shape (t = |dr|^2 / rc^2, no normalisation) chosen at run time.

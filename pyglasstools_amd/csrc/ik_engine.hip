@@ -627,7 +627,7 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     if (j.D == 2) j.ebytes = j.fp32 ? bond_entry_bytes<2, 2, float>(fields) : bond_entry_bytes<2, 2, double>(fields);
     else if (j.OD == 2) j.ebytes = bond_entry_bytes<3, 2, double>(fields);
     else j.ebytes = j.fp32 ? bond_entry_bytes<3, 3, float>(fields) : bond_entry_bytes<3, 3, double>(fields);
-    j.block = j.adaptive ? 128 : e->block;  // k_gather_adaptive runs 128-thread workgroups
+    j.block = j.adaptive ? 64 : e->block;  // k_gather_adaptive runs 64-thread workgroups
     j.pl = j.adaptive ? 1 : gather_pl(e->points_per_lane, e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD);
     j.tile = allow_tile && !j.adaptive && n <= kTileMaxParticles && e->ntiles > 0 &&
              (e->gather_mode == 1 ? tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32)
@@ -638,9 +638,8 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
         j.tp = tile_part(e, j.g, j.D, n, (int64_t)e->ntiles * nf);
         j.gwaves = (int64_t)e->ntiles * (kTilePoints / j.tp);
     } else {
-        // the adaptive gather deals each point's integrals to several lanes
-        const int64_t lanes = j.adaptive ? e->G * adaptive_lanes(e->G) : (e->G + j.pl - 1) / j.pl;
-        j.gwaves = (lanes + j.block - 1) / j.block * (j.block / 64);
+        const int64_t lanes = (e->G + j.pl - 1) / j.pl;
+        j.gwaves = j.adaptive ? adaptive_waves(e->G) : (lanes + j.block - 1) / j.block * (j.block / 64);
     }
     return j;
 }
@@ -951,8 +950,7 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
             // the job again with tables of the limit in global memory, as
             // many frames per launch as kQagWorkspaceBytes holds
             if (j.qag_global) return fail(PGT_ERR_STATE, "adaptive workspace overflow with the caller's limit");
-            const size_t per_frame =
-                (((size_t)e->G * adaptive_lanes(e->G) + 127) / 128) * 128 * 4 * (size_t)e->prm.adapt_limit;
+            const size_t per_frame = (size_t)adaptive_waves(e->G) * 64 * 4 * (size_t)e->prm.adapt_limit;
             const size_t fit = kQagWorkspaceBytes / sizeof(double) / per_frame;
             if (fit < 1)
                 return fail(PGT_ERR_RANGE, "an adaptive bond integral needs more than " + std::to_string(kQagMax) +

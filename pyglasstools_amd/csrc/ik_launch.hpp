@@ -71,15 +71,20 @@ void launch_gather_3d32(const LaunchCtx &c, unsigned fields, int cg);  // ik_gat
 // The tile gather with rules other than the Octic 5-node one, FP64 entries.
 void launch_tile_rules_2d(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_rules_2d.hip
 void launch_tile_rules_3d(const LaunchCtx &c, unsigned fields, int cg);  // ik_gather_rules_3d.hip
-// Lanes per grid point of the adaptive gather: the point's bond integrals
-// are dealt to them, so that a small grid still fills the GPU (about 64K
-// lanes per frame; a power of two from 1 to 32).  Measured on a 1,024-point
-// frame: 8 lanes 5.6 ms, 16 lanes 3.4 ms, 32 lanes 2.2 ms (Octic).
+// Lanes per grid point of the adaptive gather, a power of two from 1 to 32:
+// about 64K lanes per frame, so that a small grid still fills the GPU.  Two
+// points to a wavefront leave about 28 integrals to bisect in 2D, two lanes
+// each (58 us a frame of 1,024 points; four points, a lane each, 106 us).
 inline int adaptive_lanes(int64_t G)
 {
     int l = 1;
     while (l < 32 && (int64_t)l * G < 65536) l <<= 1;
     return l;
+}
+inline int64_t adaptive_waves(int64_t G)
+{
+    const int64_t np = 64 / adaptive_lanes(G);
+    return (G + np - 1) / np;
 }
 
 // Field gather with the adaptive (QAG) bond integral.  ws null: each

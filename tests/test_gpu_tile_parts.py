@@ -154,3 +154,36 @@ def test_bond_windows_match_the_oracle(gpu, dim, N, keep, reach, rc):
     print("  max scaled err %.2e" % err, flush=True)
     assert err <= 1e-10
     assert e.stats()["n_contrib"] == ref["n_nonzero"] and e.stats()["n_ball"] == ref["n_ball"]
+
+
+@pytest.mark.parametrize("dim,side,fields,cg", [(2, 1, ("virial",), "octic"), (2, 3, ("virial", "kinetic"), "rect"),
+                                                (2, 9, ("virial", "elastic"), "mollifier"), (2, 70, ("kinetic",), "octic"),
+                                                (3, 3, ("virial", "kinetic", "elastic"), "octic"),
+                                                (3, 4, ("virial",), "rect")])
+def test_adaptive_shapes_match_the_oracle(gpu, dim, side, fields, cg):
+    """The adaptive gather with one point, points that do not fill a wavefront,
+    two frames, one to three fields.  The rule is asked for 1e-10 of each
+    integral; a decision at a near-tie can differ, so 1e-8 of each component's
+    scale, as the other adaptive fields are held to."""
+    adapt = (100, 1e-10, 1e-12)
+    frames = [_system(500 if dim == 2 else 400, dim, 9700 + f) for f in range(2)]
+    L = frames[0]["L"][0]
+    grid = workload.cartesian_grid_2d(L, side) if dim == 2 else workload.cartesian_grid_3d(L, side)
+    grid = grid * 0.83
+    print("adaptive %dD side %d %s %s" % (dim, side, fields, cg), flush=True)
+    e = engine.Engine(dim=dim, max_rcut=1.25 * 1.62, cg=cg, adaptive=adapt)
+    e.set_box(frames[0]["L"], frames[0]["periodic"])
+    e.set_grid(grid)
+    got, st = _frames(e, frames, fields)
+    ball = 0
+    for f, s in enumerate(frames):
+        ref = oracle.ik_compute(s, grid, fields=fields, max_rcut=1.25 * 1.62, cg=cg, adaptive=adapt, with_abs=True)
+        ball += ref["n_ball"]
+        for k in fields:
+            if k == "kinetic":
+                err = np.abs(got[k][f] - ref[k]).max() / np.abs(ref[k]).max()
+            else:
+                err = scaled_error(got[k][f], ref[k], ref["virial_abs"], floor=1e-4).max()
+            print("  %s: max scaled err %.2e" % (k, err), flush=True)
+            assert err <= 1e-8, (k, err)
+    assert st["n_ball"] == ball
