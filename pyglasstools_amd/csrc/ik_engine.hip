@@ -1101,10 +1101,18 @@ int prepare_pairs(pgt_ik_engine *e, int64_t *np, bool write, float *xin)
     return 0;
 }
 
-// H1 H2 H3 dZa dZb (64 n each), Y, dY (n each), loss partials (doubles),
-// gradient partials (kGradSplit rows of 64 * 64 + 64)
-size_t mlp_part_offset(int64_t n) { return (size_t)n * 322 + 2 * (size_t)((n + 255) / 256) + 2; }
-size_t mlp_work_floats(int64_t n) { return mlp_part_offset(n) + (size_t)kGradSplit * (kMlpW * kMlpW + kMlpW); }
+// Workspace of the network calls: pgt_mlp_forward's activations (64 n floats
+// for each of three layers), or pgt_mlp_grad's rows.  The size is what callers
+// have been told to allocate, more than either takes.
+constexpr int kMlpWorkRows = 64;
+size_t mlp_work_floats(int64_t n)
+{
+    return (size_t)n * 322 + 2 * (size_t)((n + 255) / 256) + 2 + (size_t)kMlpWorkRows * (kMlpW * kMlpW + kMlpW);
+}
+// (rows of 16 samples: at most 64 of them; rows of 32: 322 x 32 floats each)
+static_assert((size_t)kMlpWorkRows * (kMlpW * kMlpW + kMlpW) + 322 * 16 * 63 >= (size_t)64 * kGradRow &&
+                  322 * 32 >= kGradRow,
+              "the rows fit the workspace");
 
 unsigned blocks_for(int64_t threads) { return (unsigned)((threads + 255) / 256); }
 
@@ -1748,32 +1756,12 @@ int pgt_mlp_grad(const float *d_params, int64_t n, const float *d_x, const float
     if (n <= 0 || !d_params || !d_x || !d_t || !d_grad || !d_loss || !d_work)
         return fail(PGT_ERR_ARG, "bad network arguments");
     hipStream_t s = (hipStream_t)stream;
-    const float *P = d_params;
-    float *H1 = d_work, *H2 = d_work + 64 * n, *H3 = d_work + 128 * n, *dZa = d_work + 192 * n,
-          *dZb = d_work + 256 * n, *Y = d_work + 320 * n, *dY = d_work + 321 * n;
-    double *part = reinterpret_cast<double *>(d_work + 322 * n);
-    int rc;
-    if ((rc = pgt_mlp_forward(d_params, n, d_x, Y, d_work, stream))) return rc;
-    const unsigned nb = blocks_for(n);
-    hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, s, n, Y, d_t, dY, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, s, (int)nb, part, n, d_loss);
-    float *g = d_grad;
-    float *gpart = d_work + mlp_part_offset(n);
-    // weight and bias gradient of a layer with K inputs X (row stride ldx), N outputs, error dZ
-    auto wgrad = [&](int K, int N, const float *X, int ldx, const float *dZ, float *gW, float *gb) {
-        const int M = K * N + N;
-        hipLaunchKernelGGL(k_dense_bwd_weight, dim3(kGradSplit), dim3(256), 0, s, n, K, N, X, ldx, dZ, gpart);
-        hipLaunchKernelGGL(k_sum_split, dim3(blocks_for(M)), dim3(256), 0, s, K, N, gpart, gW, gb);
-    };
-    wgrad(kMlpW, 1, H3, kMlpW, dY, g + kOffW4, g + kOffB4);
-    hipLaunchKernelGGL(k_dense_bwd_data<1>, dim3(blocks_for(n * 64)), dim3(256), 0, s, n, dY, P + kOffW4, H3, dZa);
-    wgrad(kMlpW, kMlpW, H2, kMlpW, dZa, g + kOffW3, g + kOffB3);
-    hipLaunchKernelGGL(k_dense_bwd_data<kMlpW>, dim3(blocks_for(n * 64)), dim3(256), 0, s, n, dZa, P + kOffW3, H2,
-                       dZb);
-    wgrad(kMlpW, kMlpW, H1, kMlpW, dZb, g + kOffW2, g + kOffB2);
-    hipLaunchKernelGGL(k_dense_bwd_data<kMlpW>, dim3(blocks_for(n * 64)), dim3(256), 0, s, n, dZb, P + kOffW2, H1,
-                       dZa);
-    wgrad(kMlpIn, kMlpW, d_x, kMlpInPad, dZa, g + kOffW1, g + kOffB1);
+    const int rows = grad_rows(n);  // of kGradRow floats each, fewer than mlp_work_floats(n) in all
+    if (grad_chunk(n) == 16)
+        hipLaunchKernelGGL(k_mlp_grad<16>, dim3(rows), dim3(256), 0, s, n, d_params, d_x, d_t, d_work);
+    else
+        hipLaunchKernelGGL(k_mlp_grad<32>, dim3(rows), dim3(256), 0, s, n, d_params, d_x, d_t, d_work);
+    hipLaunchKernelGGL(k_grad_sum, dim3((kMlpNParam + 1 + 63) / 64), dim3(256), 0, s, rows, d_work, n, d_grad, d_loss);
     HIPCHK(hipGetLastError());
     return PGT_OK;
 }

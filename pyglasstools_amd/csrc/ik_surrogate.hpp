@@ -54,145 +54,264 @@ __global__ __launch_bounds__(256) void k_dense_fwd(int64_t n, const float *__res
     Y[idx] = tanh_act ? tanhf(acc) : acc;
 }
 
-// Mean-squared loss over n outputs: dY = 2 (Y - T) / n and per-block sums of
-// (Y - T)^2 into part[blockIdx.x] (folded by k_sum_parts).
-__global__ __launch_bounds__(256) void k_mse(int64_t n, const float *__restrict__ Y, const float *__restrict__ T,
-                                             float *__restrict__ dY, double *__restrict__ part)
+// Gradient of the mean-squared loss in one launch.  A workgroup takes chunks
+// of C samples (chunk c, c + gridDim.x, ...) through the forward pass and
+// back with every activation and error in LDS, and keeps its share of all
+// weight gradients in registers; it then stores them, its bias gradients and
+// its loss as row blockIdx.x of `part` (k_grad_sum adds the rows in order).
+// As seventeen launches, one per layer and direction, the step of 1,024
+// samples was bound by the launches and their tails: 65 us of kernels; this
+// takes 9 us, the sum of the rows 5.
+//
+// The products run on the matrix cores in FP32 (v_mfma_f32_16x16x4_f32):
+// wave w computes columns 16 w .. 16 w + 15.  Lane l = 16 q + c holds
+// A[c][k] and B[k][c] of a step's four k, one per q, and D[4 q + r][c]; a
+// product's k may come in any order, so that of step t is t + (K / 4) q, which
+// makes a lane's A values neighbours.  The row strides (66 for activations and
+// errors, 65 for weights) put the 64 lanes' words on distinct LDS banks.
+constexpr int kGradMaxRows = 256;                   // workgroups
+constexpr int kGradRow = (kMlpNParam + 3) / 4 * 4;  // floats of a row: the parameters' gradients, then
+                                                    // (8-byte aligned, in the last two) the loss sum
+static_assert(kGradRow >= ((kMlpNParam + 1) & ~1) + 2, "room for the loss");
+
+// Samples of a chunk: 16 while they leave the GPU's CUs a chunk or less each
+// (64 workgroups for 1,024 samples: 9.4 us a launch; 32 samples each on 32
+// workgroups, with the bias sums in one wavefront, 16.9).
+inline int grad_chunk(int64_t n) { return n <= 1024 ? 16 : 32; }
+inline int grad_rows(int64_t n)
 {
-    __shared__ double sh[256];
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double e2 = 0.0;
-    if (s < n) {
-        const float d = Y[s] - T[s];
-        dY[s] = 2.0f * d / (float)n;
-        e2 = (double)d * d;
+    const int64_t c = (n + grad_chunk(n) - 1) / grad_chunk(n);
+    return (int)(c < kGradMaxRows ? c : kGradMaxRows);
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void k_mlp_grad(int64_t n, const float *__restrict__ P, const float *__restrict__ X,
+                                                  const float *__restrict__ T, float *__restrict__ part)
+{
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int W = kMlpW, AS = 66, WS = 65, NT = C / 16, KQ = C / 4;  // row tiles, samples per q
+    __shared__ float s_w1[kMlpInPad][WS];  // rows past the inputs are zero
+    __shared__ float s_w2[W][WS], s_w3[W][WS], s_w4[W], s_b[3][W];
+    __shared__ float s_x[C][kMlpInPad + 2], s_h[3][C][AS], s_z[2][C][AS], s_dy[C];
+    __shared__ double s_loss[4];
+    __shared__ float s_gb4[4];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63, q = l >> 4, c = l & 15;
+    const int col = 16 * w + c;
+    {
+        float v2[W * W / 256], v3[W * W / 256];  // all loads in flight together
+#pragma unroll
+        for (int k = 0; k < W * W / 256; ++k) {
+            v2[k] = P[kOffW2 + 256 * k + t];
+            v3[k] = P[kOffW3 + 256 * k + t];
+        }
+        for (int k = t; k < kMlpInPad * W; k += 256) s_w1[k / W][k % W] = k < kMlpIn * W ? P[kOffW1 + k] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < W * W / 256; ++k) {
+            s_w2[4 * k + w][l] = v2[k];
+            s_w3[4 * k + w][l] = v3[k];
+        }
     }
-    sh[threadIdx.x] = e2;
+    if (t < W) {
+        s_w4[t] = P[kOffW4 + t];
+        s_b[0][t] = P[kOffB1 + t];
+        s_b[1][t] = P[kOffB2 + t];
+        s_b[2][t] = P[kOffB3 + t];
+    }
+    const float b4 = P[kOffB4];
+
+    f32x4 g1{}, g2[4], g3[4];  // weight gradients: rows 16 i + 4 q + r of column col
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g2[i] = g3[i] = f32x4{};
+    float gw4 = 0.0f, gb[3] = {0.0f, 0.0f, 0.0f};  // of unit col
+    float gb4 = 0.0f;   // of this thread's sample
+    double loss = 0.0;
+
+    // D = A (C x 64 activations or errors) B (64 x 64) for the wave's columns
+    auto product = [&](const float (&A)[C][AS], auto bval, f32x4 (&d)[NT]) {
+        float b[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) b[k] = bval(16 * q + k);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            d[i] = f32x4{};
+            float a[16];
+#pragma unroll
+            for (int k = 0; k < 16; k += 2) {
+                const float2 v = *reinterpret_cast<const float2 *>(&A[16 * i + c][16 * q + k]);
+                a[k] = v.x;
+                a[k + 1] = v.y;
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) d[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], b[k], d[i], 0, 0, 0);
+        }
+    };
+    // sum over the chunk's samples from the lane's KQ of them
+    auto over_samples = [&](float v) {
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
+    };
+    // G += A^T Z over the chunk's samples, and b += the sum of Z
+    auto outer = [&](const float (&A)[C][AS], const float (&Z)[C][AS], f32x4 (&g)[4], float &b) {
+        float z[KQ], v = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KQ; ++k) {
+            z[k] = Z[KQ * q + k][col];
+            v += z[k];
+        }
+        b += over_samples(v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int k = 0; k < KQ; ++k)
+                g[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[KQ * q + k][16 * i + c], z[k], g[i], 0, 0, 0);
+    };
+    // the hidden layer's output from its pre-activations
+    auto activate = [&](const f32x4 (&d)[NT], int layer) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s_h[layer][16 * i + 4 * q + r][col] = tanhf(d[i][r] + s_b[layer][col]);
+    };
+    // the error at a hidden layer's pre-activations
+    auto error = [&](const f32x4 (&d)[NT], int layer, float (&Z)[C][AS]) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float h = s_h[layer][16 * i + 4 * q + r][col];
+                Z[16 * i + 4 * q + r][col] = d[i][r] * (1.0f - h * h);
+            }
+    };
+    for (int64_t s0 = (int64_t)blockIdx.x * C; s0 < n; s0 += (int64_t)gridDim.x * C) {
+        if (t < 8 * C) {
+            const int r = t >> 3, k = t & 7;
+            s_x[r][k] = s0 + r < n && k < kMlpIn ? X[(s0 + r) * kMlpInPad + k] : 0.0f;
+        }
+        __syncthreads();
+        f32x4 d[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            d[i] = f32x4{};
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                d[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_x[16 * i + c][2 * q + k], s_w1[2 * q + k][col], d[i], 0, 0,
+                                                            0);
+        }
+        activate(d, 0);
+        __syncthreads();
+        product(s_h[0], [&](int k) { return s_w2[k][col]; }, d);
+        activate(d, 1);
+        __syncthreads();
+        product(s_h[1], [&](int k) { return s_w3[k][col]; }, d);
+        activate(d, 2);
+        __syncthreads();
+        if (t < 8 * C) {  // the output and its error, eight threads per sample
+            const int r = t >> 3, k0 = (t & 7) * 8;
+            float y = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) y = fmaf(s_h[2][r][k0 + k], s_w4[k0 + k], y);
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) y += __shfl_xor(y, off, 64);
+            if ((t & 7) == 0 && s0 + r < n) {
+                const float e = y + b4 - T[s0 + r];
+                const float dy = 2.0f * e / (float)n;
+                s_dy[r] = dy;
+                gb4 += dy;
+                loss += (double)e * e;
+            } else if ((t & 7) == 0) {
+                s_dy[r] = 0.0f;
+            }
+        }
+        __syncthreads();
+        {
+            float v = 0.0f;
+#pragma unroll
+            for (int k = 0; k < KQ; ++k) {
+                const int r = KQ * q + k;
+                const float h = s_h[2][r][col], dy = s_dy[r];
+                v = fmaf(h, dy, v);
+                s_z[0][r][col] = dy * s_w4[col] * (1.0f - h * h);
+            }
+            gw4 += over_samples(v);
+        }
+        __syncthreads();
+        outer(s_h[1], s_z[0], g3, gb[2]);
+        product(s_z[0], [&](int k) { return s_w3[col][k]; }, d);
+        error(d, 1, s_z[1]);
+        __syncthreads();
+        outer(s_h[0], s_z[1], g2, gb[1]);
+        product(s_z[1], [&](int k) { return s_w2[col][k]; }, d);
+        error(d, 0, s_z[0]);
+        __syncthreads();
+        {
+            float v = 0.0f;
+#pragma unroll
+            for (int k = 0; k < KQ; ++k) {
+                const float z = s_z[0][KQ * q + k][col];
+                v += z;
+                g1 = __builtin_amdgcn_mfma_f32_16x16x4f32(c < kMlpIn ? s_x[KQ * q + k][c] : 0.0f, z, g1, 0, 0, 0);
+            }
+            gb[0] += over_samples(v);
+        }
+        __syncthreads();
+    }
+
+    // the samples' threads: a fixed butterfly, then the four wavefronts in order
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1) {
+        gb4 += __shfl_xor(gb4, off, 64);
+        loss += __shfl_xor(loss, off, 64);
+    }
+    if (l == 0) {
+        s_gb4[w] = gb4;
+        s_loss[w] = loss;
+    }
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
+    float *out = part + (size_t)blockIdx.x * kGradRow;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (4 * q + r < kMlpIn) out[kOffW1 + (4 * q + r) * W + col] = g1[r];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            out[kOffW2 + (16 * i + 4 * q + r) * W + col] = g2[i][r];
+            out[kOffW3 + (16 * i + 4 * q + r) * W + col] = g3[i][r];
+        }
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    if (q == 0) {
+        out[kOffB1 + col] = gb[0];
+        out[kOffB2 + col] = gb[1];
+        out[kOffB3 + col] = gb[2];
+        out[kOffW4 + col] = gw4;
+    }
+    if (t == 0) {
+        out[kOffB4] = s_gb4[0] + s_gb4[1] + s_gb4[2] + s_gb4[3];
+        *reinterpret_cast<double *>(out + kGradRow - 2) = s_loss[0] + s_loss[1] + s_loss[2] + s_loss[3];
+    }
 }
 
-// out[0] = sum(part[0..np)) / n, in a fixed order (one workgroup).
-__global__ __launch_bounds__(256) void k_sum_parts(int np, const double *__restrict__ part, int64_t n,
-                                                   float *__restrict__ out)
+// grad = the sum of the rows of part, loss = the sum of their losses / n, each
+// as four sums of consecutive rows added in order (64 parameters a workgroup).
+__global__ __launch_bounds__(256) void k_grad_sum(int rows, const float *__restrict__ part, int64_t n,
+                                                  float *__restrict__ grad, float *__restrict__ loss)
 {
-    __shared__ double sh[256];
-    double s = 0.0;
-    for (int k = threadIdx.x; k < np; k += blockDim.x) s += part[k];
-    sh[threadIdx.x] = s;
+    __shared__ double sh[4][64];
+    const int o = threadIdx.x & 63, u = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + o;
+    const int r0 = rows * u / 4, r1 = rows * (u + 1) / 4;
+    double v = 0.0;
+    if (k < kMlpNParam) {
+        float f = 0.0f;
+#pragma unroll 8
+        for (int r = r0; r < r1; ++r) f += part[(size_t)r * kGradRow + k];
+        v = f;
+    } else if (k == kMlpNParam) {
+        for (int r = r0; r < r1; ++r) v += *reinterpret_cast<const double *>(part + (size_t)(r + 1) * kGradRow - 2);
+    }
+    sh[u][o] = v;
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = (float)(sh[0] / (double)n);
-}
-
-// dZp[s][k] = (sum_o dZ[s][o] W[k][o]) * (1 - H[s][k]^2): the error at the
-// pre-activation of the previous (tanh) layer of K = kMlpW units, H being
-// that layer's output; N outputs (a template argument, for the same reason
-// as in k_dense_fwd).
-template <int N>
-__global__ __launch_bounds__(256) void k_dense_bwd_data(int64_t n, const float *__restrict__ dZ,
-                                                        const float *__restrict__ W, const float *__restrict__ H,
-                                                        float *__restrict__ dZp)
-{
-    constexpr int K = kMlpW;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * K) return;
-    const int64_t s = idx / K;
-    const int k = (int)(idx % K);
-    float z[N];
-#pragma unroll
-    for (int o = 0; o < N; ++o) z[o] = dZ[s * N + o];
-    float acc = 0.0f;
-#pragma unroll
-    for (int o = 0; o < N; ++o) acc = fmaf(z[o], W[k * N + o], acc);
-    const float h = H[idx];
-    dZp[idx] = acc * (1.0f - h * h);
-}
-
-// Weight and bias gradients in two deterministic stages.  Stage 1: workgroup
-// c (of S = gridDim.x) sums samples [n c / S, n (c+1) / S) into
-// part[c][k*N + o] = sum X[s][k] dZ[s][o] and part[c][K*N + o] = sum dZ[s][o]
-// (K, N <= 64).  The slice is staged through LDS kWChunk samples at a time
-// (the X and dZ rows of the chunk), and thread t keeps the 4 x 4 outputs
-// k = 4 (t / 16) + i, o = 4 (t % 16) + j in registers, adding the chunk's
-// samples in order: 16 FMAs per pair of 16-byte LDS reads, against a
-// dependent chain of global loads per output before.  Stage 2 (k_sum_split)
-// adds the S rows in order.
-constexpr int kGradSplit = 64;
-constexpr int kWChunk = 32;
-__global__ __launch_bounds__(256) void k_dense_bwd_weight(int64_t n, int K, int N, const float *__restrict__ X,
-                                                          int ldx, const float *__restrict__ dZ,
-                                                          float *__restrict__ part)
-{
-    __shared__ float4 sx[kWChunk][kMlpW / 4];  // X rows of the chunk, zero past K
-    __shared__ float4 sz[kWChunk][kMlpW / 4];  // dZ rows, zero past N
-    const int t = threadIdx.x;
-    const int ty = t >> 4, tx = t & 15;
-    const int c = blockIdx.x, S = gridDim.x;
-    const int64_t s0 = n * c / S, s1 = n * (c + 1) / S;
-    float acc[4][4], bacc = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-    float *fx = reinterpret_cast<float *>(sx), *fz = reinterpret_cast<float *>(sz);
-    for (int64_t b = s0; b < s1; b += kWChunk) {
-        __syncthreads();  // the previous chunk's reads are done
-        for (int q = t; q < kWChunk * kMlpW; q += 256) {
-            const int r = q / kMlpW, k = q % kMlpW;
-            const int64_t smp = b + r;
-            const bool ok = smp < s1;
-            fx[q] = (ok && k < K) ? X[smp * ldx + k] : 0.0f;
-            fz[q] = (ok && k < N) ? dZ[smp * N + k] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int r = 0; r < kWChunk; ++r) {
-            const float4 a = sx[r][ty], z = sz[r][tx];
-            const float av[4] = {a.x, a.y, a.z, a.w}, zv[4] = {z.x, z.y, z.z, z.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], zv[j], acc[i][j]);
-        }
-        if (t < N)
-            for (int r = 0; r < kWChunk; ++r) bacc += fz[r * kMlpW + t];
-    }
-    const int M = K * N + N;
-    float *out = part + (size_t)c * M;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k = 4 * ty + i, o = 4 * tx + j;
-            if (k < K && o < N) out[k * N + o] = acc[i][j];
-        }
-    if (t < N) out[K * N + t] = bacc;
-}
-
-// gW, gb = the sum of the kGradSplit rows of part, in row order (the rows'
-// loads issue together).
-__global__ __launch_bounds__(256) void k_sum_split(int K, int N, const float *__restrict__ part,
-                                                   float *__restrict__ gW, float *__restrict__ gb)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int M = K * N + N;
-    if (t >= M) return;
-    float v[kGradSplit];
-#pragma unroll
-    for (int c = 0; c < kGradSplit; ++c) v[c] = part[(size_t)c * M + t];
-    float acc = 0.0f;
-#pragma unroll
-    for (int c = 0; c < kGradSplit; ++c) acc += v[c];
-    if (t < K * N) gW[t] = acc;
-    else gb[t - K * N] = acc;
+    if (u) return;
+    if (k < kMlpNParam) grad[k] = (float)sh[0][o] + (float)sh[1][o] + (float)sh[2][o] + (float)sh[3][o];
+    else if (k == kMlpNParam) loss[0] = (float)((sh[0][o] + sh[1][o] + sh[2][o] + sh[3][o]) / (double)n);
 }
 
 // Adam (Kingma & Ba 2015), bias-corrected, on np parameters.

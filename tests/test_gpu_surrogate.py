@@ -203,3 +203,32 @@ def test_surrogate_form_rejects_unsupported_settings(gpu):
         assert ex.value.code == -5, kw
         with pytest.raises(engine.PGTError):
             e.bond_samples()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1024, 1025, 8200])
+def test_mlp_gradient_chunks_match_oracle(gpu, n):
+    """Chunks of 16 samples (up to 1,024) and of 32, the last one partly
+    filled, and more chunks than workgroups (8,200).  FP32 sums of up to 8,200
+    terms against FP64, and an output error of a few FP32 roundings: 2e-5 of
+    each block's largest gradient, 1e-5 of the loss."""
+    import torch
+
+    dev = torch.device("cuda:0")
+    print("mlp gradient n=%d" % n, flush=True)
+    rng = np.random.default_rng(n)
+    x = _rows(n, n + 1)
+    t = rng.uniform(0.0, 1.0, n).astype(np.float32)
+    p = surrogate.init_params(7)
+    d = [torch.tensor(a, device=dev) for a in (p, x, t)]
+    g = torch.full((engine.mlp_nparam(),), np.nan, dtype=torch.float32, device=dev)
+    loss = torch.zeros(1, dtype=torch.float32, device=dev)
+    work = torch.empty(engine.mlp_work_floats(n), dtype=torch.float32, device=dev)
+    engine.mlp_grad(d[0], d[1], d[2], g, loss, work)
+    torch.cuda.synchronize()
+    ref_loss, ref = omlp.loss_grad(p, x, t)
+    got = g.cpu().numpy().astype(np.float64)
+    assert abs(float(loss.item()) - ref_loss) <= 1e-5 * abs(ref_loss)
+    at = 0
+    for k in (320, 64, 4096, 64, 4096, 64, 64, 1):
+        assert np.abs(got[at:at + k] - ref[at:at + k]).max() <= 2e-5 * np.abs(ref[at:at + k]).max(), (at, k)
+        at += k
