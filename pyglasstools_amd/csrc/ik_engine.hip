@@ -535,6 +535,7 @@ struct JobShape {
     int D, OD, KN, PS;
     bool pairs, kin, ela, fp32, adaptive;
     Geom g;
+    bool small;  // the cell list of k_sort_small
     int npass, nbits, radix;
     size_t ebytes;
     int block, pl;
@@ -618,6 +619,7 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     j.fp32 = e->prm.precision == PGT_PREC_FP32 && !(j.D == 3 && j.OD == 2);
     j.adaptive = e->prm.quad_mode == PGT_QUAD_ADAPTIVE && j.pairs;
     j.g = make_geom(e, j.D);
+    j.small = n <= kSmallParticles && j.g.ncell <= kSmallCells;
     // radix sort of the cell keys: digits of nbits bits, npass passes
     int kbits = 0;
     while ((1 << kbits) < j.g.ncell) ++kbits;
@@ -738,7 +740,7 @@ size_t work_carve(const JobShape &j, int nf, int64_t n, int64_t G, int cap, unsi
 int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int nf, int64_t n_particles,
                const double *pos, const double *diam, const double *mass, const double *vel, const double *disp,
                unsigned fields, double *ovir, double *okin, double *oela, hipEvent_t ev_begin, hipEvent_t ev_gather,
-               hipEvent_t ev_end, bool bonds_only)
+               hipEvent_t ev_end, bool bonds_only, bool clear)
 {
     const int D = j.D, OD = j.OD;
     const int n = (int)n_particles;
@@ -756,12 +758,20 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     hipStream_t s = e->stream;
     if (ev_begin) HIPCHK(hipEventRecord(ev_begin, s));
     const int *keys = nullptr;  // sorted cell keys
-    // cell list: per pass a histogram, a scan and a scatter of one digit of
-    // the cell keys; frames are dealt to XCDs whole (frame_block)
+    if (clear && !j.small) {  // k_sort_small clears the counters itself
+        if (int rc = fill_async(w.maxcount, 0, 2, s)) return rc;
+        if (int rc = fill_async(w.stats, 0ull, 2, s)) return rc;
+    }
+    // cell list: sorted keys and input indices, by one launch for small frames,
+    // else per pass a histogram, a scan and a scatter of one digit of the cell
+    // keys; frames are dealt to XCDs whole (frame_block)
     {
         const dim3 cgrid((unsigned)nchunk, (unsigned)frame_rows(nf));
         int *kb[2] = {w.get<int>(W_KEYS0), w.get<int>(W_KEYS1)}, *vb[2] = {w.get<int>(W_VALS0), w.get<int>(W_VALS1)};
-        for (int p = 0; p < j.npass; ++p) {
+        if (j.small)
+            hipLaunchKernelGGL(k_sort_small, dim3(nf), dim3(kSmallBlock), 0, s, g, n, g.ncell, pos, kb[j.npass & 1],
+                               vb[j.npass & 1], clear ? w.maxcount : nullptr, clear ? w.stats : nullptr);
+        for (int p = 0; p < j.npass && !j.small; ++p) {
             const int shift = p * j.nbits, radix = j.radix;
             int *kin = kb[p & 1], *vin = vb[p & 1], *kout = kb[(p + 1) & 1], *vout = vb[(p + 1) & 1];
             if (p == 0) {
@@ -899,16 +909,17 @@ struct FrameSet {
     bool bonds_only;  // build the cell and bond lists only (no field gather)
 };
 
-// Launch batch f0 .. f0 + nf - 1 of a job with work arrays w.
+// Launch batch f0 .. f0 + nf - 1 of a job with work arrays w.  clear: zero the
+// job's counters first.
 int run_batch(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, const FrameSet &fs, unsigned fields, int f0,
-              int nf, hipEvent_t e0, hipEvent_t e1, hipEvent_t e2)
+              int nf, bool clear, hipEvent_t e0, hipEvent_t e1, hipEvent_t e2)
 {
     const size_t fsz = (size_t)e->G * j.OD * j.OD;
     const size_t po = (size_t)f0 * fs.n;
     return run_frames(e, j, w, cap, nf, fs.n, fs.pos + po * 3, fs.diam + po, fs.mass ? fs.mass + po : nullptr,
                       fs.vel ? fs.vel + po * 3 : nullptr, fs.disp ? fs.disp + po * 3 : nullptr, fields,
                       fs.vir ? fs.vir + (size_t)f0 * fsz : nullptr, fs.kin ? fs.kin + (size_t)f0 * fsz : nullptr,
-                      fs.ela ? fs.ela + (size_t)f0 * fsz : nullptr, e0, e1, e2, fs.bonds_only);
+                      fs.ela ? fs.ela + (size_t)f0 * fsz : nullptr, e0, e1, e2, fs.bonds_only, clear);
 }
 
 // Run every batch of a job on the engine's stream, then check the bond-list
@@ -926,10 +937,9 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     for (int attempt = 0; attempt < 4; ++attempt) {
         Work w{};
         if ((rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, false, w))) return rc;
-        if ((rc = fill_async(w.maxcount, 0, 2, e->stream)) || (rc = fill_async(w.stats, 0ull, 2, e->stream))) return rc;
         for (int b = 0; b < nb; ++b) {
             const int f0 = b * fpl;
-            rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), e->ev[3 * b],
+            rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), b == 0, e->ev[3 * b],
                            e->ev[3 * b + 1], e->ev[3 * b + 2]);
             if (rc) return rc;
         }
@@ -1011,8 +1021,8 @@ int enqueue_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     if (int rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, true, w)) return rc;
     for (int b = 0; b < nb; ++b) {
         const int f0 = b * fpl;
-        const int rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), nullptr, nullptr,
-                                 nullptr);
+        const int rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), false, nullptr,
+                                 nullptr, nullptr);
         if (rc) return rc;
     }
     return 0;
@@ -1587,9 +1597,9 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
         work_carve(j, nf, n, e->G, cap, e->scratch, &w);
         // counters start at zero on every call (the array keeps the last call's contents)
         int rc;
-        if ((rc = fill_async(w.maxcount, 0, 2, s)) || (rc = fill_async(w.stats, 0ull, 2, s))) return rc;
         for (int f0 = 0; f0 < nframes; f0 += nf)
-            if ((rc = run_batch(e, j, w, cap, fs, fields, f0, std::min(nf, nframes - f0), nullptr, nullptr, nullptr)))
+            if ((rc = run_batch(e, j, w, cap, fs, fields, f0, std::min(nf, nframes - f0), f0 == 0, nullptr, nullptr,
+                                nullptr)))
                 return rc;
         int flags[2] = {0, 0};
         HIPCHK(hipMemcpyAsync(flags, w.maxcount, sizeof(flags), hipMemcpyDeviceToHost, s));

@@ -2,7 +2,8 @@
 // stress-field engine (gfx950).  Included once, by ik_engine.hip; the field
 // gathers live in their own translation units (ik_gather_*.hip).
 //
-//   cell list   k_sort_hist -> k_sort_scan -> k_sort_scatter (per digit), k_sort_finish
+//   cell list   k_sort_hist -> k_sort_scan -> k_sort_scatter (per digit), or k_sort_small;
+//               k_sort_finish
 //   bond list   k_bonds   (ik_bonds.hpp)
 //   fields      k_gather  (ik_gather.hpp); with the adaptive bond integral
 //               k_gather_adaptive (ik_gather_adaptive.hpp)
@@ -185,32 +186,22 @@ __global__ __launch_bounds__(kSortBlock) void k_sort_scatter(int n, int nf, int 
                              kout + fo, vout + fo);
 }
 
-// Write the cell-sorted particle arrays (slot k takes input particle
-// vals[k]) and the cell starts: cstart[c] = first slot of cell c, and
-// cstart[ncell] = n (keys are sorted, so slot k writes the starts of the
-// cells after its predecessor's up to its own).  Positions are wrapped into
-// the box along periodic axes (x - L floor((x - lo) / L): unchanged, bit for
-// bit, inside the box), so a particle sits where its cell says.  In 3D with
-// bonds it also writes each particle's FP32 record (x, y, z; the bond kernel
-// adds the count) for the candidate scans' FP32 pre-tests.
+// Write sorted slot k of a frame's particle arrays from its input particle
+// fi.  Positions are wrapped into the box along periodic axes (x - L floor((x -
+// lo) / L): unchanged, bit for bit, inside the box), so a particle sits where
+// its cell says.  In 3D with bonds it also writes the particle's FP32 record
+// (x, y, z; the bond kernel adds the count) for the lane gather's FP32
+// pre-test.
 template <int D, int OD>
-__device__ __forceinline__ void sort_finish_body(const Geom &g, int n, int k, int ncell, const int *__restrict__ keys,
-                                                 const int *__restrict__ vals, const double *__restrict__ pos,
-                                                 const double *__restrict__ diam, const double *__restrict__ mass,
-                                                 const double *__restrict__ vel, const double *__restrict__ disp,
-                                                 int *__restrict__ st, double *__restrict__ spos,
-                                                 double *__restrict__ sdiam, double *__restrict__ skin,
-                                                 double *__restrict__ sdisp, float4 *__restrict__ rec)
+__device__ __forceinline__ void sorted_particle(const Geom &g, int k, size_t fi, const double *__restrict__ pos,
+                                                const double *__restrict__ diam, const double *__restrict__ mass,
+                                                const double *__restrict__ vel, const double *__restrict__ disp,
+                                                double *__restrict__ spos, double *__restrict__ sdiam,
+                                                double *__restrict__ skin, double *__restrict__ sdisp,
+                                                float4 *__restrict__ rec)
 {
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
-    if (k >= n) return;
-    const int c = keys[k];
-    const int cp = k == 0 ? -1 : keys[k - 1];
-    for (int q = cp + 1; q <= c; ++q) st[q] = k;
-    if (k == n - 1)
-        for (int q = c + 1; q <= ncell; ++q) st[q] = n;
-    const size_t fi = (size_t)vals[k];
     const double *p = pos + fi * 3;
     double *sp = spos + (size_t)k * PS;
     auto wrap = [&](int a) {
@@ -219,8 +210,6 @@ __device__ __forceinline__ void sort_finish_body(const Geom &g, int n, int k, in
     sp[0] = wrap(0);
     sp[1] = wrap(1);
     if (D == 3) { sp[2] = wrap(2); sp[3] = 0.0; }
-    // 3D with bonds: the FP32 record of the candidate scans (its last word,
-    // the bond count, is filled in by the bond kernel)
     if (D == 3 && rec) rec[k] = make_float4((float)sp[0], (float)sp[1], (float)sp[2], 0.0f);
     sdiam[k] = diam[fi];
     if (skin) {
@@ -235,6 +224,28 @@ __device__ __forceinline__ void sort_finish_body(const Geom &g, int n, int k, in
     }
     if (sdisp)
         for (int a = 0; a < 3; ++a) sdisp[(size_t)k * 3 + a] = disp ? disp[fi * 3 + a] : 0.0;
+}
+
+// Write the cell-sorted particle arrays (slot k takes input particle
+// vals[k]) and the cell starts: cstart[c] = first slot of cell c, and
+// cstart[ncell] = n (keys are sorted, so slot k writes the starts of the
+// cells after its predecessor's up to its own).
+template <int D, int OD>
+__device__ __forceinline__ void sort_finish_body(const Geom &g, int n, int k, int ncell, const int *__restrict__ keys,
+                                                 const int *__restrict__ vals, const double *__restrict__ pos,
+                                                 const double *__restrict__ diam, const double *__restrict__ mass,
+                                                 const double *__restrict__ vel, const double *__restrict__ disp,
+                                                 int *__restrict__ st, double *__restrict__ spos,
+                                                 double *__restrict__ sdiam, double *__restrict__ skin,
+                                                 double *__restrict__ sdisp, float4 *__restrict__ rec)
+{
+    if (k >= n) return;
+    const int c = keys[k];
+    const int cp = k == 0 ? -1 : keys[k - 1];
+    for (int q = cp + 1; q <= c; ++q) st[q] = k;
+    if (k == n - 1)
+        for (int q = c + 1; q <= ncell; ++q) st[q] = n;
+    sorted_particle<D, OD>(g, k, (size_t)vals[k], pos, diam, mass, vel, disp, spos, sdiam, skin, sdisp, rec);
 }
 
 template <int D, int OD>
@@ -256,6 +267,101 @@ __global__ __launch_bounds__(256) void k_sort_finish(Geom g, int n, int nf, int 
                             disp ? disp + fo * 3 : nullptr, cstart + (size_t)f * (ncell + 1), spos + fo * PS,
                             sdiam + fo, skin ? skin + fo * KN : nullptr, sdisp ? sdisp + fo * 3 : nullptr,
                             rec ? rec + fo : nullptr);
+}
+
+// ------------------------------------------------------------------------
+// cell list of small frames: one workgroup per frame, counts and order in LDS
+// ------------------------------------------------------------------------
+// A counting sort by cell: cell sizes by LDS atomics, their scan, then every
+// particle takes a slot of its cell in whatever order the atomics give, and
+// finally counts the particles of its cell with a lower input index, which is
+// its place: the radix sort's keys and values from one launch instead of six.
+// Those launches, a few microseconds each whatever their size, were a third
+// of a small frame's time on the GPU: N = 2,000 6 us against 20 in six kernels
+// (and their gaps), N = 4,000 10 us; a driver call on them 147 -> 125 and 194 ->
+// 173 us.  With clear0 and clear1 not null the first workgroup also zeroes
+// the job's counters.
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallParticles = 8192;  // most particles of a frame, eight per thread
+constexpr int kSmallCells = 8192;      // most cells (32 KB of LDS each for cells and particles)
+
+__global__ __launch_bounds__(kSmallBlock) void k_sort_small(Geom g, int n, int ncell, const double *__restrict__ pos,
+                                                            int *__restrict__ keys, int *__restrict__ vals,
+                                                            int *__restrict__ clear0,
+                                                            unsigned long long *__restrict__ clear1)
+{
+    constexpr int PER = kSmallParticles / kSmallBlock, CPT = kSmallCells / kSmallBlock;
+    __shared__ int s_cell[kSmallCells];  // counts, then each cell's next slot
+    __shared__ int s_order[kSmallParticles];
+    __shared__ int s_wave[kSmallBlock / 64];
+    const int t = threadIdx.x, f = blockIdx.x;
+    const size_t fo = (size_t)f * n;
+    pos += fo * 3;
+    keys += fo;
+    vals += fo;
+    if (f == 0 && t < 2 && clear0) {
+        clear0[t] = 0;
+        clear1[t] = 0ull;
+    }
+    double x[PER][3];  // the frame's positions, in flight together
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (u * kSmallBlock >= n) continue;
+        const double *p = pos + (size_t)min(u * kSmallBlock + t, n - 1) * 3;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) x[u][a] = p[a];
+    }
+    for (int c = t; c < ncell; c += kSmallBlock) s_cell[c] = 0;
+    __syncthreads();
+    int key[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        key[u] = -1;
+        if (u * kSmallBlock + t < n) {
+            key[u] = cell_of(g, x[u]);
+            atomicAdd(&s_cell[key[u]], 1);
+        }
+    }
+    __syncthreads();
+    // exclusive scan of the counts, `per` consecutive cells per thread
+    const int per = (ncell + kSmallBlock - 1) / kSmallBlock;
+    int own[CPT], sum = 0;
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        own[q] = q < per && t * per + q < ncell ? s_cell[t * per + q] : 0;
+        sum += own[q];
+    }
+    int v = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int w = __shfl_up(v, off, 64);
+        if ((t & 63) >= off) v += w;
+    }
+    if ((t & 63) == 63) s_wave[t >> 6] = v;
+    __syncthreads();
+    int run = v - sum;
+#pragma unroll
+    for (int w = 0; w < kSmallBlock / 64; ++w) run += w < (t >> 6) ? s_wave[w] : 0;
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        if (q < per && t * per + q < ncell) s_cell[t * per + q] = run;
+        run += own[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u)
+        if (key[u] >= 0) s_order[atomicAdd(&s_cell[key[u]], 1)] = u * kSmallBlock + t;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (key[u] < 0) continue;
+        const int i = u * kSmallBlock + t;
+        const int begin = key[u] ? s_cell[key[u] - 1] : 0, end = s_cell[key[u]];
+        int k = begin;
+        for (int q = begin; q < end; ++q) k += s_order[q] < i ? 1 : 0;
+        keys[k] = key[u];
+        vals[k] = i;
+    }
 }
 
 // Clears that a captured HIP graph can hold (a memset node is avoided there).

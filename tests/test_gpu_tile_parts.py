@@ -187,3 +187,37 @@ def test_adaptive_shapes_match_the_oracle(gpu, dim, side, fields, cg):
             print("  %s: max scaled err %.2e" % (k, err), flush=True)
             assert err <= 1e-8, (k, err)
     assert st["n_ball"] == ball
+
+
+@pytest.mark.parametrize("N,nf,keep,lengths", [(1, 1, 1.0, None), (1023, 1, 1.0, None), (1025, 3, 1.0, None),
+                                               (8192, 2, 1.0, None), (8193, 1, 1.0, None), (33000, 1, 0.2, None),
+                                               (39000, 1, 0.2, None), (900, 1, 1.0, (4.2, 220.0, 1.0))])
+def test_small_frames_match_the_oracle(gpu, N, nf, keep, lengths):
+    """Frames on both sides of the one-launch cell list's limits (8,192
+    particles, 8,192 cells: dilute boxes of 7,921 and 9,409 cells), one cell
+    with most of the particles (a strip), several frames.  FP64 drop-in bar."""
+    frames = []
+    for f in range(nf):
+        s = workload.make_system(max(N, 30), 2, 9800 + f)
+        n = max(1, int(N * keep))
+        s = dict(s, **{k: s[k][:n].copy() for k in ("pos", "diam", "mass", "vel")})
+        if lengths is not None:
+            s["pos"][:, :2] *= np.array(lengths[:2]) / s["L"][0]
+            s["pos"][: n * 3 // 4, 1] *= 0.02
+            s["L"] = np.array(lengths)
+        frames.append(s)
+    L = frames[0]["L"]
+    grid = np.stack([a.ravel() for a in np.meshgrid(np.linspace(-0.5, 0.5, 12) * L[0], np.linspace(-0.5, 0.5, 12) * L[1],
+                                                    [0.0], indexing="ij")], axis=1)
+    print("small frames N=%d x %d keep %.1f" % (N, nf, keep), flush=True)
+    e = engine.Engine(dim=2, max_rcut=1.25 * 1.62)
+    e.set_box(L, [1, 1, 0])
+    e.set_grid(grid)
+    got, st = _frames(e, frames, ("virial", "kinetic"))
+    contrib = 0
+    for f, s in enumerate(frames):
+        ref = oracle.ik_compute(s, grid, fields=("virial", "kinetic"), max_rcut=1.25 * 1.62, with_abs=True)
+        contrib += ref["n_nonzero"]
+        assert scaled_error(got["virial"][f], ref["virial"], ref["virial_abs"]).max() <= 1e-10
+        assert np.abs(got["kinetic"][f] - ref["kinetic"]).max() <= 1e-10 * max(np.abs(ref["kinetic"]).max(), 1e-300)
+    assert st["n_contrib"] == contrib
