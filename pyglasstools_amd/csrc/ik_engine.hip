@@ -188,6 +188,36 @@ struct GridOrder {
     double step[3] = {0.0, 0.0, 0.0};  // of the lattice
 };
 
+// The bits of a site number, a place apart for the other axis of a 2D Morton
+// key (16 bits) or two for the others of a 3D one (10 bits).
+uint32_t spread_bits(uint32_t x, bool three)
+{
+    if (three) {
+        x = (x | x << 16) & 0x030000ffu;
+        x = (x | x << 8) & 0x0300f00fu;
+        x = (x | x << 4) & 0x030c30c3u;
+        return (x | x << 2) & 0x09249249u;
+    }
+    x = (x | x << 8) & 0x00ff00ffu;
+    x = (x | x << 4) & 0x0f0f0f0fu;
+    x = (x | x << 2) & 0x33333333u;
+    return (x | x << 1) & 0x55555555u;
+}
+
+// perm (0, 1, ...) by ascending key, equal keys in order: a radix sort of the
+// key bits in use, 11 at a time.
+void sort_by_key(const std::vector<uint32_t> &key, uint32_t used_bits, std::vector<int> &perm)
+{
+    std::vector<int> other(perm.size());
+    for (int shift = 0; shift < 32 && used_bits >> shift; shift += 11) {
+        size_t start[2049] = {};
+        for (int i : perm) ++start[((key[(size_t)i] >> shift) & 2047u) + 1];
+        for (int b = 0; b < 2048; ++b) start[b + 1] += start[b];
+        for (int i : perm) other[start[(key[(size_t)i] >> shift) & 2047u]++] = i;
+        perm.swap(other);
+    }
+}
+
 GridOrder order_grid(int64_t G, const double *grid, bool use_z)
 {
     GridOrder o;
@@ -207,17 +237,17 @@ GridOrder order_grid(int64_t G, const double *grid, bool use_z)
     for (int a = 0; a < 3; ++a) o.step[a] = h[a] = std::max(hi[a] - lo[a], 1e-300) / (nside - 1.0);
     const int bits = use_z ? 10 : 16;
     const double qmax = (double)((1u << bits) - 1);
-    std::vector<uint64_t> key((size_t)G);
+    std::vector<uint32_t> key((size_t)G);
+    uint32_t used_bits = 0;
     for (int64_t i = 0; i < G; ++i) {
-        uint64_t k = 0;
-        uint32_t q[3] = {0, 0, 0};
+        uint32_t k = 0;
         for (int a = 0; a < d; ++a)
-            q[a] = (uint32_t)std::min(qmax, std::max(0.0, std::floor((grid[3 * i + a] - lo[a]) / h[a] + 0.5)));
-        for (int b = bits - 1; b >= 0; --b)
-            for (int a = d - 1; a >= 0; --a) k = (k << 1) | ((q[a] >> b) & 1u);
+            k |= spread_bits((uint32_t)std::min(qmax, std::max(0.0, std::floor((grid[3 * i + a] - lo[a]) / h[a] + 0.5))),
+                             use_z) << a;
         key[(size_t)i] = k;
+        used_bits |= k;
     }
-    std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return key[(size_t)x] < key[(size_t)y]; });
+    sort_by_key(key, used_bits, perm);
     const int side = use_z ? 4 : 8;  // sites of a block along an axis
     for (int64_t t0 = 0, t1; t0 < G; t0 = t1) {
         for (t1 = t0 + 1; t1 < G && t1 - t0 < kTilePoints && key[(size_t)perm[t1]] >> 6 == key[(size_t)perm[t0]] >> 6;)
@@ -229,7 +259,7 @@ GridOrder order_grid(int64_t G, const double *grid, bool use_z)
         uint64_t used = 0;
         bool product = true;
         for (int64_t t = t0; t < t1 && product; ++t) {
-            const uint64_t k = key[(size_t)perm[t]];
+            const uint32_t k = key[(size_t)perm[t]];
             int at[3] = {0, 0, 0};  // the site in its block: the key's low 6 bits, de-interleaved
             for (int b = 0; b < 6; ++b) at[b % d] |= (int)((k >> b) & 1u) << (b / d);
             const int j = use_z ? ((at[2] >> 1) * 2 + (at[1] >> 1)) * 16 + (at[2] & 1) * 8 + (at[1] & 1) * 4 + at[0]
@@ -351,6 +381,11 @@ struct pgt_ik_engine {
     // pinned host copy of a job's counters (flags, then the two totals), read
     // back with one synchronisation per job
     unsigned long long *h_counts = nullptr;
+    // pinned host memory for a frame's arrays (stage_for); stage_busy: an
+    // upload that reads it may still be under way
+    double *h_stage = nullptr;
+    size_t stage_bytes = 0;
+    bool stage_busy = false;
     pgt_ik_stats stats{};
 };
 
@@ -398,6 +433,37 @@ int fail_held()
     return fail(PGT_ERR_STATE, "device buffers are held by enqueued work that a captured graph may replay: call "
                                "pgt_ik_release_enqueued before a call that would regrow or replace them, and capture "
                                "again afterwards");
+}
+
+// A frame's arrays of at most this much go through pinned memory of the
+// engine's and a copy kernel, without a synchronisation of their own, larger
+// ones by the runtime's copies of the caller's pageable arrays.  set_particles
+// and compute together, pageable -> staged: N = 2,000 with a 32 x 32 grid
+// (125 + 64 KB) 115 -> 78 us, 16,000 with 180 x 180 (1 + 2 MB) 261 -> 223,
+// 65,536 with 256 x 256 (4 + 4 MB) 538 -> 492.  The gain goes on above (16 MB in:
+// 881 -> 787); the line bounds the pinned memory that an engine holds.
+constexpr size_t kStageBytes = (size_t)8 << 20;
+
+// The staging memory for `bytes`, or null: too large, or none to be had.
+double *stage_for(pgt_ik_engine *e, size_t bytes)
+{
+    if (bytes > kStageBytes) return nullptr;
+    if (bytes > e->stage_bytes) {
+        if (e->stage_busy && hipStreamSynchronize(e->stream) != hipSuccess) return nullptr;
+        e->stage_busy = false;
+        if (e->h_stage) (void)hipHostFree(e->h_stage);
+        e->h_stage = nullptr;
+        e->stage_bytes = 0;
+        size_t want = (size_t)256 << 10;
+        while (want < bytes) want *= 2;
+        if (hipHostMalloc((void **)&e->h_stage, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            e->h_stage = nullptr;
+            return nullptr;
+        }
+        e->stage_bytes = want;
+    }
+    return e->h_stage;
 }
 
 int ensure_events(pgt_ik_engine *e, size_t want)
@@ -736,11 +802,43 @@ size_t work_carve(const JobShape &j, int nf, int64_t n, int64_t G, int cap, unsi
     return off;
 }
 
+// What a job's last launch writes into pinned host memory: its counters, and
+// copies of small outputs.
+struct Deliver {
+    unsigned long long *counts;
+    CopySegs out;
+};
+
+// k_reduce_stats of a batch; with dv, the job's last one.
+int reduce_stats(int nrb, int nw, const unsigned long long *wave_counts, int nm, const int *wmax,
+                 unsigned long long *stats, int *maxcount, const Deliver *dv, hipStream_t s)
+{
+    constexpr int kCopyBlocks = 64;  // of 1024 threads: 512 KB in one pass
+    unsigned long long *hc = dv ? dv->counts : nullptr;
+    const CopySegs out = dv ? dv->out : CopySegs{};
+    int most = 0;
+    for (int k = 0; k < 5; ++k) most = std::max(most, out.n[k]);
+    const int ncopy = std::min(kCopyBlocks, (most + 1023) / 1024);
+    if (nrb > 1) {
+        hipLaunchKernelGGL(k_reduce_stats, dim3(nrb), dim3(1024), 0, s, nrb, nw, wave_counts, nm, wmax, stats, maxcount,
+                           (unsigned long long *)nullptr, CopySegs{});
+        nw = nm = 0;
+        if (!dv) {
+            HIPCHK(hipGetLastError());
+            return 0;
+        }
+    }
+    hipLaunchKernelGGL(k_reduce_stats, dim3(1 + ncopy), dim3(1024), 0, s, 1, nw, wave_counts, nm, wmax, stats, maxcount,
+                       hc, out);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 // Launch the cell list, bond list and gather for nf frames (no host sync).
 int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int nf, int64_t n_particles,
                const double *pos, const double *diam, const double *mass, const double *vel, const double *disp,
                unsigned fields, double *ovir, double *okin, double *oela, hipEvent_t ev_begin, hipEvent_t ev_gather,
-               hipEvent_t ev_end, bool bonds_only, bool clear)
+               hipEvent_t ev_end, bool bonds_only, bool clear, const Deliver *dv)
 {
     const int D = j.D, OD = j.OD;
     const int n = (int)n_particles;
@@ -758,10 +856,8 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     hipStream_t s = e->stream;
     if (ev_begin) HIPCHK(hipEventRecord(ev_begin, s));
     const int *keys = nullptr;  // sorted cell keys
-    if (clear && !j.small) {  // k_sort_small clears the counters itself
-        if (int rc = fill_async(w.maxcount, 0, 2, s)) return rc;
-        if (int rc = fill_async(w.stats, 0ull, 2, s)) return rc;
-    }
+    int *const clear_max = clear ? w.maxcount : nullptr;  // cleared by the first launch
+    unsigned long long *const clear_stats = clear ? w.stats : nullptr;
     // cell list: sorted keys and input indices, by one launch for small frames,
     // else per pass a histogram, a scan and a scatter of one digit of the cell
     // keys; frames are dealt to XCDs whole (frame_block)
@@ -770,19 +866,19 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         int *kb[2] = {w.get<int>(W_KEYS0), w.get<int>(W_KEYS1)}, *vb[2] = {w.get<int>(W_VALS0), w.get<int>(W_VALS1)};
         if (j.small)
             hipLaunchKernelGGL(k_sort_small, dim3(nf), dim3(kSmallBlock), 0, s, g, n, g.ncell, pos, kb[j.npass & 1],
-                               vb[j.npass & 1], clear ? w.maxcount : nullptr, clear ? w.stats : nullptr);
+                               vb[j.npass & 1], clear_max, clear_stats);
         for (int p = 0; p < j.npass && !j.small; ++p) {
             const int shift = p * j.nbits, radix = j.radix;
             int *kin = kb[p & 1], *vin = vb[p & 1], *kout = kb[(p + 1) & 1], *vout = vb[(p + 1) & 1];
             if (p == 0) {
                 hipLaunchKernelGGL(k_sort_hist<true>, cgrid, dim3(kSortBlock), 0, s, g, n, nf, shift, radix, pos, kin,
-                                   hist);
+                                   hist, clear_max, clear_stats);
                 hipLaunchKernelGGL(k_sort_scan, dim3(nf), dim3(1024), 0, s, radix * nchunk, hist);
                 hipLaunchKernelGGL(k_sort_scatter<true>, cgrid, dim3(kSortBlock), 0, s, n, nf, shift, radix, kin, vin,
                                    hist, kout, vout);
             } else {
                 hipLaunchKernelGGL(k_sort_hist<false>, cgrid, dim3(kSortBlock), 0, s, g, n, nf, shift, radix, pos,
-                                   kin, hist);
+                                   kin, hist, (int *)nullptr, (unsigned long long *)nullptr);
                 hipLaunchKernelGGL(k_sort_scan, dim3(nf), dim3(1024), 0, s, radix * nchunk, hist);
                 hipLaunchKernelGGL(k_sort_scatter<false>, cgrid, dim3(kSortBlock), 0, s, n, nf, shift, radix, kin,
                                    vin, hist, kout, vout);
@@ -894,10 +990,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     if (ev_end) HIPCHK(hipEventRecord(ev_end, s));
     const int nwg = bonds_only ? 0 : nw_gather;
     const int nrb = std::max(1, std::min(256, (std::max(nwg, nw_bonds) + 4095) / 4096));
-    hipLaunchKernelGGL(k_reduce_stats, dim3(nrb), dim3(1024), 0, s, nwg, c.out.wave_counts, nw_bonds, wmax, w.stats,
-                       w.maxcount);
-    HIPCHK(hipGetLastError());
-    return 0;
+    return reduce_stats(nrb, nwg, c.out.wave_counts, nw_bonds, wmax, w.stats, w.maxcount, dv, s);
 }
 
 struct FrameSet {
@@ -907,19 +1000,20 @@ struct FrameSet {
     double *vir, *kin, *ela;  // device outputs, nframes * G * D * D each
     bool z_flat;
     bool bonds_only;  // build the cell and bond lists only (no field gather)
+    CopySegs host;    // outputs that the last launch copies to pinned host memory
 };
 
 // Launch batch f0 .. f0 + nf - 1 of a job with work arrays w.  clear: zero the
 // job's counters first.
 int run_batch(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, const FrameSet &fs, unsigned fields, int f0,
-              int nf, bool clear, hipEvent_t e0, hipEvent_t e1, hipEvent_t e2)
+              int nf, bool clear, hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, const Deliver *dv)
 {
     const size_t fsz = (size_t)e->G * j.OD * j.OD;
     const size_t po = (size_t)f0 * fs.n;
     return run_frames(e, j, w, cap, nf, fs.n, fs.pos + po * 3, fs.diam + po, fs.mass ? fs.mass + po : nullptr,
                       fs.vel ? fs.vel + po * 3 : nullptr, fs.disp ? fs.disp + po * 3 : nullptr, fields,
                       fs.vir ? fs.vir + (size_t)f0 * fsz : nullptr, fs.kin ? fs.kin + (size_t)f0 * fsz : nullptr,
-                      fs.ela ? fs.ela + (size_t)f0 * fsz : nullptr, e0, e1, e2, fs.bonds_only, clear);
+                      fs.ela ? fs.ela + (size_t)f0 * fsz : nullptr, e0, e1, e2, fs.bonds_only, clear, dv);
 }
 
 // Run every batch of a job on the engine's stream, then check the bond-list
@@ -933,6 +1027,7 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
     if ((rc = e->d_maxcount.ensure(2)) || (rc = e->d_stats.ensure(2))) return rc;
     if (j.pairs && e->cap < 1) e->cap = j.D == 3 ? 32 : 16;
+    const Deliver dv{e->h_counts, fs.host};
     int mx = 0;
     for (int attempt = 0; attempt < 4; ++attempt) {
         Work w{};
@@ -940,16 +1035,13 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
         for (int b = 0; b < nb; ++b) {
             const int f0 = b * fpl;
             rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), b == 0, e->ev[3 * b],
-                           e->ev[3 * b + 1], e->ev[3 * b + 2]);
+                           e->ev[3 * b + 1], e->ev[3 * b + 2], b == nb - 1 ? &dv : nullptr);
             if (rc) return rc;
         }
-        // flags and totals into pinned memory, one synchronisation
-        int *hf = reinterpret_cast<int *>(e->h_counts);
-        HIPCHK(hipMemcpyAsync(hf, e->d_maxcount.p, 2 * sizeof(int), hipMemcpyDeviceToHost, e->stream));
-        HIPCHK(hipMemcpyAsync(e->h_counts + 1, e->d_stats.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                              e->stream));
+        // flags and totals are in pinned memory then
         HIPCHK(hipStreamSynchronize(e->stream));
-        const int flags[2] = {hf[0], hf[1]};
+        e->stage_busy = false;
+        const int flags[2] = {(int)(e->h_counts[0] & 0xffffffffu), (int)(e->h_counts[0] >> 32)};
         mx = flags[0];
         const bool grow = j.pairs && mx > e->cap;
         if (grow && mx > 65535) return fail(PGT_ERR_RANGE, "a particle has more than 65535 interacting neighbours");
@@ -1022,7 +1114,7 @@ int enqueue_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     for (int b = 0; b < nb; ++b) {
         const int f0 = b * fpl;
         const int rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), false, nullptr,
-                                 nullptr, nullptr);
+                                 nullptr, nullptr, nullptr);
         if (rc) return rc;
     }
     return 0;
@@ -1219,6 +1311,7 @@ void pgt_ik_destroy(pgt_ik_engine *e)
     e->d_stats.release();
     for (hipEvent_t v : e->ev) (void)hipEventDestroy(v);
     if (e->h_counts) (void)hipHostFree(e->h_counts);
+    if (e->h_stage) (void)hipHostFree(e->h_stage);
     if (e->own_stream) (void)hipStreamDestroy(e->own_stream);
     delete e;
 }
@@ -1258,22 +1351,54 @@ int pgt_ik_set_particles(pgt_ik_engine *e, int64_t n, const double *pos, const d
     e->have_mass = mass != nullptr;
     e->have_vel = vel != nullptr;
     e->have_disp = disp != nullptr;
+    bool staged = false;
     if (n > 0) {
-        // straight from the caller's (pageable) arrays: the runtime stages
-        // them through its own pinned buffers with the copies pipelined,
-        // which measured faster than one host copy into pinned memory of
-        // ours followed by the DMA
         const double *src[5] = {pos, diam, mass, vel, disp};
         double *dst[5] = {e->d_pos.p, e->d_diam.p, e->d_mass.p, e->d_vel.p, e->d_disp.p};
         const size_t cnt[5] = {3, 1, 1, 3, 3};
-        for (int k = 0; k < 5; ++k)
-            if (src[k])
-                HIPCHK(hipMemcpyAsync(dst[k], src[k], sizeof(double) * cnt[k] * (size_t)n, hipMemcpyHostToDevice, s));
+        size_t per = 0;
+        for (int k = 0; k < 5; ++k) per += src[k] ? cnt[k] : 0;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(s, &cap));
+        if (cap != hipStreamCaptureStatusNone)
+            return fail(PGT_ERR_HIP, "the stream is capturing a graph: particles are uploaded outside of it");
+        if (double *h = stage_for(e, sizeof(double) * per * (size_t)n)) {
+            if (e->stage_busy) HIPCHK(hipStreamSynchronize(s));
+            e->stage_busy = staged = true;
+            // a launch per 512 KB or more, so that the transfer of one array
+            // runs beside the host copy of the next
+            CopySegs c{};
+            int most = 0, last = 4;
+            size_t held = 0;
+            while (!src[last]) --last;
+            for (int k = 0; k <= last; ++k) {
+                if (src[k]) {
+                    c.src[k] = h;
+                    c.dst[k] = dst[k];
+                    c.n[k] = (int)cnt[k] * (int)n;
+                    std::memcpy(h, src[k], sizeof(double) * (size_t)c.n[k]);
+                    h += c.n[k];
+                    held += (size_t)c.n[k];
+                    most = std::max(most, c.n[k]);
+                }
+                if (k == last || held >= (size_t)65536) {
+                    hipLaunchKernelGGL(k_copy_segs, dim3((unsigned)((most + 255) / 256)), dim3(256), 0, s, c);
+                    HIPCHK(hipGetLastError());
+                    c = CopySegs{};
+                    held = 0;
+                    most = 0;
+                }
+            }
+        } else {
+            for (int k = 0; k < 5; ++k)
+                if (src[k])
+                    HIPCHK(hipMemcpyAsync(dst[k], src[k], sizeof(double) * cnt[k] * (size_t)n, hipMemcpyHostToDevice, s));
+        }
     }
     bool flat = true;
     for (int64_t i = 0; i < n && flat; ++i) flat = pos[3 * i + 2] == 0.0;
     e->z_flat = flat;
-    HIPCHK(hipStreamSynchronize(s));
+    if (!staged) HIPCHK(hipStreamSynchronize(s));
     e->n = n;
     e->have_particles = true;
     return PGT_OK;
@@ -1403,6 +1528,7 @@ int pgt_ik_set_stream(pgt_ik_engine *e, void *hip_stream)
 {
     if (int rc = check_engine(e)) return rc;
     HIPCHK(hipStreamSynchronize(e->stream));
+    e->stage_busy = false;
     e->stream = hip_stream ? (hipStream_t)hip_stream : e->own_stream;
     return PGT_OK;
 }
@@ -1483,11 +1609,28 @@ int pgt_ik_compute(pgt_ik_engine *e, unsigned fields, double *virial, double *ki
     fs.kin = e->d_out.p + fsz;
     fs.ela = e->d_out.p + 2 * fsz;
     fs.z_flat = e->z_flat && e->grid_z_flat;
-    if ((rc = run_job(e, fs, fields))) return rc;
-    // straight into the caller's arrays (see pgt_ik_set_particles)
     const unsigned bits[3] = {PGT_FIELD_VIRIAL, PGT_FIELD_KINETIC, PGT_FIELD_ELASTIC};
     const double *dsrc[3] = {fs.vir, fs.kin, fs.ela};
     double *hdst[3] = {virial, kinetic, elastic};
+    size_t nout = 0;
+    for (int k = 0; k < 3; ++k) nout += (fields & bits[k]) ? fsz : 0;
+    if (double *h = stage_for(e, nout * sizeof(double))) {
+        // (an upload still under way reads the memory before the job's last
+        // launch writes it; outputs in two halves, one crossing the bus while
+        // the host copies the other, gained nothing below 8 MB)
+        for (int k = 0; k < 3; ++k) {
+            if (!(fields & bits[k])) continue;
+            fs.host.src[k] = dsrc[k];
+            fs.host.dst[k] = h;
+            fs.host.n[k] = (int)fsz;
+            h += fsz;
+        }
+        if ((rc = run_job(e, fs, fields))) return rc;
+        for (int k = 0; k < 3; ++k)
+            if (fields & bits[k]) std::memcpy(hdst[k], fs.host.dst[k], fsz * sizeof(double));
+        return PGT_OK;
+    }
+    if ((rc = run_job(e, fs, fields))) return rc;
     for (int k = 0; k < 3; ++k)
         if (fields & bits[k])
             HIPCHK(hipMemcpyAsync(hdst[k], dsrc[k], fsz * sizeof(double), hipMemcpyDeviceToHost, e->stream));
@@ -1582,6 +1725,7 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
     int cap = e->scratch_cap;
     if (j.pairs && cap < 1) cap = j.D == 3 ? 32 : 16;
     if (!j.pairs) cap = 1;
+    const Deliver dv{e->h_counts, {}};
     int mx = 0;
     unsigned long long h[2] = {0, 0};
     for (int attempt = 0; attempt < 3; ++attempt) {
@@ -1599,12 +1743,12 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
         int rc;
         for (int f0 = 0; f0 < nframes; f0 += nf)
             if ((rc = run_batch(e, j, w, cap, fs, fields, f0, std::min(nf, nframes - f0), f0 == 0, nullptr, nullptr,
-                                nullptr)))
+                                nullptr, f0 + nf >= nframes ? &dv : nullptr)))
                 return rc;
-        int flags[2] = {0, 0};
-        HIPCHK(hipMemcpyAsync(flags, w.maxcount, sizeof(flags), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(h, w.stats, sizeof(h), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
+        const int flags[2] = {(int)(e->h_counts[0] & 0xffffffffu), (int)(e->h_counts[0] >> 32)};
+        h[0] = e->h_counts[1];
+        h[1] = e->h_counts[2];
         mx = flags[0];
         if (flags[1] & 1)
             return fail(PGT_ERR_RANGE, "an adaptive bond integral needed more than " + std::to_string(kQagMax) +
@@ -1918,6 +2062,7 @@ struct pgt_ik_sweep {
     DBuf<unsigned char> d_bonds, d_wcounts, d_wmax, d_rec;
     DBuf<int> d_maxcount;                // [0] largest bond count, [1] tile overflow bits
     DBuf<unsigned long long> d_stats;    // balls, contributions
+    unsigned long long *h_counts = nullptr;  // pinned: the counters of a run
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     pgt_ik_stats stats{};
 };
@@ -1961,10 +2106,12 @@ int sweep_buffers(pgt_ik_sweep *s)
     return s->d_stats.ensure(2);
 }
 
-// Every launch of the sweep on its stream, no host synchronisation.  With
-// timed, events around the whole and around the gather.
-int sweep_launch(pgt_ik_sweep *s, bool timed)
+// Every launch of the sweep on its stream, no host synchronisation.  With run
+// (pgt_ik_sweep_run) events around the whole and around the gather, and
+// counters that start at zero and end in pinned memory.
+int sweep_launch(pgt_ik_sweep *s, bool run)
 {
+    const bool timed = run;
     hipStream_t st = s->stream;
     const SweepSys *T = s->d_tab.p;
     const int ns = s->ns;
@@ -1977,12 +2124,14 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
         const int shift = p * s->nbits, radix = s->radix;
         int *kin = kb[p & 1], *vin = vb[p & 1], *kout = kb[(p + 1) & 1], *vout = vb[(p + 1) & 1];
         if (p == 0) {
-            hipLaunchKernelGGL(k_sweep_hist<true>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, hist);
+            hipLaunchKernelGGL(k_sweep_hist<true>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, hist,
+                               run ? s->d_maxcount.p : nullptr, run ? s->d_stats.p : nullptr);
             hipLaunchKernelGGL(k_sweep_scan, dim3((unsigned)s->nframes), dim3(1024), 0, st, T, ns, radix, hist);
             hipLaunchKernelGGL(k_sweep_scatter<true>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, vin,
                                hist, kout, vout);
         } else {
-            hipLaunchKernelGGL(k_sweep_hist<false>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, hist);
+            hipLaunchKernelGGL(k_sweep_hist<false>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, hist,
+                               (int *)nullptr, (unsigned long long *)nullptr);
             hipLaunchKernelGGL(k_sweep_scan, dim3((unsigned)s->nframes), dim3(1024), 0, st, T, ns, radix, hist);
             hipLaunchKernelGGL(k_sweep_scatter<false>, sg, dim3(kSortBlock), 0, st, T, ns, shift, radix, kin, vin,
                                hist, kout, vout);
@@ -2037,10 +2186,8 @@ int sweep_launch(pgt_ik_sweep *s, bool timed)
     if (timed) HIPCHK(hipEventRecord(s->ev[2], st));
     const int nwg = s->blocks[SW_GATHER], nwb = s->vir ? s->blocks[SW_BONDS] : 0;
     const int nrb = std::max(1, std::min(256, (std::max(nwg, nwb) + 4095) / 4096));
-    hipLaunchKernelGGL(k_reduce_stats, dim3(nrb), dim3(1024), 0, st, nwg, c.wave_counts, nwb, wmax, s->d_stats.p,
-                       s->d_maxcount.p);
-    HIPCHK(hipGetLastError());
-    return 0;
+    const Deliver dv{s->h_counts, {}};
+    return reduce_stats(nrb, nwg, c.wave_counts, nwb, wmax, s->d_stats.p, s->d_maxcount.p, run ? &dv : nullptr, st);
 }
 
 int sweep_flags_error(int flags1)
@@ -2201,6 +2348,10 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
     }
     if (hipMemcpy(s->d_tab.p, s->tab.data(), sizeof(SweepSys) * (size_t)nsys, hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(PGT_ERR_HIP, "uploading the sweep's table"));
+    if (hipHostMalloc((void **)&s->h_counts, 4 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+        s->h_counts = nullptr;
+        return bail(fail(PGT_ERR_HIP, "hipHostMalloc"));
+    }
     if (hipStreamCreate(&s->own_stream) != hipSuccess) return bail(fail(PGT_ERR_HIP, "hipStreamCreate"));
     s->stream = hip_stream ? (hipStream_t)hip_stream : s->own_stream;
     for (auto &v : s->ev)
@@ -2225,6 +2376,7 @@ void pgt_ik_sweep_destroy(pgt_ik_sweep *s)
     s->d_stats.release();
     for (hipEvent_t v : s->ev)
         if (v) (void)hipEventDestroy(v);
+    if (s->h_counts) (void)hipHostFree(s->h_counts);
     if (s->own_stream) (void)hipStreamDestroy(s->own_stream);
     delete s;
 }
@@ -2236,12 +2388,9 @@ int pgt_ik_sweep_run(pgt_ik_sweep *s)
     for (int attempt = 0; attempt < 4; ++attempt) {
         int rc;
         if ((rc = sweep_buffers(s))) return rc;
-        if ((rc = fill_async(s->d_maxcount.p, 0, 2, s->stream)) || (rc = fill_async(s->d_stats.p, 0ull, 2, s->stream)))
-            return rc;
         if ((rc = sweep_launch(s, true))) return rc;
-        int flags[2] = {0, 0};
-        HIPCHK(hipMemcpyAsync(flags, s->d_maxcount.p, sizeof(flags), hipMemcpyDeviceToHost, s->stream));
         HIPCHK(hipStreamSynchronize(s->stream));
+        const int flags[2] = {(int)(s->h_counts[0] & 0xffffffffu), (int)(s->h_counts[0] >> 32)};
         if ((rc = sweep_flags_error(flags[1]))) return rc;
         mx = flags[0];
         if (!(s->vir && mx > s->cap)) break;
@@ -2250,8 +2399,7 @@ int pgt_ik_sweep_run(pgt_ik_sweep *s)
         s->cap = ((mx + 7) / 8) * 8;
         if (attempt == 3) return fail(PGT_ERR_HIP, "bond list capacity did not settle");
     }
-    unsigned long long h[2] = {0, 0};
-    HIPCHK(hipMemcpy(h, s->d_stats.p, sizeof(h), hipMemcpyDeviceToHost));
+    const unsigned long long h[2] = {s->h_counts[1], s->h_counts[2]};
     float g_ms = 0.0f, tot = 0.0f;
     (void)hipEventElapsedTime(&g_ms, s->ev[1], s->ev[2]);
     (void)hipEventElapsedTime(&tot, s->ev[0], s->ev[2]);

@@ -66,13 +66,25 @@ __device__ __forceinline__ void sort_hist_body(const Geom &g, int n, int ch, int
     if (t < radix) hf[(size_t)t * nchunk + ch] = h[t];
 }
 
+// A job's first launch zeroes its counters on the way (maxcount null: not the
+// first launch of a job).
+__device__ __forceinline__ void clear_counts(int *maxcount, unsigned long long *stats)
+{
+    if (maxcount && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) {
+        maxcount[threadIdx.x] = 0;
+        stats[threadIdx.x] = 0;
+    }
+}
+
 // One frame per y row (frames dealt to XCDs whole), one chunk per workgroup:
 // hist[f][digit][chunk].
 template <bool FIRST>
 __global__ __launch_bounds__(kSortBlock) void k_sort_hist(Geom g, int n, int nf, int shift, int radix,
                                                           const double *__restrict__ pos, int *__restrict__ keys,
-                                                          int *__restrict__ hist)
+                                                          int *__restrict__ hist, int *__restrict__ maxcount,
+                                                          unsigned long long *__restrict__ stats)
 {
+    if constexpr (FIRST) clear_counts(maxcount, stats);
     int f, ch;
     if (!frame_block(nf, f, ch)) return;
     sort_hist_body<FIRST>(g, n, ch, gridDim.x, shift, radix, pos + (size_t)f * n * 3, keys + (size_t)f * n,
@@ -372,20 +384,51 @@ __global__ void k_fill(T *__restrict__ p, T v, size_t n)
     if (i < n) p[i] = v;
 }
 
+// Up to five arrays of doubles copied by one launch between device memory and
+// pinned host memory, which a kernel reads and writes over PCIe like its own:
+// for the arrays of a small frame the copy engines' start and hand-over cost
+// several times the transfer (pgt_ik_set_particles, pgt_ik_compute).
+struct CopySegs {
+    const double *src[5];
+    double *dst[5];
+    int n[5];
+};
+
+__device__ __forceinline__ void copy_segs(const CopySegs &c, int tid, int stride)
+{
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        for (int i = tid; i < c.n[k]; i += stride) c.dst[k][i] = c.src[k][i];
+}
+
+__global__ __launch_bounds__(256) void k_copy_segs(CopySegs c)
+{
+    copy_segs(c, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
 // Fold the per-wavefront statistics of one batch into the job totals: sums
 // of (balls, contributions) into stats[0..1], the largest bond count into
-// maxcount[0].  Each workgroup reduces a stretch of the per-wavefront arrays
-// and adds its result with one atomic per total (a few hundred atomics per
-// batch, against one per wavefront of the batch's kernels before).
-__global__ __launch_bounds__(1024) void k_reduce_stats(int nw, const unsigned long long *__restrict__ wave_counts,
+// maxcount[0].  The first nrb workgroups reduce a stretch of the per-wavefront
+// arrays each and add their result with one atomic per total (a few hundred
+// atomics per batch, against one per wavefront of the batch's kernels before);
+// the rest copy the segments of `out`.  host_counts (nrb = 1 only): pinned
+// host memory that takes the job's counters, maxcount[0..1] in the first word
+// and the two totals after it, so that a job ends with its last kernel and one
+// synchronisation, without copies of a few bytes behind it.
+__global__ __launch_bounds__(1024) void k_reduce_stats(int nrb, int nw, const unsigned long long *__restrict__ wave_counts,
                                                        int nm, const int *__restrict__ wave_max,
-                                                       unsigned long long *__restrict__ stats, int *__restrict__ maxcount)
+                                                       unsigned long long *__restrict__ stats, int *__restrict__ maxcount,
+                                                       unsigned long long *__restrict__ host_counts, CopySegs out)
 {
+    if ((int)blockIdx.x >= nrb) {
+        copy_segs(out, (blockIdx.x - nrb) * blockDim.x + threadIdx.x, (gridDim.x - nrb) * blockDim.x);
+        return;
+    }
     __shared__ unsigned long long s0[16], s1[16];
     __shared__ int sm[16];
     unsigned long long a = 0, b = 0;
     int m = 0;
-    const int stride = gridDim.x * blockDim.x;
+    const int stride = nrb * blockDim.x;
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nw; k += stride) {
         a += wave_counts[2 * k];
         b += wave_counts[2 * k + 1];
@@ -409,9 +452,21 @@ __global__ __launch_bounds__(1024) void k_reduce_stats(int nw, const unsigned lo
             b += s1[k];
             m = max(m, sm[k]);
         }
-        if (a) atomicAdd(&stats[0], a);
-        if (b) atomicAdd(&stats[1], b);
-        if (m) atomicMax(maxcount, m);
+        if (host_counts) {  // the only workgroup: no other adds beside it
+            a += stats[0];
+            b += stats[1];
+            m = max(m, maxcount[0]);
+            stats[0] = a;
+            stats[1] = b;
+            maxcount[0] = m;
+            host_counts[0] = (unsigned long long)(unsigned)m | ((unsigned long long)(unsigned)maxcount[1] << 32);
+            host_counts[1] = a;
+            host_counts[2] = b;
+        } else {
+            if (a) atomicAdd(&stats[0], a);
+            if (b) atomicAdd(&stats[1], b);
+            if (m) atomicMax(maxcount, m);
+        }
     }
 }
 

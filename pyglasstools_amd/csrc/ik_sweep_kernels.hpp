@@ -13,8 +13,11 @@ namespace pgt {
 
 template <bool FIRST>
 __global__ __launch_bounds__(kSortBlock) void k_sweep_hist(const SweepSys *__restrict__ T, int ns, int shift,
-                                                           int radix, int *__restrict__ keys, int *__restrict__ hist)
+                                                           int radix, int *__restrict__ keys, int *__restrict__ hist,
+                                                           int *__restrict__ maxcount,
+                                                           unsigned long long *__restrict__ stats)
 {
+    if constexpr (FIRST) clear_counts(maxcount, stats);
     const SweepSys &S = T[sweep_system(T, ns, SW_SORT, blockIdx.x)];
     int f, ch;
     if (!sweep_frame_block(S, SW_SORT, blockIdx.x, f, ch)) return;

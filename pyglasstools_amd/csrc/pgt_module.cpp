@@ -565,8 +565,9 @@ struct IrvingKirkwood : Calculator {
         const ParticleSystem &s = *m_sysdata;
         int per[3] = {s.simbox->periodic[0] != 0, s.simbox->periodic[1] != 0, s.simbox->periodic[2] != 0};
         check(pgt_ik_set_box(engine, s.simbox->boxsize, s.simbox->lowerbound, per), "IrvingKirkwood.compute");
-        check(pgt_ik_set_particles(engine, (int64_t)s.n, s.position.data(), s.diameter.data(), s.mass.data(),
-                                   s.velocity.data(), fe ? s.displacement.data() : nullptr),
+        check(pgt_ik_set_particles(engine, (int64_t)s.n, s.position.data(), s.diameter.data(),
+                                   fk ? s.mass.data() : nullptr, fk ? s.velocity.data() : nullptr,
+                                   fe ? s.displacement.data() : nullptr),
               "IrvingKirkwood.compute");
         check(pgt_ik_set_grid(engine, (int64_t)G, grid.data()), "IrvingKirkwood.compute");
         unsigned fields = (fv ? PGT_FIELD_VIRIAL : 0) | (fe ? PGT_FIELD_ELASTIC : 0) | (fk ? PGT_FIELD_KINETIC : 0);

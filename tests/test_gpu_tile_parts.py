@@ -221,3 +221,33 @@ def test_small_frames_match_the_oracle(gpu, N, nf, keep, lengths):
         assert scaled_error(got["virial"][f], ref["virial"], ref["virial_abs"]).max() <= 1e-10
         assert np.abs(got["kinetic"][f] - ref["kinetic"]).max() <= 1e-10 * max(np.abs(ref["kinetic"]).max(), 1e-300)
     assert st["n_contrib"] == contrib
+
+
+@pytest.mark.parametrize("sizes", [(1, 700, 40), (3000, 3001, 5), (16384, 131072, 131073, 2000)])
+def test_host_arrays_match_device_arrays(gpu, sizes):
+    """One engine's host entry, sizes up and down across the staging memory's
+    growth and its limit (8 MB of particles: 131,072 of them), an upload
+    replaced before it is used, against the same frames from device memory:
+    the same launches, so the same bits."""
+    import torch
+
+    frames = [workload.make_system(max(N, 30), 2, 8800 + N) for N in sizes]
+    frames = [dict(s, **{k: s[k][:N].copy() for k in ("pos", "diam", "mass", "vel")}) for s, N in zip(frames, sizes)]
+    e = engine.Engine(dim=2, max_rcut=1.25 * 1.62)
+    for s, N in zip(frames, sizes):
+        print("host arrays N=%d" % N, flush=True)
+        grid = workload.cartesian_grid_2d(s["L"][0], 33 if N < 131072 else 300)
+        e.set_box(s["L"], s["periodic"])
+        e.set_grid(grid)
+        e.set_particles(s["pos"] * 0.5, s["diam"][::-1].copy(), s["mass"] * 2, s["vel"])
+        e.set_particles(s["pos"], s["diam"], s["mass"], s["vel"])
+        got = e.compute(("virial", "kinetic"))
+        ball = e.stats()["n_ball"]
+        d = {k: torch.tensor(s[k], device="cuda") for k in ("pos", "diam", "mass", "vel")}
+        o = {k: torch.zeros(len(grid), 2, 2, dtype=torch.float64, device="cuda") for k in ("virial", "kinetic")}
+        torch.cuda.synchronize()
+        e.compute_frames(1, N, d["pos"], d["diam"], d["mass"], d["vel"], fields=("virial", "kinetic"),
+                         d_virial=o["virial"], d_kinetic=o["kinetic"])
+        assert e.stats()["n_ball"] == ball
+        for k in o:
+            assert np.array_equal(o[k].cpu().numpy(), got[k]), k
