@@ -43,8 +43,8 @@ struct BondLayout {
     static_assert(GV % PER16 == 0, "a read group is a whole number of 16-byte pieces");
 };
 
-// One wavefront per 64 consecutive cell-sorted particles, one particle per
-// lane.
+// One wavefront per 64 (small jobs: 16) consecutive cell-sorted particles, one
+// particle per lane.
 //
 // The particles sit in one or a few runs of cells of one row each (pieces),
 // and a lane's candidates in the rows within reach of its own.  For every
@@ -56,11 +56,12 @@ struct BondLayout {
 // it is the plain difference.  Read from memory instead, each lane's
 // candidates are scattered loads: a CU takes about one lane's 16 bytes a
 // cycle of them, which was 69% of this kernel's time on the 2D N = 65,536
-// job.  Measured, from memory / this (one launch): that job, 100 frames 753 /
-// 538 us; 2D FP32 form, N = 30,011, 33 frames 119 / 81 us; 3D N = 131,072, FP32
-// form, 20 frames 1,259 / 940 us; 3D FP64, N = 20,011, 5 frames 126 / 84 us; one
-// frame of 2,000 particles 24 / 17 us.  What is left is latency: half of the
-// wavefronts' time is waits, with VALU issue at 65%.
+// job.  Measured, from memory / from LDS with a compare and a listing per
+// candidate / this (one launch): that job, 100 frames 753 / 505 / 462 us; 2D
+// FP32 form, N = 30,011, 33 frames 119 / 81 / 73 us; 3D N = 131,072, FP32 form,
+// 20 frames 1,259 / 866 / 758 us; 3D FP64, N = 20,011, 5 frames 126 / 82 / 73 us.
+// VALU issue is at 75%: 1,700 instructions a wavefront in 2D, half of them in
+// pass 2 (three FP64 divisions a pair).
 //
 // Pass 1 lists a lane's candidates within max_rcut and (without elastic
 // terms) within a bound of their own pair cutoff, about 4 of 37 in 2D and 7 of
@@ -77,14 +78,13 @@ struct BondLayout {
 // The body works on one frame's arrays (sorted cell keys kf, cell starts st,
 // sorted positions sp, diameters sd, displacements sdp, counts bc, entries
 // bd, FP32 records rf) for the particles of block pb, and stores the
-// wavefront's largest count at *wmax.
-constexpr int kBondBlock = 64;  // particles of a block, one per lane
+// wavefront's largest count at *wmax.  pw: particles per block.
+constexpr int kBondBlock = 64;  // lanes, and at most as many particles, of a block
 constexpr int kBondWin = 256;   // candidates in LDS
 // Wavefronts per SIMD the registers are held to: four in 2D without elastic
-// terms (131 registers otherwise, three wavefronts; 4 spilled: 588 -> 538 us
-// on the 2D N = 65,536 job), left to the compiler elsewhere (the 3D forms
-// would spill 64 bytes a lane: 992 us at four against 940 at three on the 3D
-// N = 131,072 FP32 job).
+// terms (a few registers over otherwise, three wavefronts; 588 -> 538 us on
+// the 2D N = 65,536 job when this was set), left to the compiler elsewhere (the 3D forms
+// would spill 110 bytes a lane, and their LDS lets 13 wavefronts onto a CU).
 constexpr int bond_waves(int D, bool ELA) { return D == 2 && !ELA ? 4 : 1; }
 
 // Where the particles of cell c of a row start, in the frame's sorted order
@@ -101,7 +101,7 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
                                            const int *__restrict__ kf, const int *__restrict__ st,
                                            const double *__restrict__ sp, const double *__restrict__ sd,
                                            const double *__restrict__ sdp, int cap, int *__restrict__ bc,
-                                           ER *__restrict__ bd, int *__restrict__ wmax, float4 *__restrict__ rf, int pb)
+                                           ER *__restrict__ bd, int *__restrict__ wmax, float4 *__restrict__ rf, int pb, int pw)
 {
     constexpr int PS = (D == 2) ? 2 : 4;
     using LY = BondLayout<D, OD, ELA, ER>;
@@ -112,8 +112,8 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
     constexpr int NB = 4;      // candidates per step of pass 1
     constexpr int NROW = 3;    // rows whose ranges are loaded together
     static_assert(kBondWin <= 256, "list entries are bytes");
-    __shared__ double s_x[kBondWin][D];       // candidates: positions,
-    __shared__ double s_d[kBondWin];          // diameters,
+    __shared__ double s_x[kBondWin + NB][D];  // candidates: positions,
+    __shared__ double s_d[kBondWin + NB];     // diameters (the last step of a scan may read past the window),
     __shared__ int s_id[ELA ? kBondWin : 1];  // sorted indices
     __shared__ unsigned char lq[MAXC][64];    // each lane's list
     // segments: first candidate, sorted index of the first particle (as
@@ -129,11 +129,11 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
     } s_u;
 
     const int lane = threadIdx.x;
-    const int p0 = pb * kBondBlock;
+    const int p0 = pb * pw, pn = min(pw, n - p0);
     // lanes past the end shadow the last particle without writing, so the
     // whole wavefront takes part in the staging and in the maximum at the end
-    const bool live = p0 + lane < n;
-    const int p = live ? p0 + lane : n - 1;
+    const bool live = lane < pn;
+    const int p = p0 + min(lane, pn - 1);
     double xi[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) xi[a] = sp[(size_t)p * PS + a];
@@ -147,23 +147,31 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
 #pragma unroll
     for (int a = 0; a < D; ++a) one_cell = one_cell || (g.nc[a] == 1 && g.periodic[a]);
 
-    // force of particle i (position x, diameter d) and candidate q; writes the
-    // entry to slot k of the particle's list and returns true unless it is zero
+    ER *const bd0 = bd + (size_t)p0 * (size_t)cap * ES;  // the block's entries
+
+    // force of particle p0 + i (position x, diameter d) and candidate q; writes
+    // the entry to slot k of the particle's list and returns true unless it is zero
     auto bond = [&](int i, const double *x, double d, int q, int k, bool write) {
         const double dj = s_d[q];
         double b[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             b[a] = s_x[q][a] - x[a];
-            if (img) b[a] = minimg(b[a], g.L[a], g.pinvL[a]);
+            if (img) {
+                asm volatile("");  // a branch: most blocks have none of these
+                b[a] = minimg(b[a], g.L[a], g.pinvL[a]);
+            }
         }
         const double rsq = fma(b[2], b[2], fma(b[1], b[1], b[0] * b[0]));
+        // false for numbers that are none, which the list may hold (force_divr
+        // ends with the same test of the pair's own cutoff)
+        if (!(rsq < g.mr2)) return false;
         double f0, f1 = 0.0;
         double ur[3] = {0, 0, 0};
         if constexpr (std::is_same<ER, double>::value) f0 = force_divr<double>(P, rsq, d, dj);
         else f0 = (double)force_divr<float>(P, (float)rsq, (float)d, (float)dj);
         if constexpr (ELA) {
-            for (int a = 0; a < 3; ++a) ur[a] = sdp[(size_t)s_id[q] * 3 + a] - sdp[(size_t)i * 3 + a] + b[a];
+            for (int a = 0; a < 3; ++a) ur[a] = sdp[(size_t)s_id[q] * 3 + a] - sdp[(size_t)(p0 + i) * 3 + a] + b[a];
             const double ursq = ur[0] * ur[0] + ur[1] * ur[1] + ur[2] * ur[2];
             if constexpr (std::is_same<ER, double>::value) f1 = force_divr<double>(P, ursq, d, dj);
             else f1 = (double)force_divr<float>(P, (float)ursq, (float)d, (float)dj);
@@ -182,7 +190,7 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
                 if (OD == 2) t[2] = (ER)T(0, 1);
                 else { t[3] = (ER)T(0, 1); t[4] = (ER)T(0, 2); t[5] = (ER)T(1, 2); }
             }
-            ER *e = bd + ((size_t)i * (size_t)cap + (size_t)k) * ES;
+            ER *e = bd0 + (unsigned)((i * cap + k) * ES);
             if constexpr (ES % LY::PER16 == 0) {
                 using V = typename std::conditional<std::is_same<ER, double>::value, double2, float4>::type;
                 V t[ES / LY::PER16];
@@ -222,7 +230,7 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
 #pragma unroll
                     for (int a = 0; a < D; ++a) x[a] = __shfl(xi[a], i, 64);
                     const double d = __shfl(di, i, 64);
-                    if (k < total && !bond(p0 + i, x, d, w >> 6, k + s_slot[i], true)) zero = true;
+                    if (k < total && !bond(i, x, d, w >> 6, k + s_slot[i], true)) zero = true;
                 }
                 alone = __builtin_amdgcn_ballot_w64(zero) != 0ull;
                 if (!alone) cnt += mine;
@@ -231,51 +239,56 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
         }
         if (alone)
             for (int k = 0; k < m; ++k)
-                if (bond(p, xi, di, lq[k][lane], cnt, live)) ++cnt;
+                if (bond(p - p0, xi, di, lq[k][lane], cnt, live)) ++cnt;
     };
 
-    // a bound of the pair's cutoff radius squared, loose enough for the FP32
-    // form's own rounding (the force decides)
-    const double lim = P.rcutsq * 0.25 * (1.0 + 1e-5);
     // pass 1 over candidates b .. e - 1 (self: the particle itself): m counts
-    // those within reach, of which numbers skip .. skip + MAXC - 1 are listed
+    // those within reach, of which numbers skip .. skip + MAXC - 1 are listed.
+    // Up to 32 candidates set the bits of a mask, each by the sign of a
+    // difference (one instruction moves it in; a compare and a listing under
+    // it, which some lane of 64 nearly always takes, would be eight), the last
+    // candidate first; then a lane lists its few.
     auto scan = [&](int b, int e, int self, int skip, int &m, auto image) {
-        for (int k = b; k < e; k += NB) {
-            double c[NB][D], dj[NB];
+        for (; b < e; b += 32) {
+            const int len = min(e - b, 32);
+            unsigned mask = 0u;
+            for (int j = (len - 1) & ~(NB - 1); j >= 0; j -= NB) {
+                double c[NB][D], dj[NB];
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                const int q = min(k + u, kBondWin - 1);
+                for (int u = 0; u < NB; ++u) {
 #pragma unroll
-                for (int a = 0; a < D; ++a) c[u][a] = s_x[q][a];
-                dj[u] = s_d[q];
+                    for (int a = 0; a < D; ++a) c[u][a] = s_x[b + j + u][a];
+                    dj[u] = s_d[b + j + u];
+                }
+#pragma unroll
+                for (int u = NB - 1; u >= 0; --u) {
+                    double b2 = 0.0;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) {
+                        double d = c[u][a] - xi[a];
+                        if constexpr (decltype(image)::value) d = minimg(d, g.L[a], g.pinvL[a]);
+                        b2 = a == 0 ? d * d : fma(d, d, b2);
+                    }
+                    double r2 = g.mr2;
+                    if constexpr (!ELA) {
+                        const double s = (di + dj[u]) * fma(P.leps, fabs(di - dj[u]), P.lim);
+                        r2 = fmin(s * s, r2);
+                    }
+                    mask = __builtin_amdgcn_alignbit(
+                        mask, (unsigned)((unsigned long long)__double_as_longlong(b2 - r2) >> 32), 31);
+                }
             }
-#pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                double b2 = 0.0;
-#pragma unroll
-                for (int a = 0; a < D; ++a) {
-                    double d = c[u][a] - xi[a];
-                    if constexpr (decltype(image)::value) d = minimg(d, g.L[a], g.pinvL[a]);
-                    b2 = a == 0 ? d * d : fma(d, d, b2);
-                }
-                bool in = b2 < g.mr2 && k + u < e && k + u != self;
-                if constexpr (!ELA) {
-                    // rcutsq sigma^2, sigma = (d_i + d_j)/2 (1 - eps |d_i - d_j|)
-                    const double sg = (di + dj[u]) * fma(-P.eps, fabs(di - dj[u]), 1.0);
-                    in = in && b2 < lim * (sg * sg);
-                }
-                if (in) {
-                    if ((unsigned)(m - skip) < (unsigned)MAXC) lq[m - skip][lane] = (unsigned char)(k + u);
-                    ++m;
-                }
-            }
+            mask &= ~0u >> (32 - len);
+            if ((unsigned)(self - b) < 32u) mask &= ~(1u << (self - b));
+            for (; mask; mask &= mask - 1u, ++m)
+                if ((unsigned)(m - skip) < (unsigned)MAXC) lq[m - skip][lane] = (unsigned char)(b + __builtin_ctz(mask));
         }
     };
 
     // the lane's cell, and the pieces: runs of lanes of one row
     const int nx = g.nc[0], ny = g.nc[1], nz = g.nc[2], R = g.reach;
     const int key = kf[p];
-    const int row = (int)(((double)key + 0.5) / (double)nx);
+    const int row = (int)(((double)key + 0.5) * g.inv_nc[0]);  // (exact: a cell's half is far from rounding)
     const int cx = key - row * nx;
     const int prow = __shfl_up(row, 1, 64);
     const unsigned long long starts = __builtin_amdgcn_ballot_w64(lane == 0 || row != prow);
@@ -285,7 +298,7 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
                       (int)((starts >> lane) & 1ull) - 1;
     const int ry = ny == 1 ? 1 : 2 * R + 1, rz = nz == 1 ? 1 : 2 * R + 1, nrow = ry * rz;
     const int own = (nz == 1 ? 0 : R) * ry + (ny == 1 ? 0 : R);  // the row of the lane's own cell
-    const float inv_npiece = 1.0f / (float)npiece, inv_ry = 1.0f / (float)ry;
+    const float inv_npiece = __builtin_amdgcn_rcpf((float)npiece), inv_ry = __builtin_amdgcn_rcpf((float)ry);
     // a lane's candidates of a row: cells lx .. hx - 1, relative to its own
     const int lx = nx == 1 ? -cx : -R, hx = nx == 1 ? 1 - cx : R + 1;
 
@@ -301,12 +314,12 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
         __syncthreads();
         int len = 0, begin = 0;
         {
-            // quotients of small integers, exact in floating point
+            // quotients of integers below 2^7, half a step from the next
             const int sg = min(lane, nseg - 1);
             const int rr = (int)(((float)sg + 0.5f) * inv_npiece), q = sg - rr * npiece, r = r0 + rr;
             const int dz = D == 2 ? 0 : (int)(((float)r + 0.5f) * inv_ry), dy = r - dz * ry;
             const int pr = s_u.piece.row[q];
-            const int cz = D == 2 ? 0 : (int)(((double)pr + 0.5) / (double)ny), cy = pr - cz * ny;
+            const int cz = D == 2 ? 0 : (int)(((double)pr + 0.5) * g.inv_nc[1]), cy = pr - cz * ny;
             int z = 0, y = 0, k = 0;
             if (nz > 1) {
                 z = cz + dz - R;
@@ -432,7 +445,7 @@ __device__ __forceinline__ void bonds_body(const Geom &g, int n, const PotParams
 // xcd_tile(x, gridDim.x), so each XCD works through a contiguous eighth of
 // the frame.
 template <int D, int OD, bool VIR, bool ELA, typename ER>
-__global__ __launch_bounds__(kBondBlock, bond_waves(D, ELA)) void k_bonds(Geom g, int n, PotParams P, double cgnorm,
+__global__ __launch_bounds__(kBondBlock, bond_waves(D, ELA)) void k_bonds(Geom g, int n, int pw, PotParams P, double cgnorm,
                                                const int *__restrict__ keys, const int *__restrict__ cstart, const double *__restrict__ spos,
                                                const double *__restrict__ sdiam, const double *__restrict__ sdisp,
                                                int cap, int *__restrict__ bcount, ER *__restrict__ bonds,
@@ -446,7 +459,7 @@ __global__ __launch_bounds__(kBondBlock, bond_waves(D, ELA)) void k_bonds(Geom g
         g, n, P, cgnorm, keys + fo, cstart + (size_t)f * (g.ncell + 1), spos + fo * PS, sdiam + fo,
         ELA ? sdisp + fo * 3 : nullptr, cap, bcount + fo, bonds + fo * (size_t)cap * ES,
         wave_max + (size_t)blockIdx.y * gridDim.x + blockIdx.x, D == 3 ? rec + fo : nullptr,
-        xcd_tile(blockIdx.x, gridDim.x));
+        xcd_tile(blockIdx.x, gridDim.x), pw);
 }
 
 }  // namespace pgt

@@ -17,6 +17,9 @@ struct PotParams {
     int kind;
     double v0, eps, c0, c1, c2, c3;
     double rcutsq;  // scaled_rcut^2
+    // the bond search's bound of a pair's cutoff radius, lim sigma with sigma
+    // = (d_i + d_j) (1 - eps |d_i - d_j|), and -eps lim
+    double lim, leps;
 };
 
 // F/r of the polydisperse m-n family with its even-polynomial smoothing.

@@ -487,6 +487,9 @@ PotParams make_pot(const pgt_ik_params &p)
     P.c2 = p.pot_params[4];
     P.c3 = p.n_pot_params > 5 ? p.pot_params[5] : 0.0;
     P.rcutsq = p.scaled_rcut * p.scaled_rcut;
+    // loose enough for the FP32 form's own rounding (the force decides)
+    P.lim = std::sqrt(P.rcutsq * 0.25 * (1.0 + 1e-5));
+    P.leps = -P.eps * P.lim;
     return P;
 }
 
@@ -545,6 +548,7 @@ Geom make_geom(const pgt_ik_engine *e, int D)
     g.rc2 = e->prm.cg_rcut * e->prm.cg_rcut;
     g.inv_rc = 1.0 / e->prm.cg_rcut;
     g.inv_rc2 = 1.0 / g.rc2;
+    for (int a = 0; a < 2; ++a) g.inv_nc[a] = 1.0 / (double)g.nc[a];
     g.mr2 = e->prm.max_rcut * e->prm.max_rcut;
     // FP32 pre-test bounds for the two search radii (r_cg for the gather,
     // max_rcut for the bond list): fp32_band, with M the largest coordinate
@@ -572,19 +576,19 @@ Geom make_geom(const pgt_ik_engine *e, int D)
 // launch dispatch
 // ------------------------------------------------------------------------
 template <int D, int OD, typename ER>
-void launch_bonds_t(const LaunchCtx &c, unsigned fields, const PotParams &P, const int *keys, const double *sdiam,
+void launch_bonds_t(const LaunchCtx &c, unsigned fields, int pw, const PotParams &P, const int *keys, const double *sdiam,
                     const double *sdisp, int *bcount, void *bonds, int *wave_max, float4 *rec)
 {
     const bool V = fields & PGT_FIELD_VIRIAL, E = fields & PGT_FIELD_ELASTIC;
-    dim3 grid((unsigned)((c.n + kBondBlock - 1) / kBondBlock), (unsigned)c.nf);
+    dim3 grid((unsigned)((c.n + pw - 1) / pw), (unsigned)c.nf);
     if (V && E)
-        hipLaunchKernelGGL((k_bonds<D, OD, true, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+        hipLaunchKernelGGL((k_bonds<D, OD, true, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, pw, P,
                            c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
     else if (E)
-        hipLaunchKernelGGL((k_bonds<D, OD, false, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+        hipLaunchKernelGGL((k_bonds<D, OD, false, true, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, pw, P,
                            c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
     else
-        hipLaunchKernelGGL((k_bonds<D, OD, true, false, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, P,
+        hipLaunchKernelGGL((k_bonds<D, OD, true, false, ER>), grid, dim3(kBondBlock), 0, c.stream, c.g, c.n, pw, P,
                            c.cgnorm, keys, c.cstart, c.spos, sdiam, sdisp, c.cap, bcount, (ER *)bonds, wave_max, rec);
 }
 
@@ -602,6 +606,7 @@ struct JobShape {
     bool pairs, kin, ela, fp32, adaptive;
     Geom g;
     bool small;  // the cell list of k_sort_small
+    int bp;      // particles per wavefront of the bond kernel
     int npass, nbits, radix;
     size_t ebytes;
     int block, pl;
@@ -670,6 +675,14 @@ int launch_frames(const pgt_ik_engine *e, int64_t n, int nframes)
 // n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
 // gather even where the tile gather is selected (the fallback when a tile
 // reports an overflow)
+// Particles per wavefront of the bond kernel: one a lane, or a quarter of that
+// where the GPU is nearly empty even so (512 wavefronts, half of its SIMDs) and
+// the time is one wavefront's: fewer candidates to stage and fewer rounds of
+// pairs.  Cell and bond lists of one frame, 64 / 16 a wavefront: 2D, N = 2,000
+// 26 / 22 us, 8,000 36 / 32, 32,000 52 / 56; with elastic terms 39 / 32, 50 /
+// 43, 70 / 66; 3D, N = 1,000 81 / 67, 8,000 81 / 73, 16,000 85 / 92.
+int bond_block(int64_t particles) { return particles <= 512 * 16 ? 16 : kBondBlock; }
+
 JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nf, bool allow_tile = true)
 {
     JobShape j{};
@@ -686,6 +699,7 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     j.adaptive = e->prm.quad_mode == PGT_QUAD_ADAPTIVE && j.pairs;
     j.g = make_geom(e, j.D);
     j.small = n <= kSmallParticles && j.g.ncell <= kSmallCells;
+    j.bp = bond_block(n * nf);
     // radix sort of the cell keys: digits of nbits bits, npass passes
     int kbits = 0;
     while ((1 << kbits) < j.g.ncell) ++kbits;
@@ -733,7 +747,7 @@ void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, size_t
     const size_t fn = (size_t)nf * (size_t)n;
     const size_t nchunk = (size_t)((n + kSortChunk - 1) / kSortChunk);
     const size_t nw_gather_max = (size_t)std::max<int64_t>(j.gwaves, (G + j.block - 1) / j.block * (j.block / 64)) * nf;
-    const size_t nw_bonds = j.pairs ? (size_t)((n + kBondBlock - 1) / kBondBlock) * nf : 0;
+    const size_t nw_bonds = j.pairs ? (size_t)((n + j.bp - 1) / j.bp) * nf : 0;
     for (int k = 0; k < W_NARRAYS; ++k) out[k] = 0;
     out[W_KEYS0] = out[W_VALS0] = out[W_KEYS1] = out[W_VALS1] = fn * sizeof(int);
     out[W_HIST] = (size_t)nf * j.radix * std::max<size_t>(nchunk, 1) * sizeof(int);
@@ -932,7 +946,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     // per-wavefront statistics of this batch (see k_reduce_stats)
     c.pl = j.pl;
     const int nw_gather = (int)(j.gwaves * nf);
-    const int nw_bonds = j.pairs ? (int)(((size_t)n + kBondBlock - 1) / kBondBlock) * nf : 0;
+    const int nw_bonds = j.pairs ? (int)(((size_t)n + j.bp - 1) / j.bp) * nf : 0;
     c.out.wave_counts = w.get<unsigned long long>(W_WCOUNTS);
     int *wmax = w.get<int>(W_WMAX);
     void *bonds = w.p[W_BONDS];
@@ -942,13 +956,13 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         c.cap = cap;
         const PotParams P = make_pot(e->prm);
         if (D == 2) {
-            if (j.fp32) launch_bonds_t<2, 2, float>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
-            else launch_bonds_t<2, 2, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            if (j.fp32) launch_bonds_t<2, 2, float>(c, fields, j.bp, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            else launch_bonds_t<2, 2, double>(c, fields, j.bp, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         } else if (OD == 2) {
-            launch_bonds_t<3, 2, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            launch_bonds_t<3, 2, double>(c, fields, j.bp, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         } else {
-            if (j.fp32) launch_bonds_t<3, 3, float>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
-            else launch_bonds_t<3, 3, double>(c, fields, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            if (j.fp32) launch_bonds_t<3, 3, float>(c, fields, j.bp, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
+            else launch_bonds_t<3, 3, double>(c, fields, j.bp, P, keys, sdiam, sdisp, bcount, bonds, wmax, rec);
         }
         HIPCHK(hipGetLastError());
     } else {

@@ -22,6 +22,7 @@ struct Geom {
     double inv_rc;   // 1/cg_rcut
     double inv_rc2;  // 1/cg_rcut^2
     double mr2;      // max_rcut^2
+    double inv_nc[2];  // 1/nc[0], 1/nc[1]
     // FP32 pre-tests of the 3D candidate scans: with |a|^2 from FP32 copies
     // of the positions, |a|^2 < in32 means inside the coarse-graining ball
     // and |a|^2 > out32 outside, whatever the FP64 rounding; in between the

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kBondBlock, bond_waves(D, false)) void k_sweep_bond
     bonds_body<D, OD, true, false, ER>(g, n, P, S.cgnorm, keys + fo,
                                        cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1), spos + fo * PS, sdiam + fo,
                                        nullptr, cap, bcount + fo, bonds + fo * (size_t)cap * ES, wm,
-                                       D == 3 ? rec + fo : nullptr, pb);
+                                       D == 3 ? rec + fo : nullptr, pb, kBondBlock);
 }
 
 }  // namespace pgt

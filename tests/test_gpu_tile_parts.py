@@ -251,3 +251,35 @@ def test_host_arrays_match_device_arrays(gpu, sizes):
         assert e.stats()["n_ball"] == ball
         for k in o:
             assert np.array_equal(o[k].cpu().numpy(), got[k]), k
+
+
+@pytest.mark.parametrize("dim,N,nf,cells", [(2, 17, 1, 0), (2, 1000, 8, 0), (2, 1025, 8, 0), (3, 1025, 2, 0),
+                                            (2, 9000, 1, 40), (3, 9000, 1, 30)])
+def test_bond_scan_masks_match_the_oracle(gpu, dim, N, nf, cells):
+    """Both sizes of the bond kernel's blocks (8,192 particles in a launch is
+    the line), and rows of candidates longer than a 32-candidate mask and than
+    the window (cells > 0: that many times the density along x).  FP64 drop-in
+    bar."""
+    frames = []
+    for f in range(nf):
+        s = workload.make_system(N, dim, 9900 + f)
+        if cells:  # short cutoffs, many candidates a cell
+            s = dict(s, pos=s["pos"] / np.sqrt(cells), diam=s["diam"] / np.sqrt(cells), L=s["L"] / np.sqrt(cells))
+            if dim == 2:
+                s["L"][2] = 1.0
+        frames.append(s)
+    print("bond masks dim %d N %d x %d cells %d L %s" % (dim, N, nf, cells, frames[0]["L"]), flush=True)
+    L = frames[0]["L"][0]
+    rmax = 1.25 * 1.62 / (np.sqrt(cells) if cells else 1.0)
+    rc = 0.45 * L if L < 4.2 else 2.0
+    grid = workload.cartesian_grid_2d(L, 9) if dim == 2 else workload.cartesian_grid_3d(L, 5)
+    e = engine.Engine(dim=dim, max_rcut=rmax, cg_rcut=rc)
+    e.set_box(frames[0]["L"], frames[0]["periodic"])
+    e.set_grid(grid)
+    got, st = _frames(e, frames, ("virial",))
+    contrib = 0
+    for f, s in enumerate(frames):
+        ref = oracle.ik_compute(s, grid, fields=("virial",), max_rcut=rmax, cg_rcut=rc, with_abs=True)
+        contrib += ref["n_nonzero"]
+        assert scaled_error(got["virial"][f], ref["virial"], ref["virial_abs"]).max() <= 1e-10
+    assert st["n_contrib"] == contrib
