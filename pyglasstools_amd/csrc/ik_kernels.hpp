@@ -93,28 +93,57 @@ __global__ __launch_bounds__(kSortBlock) void k_sort_hist(Geom g, int n, int nf,
 
 // In-place exclusive scan of the len ints at a, by one 1024-thread
 // workgroup: a frame's hist[digit][chunk] becomes the first output slot of
-// that digit's items of that chunk.
+// that digit's items of that chunk.  8,192 at a time, eight consecutive ones a
+// thread in two loads; each thread walking its 1,024th of the whole array an
+// int at a time waited for every one of its loads (one launch, before
+// / after: 100 frames of 8,192 13.4 / 5.1 us, a sweep's 128 of up to 24,576
+// 42 / 7.9, 20 of 16,384 26 / 4.9).
 __device__ __forceinline__ void scan_body(int len, int *__restrict__ a)
 {
-    const int T = blockDim.x, t = threadIdx.x;
-    const int chunk = (len + T - 1) / T;
-    const int b0 = min(len, t * chunk), b1 = min(len, b0 + chunk);
-    int s = 0;
-    for (int k = b0; k < b1; ++k) s += a[k];
-    __shared__ int sh[1024];
-    sh[t] = s;
-    __syncthreads();
-    for (int off = 1; off < T; off <<= 1) {
-        const int v = t >= off ? sh[t - off] : 0;
-        __syncthreads();
-        sh[t] += v;
-        __syncthreads();
-    }
-    int run = sh[t] - s;
-    for (int k = b0; k < b1; ++k) {
-        const int v = a[k];
-        a[k] = run;
-        run += v;
+    constexpr int PER = 8, NW = 1024 / 64;
+    __shared__ int s_wave[2][NW];
+    const int t = threadIdx.x, w = t >> 6;
+    int base = 0;
+    for (int t0 = 0, turn = 0; t0 < len; t0 += 1024 * PER, turn ^= 1) {
+        const int k = t0 + t * PER;
+        int x[PER];
+        if (k + PER <= len) {
+            __builtin_memcpy(x, a + k, sizeof(x));
+        } else {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) x[q] = k + q < len ? a[k + q] : 0;
+        }
+        int sum = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int v = x[q];
+            x[q] = sum;
+            sum += v;
+        }
+        int v = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(v, off, 64);
+            if ((t & 63) >= off) v += u;
+        }
+        if ((t & 63) == 63) s_wave[turn][w] = v;
+        __syncthreads();  // (the other turn's sums are read before this one's next barrier)
+        int first = base + v - sum;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            const int c = s_wave[turn][q];
+            if (q < w) first += c;
+            base += c;
+        }
+#pragma unroll
+        for (int q = 0; q < PER; ++q) x[q] += first;
+        if (k + PER <= len) {
+            __builtin_memcpy(a + k, x, sizeof(x));
+        } else {
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                if (k + q < len) a[k + q] = x[q];
+        }
     }
 }
 
@@ -214,7 +243,23 @@ __device__ __forceinline__ void sorted_particle(const Geom &g, int k, size_t fi,
 {
     constexpr int PS = (D == 2) ? 2 : 4;
     constexpr int KN = OD * (OD + 1) / 2;
-    const double *p = pos + fi * 3;
+    // Every load first.  The rows of the inputs lie anywhere in the frame: four
+    // lines a particle, one lane's at a time, bound this kernel (274 us for 100
+    // frames of 65,536; its bytes alone take 156).  Streaming the inputs and
+    // scattering the sorted arrays instead wrote partly filled lines (900 MB
+    // for 320): 321 us; reading the frame once in order before: 294.
+    const double p[3] = {pos[fi * 3], pos[fi * 3 + 1], D == 3 ? pos[fi * 3 + 2] : 0.0};
+    const double d = diam[fi];
+    double m = 1.0, v[3] = {0.0, 0.0, 0.0}, u[3] = {0.0, 0.0, 0.0};
+    if (skin && mass) m = mass[fi];
+    if (skin && vel) {
+#pragma unroll
+        for (int a = 0; a < OD; ++a) v[a] = vel[fi * 3 + a];
+    }
+    if (sdisp && disp) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) u[a] = disp[fi * 3 + a];
+    }
     double *sp = spos + (size_t)k * PS;
     auto wrap = [&](int a) {
         return g.periodic[a] ? p[a] - g.L[a] * floor((p[a] - g.lo[a]) * g.invL[a]) : p[a];
@@ -223,11 +268,8 @@ __device__ __forceinline__ void sorted_particle(const Geom &g, int k, size_t fi,
     sp[1] = wrap(1);
     if (D == 3) { sp[2] = wrap(2); sp[3] = 0.0; }
     if (D == 3 && rec) rec[k] = make_float4((float)sp[0], (float)sp[1], (float)sp[2], 0.0f);
-    sdiam[k] = diam[fi];
+    sdiam[k] = d;
     if (skin) {
-        const double m = mass ? mass[fi] : 1.0;
-        double v[3] = {0, 0, 0};
-        if (vel) { v[0] = vel[fi * 3]; v[1] = vel[fi * 3 + 1]; v[2] = vel[fi * 3 + 2]; }
         double *kk = skin + (size_t)k * KN;
         // symmetric packing: diagonal, then (0,1) [, (0,2), (1,2)]
         for (int a = 0; a < OD; ++a) kk[a] = m * v[a] * v[a];
@@ -235,7 +277,7 @@ __device__ __forceinline__ void sorted_particle(const Geom &g, int k, size_t fi,
         else { kk[3] = m * v[0] * v[1]; kk[4] = m * v[0] * v[2]; kk[5] = m * v[1] * v[2]; }
     }
     if (sdisp)
-        for (int a = 0; a < 3; ++a) sdisp[(size_t)k * 3 + a] = disp ? disp[fi * 3 + a] : 0.0;
+        for (int a = 0; a < 3; ++a) sdisp[(size_t)k * 3 + a] = u[a];
 }
 
 // Write the cell-sorted particle arrays (slot k takes input particle
@@ -252,12 +294,12 @@ __device__ __forceinline__ void sort_finish_body(const Geom &g, int n, int k, in
                                                  double *__restrict__ sdisp, float4 *__restrict__ rec)
 {
     if (k >= n) return;
-    const int c = keys[k];
-    const int cp = k == 0 ? -1 : keys[k - 1];
+    const int c = keys[k], i = vals[k], cb = keys[max(k - 1, 0)];
+    const int cp = k == 0 ? -1 : cb;
+    sorted_particle<D, OD>(g, k, (size_t)i, pos, diam, mass, vel, disp, spos, sdiam, skin, sdisp, rec);
     for (int q = cp + 1; q <= c; ++q) st[q] = k;
     if (k == n - 1)
         for (int q = c + 1; q <= ncell; ++q) st[q] = n;
-    sorted_particle<D, OD>(g, k, (size_t)vals[k], pos, diam, mass, vel, disp, spos, sdiam, skin, sdisp, rec);
 }
 
 template <int D, int OD>

@@ -283,3 +283,29 @@ def test_bond_scan_masks_match_the_oracle(gpu, dim, N, nf, cells):
         contrib += ref["n_nonzero"]
         assert scaled_error(got["virial"][f], ref["virial"], ref["virial_abs"]).max() <= 1e-10
     assert st["n_contrib"] == contrib
+
+
+@pytest.mark.parametrize("N,nf,keep", [(8193, 3, 1.0), (66000, 1, 1.0), (100001, 2, 1.0), (300000, 1, 0.03)])
+def test_histogram_scan_sizes_match_the_oracle(gpu, N, nf, keep):
+    """Cell lists whose digit histograms (digits x chunks of 1,024 particles)
+    are below (576), just past (8,320) and several times (25,088) the 8,192
+    entries that the scan takes at a time, and three digits.  FP64 drop-in bar."""
+    frames = []
+    for f in range(nf):
+        s = workload.make_system(N, 2, 9700 + f)
+        n = int(N * keep)
+        frames.append(dict(s, **{k: s[k][:n].copy() for k in ("pos", "diam", "mass", "vel")}))
+    L = frames[0]["L"][0]
+    grid = workload.cartesian_grid_2d(L, 24)
+    print("scan N=%d x %d keep %.2f" % (N, nf, keep), flush=True)
+    e = engine.Engine(dim=2, max_rcut=1.25 * 1.62)
+    e.set_box(frames[0]["L"], frames[0]["periodic"])
+    e.set_grid(grid)
+    got, st = _frames(e, frames, ("virial", "kinetic"))
+    contrib = 0
+    for f, s in enumerate(frames):
+        ref = oracle.ik_compute(s, grid, fields=("virial", "kinetic"), max_rcut=1.25 * 1.62, with_abs=True)
+        contrib += ref["n_nonzero"]
+        assert scaled_error(got["virial"][f], ref["virial"], ref["virial_abs"]).max() <= 1e-10
+        assert np.abs(got["kinetic"][f] - ref["kinetic"]).max() <= 1e-10 * np.abs(ref["kinetic"]).max()
+    assert st["n_contrib"] == contrib
