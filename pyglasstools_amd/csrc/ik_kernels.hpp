@@ -153,64 +153,97 @@ __global__ __launch_bounds__(1024) void k_sort_scan(int len, int *__restrict__ h
     scan_body(len, hist + (size_t)blockIdx.x * len);
 }
 
-// Move the items of one chunk to their slots for this digit.  A chunk is
-// taken row by row (kSortBlock consecutive items); inside a row an item's
-// slot is the chunk's offset for its digit, plus the items of that digit in
-// earlier rows, in earlier wavefronts of the row, and in lower lanes of its
-// wavefront (found with one ballot per digit bit).  With FIRST the value is
-// the input index.
+// Move the items of one chunk to their slots for this digit.  A chunk's items
+// lie in rows of kSortBlock; an item's slot is the chunk's offset for its
+// digit, plus the items of that digit in earlier rows, in earlier wavefronts
+// of its row, and in lower lanes of its wavefront (found with one ballot per
+// digit bit).  The chunk is put in order in LDS first, so that neighbouring
+// lanes store to neighbouring slots: stored from their input order, 64 lanes'
+// items went to as many lines, one lane a cycle.  One launch on 100 frames of
+// 65,536: 57 -> 24 us, the eight-system sweep's 46 and 36 -> 26 and 21.  With
+// FIRST the value is the input index.
 template <bool FIRST>
 __device__ __forceinline__ void sort_scatter_body(int n, int ch, int nchunk, int shift, int radix,
                                                   const int *__restrict__ kin, const int *__restrict__ vin,
                                                   const int *__restrict__ hf, int *__restrict__ kout,
                                                   int *__restrict__ vout)
 {
-    constexpr int NW = kSortBlock / 64;
-    __shared__ int run[kSortMaxRadix];     // next slot of each digit
-    __shared__ int wc[NW][kSortMaxRadix];  // per-wavefront digit counts of a row, then their slots
+    constexpr int NW = kSortBlock / 64, NE = kSortRows * NW;
+    static_assert(kSortBlock == kSortMaxRadix, "a thread per digit");
+    __shared__ unsigned short wc[NE][kSortMaxRadix];  // digit counts of each row's wavefronts, then their first places
+    __shared__ int s_key[kSortChunk], s_val[kSortChunk];  // the chunk in order
+    __shared__ int s_off[kSortMaxRadix];                  // a digit's first slot less its first place
+    __shared__ int s_wave[NW];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (t < radix) run[t] = hf[(size_t)t * nchunk + ch];
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;  // lanes under this one
-    int nbits = 0;
-    while ((1 << nbits) < radix) ++nbits;
-    const int base = ch * kSortChunk;
+    const int base = ch * kSortChunk, items = min(kSortChunk, n - base);
+    int key[kSortRows], val[kSortRows], rank[kSortRows];
+#pragma unroll
     for (int r = 0; r < kSortRows; ++r) {
-        if (base + r * kSortBlock >= n) break;  // uniform over the workgroup
-        for (int k = t; k < NW * kSortMaxRadix; k += kSortBlock) wc[k / kSortMaxRadix][k % kSortMaxRadix] = 0;
-        __syncthreads();
-        const int i = base + r * kSortBlock + t;
-        const bool valid = i < n;
-        int key = 0, val = 0, d = 0;
-        if (valid) {
-            key = kin[i];
-            val = FIRST ? i : vin[i];
-            d = (key >> shift) & (radix - 1);
-        }
+        const int i = base + min(r * kSortBlock + t, items - 1);
+        key[r] = kin[i];
+        val[r] = FIRST ? i : vin[i];
+    }
+    const int first = t < radix ? hf[(size_t)t * nchunk + ch] : 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) wc[e][t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRows; ++r) {
+        const bool valid = r * kSortBlock + t < items;
+        const int d = (key[r] >> shift) & (radix - 1);
         unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < nbits; ++b) {
-            const bool bit = (d >> b) & 1;
+        for (int b = 1; b < radix; b <<= 1) {
+            const bool bit = d & b;
             const unsigned long long m = __ballot(bit);
             peers &= bit ? m : ~m;
         }
-        const int rank = __popcll(peers & below);
-        if (valid && rank == 0) wc[w][d] = __popcll(peers);
-        __syncthreads();
-        if (t < radix) {
-            int acc = run[t];
-            for (int q = 0; q < NW; ++q) {
-                const int c = wc[q][t];
-                wc[q][t] = acc;
-                acc += c;
-            }
-            run[t] = acc;
-        }
-        __syncthreads();
-        if (valid) {
-            const int slot = wc[w][d] + rank;
-            kout[slot] = key;
-            vout[slot] = val;
-        }
-        __syncthreads();
+        rank[r] = __popcll(peers & below);
+        if (valid && rank[r] == 0) wc[r * NW + w][d] = (unsigned short)__popcll(peers);
+    }
+    __syncthreads();
+    // thread t: the places of digit t
+    int c[NE], sum = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        c[e] = wc[e][t];
+        sum += c[e];
+    }
+    int place = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(place, off, 64);
+        if (lane >= off) place += u;
+    }
+    if (lane == 63) s_wave[w] = place;
+    __syncthreads();
+    place -= sum;
+#pragma unroll
+    for (int q = 0; q < NW; ++q)
+        if (q < w) place += s_wave[q];
+    s_off[t] = first - place;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        wc[e][t] = (unsigned short)place;
+        place += c[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRows; ++r) {
+        if (r * kSortBlock + t >= items) continue;
+        const int k = wc[r * NW + w][(key[r] >> shift) & (radix - 1)] + rank[r];
+        s_key[k] = key[r];
+        s_val[k] = val[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRows; ++r) {
+        const int k = r * kSortBlock + t;
+        if (k >= items) continue;
+        const int kk = s_key[k];
+        const int slot = s_off[(kk >> shift) & (radix - 1)] + k;
+        kout[slot] = kk;
+        vout[slot] = s_val[k];
     }
 }
 
