@@ -672,9 +672,6 @@ int launch_frames(const pgt_ik_engine *e, int64_t n, int nframes)
     return (int)std::min<int64_t>(nframes, std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
 }
 
-// n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
-// gather even where the tile gather is selected (the fallback when a tile
-// reports an overflow)
 // Particles per wavefront of the bond kernel: one a lane, or a quarter of that
 // where the GPU is nearly empty even so (512 wavefronts, half of its SIMDs) and
 // the time is one wavefront's: fewer candidates to stage and fewer rounds of
@@ -683,6 +680,9 @@ int launch_frames(const pgt_ik_engine *e, int64_t n, int nframes)
 // 43, 70 / 66; 3D, N = 1,000 81 / 67, 8,000 81 / 73, 16,000 85 / 92.
 int bond_block(int64_t particles) { return particles <= 512 * 16 ? 16 : kBondBlock; }
 
+// n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
+// gather even where the tile gather is selected (the fallback when a tile
+// reports an overflow)
 JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nf, bool allow_tile = true)
 {
     JobShape j{};
@@ -1746,6 +1746,14 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
         // the most frames per launch whose work arrays fit the scratch array
         int nf = fpl;
         while (nf > 0 && work_carve(j, nf, n, e->G, cap, nullptr, nullptr) > kScratchBytes) nf = nf / 2;
+        if (nf < 1 && (j.tile || j.bp != kBondBlock)) {
+            // the tile gather's counters and those of quarter bond blocks take
+            // a few KB more than the lane gather's, which may be the ones that
+            // do not fit
+            j = job_shape(e, fields, fs.z_flat, fs.n, 1, false);
+            j.bp = kBondBlock;
+            nf = work_carve(j, 1, n, e->G, cap, nullptr, nullptr) > kScratchBytes ? 0 : 1;
+        }
         if (nf < 1)
             return fail(PGT_ERR_RANGE, "one frame of this job needs " +
                                            std::to_string(work_carve(j, 1, n, e->G, cap, nullptr, nullptr)) +
