@@ -307,8 +307,9 @@ int pgt_ik_set_tuning(pgt_ik_engine *e, int threads_per_block, int frames_per_la
  * more than 255 bonds makes the job run again with the lane gather.  An
  * engine on which neither this nor the lane gather's settings
  * (pgt_ik_set_tuning's threads_per_block, points_per_lane) were chosen takes
- * the tile gather for FP64 entries with at most 255 bond slots a particle,
- * the lane gather otherwise.  No counterpart in the reference. */
+ * the tile gather where it has the form, with at most 255 bond slots a
+ * particle, the lane gather otherwise (and for the elastic field alone in the
+ * FP32 form); its FP32 terms are then rounded as the lane gather's.  No counterpart in the reference. */
 int pgt_ik_set_gather_mode(pgt_ik_engine *e, int mode);
 
 int pgt_ik_get_stats(pgt_ik_engine *e, pgt_ik_stats *out);

@@ -617,16 +617,24 @@ struct JobShape {
 };
 
 // Whether an engine whose gather was not chosen takes the tile gather: where
-// it has the form, with FP64 entries (the two gathers round the FP32 form's
-// terms differently) and at most 255 bond slots a particle (the lane gather
-// holds more), unless the caller set one of the lane gather's knobs.  It is
-// the faster one from the smallest jobs to the largest: gather of one frame
+// it has the form, with at most 255 bond slots a particle (the lane gather
+// holds more), unless the caller set one of the lane gather's knobs.  With
+// FP32 entries it rounds the terms as the lane gather does (lane_terms), which
+// it has for the virial field, with others or alone; the elastic field alone
+// stays with the lane gather.  It is the faster one from the smallest jobs to the largest: gather of one frame
 // of N = 2,000, 32^2 grid 77 -> 8 us, N = 1,024, 128^2 grid 54 -> 12 us, N = 65,536,
 // 256^2 grid 74 -> 25 us, a 10-node Mollifier rule on N = 4,000, 97^2 grid
 // 202 -> 41 us, 24 frames with elastic terms, N = 16,384, 128^2 grid 252 -> 95 us.
-bool default_tile(const pgt_ik_engine *e, const JobShape &j)
+// Whole FP32-form jobs, lane / tile gather: 2D, N = 1,000, one frame, 32^2 grid
+// 128 / 63 us; N = 12,874, 4 frames, 173^2 163 / 108; N = 65,536, 32 frames,
+// 256^2 828 / 590; with elastic terms, N = 20,000, 8 frames, 200^2 202 / 171; 3D,
+// N = 4,000, one frame, 12^3 872 / 120; N = 94,181, 4 frames, 60^3 1,624 / 787;
+// N = 29,763, 11 frames, 12^3 9,313 / 292 (a coarse grid gives the lane gather few
+// lanes, each with a long list of its own).
+bool default_tile(const pgt_ik_engine *e, const JobShape &j, unsigned fields)
 {
-    return !e->lane_knobs && !j.fp32 && e->cap <= 255 &&
+    const bool terms = !j.fp32 || (fields & PGT_FIELD_VIRIAL) || !j.pairs;
+    return !e->lane_knobs && terms && e->cap <= 255 &&
            tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32);
 }
 
@@ -713,7 +721,7 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     j.pl = j.adaptive ? 1 : gather_pl(e->points_per_lane, e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD);
     j.tile = allow_tile && !j.adaptive && n <= kTileMaxParticles && e->ntiles > 0 &&
              (e->gather_mode == 1 ? tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32)
-                                  : e->gather_mode == -1 && default_tile(e, j));
+                                  : e->gather_mode == -1 && default_tile(e, j, fields));
     if (j.tile) {
         j.block = kTileThreads;
         j.pl = 1;
@@ -925,6 +933,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     c.tperm = e->d_tperm.p;
     c.ntiles = e->ntiles;
     c.tp = j.tp;
+    c.lane_terms = e->gather_mode == -1;
     c.R.n = (int)e->gl_s.size();
     for (int k = 0; k < c.R.n && k < kMaxQArg; ++k) {
         c.R.s[k] = e->gl_s[k];

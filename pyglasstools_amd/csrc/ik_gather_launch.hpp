@@ -58,13 +58,15 @@ void launch_gather_f(const LaunchCtx &c, unsigned fields)
     else launch_gather_b<D, OD, CG, NQ, false, false, ER>(c);
 }
 
-template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
+template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
 void launch_tile_t(const LaunchCtx &c)
 {
+    if constexpr (VIR && std::is_same<ER, float>::value && !LT)
+        if (c.lane_terms) return launch_tile_t<D, OD, CG, NQ, VIR, ELA, KIN, ER, true>(c);
     using CP = TileCaps;
     const dim3 grid((unsigned)(c.ntiles * (CP::TP / c.tp)), (unsigned)c.nf);
     c.pl_launched = 1;
-    hipLaunchKernelGGL((k_gather_tile<D, OD, CG, NQ, VIR, ELA, KIN, ER>), grid, dim3(CP::BLK), 0, c.stream, c.g, c.n, c.G,
+    hipLaunchKernelGGL((k_gather_tile<D, OD, CG, NQ, VIR, ELA, KIN, ER, LT>), grid, dim3(CP::BLK), 0, c.stream, c.g, c.n, c.G,
                        c.grid, c.tiles, c.tperm, c.tp, c.R, c.gld, c.cgnorm, c.cstart, c.spos, c.skin, c.cap,
                        c.bcount, (const ER *)c.bonds, c.out, c.flags);
 }

@@ -128,8 +128,10 @@ __device__ __forceinline__ double uniform(double v)
 // sp, kinetic terms sk, bond counts bc, entries bd; out's field pointers at
 // the frame's first value) for slots j0 .. j0 + tp - 1 of tile record tr (tp:
 // 64, 16 or 4, j0 a multiple of it), whose grid points are tperm[0 .. 63],
-// and stores its counts at out.wave_counts[2 wi ..].
-template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
+// and stores its counts at out.wave_counts[2 wi ..].  LT: FP32 terms rounded
+// as the lane gather of two points a lane rounds them, so that an engine whose
+// gather was not chosen may take either.
+template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
 __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__restrict__ grid,
                                                  const TileRec &tr, const int *__restrict__ tperm, int j0, int tp,
                                                  const GLRule &R, const double *__restrict__ gld, double cgnorm,
@@ -298,7 +300,9 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                     if constexpr (FOLD)
 #pragma unroll
                         for (int q = 0; q < 3; ++q) Aq[q] = A * R.oct_a[q];
-                    auto one = [&](const ER (&Gv)[GV], auto O, auto odd) {
+                    // site: 0 and 1, the loop's even and odd groups; 2, the
+                    // last of an odd number of groups
+                    auto one = [&](const ER (&Gv)[GV], auto O, auto site) {
                         constexpr int o = decltype(O)::value;
                         const ER *e = Gv + o;
                         ER C = e[0] * e[0];
@@ -309,9 +313,13 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                         // contracts each copy: results of earlier builds
                         // repeat bit for bit with y's product rounded first
                         // in the odd groups and in 3D without elastic terms,
-                        // x's elsewhere.
+                        // x's elsewhere.  The lane gather's virial forms have
+                        // y's rounded first, but for the last of an odd number
+                        // of groups in 3D without elastic terms.
+                        constexpr int S = decltype(site)::value;
+                        constexpr bool YF = LT ? D == 2 || ELA || S != 2 : (D == 3 && !ELA) || S == 1;
                         ER B;
-                        if constexpr ((D == 3 && !ELA) || decltype(odd)::value) B = fma(ta[0], e[0], ta[1] * e[1]);
+                        if constexpr (YF) B = fma(ta[0], e[0], ta[1] * e[1]);
                         else B = fma(ta[1], e[1], ta[0] * e[0]);
                         if constexpr (D == 3) B = fma(ta[2], e[2], B);
                         ER wq;
@@ -363,14 +371,14 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                             }
                         }
                     };
-                    auto group = [&](const ER (&Gv)[GV], int kk2, auto odd) {
-                        one(Gv, std::integral_constant<int, 0>(), odd);
+                    auto group = [&](const ER (&Gv)[GV], int kk2, auto site) {
+                        one(Gv, std::integral_constant<int, 0>(), site);
                         if constexpr (GRP >= 2)
-                            if (GRP * kk2 + 1 < nb) one(Gv, std::integral_constant<int, ES>(), odd);
+                            if (GRP * kk2 + 1 < nb) one(Gv, std::integral_constant<int, ES>(), site);
                         if constexpr (GRP >= 3)
-                            if (GRP * kk2 + 2 < nb) one(Gv, std::integral_constant<int, 2 * ES>(), odd);
+                            if (GRP * kk2 + 2 < nb) one(Gv, std::integral_constant<int, 2 * ES>(), site);
                         if constexpr (GRP >= 4)
-                            if (GRP * kk2 + 3 < nb) one(Gv, std::integral_constant<int, 3 * ES>(), odd);
+                            if (GRP * kk2 + 3 < nb) one(Gv, std::integral_constant<int, 3 * ES>(), site);
                     };
                     const ER *ptr = bd + (size_t)s_wid[slot] * cap * ES;
                     const int ng = (nb + GRP - 1) / GRP;
@@ -378,11 +386,11 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                     int kk2 = 0;
                     for (; kk2 + 1 < ng; kk2 += 2) {
                         load_entry<ER, GV>(ptr + (size_t)(kk2 + 1) * GV, E1);
-                        group(E0, kk2, std::false_type());
+                        group(E0, kk2, std::integral_constant<int, 0>());
                         if (kk2 + 2 < ng) load_entry<ER, GV>(ptr + (size_t)(kk2 + 2) * GV, E0);
-                        group(E1, kk2 + 1, std::true_type());
+                        group(E1, kk2 + 1, std::integral_constant<int, 1>());
                     }
-                    if (kk2 < ng) group(E0, kk2, std::false_type());
+                    if (kk2 < ng) group(E0, kk2, std::integral_constant<int, 2>());
                 }
 #pragma unroll
                 for (int q = 0; q < KT; ++q)
@@ -679,7 +687,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
 // One frame per y row; block x takes part b mod (64 / tp) of tile b / (64 /
 // tp), b = xcd_tile(x, gridDim.x), so each XCD works through a contiguous
 // eighth of the frame's tiles.
-template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER>
+template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
 __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gather_tile(
     Geom g, int n, int G, const double *__restrict__ grid, const TileRec *__restrict__ tiles,
     const int *__restrict__ tperm, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
@@ -696,7 +704,7 @@ __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gat
     if (ELA) of.ela = out.ela + oo;
     if (KIN) of.kin = out.kin + oo;
     const int b = xcd_tile(blockIdx.x, gridDim.x), sub = kTilePoints / tp, k = b / sub;
-    gather_tile_body<D, OD, CG, NQ, VIR, ELA, KIN, ER>(
+    gather_tile_body<D, OD, CG, NQ, VIR, ELA, KIN, ER, LT>(
         g, grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - k * sub) * tp, tp, R, gld, cgnorm,
         cstart + (size_t)f * (g.ncell + 1), spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, bcount + fo,
         bonds + fo * (size_t)cap * ES, of, (size_t)blockIdx.y * gridDim.x + blockIdx.x, overflow);

@@ -85,3 +85,49 @@ def test_noalloc_refuses_a_frame_larger_than_its_scratch(gpu):
     out = torch.zeros((1, 64, 2, 2), dtype=torch.float64, device=dev)
     with pytest.raises(engine.PGTError, match="PGT_ERR_RANGE"):
         e.compute_frames_noalloc(1, N, pos, diam, fields=("virial",), d_virial=out)
+
+
+def test_noalloc_takes_the_largest_frame_by_default_too(gpu):
+    """The largest frame that fits the fixed work memory with the lane gather:
+    an engine whose gather was not chosen takes it as well.  The other gather's
+    counters (30 KB more on this grid, 65 particles' worth) do not fit beside
+    it.  The same launches run on both engines, so the fields are equal."""
+    import torch
+
+    dev = torch.device("cuda:0")
+    N = 160_000
+    s = workload.make_system(N, 2, 5)
+    pos = torch.tensor(s["pos"], dtype=torch.float64, device=dev)
+    diam = torch.tensor(s["diam"], dtype=torch.float64, device=dev)
+    order = torch.randperm(N, generator=torch.Generator().manual_seed(5)).to(dev)
+    grid = workload.cartesian_grid_2d(np.sqrt(N), 200)
+    engines = {}
+    for mode in ("lane", None):
+        e = engines[mode] = engine.Engine(dim=2, max_rcut=1.25 * 1.62)
+        if mode:
+            e.set_gather_mode(mode)
+        e.set_box([np.sqrt(N), np.sqrt(N), 1.0], [1, 1, 0])
+        e.set_grid(grid)
+
+    def fields(mode, n):
+        out = torch.full((1, len(grid), 2, 2), np.nan, dtype=torch.float64, device=dev)
+        p, d = pos[order[:n]].contiguous(), diam[order[:n]].contiguous()
+        torch.cuda.synchronize()
+        try:
+            engines[mode].compute_frames_noalloc(1, n, p, d, fields=("virial",), d_virial=out)
+        except engine.PGTError as err:
+            assert "PGT_ERR_RANGE" in str(err)
+            return None
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    lo, hi = 60_000, N
+    assert fields("lane", lo) is not None and fields("lane", hi) is None
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if fields("lane", mid) is None else (mid, hi)
+    print("noalloc: largest 2D frame %d particles" % lo, flush=True)
+    a, b = fields("lane", lo), fields(None, lo)
+    assert b is not None
+    assert np.isfinite(a).all() and np.array_equal(a, b)
+    assert fields(None, hi) is None
