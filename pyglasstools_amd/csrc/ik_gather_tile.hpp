@@ -713,16 +713,17 @@ __global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gat
 // The sweep's field gather (2D or 3D, virial and/or kinetic): each
 // workgroup finds its system, frame and tile in the sweep's table
 // (ik_sweep.hpp).  Padding workgroups store zero counts for their slot, so
-// k_reduce_stats can read every slot.  Three waves per SIMD: the system's
+// k_reduce_stats can read every slot.  Four waves per SIMD in 2D: the system's
 // geometry and pointers come from the table and stay in registers (a kernel
-// argument would be reloaded instead), which at the single-system kernel's
-// four waves spills 24 bytes a lane in the 2D FP64 form; with the room of
-// three there is no spill, and the eight-system 2D sweep's gather takes
-// 5.87 ms against 5.89 at four.
-constexpr int kSweepGatherWaves = 3;
+// argument would be reloaded instead), so the forms with both fields spill 28
+// to 36 bytes a lane, and are the faster for the fourth wave: the eight-system
+// sweep's job 1,246 us at three, 1,188 at four; with 125 frames a system, gather
+// 4.15 -> 3.85 ms FP64, 3.62 -> 3.22 FP32 form.  3D: three, as the single-system
+// kernel.
+constexpr int sweep_gather_waves(int D) { return D == 2 ? 4 : 3; }
 
 template <int D, int OD, bool VIR, bool KIN, typename ER>
-__global__ __launch_bounds__(64, kSweepGatherWaves) void k_sweep_gather(
+__global__ __launch_bounds__(64, sweep_gather_waves(D)) void k_sweep_gather(
     const SweepSys *__restrict__ T, int ns, const TileRec *__restrict__ tiles, const int *__restrict__ tperm,
     GLRule R, const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap, const int *__restrict__ bcount,
     const ER *__restrict__ bonds, unsigned long long *__restrict__ wave_counts,
