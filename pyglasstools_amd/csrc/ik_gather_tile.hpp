@@ -89,12 +89,17 @@ __device__ __forceinline__ T wave_min(T v)
 // without elastic terms (a few registers spilled at most) and for the 3D FP32
 // virial form (126 registers, no spill; 131 and three waves unbounded, with
 // the gather 7% slower on the 3D N = 131,072 job), which hides more memory
-// latency; the others are left to the compiler (two or three: the 3D FP64
-// virial form would spill 88 bytes a lane at four).
+// latency; three for the 3D FP64 virial + kinetic form (184 registers and two
+// waves unbounded, 36 bytes a lane spilled: N = 20,011, 37^3 grid, 5 frames, the
+// job 455 -> 446 us; N = 19,459, 18^3, 19 frames 454 -> 443); the others are left
+// to the compiler (one to three: the 3D FP64 virial form would spill 88 bytes a
+// lane at four).
 template <int D, bool ELA, bool KIN, typename ER>
 struct TileWaves {
     static constexpr bool F32 = std::is_same<ER, float>::value;
-    static constexpr int value = ((D == 2 && !ELA) || (D == 3 && F32 && !ELA && !KIN)) ? 4 : 1;
+    static constexpr int value = ((D == 2 && !ELA) || (D == 3 && F32 && !ELA && !KIN)) ? 4
+                               : D == 3 && !F32 && !ELA && KIN                                ? 3
+                                                                                              : 1;
 };
 
 // Cells of one axis that hold every particle within r of [lo, hi]: w0 (in
