@@ -91,15 +91,17 @@ __device__ __forceinline__ T wave_min(T v)
 // the gather 7% slower on the 3D N = 131,072 job), which hides more memory
 // latency; three for the 3D FP64 virial + kinetic form (184 registers and two
 // waves unbounded, 36 bytes a lane spilled: N = 20,011, 37^3 grid, 5 frames, the
-// job 455 -> 446 us; N = 19,459, 18^3, 19 frames 454 -> 443); the others are left
+// job 455 -> 446 us; N = 19,459, 18^3, 19 frames 454 -> 443; Rect, 5 nodes, 641 ->
+// 555) but for the Mollifier kernel, which would spill 144 (10 nodes 1,969 ->
+// 2,014 us); in 2D that kernel is as fast at three as at four; the others are left
 // to the compiler (one to three: the 3D FP64 virial form would spill 88 bytes a
 // lane at four).
-template <int D, bool ELA, bool KIN, typename ER>
+template <int D, int CG, bool ELA, bool KIN, typename ER>
 struct TileWaves {
     static constexpr bool F32 = std::is_same<ER, float>::value;
-    static constexpr int value = ((D == 2 && !ELA) || (D == 3 && F32 && !ELA && !KIN)) ? 4
-                               : D == 3 && !F32 && !ELA && KIN                                ? 3
-                                                                                              : 1;
+    static constexpr bool four = (D == 2 && !ELA) || (D == 3 && F32 && !ELA && !KIN);
+    static constexpr bool three = D == 3 && CG != 2 && !F32 && !ELA && KIN;
+    static constexpr int value = four ? 4 : three ? 3 : 1;
 };
 
 // Cells of one axis that hold every particle within r of [lo, hi]: w0 (in
@@ -693,7 +695,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
 // tp), b = xcd_tile(x, gridDim.x), so each XCD works through a contiguous
 // eighth of the frame's tiles.
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
-__global__ __launch_bounds__(64, (TileWaves<D, ELA, KIN, ER>::value)) void k_gather_tile(
+__global__ __launch_bounds__(64, (TileWaves<D, CG, ELA, KIN, ER>::value)) void k_gather_tile(
     Geom g, int n, int G, const double *__restrict__ grid, const TileRec *__restrict__ tiles,
     const int *__restrict__ tperm, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
     const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap,
