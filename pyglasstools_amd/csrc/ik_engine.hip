@@ -612,6 +612,7 @@ struct JobShape {
     int block, pl;
     bool tile;       // the item-balanced tile gather
     int tp;          // its grid points per workgroup of kTileThreads lanes
+    int unit;        // and of the window that orders its sums
     int64_t gwaves;  // gather wavefronts per frame
     bool qag_global; // adaptive rule: interval tables of the caller's limit in e->d_qag
 };
@@ -638,34 +639,56 @@ bool default_tile(const pgt_ik_engine *e, const JobShape &j, unsigned fields)
            tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32);
 }
 
-// Grid points per workgroup of the tile gather: whole tiles (64), or parts of
-// them.  Two things ask for parts.  `tiles` (of all frames of a launch) must
-// fill the GPU's 4,096 wavefront slots or the launch is as long as one
-// wavefront: gather of one frame, parts of 64 / 32 / 16 / 4 points: 2D N = 2,000,
-// 16 tiles 30 / - / 14 / 8 us; N = 16,384, 256 tiles 28 / 20 / 16 / 16; N = 65,536,
-// 1,024 tiles 34 / 27 / 26 / 52; 2,048 tiles 40 / 37 / 45 / 96; 3,072 tiles
-// 48 / 54 / 63 / 138.  And on a coarse grid a whole tile's window holds many
-// particles that are near only a few of its points: with n particles per
-// frame, a part's window should hold at most about 600: N = 98,304, grid
-// spacing 2.4 (447 particles in a whole tile's window) 127 / 131 / 137 / 224 us,
-// 3.5 (812, 413 in half of it) 269 / 229 / 223 / 279, 4.9 (349 in a quarter)
-// 197 / 145 / 149 / 158, 7.8 (110 in a row of four) 391 / 334 / 270 / 223; 3D N = 131,072,
-// spacing 1.6 (708, 447) 360 / 328 / 340 / 548, 2.7 (534 in a quarter)
-// 381 / 372 / 360 / 476, 4.6 (285 in a row of four) 669 / 375 / 333 / 276.
-int tile_part(const pgt_ik_engine *e, const Geom &g, int D, int64_t n, int64_t tiles)
+// The tile gather's unit: the grid points whose window orders the sums, whole
+// tiles (64) or parts of them, and the most that a workgroup takes.  On a coarse
+// grid a whole tile's window holds many particles that are near only a few of
+// its points, and a smaller part scans the unit's window all the same.  Gather
+// in launches that fill the GPU, units of 64 / 32 / 16 / 4 points: N = 98,304,
+// grid spacing 2.4 (447 particles in a whole tile's window) 127 / 131 / 137 / 224
+// us, 3.5 (812, 413 in half of it) 269 / 229 / 223 / 279, 4.9 (349 in a quarter)
+// 197 / 145 / 149 / 158, 7.8 (110 in a row of four) 391 / 334 / 270 / 223; N = 65,536,
+// spacing 6.6 (561 in a quarter) - / - / 66 / 44; 3D N = 131,072, spacing 1.6 (708,
+// 447) 360 / 328 / 340 / 548, 2.7 (534 in a quarter) 381 / 372 / 360 / 476, 4.6 (285 in a
+// row of four) 669 / 375 / 333 / 276; N = 8,000, spacing 1.05 (367, 259) 343 / 368 /
+// 441 / -.  In launches that do not (parts of 4, 16 and 16 points), with units
+// of 64 / 32 / 16: N = 65,536, one frame, spacing 2.6 (488, 287) 32 / 21 / -; 3D N
+// = 4,000, one frame, spacing 1.4 (575, 376) - / 41 / 36; N = 131,072, two, spacing
+// 1.75 (753, 471) - / 169 / 140.  So a unit's window holds at most about 300
+// particles in 2D and 400 in 3D; the step to rows of four, which overlap most,
+// is taken above 500 and 600.  A window that reaches around a periodic axis
+// holds the whole axis, at the minimum image: a smaller unit there too, if that
+// avoids it.  The unit knows nothing of the launch: the sums must not depend on
+// how many frames or systems it holds.
+int tile_unit(const pgt_ik_engine *e, const Geom &g, int D, int64_t n)
 {
-    int tp = tiles < 192 ? 4 : tiles < 1536 ? 16 : tiles < 3072 ? 32 : 64;
+    int unit = kTilePoints;
     double density = (double)n;
     for (int a = 0; a < D; ++a) density /= g.L[a];
-    for (; tp > 4; tp = tp == 16 ? 4 : tp / 2) {
-        // steps of the lattice that a part spans along each axis
-        const double span[3] = {D == 2 && tp >= 32 ? 7.0 : 3.0, D == 2 ? (tp == 64 ? 7.0 : 3.0) : (tp >= 32 ? 3.0 : 1.0),
-                                tp == 64 ? 3.0 : 1.0};
+    for (; unit > 4; unit = unit == 16 ? 4 : unit / 2) {
+        // steps of the lattice that a unit spans along each axis
+        const double span[3] = {D == 2 && unit >= 32 ? 7.0 : 3.0,
+                                D == 2 ? (unit == 64 ? 7.0 : 3.0) : (unit >= 32 ? 3.0 : 1.0), unit == 64 ? 3.0 : 1.0};
         double window = density;
-        for (int a = 0; a < D; ++a) window *= std::min(g.L[a], span[a] * e->grid_step[a] + 2.0 * g.rc);
-        if (window <= 600.0) break;
+        bool around = false;
+        for (int a = 0; a < D; ++a) {
+            const double reach = span[a] * e->grid_step[a] + 2.0 * g.rc;
+            window *= std::min(g.L[a], reach);
+            around = around || (g.periodic[a] && reach >= 0.99 * g.L[a] && 2.0 * g.rc < 0.99 * g.L[a]);
+        }
+        if (window <= (D == 2 ? (unit > 16 ? 300.0 : 500.0) : (unit > 16 ? 400.0 : 600.0)) && !around) break;
     }
-    return tp;
+    return unit;
+}
+
+// Grid points per workgroup of the tile gather: the unit, or parts of it where
+// the `tiles` (of all frames of a launch) would not fill the GPU's 4,096
+// wavefront slots and the launch would be as long as one wavefront.  Gather of
+// one frame, parts of 64 / 32 / 16 / 4 points: 2D N = 2,000, 16 tiles 30 / - / 14 /
+// 8 us; N = 16,384, 256 tiles 28 / 20 / 16 / 16; N = 65,536, 1,024 tiles 34 / 27 /
+// 26 / 52; 2,048 tiles 40 / 37 / 45 / 96; 3,072 tiles 48 / 54 / 63 / 138.
+int tile_part(int unit, int64_t tiles)
+{
+    return std::min(unit, tiles < 192 ? 4 : tiles < 1536 ? 16 : tiles < 3072 ? 32 : 64);
 }
 
 // Frames per launch of a job where the caller set none: all of them up to
@@ -725,7 +748,8 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     if (j.tile) {
         j.block = kTileThreads;
         j.pl = 1;
-        j.tp = tile_part(e, j.g, j.D, n, (int64_t)e->ntiles * nf);
+        j.unit = tile_unit(e, j.g, j.D, n);
+        j.tp = tile_part(j.unit, (int64_t)e->ntiles * nf);
         j.gwaves = (int64_t)e->ntiles * (kTilePoints / j.tp);
     } else {
         const int64_t lanes = (e->G + j.pl - 1) / j.pl;
@@ -933,6 +957,7 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
     c.tperm = e->d_tperm.p;
     c.ntiles = e->ntiles;
     c.tp = j.tp;
+    c.unit = j.unit;
     c.lane_terms = e->gather_mode == -1;
     c.R.n = (int)e->gl_s.size();
     for (int k = 0; k < c.R.n && k < kMaxQArg; ++k) {
@@ -2335,7 +2360,8 @@ int pgt_ik_sweep_create(int nsys, const pgt_ik_sweep_system *systems, unsigned f
         S.bpf[SW_SORT] = S.nchunk;
         S.bpf[SW_FINISH] = (S.n + 255) / 256;
         S.bpf[SW_BONDS] = (S.n + kBondBlock - 1) / kBondBlock;
-        S.tp = tile_part(systems[k].engine, S.g, D, S.n, tiles);
+        S.unit = tile_unit(systems[k].engine, S.g, D, S.n);
+        S.tp = tile_part(S.unit, tiles);
         S.bpf[SW_GATHER] = systems[k].engine->ntiles * (kTilePoints / S.tp);
         for (int st = 0; st < SW_NSTAGE; ++st) {
             const int64_t nb = (st == SW_SORT || st == SW_FINISH)

@@ -67,7 +67,7 @@ void launch_tile_t(const LaunchCtx &c)
     const dim3 grid((unsigned)(c.ntiles * (CP::TP / c.tp)), (unsigned)c.nf);
     c.pl_launched = 1;
     hipLaunchKernelGGL((k_gather_tile<D, OD, CG, NQ, VIR, ELA, KIN, ER, LT>), grid, dim3(CP::BLK), 0, c.stream, c.g, c.n, c.G,
-                       c.grid, c.tiles, c.tperm, c.tp, c.R, c.gld, c.cgnorm, c.cstart, c.spos, c.skin, c.cap,
+                       c.grid, c.tiles, c.tperm, c.tp, c.unit, c.R, c.gld, c.cgnorm, c.cstart, c.spos, c.skin, c.cap,
                        c.bcount, (const ER *)c.bonds, c.out, c.flags);
 }
 

@@ -25,7 +25,19 @@
 //    and adds it to the point's FP64 accumulators in LDS.
 //
 // The wavefront runs alone in its workgroup and every step is in a fixed
-// order, so the sums are the same from run to run.
+// order, so the sums are the same from run to run.  They are also the same
+// whatever part of a tile a workgroup takes, which depends on how many tiles a
+// launch has: the window is listed in the order, and in the batches, that the
+// tile's unit gives (the part that the particles' density asks for, whatever
+// the launch), so a point's particles lie in the same batches in the same
+// order, and a smaller part only leaves out those too far from its own points.
+// Up to four batches go through steps 2 to 4 as one list, each ordered by
+// itself.  Parts scan their unit's cells for it: gather of one frame, their
+// own windows alone / this: 2D N = 2,000, 32^2 grid 12 / 15 us, N = 65,536, 256^2
+// 26 / 30; 3D N = 4,000, 12^3 25 / 41, N = 20,011, 37^3 89 / 106; whole tiles, whose
+// scan is the same, take 0.5 to 2.5% longer.  (Loading a step's candidates
+// during the one before: 2D N = 2,000 15 / 15, 3D N = 20,011 106 / 108; whole
+// tiles of a 2D sweep 2% slower, from the registers.)
 //
 // Why particles, not points, are spread over the lanes in the scan: scattered
 // loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
@@ -63,11 +75,21 @@ struct TileCaps {
     static constexpr int TP = kTilePoints;    // most grid points of a tile
     static constexpr int MAXW = 128;          // window particles listed at a time
     static constexpr int MAXI = 1024;         // items listed at a time
+    static constexpr int NBATCH = 4;          // most batches of a list
+    static constexpr int NKEY = 32;           // classes of bond counts (count_class)
     static constexpr int SBITS = 8;           // item word: window slot | point << SBITS
     static constexpr int MAXNB = 255;         // bond count of a particle (one byte); more: overflow
     static_assert(TP == 64 && BLK == 64, "one wavefront, masks of 64 points");
     static_assert(MAXW <= (1 << SBITS) && MAXW % 64 == 0, "window slots of an item word");
 };
+
+// The class that orders particles by bond count (at most MAXNB): the count
+// itself up to 16, then four classes to each doubling.
+__device__ __forceinline__ int count_class(int nb)
+{
+    const int e = 31 - __clz(nb | 1);
+    return nb < 16 ? nb : 4 * e + ((nb >> (e - 2)) & 3);
+}
 
 template <typename T>
 __device__ __forceinline__ T wave_max(T v)
@@ -134,14 +156,16 @@ __device__ __forceinline__ double uniform(double v)
 // The body works on one frame's arrays (cell starts st, sorted positions
 // sp, kinetic terms sk, bond counts bc, entries bd; out's field pointers at
 // the frame's first value) for slots j0 .. j0 + tp - 1 of tile record tr (tp:
-// 64, 16 or 4, j0 a multiple of it), whose grid points are tperm[0 .. 63],
-// and stores its counts at out.wave_counts[2 wi ..].  LT: FP32 terms rounded
-// as the lane gather of two points a lane rounds them, so that an engine whose
-// gather was not chosen may take either.
+// 64, 32, 16 or 4, j0 a multiple of it), whose grid points are tperm[0 .. 63],
+// and stores its counts at out.wave_counts[2 wi ..].  unit, at least tp, of the
+// same sizes: the slots whose window sets the order of the sums.  LT: FP32
+// terms rounded as the lane gather of two points a lane rounds them, so that an
+// engine whose gather was not chosen may take either.
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
 __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__restrict__ grid,
                                                  const TileRec &tr, const int *__restrict__ tperm, int j0, int tp,
-                                                 const GLRule &R, const double *__restrict__ gld, double cgnorm,
+                                                 int unit, const GLRule &R, const double *__restrict__ gld,
+                                                 double cgnorm,
                                                  const int *__restrict__ st, const double *__restrict__ sp,
                                                  const double *__restrict__ sk, int cap,
                                                  const int *__restrict__ bc, const ER *__restrict__ bd,
@@ -163,12 +187,17 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     constexpr int GV = LY::GV;    // values per read group
 
     __shared__ double s_pt[64][D];               // the points
+    __shared__ double s_box[2 * D];              // their box: centre, half lengths
     __shared__ double s_acc[64][KTA];            // their accumulators
     __shared__ double s_wp[MAXW][D];             // window: positions,
     __shared__ int s_wid[MAXW];                  // particles,
-    __shared__ unsigned char s_wnb[MAXW];        // bond counts,
+    __shared__ unsigned char s_wnb[MAXW];        // their batches, then bond counts,
     __shared__ unsigned short s_wof[MAXW];       // first items
-    __shared__ int s_bucket[64];                 // items per bond count, then their offsets
+    // items per batch and class of bond counts, then their offsets: two
+    // 16-bit counters a word (a list has at most MAXW TP of them)
+    constexpr int NBATCH = CP::NBATCH, NKEY = CP::NKEY;
+    __shared__ unsigned s_bucket[64];
+    static_assert(NBATCH * NKEY == 128 && MAXW * CP::TP <= 65535, "two counters a lane");
     // items in order, and one past the list for those of another piece;
     // while the window is filled, the segments' first candidates and particles
     __shared__ union {
@@ -191,49 +220,57 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     }
     const bool product = tr.product != 0;
 
-    // bounding box of the points: centre xc, half lengths xh.  When the box
-    // and its ball fit in less than a period (near), a particle has one image
-    // that can be inside any of the balls, the one nearest to xc.
+    // bounding box of the unit's points: centre xc, half lengths xh.  When the
+    // box and its ball fit in less than a period (near), a particle has one
+    // image that can be inside any of the balls, the one nearest to xc.
+    const bool part = tp < unit;
     double xc[D], xh[D];
     int w0[3] = {0, 0, 0}, wn[3] = {1, 1, 1};
     bool near = true;
     {
-        double xg[D], lo[D], hi[D];
+        const int u0 = j0 & ~(unit - 1);
+        const bool ulive = gp >= 0 && l >= u0 && l < u0 + unit;
+        double xg[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            xg[a] = live ? grid[(size_t)gp * 3 + a] : 0.0;
+            xg[a] = ulive ? grid[(size_t)gp * 3 + a] : 0.0;
             s_pt[l][a] = live ? xg[a] : __builtin_nan("");
         }
 #pragma unroll
         for (int k = 0; k < KTA; ++k) s_acc[l][k] = 0.0;
-        if (product) {
-            // over the axes' coordinates (lines without points are NaN,
-            // which the minimum and the maximum pass over)
+        // box of slots b .. b + nb - 1; in: whether the lane holds one of their points
+        auto box = [&](int b, int nb, bool in, double (&lo)[D], double (&hi)[D]) {
+            if (product) {
+                // over the axes' coordinates (lines without points are NaN,
+                // which the minimum and the maximum pass over)
 #pragma unroll
-            for (int a = 0; a < D; ++a) lo[a] = __builtin_huge_val(), hi[a] = -__builtin_huge_val();
-            const int q0 = j0 >> 4, q1 = (j0 + tp - 1) >> 4;
-            for (int q = q0; q <= q1; ++q) {
-                const double *ax = tr.ax[q];
-                // a row of four points (tp 4) has one y and one z
-                const int r = tp == 4 ? (j0 >> 2) & 3 : -1;
+                for (int a = 0; a < D; ++a) lo[a] = __builtin_huge_val(), hi[a] = -__builtin_huge_val();
+                const int q0 = b >> 4, q1 = (b + nb - 1) >> 4;
+                for (int q = q0; q <= q1; ++q) {
+                    const double *ax = tr.ax[q];
+                    // a row of four points (nb 4) has one y and one z
+                    const int r = nb == 4 ? (b >> 2) & 3 : -1;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int a = k < 4 ? 0 : ((D == 2 || k < 6) ? 1 : D - 1);
-                    if (r >= 0 && k >= 4 && (D == 2 ? k - 4 != r : a == 1 ? k - 4 != (r & 1) : k - 6 != r >> 1))
-                        continue;
-                    lo[a] = fmin(lo[a], ax[k]);
-                    hi[a] = fmax(hi[a], ax[k]);
+                    for (int k = 0; k < 8; ++k) {
+                        const int a = k < 4 ? 0 : ((D == 2 || k < 6) ? 1 : D - 1);
+                        if (r >= 0 && k >= 4 && (D == 2 ? k - 4 != r : a == 1 ? k - 4 != (r & 1) : k - 6 != r >> 1))
+                            continue;
+                        lo[a] = fmin(lo[a], ax[k]);
+                        hi[a] = fmax(hi[a], ax[k]);
+                    }
+                }
+            } else {
+                const int first = __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(in)) - 1;
+#pragma unroll
+                for (int a = 0; a < D; ++a) {
+                    const double v = in ? xg[a] : __shfl(xg[a], first, 64);
+                    lo[a] = wave_min(v);
+                    hi[a] = wave_max(v);
                 }
             }
-        } else {
-            const int first = __ffsll(points) - 1;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                const double v = live ? xg[a] : __shfl(xg[a], first, 64);
-                lo[a] = wave_min(v);
-                hi[a] = wave_max(v);
-            }
-        }
+        };
+        double lo[D], hi[D];
+        box(u0, unit, ulive, lo, hi);
 #pragma unroll
         for (int a = 0; a < D; ++a) {
             axis_cells(g, a, lo[a], hi[a], g.rc, w0[a], wn[a]);
@@ -244,6 +281,14 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh[a] + g.rc) < 0.999 * g.L[a]);
         }
         near = __builtin_amdgcn_ballot_w64(near) != 0ull;  // the same in every lane: a scalar
+        if (part && near) {
+            box(j0, tp, live, lo, hi);
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                s_box[a] = 0.5 * (lo[a] + hi[a]);
+                s_box[D + a] = 0.5 * (hi[a] - lo[a]);
+            }
+        }
     }
 
     // whether a window particle's image nearest to xc is not the particle
@@ -481,7 +526,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
 
     // ---- the items of window particles 0 .. nw - 1 --------------------------
     auto process = [&](int nw) {
-        s_bucket[l] = 0;
+        s_bucket[l] = 0u;
         __syncthreads();
         unsigned m[NR][2];
         int nbs[NR];
@@ -508,17 +553,18 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             if (nbc > CP::MAXNB && pc > 0) over = true;
             const int nb = min(nbc, CP::MAXNB);
             ncontrib += (unsigned long long)pc * (unsigned long long)nb;
-            nbs[r] = 63 - min(nb, 63);
+            nbs[r] = (int)s_wnb[ws] * NKEY + NKEY - 1 - count_class(nb);
             if (valid) {
                 s_wnb[slot] = (unsigned char)nb;
-                atomicAdd(&s_bucket[nbs[r]], pc);
+                atomicAdd(&s_bucket[nbs[r] >> 1], (unsigned)pc << (nbs[r] & 1) * 16);
             }
         }
         __syncthreads();
         int total;
         {
-            const int c = s_bucket[l];
-            int v = c;
+            const unsigned c = s_bucket[l];
+            const int mine = (int)(c & 0xffffu) + (int)(c >> 16);
+            int v = mine;
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
                 const int u = __shfl_up(v, off, 64);
@@ -527,7 +573,8 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             total = __builtin_amdgcn_readlane(v, 63);
             nball += (unsigned long long)total;
             __syncthreads();
-            s_bucket[l] = v - c;  // first item of the bond count
+            v -= mine;  // first items
+            s_bucket[l] = (unsigned)v | ((unsigned)v + (c & 0xffffu)) << 16;
         }
         __syncthreads();
         for (int base = 0; base < total; base += MAXI) {
@@ -540,7 +587,9 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                     // an LDS atomic; the lanes of one instruction are served
                     // in a fixed order
                     if (slot < nw) {
-                        k = atomicAdd(&s_bucket[nbs[r]], __popc(m[r][0]) + __popc(m[r][1]));
+                        const int sh = (nbs[r] & 1) * 16;
+                        const unsigned pc = (unsigned)(__popc(m[r][0]) + __popc(m[r][1]));
+                        k = (int)(atomicAdd(&s_bucket[nbs[r] >> 1], pc << sh) >> sh & 0xffffu);
                         s_wof[slot] = (unsigned short)k;
                     }
                 } else {
@@ -586,7 +635,9 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     int s0 = 0, c0 = 0;  // the next candidate: c0 of the segments from s0 on
     bool more = true;
     while (more) {
-        int nw = 0;
+        int nw = 0, nu = 0;              // particles listed, and those of the unit's window in this batch
+        int bs = s0, bc0 = c0, bw = 0;  // where the batch began: its first candidate and place
+        int nbatch = 0;
         bool full = false;
         for (more = false; s0 < nseg && !full;) {
             int b = 0, len = 0;
@@ -618,7 +669,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                 for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1)
                     if (lo + h < ns && s_u.seg.first[lo + h] <= c) lo += h;
                 const int id = s_u.seg.particle[lo] + c - s_u.seg.first[lo];
-                double x[D], d2 = 0.0;
+                double x[D], d2 = 0.0, p2 = 0.0;
 #pragma unroll
                 for (int a = 0; a < D; ++a) x[a] = sp[(size_t)id * PS + a];
                 bool shift = false;
@@ -629,23 +680,43 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                         shift = shift || y != x[a];
                         const double d = fabs(y - xc[a]) - xh[a];
                         d2 = fma(d > 0.0 ? d : d - d, d > 0.0 ? d : d - d, d2);
+                        if (part) {
+                            const double e = fabs(y - s_box[a]) - s_box[D + a];
+                            p2 = fma(e > 0.0 ? e : e - e, e > 0.0 ? e : e - e, p2);
+                        }
                     }
                 }
                 // not near: any image may matter, so every candidate is kept
-                const bool in = c0 + l < total && d2 < rr;
+                const bool inu = c0 + l < total && d2 < rr, in = inu && p2 < rr;
+                const int ku = __popcll(__builtin_amdgcn_ballot_w64(inu));
                 const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
                 const int k = __popcll(bm);
+                if (nu + ku > MAXW) {  // these candidates begin the next batch
+                    full = ++nbatch == NBATCH || !part;
+                    if (full) break;
+                    nu = 0;
+                    bs = s0;
+                    bc0 = c0;
+                    bw = nw;
+                }
                 full = nw + k > MAXW;
-                if (full) break;  // these candidates again with the next window
+                if (full) {  // the batch with the next list
+                    s0 = bs;
+                    c0 = bc0;
+                    nw = bw;
+                    break;
+                }
                 images = images || __builtin_amdgcn_ballot_w64(in && shift) != 0ull;
                 if (in) {
                     const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
                                                                       __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
                     s_wid[w] = id;
+                    s_wnb[w] = (unsigned char)nbatch;
 #pragma unroll
                     for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
                 }
                 nw += k;
+                nu += ku;
             }
             if (full) {
                 more = true;
@@ -697,7 +768,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
 template <int D, int OD, int CG, int NQ, bool VIR, bool ELA, bool KIN, typename ER, bool LT = false>
 __global__ __launch_bounds__(64, (TileWaves<D, CG, ELA, KIN, ER>::value)) void k_gather_tile(
     Geom g, int n, int G, const double *__restrict__ grid, const TileRec *__restrict__ tiles,
-    const int *__restrict__ tperm, int tp, GLRule R, const double *__restrict__ gld, double cgnorm,
+    const int *__restrict__ tperm, int tp, int unit, GLRule R, const double *__restrict__ gld, double cgnorm,
     const int *__restrict__ cstart, const double *__restrict__ spos, const double *__restrict__ skin, int cap,
     const int *__restrict__ bcount, const ER *__restrict__ bonds, GatherOut out, int *__restrict__ overflow)
 {
@@ -712,7 +783,7 @@ __global__ __launch_bounds__(64, (TileWaves<D, CG, ELA, KIN, ER>::value)) void k
     if (KIN) of.kin = out.kin + oo;
     const int b = xcd_tile(blockIdx.x, gridDim.x), sub = kTilePoints / tp, k = b / sub;
     gather_tile_body<D, OD, CG, NQ, VIR, ELA, KIN, ER, LT>(
-        g, grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - k * sub) * tp, tp, R, gld, cgnorm,
+        g, grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - k * sub) * tp, tp, unit, R, gld, cgnorm,
         cstart + (size_t)f * (g.ncell + 1), spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap, bcount + fo,
         bonds + fo * (size_t)cap * ES, of, (size_t)blockIdx.y * gridDim.x + blockIdx.x, overflow);
 }
@@ -757,7 +828,7 @@ __global__ __launch_bounds__(64, sweep_gather_waves(D)) void k_sweep_gather(
     of.wave_counts = wave_counts;
     const int sub = kTilePoints / S.tp, q = b / sub, k = S.tile0 + q;
     gather_tile_body<D, OD, 0, 5, VIR, false, KIN, ER>(
-        g, S.grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - q * sub) * S.tp, S.tp, R, nullptr, S.cgnorm,
+        g, S.grid, tiles[k], tperm + (size_t)k * kTilePoints, (b - q * sub) * S.tp, S.tp, S.unit, R, nullptr, S.cgnorm,
         cstart + (size_t)S.c0 + (size_t)f * (g.ncell + 1), spos + fo * PS, KIN ? skin + fo * KN : nullptr, cap,
         VIR ? bcount + fo : nullptr, VIR ? bonds + fo * (size_t)cap * ES : nullptr, of, blockIdx.x, overflow);
 }

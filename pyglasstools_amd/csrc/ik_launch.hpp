@@ -24,6 +24,7 @@ struct LaunchCtx {
     const int *tperm;      // grid point of each slot, kTilePoints per tile, -1: none
     int ntiles;
     int tp;            // tile gather: grid points per workgroup (a divisor of kTilePoints)
+    int unit;          // and of the window that orders its sums, at least tp
     GLRule R;
     const double *gld;
     double cgnorm;

@@ -38,7 +38,7 @@ struct SweepSys {
     int blk0[SW_NSTAGE], nblk[SW_NSTAGE], bpf[SW_NSTAGE];
     const double *grid;  // the sweep's copy of the system's grid (x, y, z per point)
     int tile0;           // its first tile in the sweep's copy of the tiles
-    int tp;              // grid points per gather workgroup
+    int tp, unit;        // grid points per gather workgroup, and of the window that orders its sums
     const double *pos, *diam, *mass, *vel;  // caller's frame-stacked inputs
     double *vir, *kin;                      // caller's frame-stacked outputs
 };
