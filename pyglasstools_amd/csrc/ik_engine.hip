@@ -1077,6 +1077,7 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     if (j.pairs && e->cap < 1) e->cap = j.D == 3 ? 32 : 16;
     const Deliver dv{e->h_counts, fs.host};
     int mx = 0;
+    bool allow_tile = true;
     for (int attempt = 0; attempt < 4; ++attempt) {
         Work w{};
         if ((rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, false, w))) return rc;
@@ -1119,11 +1120,13 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
             // a tile item had more bonds than its one-byte count holds:
             // run the job again with the lane gather
             if (!j.tile) return fail(PGT_ERR_STATE, "tile overflow reported by a lane gather");
-            j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes), false);
+            allow_tile = false;
         } else if (!grow) {
             break;
         }
         if (grow) e->cap = ((mx + 7) / 8) * 8;
+        // the gather follows the capacity, as it will when the job is enqueued
+        j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes), allow_tile);
         if (attempt == 3) return fail(PGT_ERR_HIP, "bond list capacity did not settle");
     }
     const unsigned long long h[2] = {e->h_counts[1], e->h_counts[2]};

@@ -106,3 +106,37 @@ def test_sweep_takes_other_parts_than_its_engines(gpu, dim, spec):
             one = _fields(y["engine"], y["frames"], fields, first=f, count=1)
             for k in fields:
                 assert np.array_equal(y[k][f].cpu().numpy(), one[k][0]), (q, f, k)
+
+
+@pytest.mark.parametrize("members", [249, 250, 256])
+def test_an_enqueued_job_repeats_the_one_that_grew_its_capacity(gpu, members):
+    """A cluster whose particles have 248, 249 or 255 bonds, for which the bond
+    capacity grows to 248 or 256 slots, on both sides of the tile gather's 255:
+    the enqueued job takes the gather that the growing one took, so the same
+    bits."""
+    import torch
+
+    N = 700
+    s = _frames(2, N, 1, 14000)[0]
+    # the cluster: a square lattice of spacing 0.05 inside every pair's cutoff
+    # (1.25 x 0.73), in place of `members` particles
+    q = np.argsort(np.abs(s["pos"]).max(1))[:members]
+    s["pos"][q, 0], s["pos"][q, 1] = 0.05 * (np.arange(members) % 16 - 7.5), 0.05 * (np.arange(members) // 16 - 7.5)
+    s["pos"][q, :2] *= 0.5
+    s["pos"][q, :2] += 1e-3 * np.random.default_rng(1).normal(size=(members, 2))
+    far = np.setdiff1d(np.nonzero(np.abs(s["pos"][:, :2]).max(1) < 4.0)[0], q)
+    s["pos"][far, :2] += 8.0
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    e.set_box(s["L"], s["periodic"])
+    e.set_grid(_grid("lattice", s["L"][0], 2, 33))
+    grown = _fields(e, [s], ("virial",))["virial"]
+    st = e.stats()
+    print("enqueue after growth: members %d, most bonds %d, capacity %d" % (members, st["max_bonds"], st["bond_capacity"]),
+          flush=True)
+    assert members - 1 <= st["max_bonds"] <= 255 and st["bond_capacity"] == (248 if members == 249 else 256)
+    out = torch.full((1, e.G, 2, 2), np.nan, dtype=torch.float64, device="cuda")
+    pos, diam = _stack([s], "pos"), _stack([s], "diam")
+    torch.cuda.synchronize()
+    e.enqueue_frames(1, N, pos, diam, fields=("virial",), d_virial=out)
+    e.finish()
+    assert np.array_equal(out.cpu().numpy(), grown)
