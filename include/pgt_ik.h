@@ -292,7 +292,8 @@ int pgt_ik_sweep_get_stats(pgt_ik_sweep *s, pgt_ik_stats *out);
  * reach (1: cells of at least the search radius, searched one cell to each
  * side; 2: cells of at least half of it, two to each side); 0 keeps the
  * current choice.  Frames per launch not set: as many as make about two
- * million particles (or grid points), at least eight.  Used by the autotuner.  No counterpart in the reference. */
+ * million particles (or grid points) and 4 GB of work arrays, at least eight,
+ * at most 65,528.  Used by the autotuner.  No counterpart in the reference. */
 int pgt_ik_set_tuning(pgt_ik_engine *e, int threads_per_block, int frames_per_launch, int points_per_lane,
                       int cell_reach);
 

@@ -691,18 +691,6 @@ int tile_part(int unit, int64_t tiles)
     return std::min(unit, tiles < 192 ? 4 : tiles < 1536 ? 16 : tiles < 3072 ? 32 : 64);
 }
 
-// Frames per launch of a job where the caller set none: all of them up to
-// about 2 M particles (or grid points) a launch, whose bond entries take
-// 0.8 GB in 2D and 2.1 GB in 3D; at least eight.  24 frames of N = 16,384 with
-// elastic terms took 518 us in three launches of eight with the lane gather,
-// 253 us in one launch with the tile gather.
-int launch_frames(const pgt_ik_engine *e, int64_t n, int nframes)
-{
-    if (e->frames_per_launch > 0) return e->frames_per_launch;
-    const int64_t per_frame = std::max<int64_t>(1, std::max(n, e->G));
-    return (int)std::min<int64_t>(nframes, std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
-}
-
 // Particles per wavefront of the bond kernel: one a lane, or a quarter of that
 // where the GPU is nearly empty even so (512 wavefronts, half of its SIMDs) and
 // the time is one wavefront's: fewer candidates to stage and fewer rounds of
@@ -795,6 +783,29 @@ void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, size_t
     // wavefronts any shape launches)
     out[W_WCOUNTS] = 2 * std::max<size_t>(nw_gather_max, 1) * sizeof(unsigned long long);
     out[W_WMAX] = std::max<size_t>(nw_bonds, 1) * sizeof(int);
+}
+
+// Frames per launch of a job where the caller set none: all of them up to
+// about 2 M particles (or grid points) a launch and kLaunchBytes of work
+// arrays (2 M particles take 1 GB in 2D and 2.3 GB in 3D at the first bond
+// capacity, more with elastic terms, in dense systems and in wide boxes of many
+// cells), at least eight, and at most what a grid's y takes in frame_rows.  24
+// frames of N = 16,384 with elastic terms took 518 us in three launches of
+// eight with the lane gather, 253 us in one launch with the tile gather.
+constexpr int kMaxLaunchFrames = 65528;
+constexpr size_t kLaunchBytes = (size_t)4 << 30;
+
+int launch_frames(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nframes, int cap)
+{
+    if (e->frames_per_launch > 0) return std::min(e->frames_per_launch, nframes);
+    const int64_t per_frame = std::max<int64_t>(1, std::max(n, e->G));
+    const int f = (int)std::min<int64_t>(std::min(nframes, kMaxLaunchFrames),
+                                         std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
+    if (f <= 8) return f;
+    size_t b[W_NARRAYS], frame = 0;
+    work_bytes(job_shape(e, fields, z_flat, n, f), 1, n, e->G, cap, b);
+    for (size_t x : b) frame += x;
+    return (int)std::max<size_t>(8, std::min<size_t>((size_t)f, kLaunchBytes / frame));
 }
 
 constexpr size_t kWorkAlign = 256;
@@ -1068,19 +1079,24 @@ int run_batch(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, const
 // capacity once; on overflow grow it and run the whole job again.
 int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 {
-    int fpl = launch_frames(e, fs.n, fs.nframes);
-    int nb = (fs.nframes + fpl - 1) / fpl;
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes));
     int rc;
-    if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
     if ((rc = e->d_maxcount.ensure(2)) || (rc = e->d_stats.ensure(2))) return rc;
+    int fpl = fs.nframes, nb = 1;
+    bool allow_tile = true, qag_global = false;
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
     if (j.pairs && e->cap < 1) e->cap = j.D == 3 ? 32 : 16;
     const Deliver dv{e->h_counts, fs.host};
     int mx = 0;
-    bool allow_tile = true;
     for (int attempt = 0; attempt < 4; ++attempt) {
+        // launches and gather as the capacity has them, which an enqueued job
+        // takes too (fpl only falls: a larger capacity, tables)
+        fpl = std::min(fpl, launch_frames(e, fields, fs.z_flat, fs.n, fs.nframes, e->cap));
+        nb = (fs.nframes + fpl - 1) / fpl;
+        j = job_shape(e, fields, fs.z_flat, fs.n, fpl, allow_tile);
+        j.qag_global = qag_global;
+        if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
         Work w{};
-        if ((rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, false, w))) return rc;
+        if ((rc = work_from_engine(e, j, fpl, fs.n, false, w))) return rc;
         for (int b = 0; b < nb; ++b) {
             const int f0 = b * fpl;
             rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), b == 0, e->ev[3 * b],
@@ -1109,10 +1125,8 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
                                                "grid exceed the " + std::to_string(kQagWorkspaceBytes >> 20) +
                                                " MiB workspace");
             fpl = (int)std::min<size_t>((size_t)fpl, fit);
-            nb = (fs.nframes + fpl - 1) / fpl;
-            if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
-            if ((rc = e->d_qag.ensure(per_frame * (size_t)std::min(fpl, fs.nframes)))) return rc;
-            j.qag_global = true;
+            if ((rc = e->d_qag.ensure(per_frame * (size_t)fpl))) return rc;
+            qag_global = true;
             if (grow) e->cap = ((mx + 7) / 8) * 8;
             continue;
         }
@@ -1125,8 +1139,6 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
             break;
         }
         if (grow) e->cap = ((mx + 7) / 8) * 8;
-        // the gather follows the capacity, as it will when the job is enqueued
-        j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes), allow_tile);
         if (attempt == 3) return fail(PGT_ERR_HIP, "bond list capacity did not settle");
     }
     const unsigned long long h[2] = {e->h_counts[1], e->h_counts[2]};
@@ -1155,13 +1167,13 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 // enqueued work shows up in pgt_ik_finish.
 int enqueue_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 {
-    const int fpl = launch_frames(e, fs.n, fs.nframes);
+    const int fpl = launch_frames(e, fields, fs.z_flat, fs.n, fs.nframes, e->cap);
     const int nb = (fs.nframes + fpl - 1) / fpl;
     if (e->cap < 1 || !e->d_maxcount.p || e->d_maxcount.n < 2 || !e->d_stats.p)
         return fail(PGT_ERR_STATE, "run pgt_ik_compute_frames of the same shape before enqueueing");
-    const JobShape j = job_shape(e, fields, fs.z_flat, fs.n, std::min(fpl, fs.nframes));
+    const JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
     Work w{};
-    if (int rc = work_from_engine(e, j, std::min(fpl, fs.nframes), fs.n, true, w)) return rc;
+    if (int rc = work_from_engine(e, j, fpl, fs.n, true, w)) return rc;
     for (int b = 0; b < nb; ++b) {
         const int f0 = b * fpl;
         const int rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), false, nullptr,
@@ -1771,11 +1783,12 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
     fs.kin = (fields & PGT_FIELD_KINETIC) ? d_out_kinetic : nullptr;
     fs.ela = (fields & PGT_FIELD_ELASTIC) ? d_out_elastic : nullptr;
     fs.z_flat = e->grid_z_flat;
-    const int fpl = std::min(launch_frames(e, n, nframes), nframes);
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
     int cap = e->scratch_cap;
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, nframes);
     if (j.pairs && cap < 1) cap = j.D == 3 ? 32 : 16;
     if (!j.pairs) cap = 1;
+    const int fpl = launch_frames(e, fields, fs.z_flat, n, nframes, cap);
+    j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
     const Deliver dv{e->h_counts, {}};
     int mx = 0;
     unsigned long long h[2] = {0, 0};

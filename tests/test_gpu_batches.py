@@ -140,3 +140,63 @@ def test_an_enqueued_job_repeats_the_one_that_grew_its_capacity(gpu, members):
     e.enqueue_frames(1, N, pos, diam, fields=("virial",), d_virial=out)
     e.finish()
     assert np.array_equal(out.cpu().numpy(), grown)
+
+
+def test_more_frames_than_a_launch_takes(gpu):
+    """70,000 frames of 20 particles on 16 points, launch settings untouched:
+    more frames than a launch's y extent holds (65,535), far fewer particles
+    than fill it.  Frames repeat a few, whose fields they must have."""
+    import torch
+
+    N, nf, kinds = 20, 70000, 5
+    frames = _frames(2, N, kinds, 15000)
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    e.set_box(frames[0]["L"], frames[0]["periodic"])
+    e.set_grid(_grid("lattice", frames[0]["L"][0], 2, 4))
+    few = _fields(e, frames, ("virial", "kinetic"))
+    t = {k: _stack(frames, k).repeat(nf // kinds, *([1] * (frames[0][k].ndim))) for k in ("pos", "diam", "mass", "vel")}
+    out = {k: torch.full((nf, 16, 2, 2), np.nan, dtype=torch.float64, device="cuda") for k in few}
+    torch.cuda.synchronize()
+    print("70,000 frames", flush=True)
+    e.compute_frames(nf, N, t["pos"], t["diam"], t["mass"], t["vel"], fields=("virial", "kinetic"),
+                     **{"d_" + k: v for k, v in out.items()})
+    torch.cuda.synchronize()
+    for k, v in out.items():
+        ref = torch.tensor(few[k], device="cuda").repeat(nf // kinds, 1, 1, 1)
+        assert torch.equal(v, ref), k
+
+
+@pytest.mark.parametrize("kind", ["dense", "wide"])
+def test_a_job_keeps_to_its_work_memory(gpu, kind):
+    """Launch settings untouched.  dense: 1,500 frames of 400 particles that are
+    all bonded to one another (400 slots of 24 bytes each: 5.8 GB of entries in
+    one launch).  wide: 3,000 frames of 30 particles in a box of 740 x 740 cells
+    (6.6 GB of cell starts).  Both fit the 4 GB of a launch in two or three of
+    them, with the fields of frames on their own."""
+    import torch
+
+    N, nf, kinds = (400, 1500, 3) if kind == "dense" else (30, 3000, 3)
+    frames = _frames(2, N, kinds, 16000)
+    L = frames[0]["L"] * (1.0 if kind == "dense" else 1500.0 / frames[0]["L"][0])
+    if kind == "dense":
+        for s in frames:
+            s["pos"][:, :2] = 0.02 * s["pos"][:, :2] + L[:2] / 6  # about a grid point
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    e.set_box([L[0], L[1], 1.0], [1, 1, 0])
+    e.set_grid(_grid("lattice", frames[0]["L"][0], 2, 4))
+    ones = [_fields(e, frames, ("virial",), first=f, count=1)["virial"][0] for f in range(kinds)]
+    e.close()
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    e.set_box([L[0], L[1], 1.0], [1, 1, 0])
+    e.set_grid(_grid("lattice", frames[0]["L"][0], 2, 4))
+    pos, diam = (_stack(frames, k).repeat(nf // kinds, *([1] * (frames[0][k].ndim))) for k in ("pos", "diam"))
+    out = torch.full((nf, 16, 2, 2), np.nan, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    e.compute_frames(nf, N, pos, diam, fields=("virial",), d_virial=out)
+    torch.cuda.synchronize()
+    took = (free - torch.cuda.mem_get_info()[0]) / 2 ** 30
+    print("%s: capacity %d, work memory %.2f GB" % (kind, e.stats()["bond_capacity"], took), flush=True)
+    assert e.stats()["bond_capacity"] >= (400 if kind == "dense" else 16)
+    assert took <= 4.2 and out.abs().max() > 0
+    assert torch.equal(out, torch.tensor(np.stack(ones), device="cuda").repeat(nf // kinds, 1, 1, 1))
