@@ -614,6 +614,10 @@ struct JobShape {
     int tp;          // its grid points per workgroup of kTileThreads lanes
     int unit;        // and of the window that orders its sums
     int64_t gwaves;  // gather wavefronts per frame
+    // most wavefronts of a launch of at most the job's frames, with any gather
+    // and launch settings: a launch of fewer frames may have more of them
+    // (tile_part, bond_block)
+    int64_t most_gwaves, most_bwaves;
     bool qag_global; // adaptive rule: interval tables of the caller's limit in e->d_qag
 };
 
@@ -690,6 +694,7 @@ int tile_part(int unit, int64_t tiles)
 {
     return std::min(unit, tiles < 192 ? 4 : tiles < 1536 ? 16 : tiles < 3072 ? 32 : 64);
 }
+constexpr int64_t kPartWaves = 6144;  // no launch has more wavefronts than this and those of its units
 
 // Particles per wavefront of the bond kernel: one a lane, or a quarter of that
 // where the GPU is nearly empty even so (512 wavefronts, half of its SIMDs) and
@@ -697,7 +702,8 @@ int tile_part(int unit, int64_t tiles)
 // pairs.  Cell and bond lists of one frame, 64 / 16 a wavefront: 2D, N = 2,000
 // 26 / 22 us, 8,000 36 / 32, 32,000 52 / 56; with elastic terms 39 / 32, 50 /
 // 43, 70 / 66; 3D, N = 1,000 81 / 67, 8,000 81 / 73, 16,000 85 / 92.
-int bond_block(int64_t particles) { return particles <= 512 * 16 ? 16 : kBondBlock; }
+constexpr int64_t kQuarterParticles = 512 * 16;
+int bond_block(int64_t particles) { return particles <= kQuarterParticles ? 16 : kBondBlock; }
 
 // n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
 // gather even where the tile gather is selected (the fallback when a tile
@@ -743,6 +749,10 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
         const int64_t lanes = (e->G + j.pl - 1) / j.pl;
         j.gwaves = j.adaptive ? adaptive_waves(e->G) : (lanes + j.block - 1) / j.block * (j.block / 64);
     }
+    const int64_t units = (int64_t)e->ntiles * (kTilePoints / tile_unit(e, j.g, j.D, n));
+    j.most_gwaves = std::max(kPartWaves, std::max({units, adaptive_waves(e->G), (e->G + 255) / 256 * 4}) * nf);
+    j.most_bwaves = std::max((n + kBondBlock - 1) / kBondBlock * nf,
+                             kQuarterParticles / 16 + std::min<int64_t>(nf, kQuarterParticles));
     return j;
 }
 
@@ -761,8 +771,9 @@ struct Work {
 };
 
 // Bytes of each work array for nf frames of n particles at bond capacity cap
-// (0 for arrays the job does not use).
-void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, size_t out[W_NARRAYS])
+// (0 for arrays the job does not use).  spare: with counters for any launch of
+// at most nf frames.
+void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, bool spare, size_t out[W_NARRAYS])
 {
     const size_t fn = (size_t)nf * (size_t)n;
     const size_t nchunk = (size_t)((n + kSortChunk - 1) / kSortChunk);
@@ -779,10 +790,9 @@ void work_bytes(const JobShape &j, int nf, int64_t n, int64_t G, int cap, size_t
     if (j.ela) out[W_SDISP] = fn * 3 * sizeof(double);
     if (j.pairs && j.D == 3) out[W_REC] = fn * sizeof(float4);
     if (j.pairs) out[W_BONDS] = fn * (size_t)cap * j.ebytes;
-    // per-wavefront statistics, sized for one point per gather lane (the most
-    // wavefronts any shape launches)
-    out[W_WCOUNTS] = 2 * std::max<size_t>(nw_gather_max, 1) * sizeof(unsigned long long);
-    out[W_WMAX] = std::max<size_t>(nw_bonds, 1) * sizeof(int);
+    // per-wavefront statistics, sized for one point per gather lane at least
+    out[W_WCOUNTS] = 2 * std::max<size_t>(nw_gather_max, spare ? (size_t)j.most_gwaves : 1) * sizeof(unsigned long long);
+    out[W_WMAX] = std::max<size_t>(nw_bonds, spare ? (size_t)j.most_bwaves : 1) * sizeof(int);
 }
 
 // Frames per launch of a job where the caller set none: all of them up to
@@ -803,7 +813,7 @@ int launch_frames(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t 
                                          std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
     if (f <= 8) return f;
     size_t b[W_NARRAYS], frame = 0;
-    work_bytes(job_shape(e, fields, z_flat, n, f), 1, n, e->G, cap, b);
+    work_bytes(job_shape(e, fields, z_flat, n, f), 1, n, e->G, cap, false, b);
     for (size_t x : b) frame += x;
     return (int)std::max<size_t>(8, std::min<size_t>((size_t)f, kLaunchBytes / frame));
 }
@@ -817,7 +827,7 @@ size_t align_up(size_t b) { return (b + kWorkAlign - 1) / kWorkAlign * kWorkAlig
 int work_from_engine(pgt_ik_engine *e, const JobShape &j, int nf, int64_t n, bool no_alloc, Work &w)
 {
     size_t b[W_NARRAYS];
-    work_bytes(j, nf, n, e->G, e->cap, b);
+    work_bytes(j, nf, n, e->G, e->cap, !no_alloc && !e->held, b);
     DBuf<unsigned char> *bufs[W_NARRAYS] = {&e->d_keys0, &e->d_vals0, &e->d_keys1, &e->d_vals1, &e->d_hist,
                                             &e->d_cstart, &e->d_spos, &e->d_sdiam, &e->d_bcount, &e->d_skin,
                                             &e->d_sdisp, &e->d_rec, &e->d_bonds, &e->d_wcounts, &e->d_wmax};
@@ -845,7 +855,7 @@ int work_from_engine(pgt_ik_engine *e, const JobShape &j, int nf, int64_t n, boo
 size_t work_carve(const JobShape &j, int nf, int64_t n, int64_t G, int cap, unsigned char *base, Work *w)
 {
     size_t b[W_NARRAYS];
-    work_bytes(j, nf, n, G, cap, b);
+    work_bytes(j, nf, n, G, cap, false, b);
     size_t off = 0;
     if (w) {
         w->stats = reinterpret_cast<unsigned long long *>(base);

@@ -200,3 +200,34 @@ def test_a_job_keeps_to_its_work_memory(gpu, kind):
     assert e.stats()["bond_capacity"] >= (400 if kind == "dense" else 16)
     assert took <= 4.2 and out.abs().max() > 0
     assert torch.equal(out, torch.tensor(np.stack(ones), device="cuda").repeat(nf // kinds, 1, 1, 1))
+
+
+@pytest.mark.parametrize("N,side,nf", [(2000, 24, 5), (4096, 256, 3)])
+def test_a_sized_engine_takes_fewer_frames(gpu, N, side, nf):
+    """Fewer frames make more wavefronts: quarter blocks of the bond kernel (5
+    frames of 2,000 particles 160 blocks, 4 of them 500), smaller parts of the
+    tiles (3 frames of 1,024 tiles 3,072 whole ones, one 4,096 quarters).  An
+    engine sized by the larger job enqueues the smaller ones, and computes them
+    while its buffers are held."""
+    import torch
+
+    frames = _frames(2, N, nf, 17000)
+    fresh = engine.Engine(dim=2, max_rcut=RMAX)
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    for x in (fresh, e):
+        x.set_box(frames[0]["L"], frames[0]["periodic"])
+        x.set_grid(_grid("lattice", frames[0]["L"][0], 2, side))
+    ref = _fields(fresh, frames, ("virial",))["virial"]
+    print("fewer frames: N=%d side %d, %d frames" % (N, side, nf), flush=True)
+    assert np.array_equal(_fields(e, frames, ("virial",))["virial"], ref)
+    pos, diam = _stack(frames, "pos"), _stack(frames, "diam")
+    for m in range(nf, 0, -1):
+        out = torch.full((m, e.G, 2, 2), np.nan, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        e.enqueue_frames(m, N, pos[:m], diam[:m], fields=("virial",), d_virial=out)
+        e.finish()
+        assert np.array_equal(out.cpu().numpy(), ref[:m]), m
+        assert np.array_equal(_fields(e, frames, ("virial",), count=m)["virial"], ref[:m]), m
+    e.set_gather_mode("lane")  # and after a change of gather
+    assert np.isfinite(_fields(e, frames, ("virial",))["virial"]).all()
+    e.release_enqueued()
