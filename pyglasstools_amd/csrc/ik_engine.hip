@@ -306,6 +306,7 @@ struct DBuf {
         hipError_t e = hipMalloc(&p, want * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();
             return fail(PGT_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
         }
         n = want;
@@ -849,6 +850,19 @@ int work_from_engine(pgt_ik_engine *e, const JobShape &j, int nf, int64_t n, boo
     return 0;
 }
 
+// The shape and work arrays of a job in launches of fpl frames, or, where the
+// caller set no frames per launch and the arrays are held, fixed or not to be
+// had, of half as many down to eight.
+int fit_launch(pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, bool allow_tile, bool no_alloc, int &fpl,
+               JobShape &j, Work &w)
+{
+    for (;; fpl = std::max(8, fpl / 2)) {
+        j = job_shape(e, fields, z_flat, n, fpl, allow_tile);
+        const int rc = work_from_engine(e, j, fpl, n, no_alloc, w);
+        if (!rc || fpl <= 8 || e->frames_per_launch > 0) return rc;
+    }
+}
+
 // Work arrays carved out of `base` (the no-allocation entry point's scratch
 // array): the job counters first, then each array, all 256-byte aligned.
 // Returns the bytes used.
@@ -1101,12 +1115,11 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
         // launches and gather as the capacity has them, which an enqueued job
         // takes too (fpl only falls: a larger capacity, tables)
         fpl = std::min(fpl, launch_frames(e, fields, fs.z_flat, fs.n, fs.nframes, e->cap));
-        nb = (fs.nframes + fpl - 1) / fpl;
-        j = job_shape(e, fields, fs.z_flat, fs.n, fpl, allow_tile);
-        j.qag_global = qag_global;
-        if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
         Work w{};
-        if ((rc = work_from_engine(e, j, fpl, fs.n, false, w))) return rc;
+        if ((rc = fit_launch(e, fields, fs.z_flat, fs.n, allow_tile, false, fpl, j, w))) return rc;
+        j.qag_global = qag_global;
+        nb = (fs.nframes + fpl - 1) / fpl;
+        if ((rc = ensure_events(e, (size_t)nb * 3))) return rc;
         for (int b = 0; b < nb; ++b) {
             const int f0 = b * fpl;
             rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), b == 0, e->ev[3 * b],
@@ -1177,13 +1190,13 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 // enqueued work shows up in pgt_ik_finish.
 int enqueue_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
 {
-    const int fpl = launch_frames(e, fields, fs.z_flat, fs.n, fs.nframes, e->cap);
-    const int nb = (fs.nframes + fpl - 1) / fpl;
     if (e->cap < 1 || !e->d_maxcount.p || e->d_maxcount.n < 2 || !e->d_stats.p)
         return fail(PGT_ERR_STATE, "run pgt_ik_compute_frames of the same shape before enqueueing");
-    const JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
+    int fpl = launch_frames(e, fields, fs.z_flat, fs.n, fs.nframes, e->cap);
+    JobShape j{};
     Work w{};
-    if (int rc = work_from_engine(e, j, fpl, fs.n, true, w)) return rc;
+    if (int rc = fit_launch(e, fields, fs.z_flat, fs.n, true, true, fpl, j, w)) return rc;
+    const int nb = (fs.nframes + fpl - 1) / fpl;
     for (int b = 0; b < nb; ++b) {
         const int f0 = b * fpl;
         const int rc = run_batch(e, j, w, e->cap, fs, fields, f0, std::min(fpl, fs.nframes - f0), false, nullptr,

@@ -231,3 +231,38 @@ def test_a_sized_engine_takes_fewer_frames(gpu, N, side, nf):
     e.set_gather_mode("lane")  # and after a change of gather
     assert np.isfinite(_fields(e, frames, ("virial",))["virial"]).all()
     e.release_enqueued()
+
+
+def test_a_sized_engine_takes_more_frames(gpu):
+    """An engine sized by eight frames, launch settings untouched, enqueues 37
+    of them and computes 37 while its buffers are held: in launches that the
+    buffers hold, the same fields.  Sized by five, it refuses eight."""
+    import torch
+
+    N, nf = 1500, 37
+    frames = _frames(2, N, nf, 18000)
+    fresh = engine.Engine(dim=2, max_rcut=RMAX)
+    e = engine.Engine(dim=2, max_rcut=RMAX)
+    for x in (fresh, e):
+        x.set_box(frames[0]["L"], frames[0]["periodic"])
+        x.set_grid(_grid("lattice", frames[0]["L"][0], 2, 24))
+    ref = _fields(fresh, frames, ("virial", "kinetic"))
+    pos, diam, mass, vel = (_stack(frames, k) for k in ("pos", "diam", "mass", "vel"))
+
+    def enqueue(m):
+        out = {k: torch.full((m, e.G, 2, 2), np.nan, dtype=torch.float64, device="cuda") for k in ref}
+        torch.cuda.synchronize()
+        e.enqueue_frames(m, N, pos[:m], diam[:m], mass[:m], vel[:m], fields=("virial", "kinetic"),
+                         **{"d_" + k: v for k, v in out.items()})
+        e.finish()
+        return {k: v.cpu().numpy() for k, v in out.items()}
+
+    _fields(e, frames, ("virial", "kinetic"), count=5)
+    with pytest.raises(engine.PGTError, match="PGT_ERR_STATE"):
+        enqueue(8)
+    _fields(e, frames, ("virial", "kinetic"), count=8)
+    print("more frames: 8, then 37", flush=True)
+    for got in (enqueue(nf), _fields(e, frames, ("virial", "kinetic")), enqueue(8)):
+        for k in ref:
+            assert np.array_equal(got[k], ref[k][:len(got[k])]), k
+    e.release_enqueued()
