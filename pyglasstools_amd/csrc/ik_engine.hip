@@ -637,10 +637,10 @@ struct JobShape {
 // N = 4,000, one frame, 12^3 872 / 120; N = 94,181, 4 frames, 60^3 1,624 / 787;
 // N = 29,763, 11 frames, 12^3 9,313 / 292 (a coarse grid gives the lane gather few
 // lanes, each with a long list of its own).
-bool default_tile(const pgt_ik_engine *e, const JobShape &j, unsigned fields)
+bool default_tile(const pgt_ik_engine *e, const JobShape &j, unsigned fields, int cap)
 {
     const bool terms = !j.fp32 || (fields & PGT_FIELD_VIRIAL) || !j.pairs;
-    return !e->lane_knobs && terms && e->cap <= 255 &&
+    return !e->lane_knobs && terms && cap <= 255 &&
            tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32);
 }
 
@@ -706,10 +706,11 @@ constexpr int64_t kPartWaves = 6144;  // no launch has more wavefronts than this
 constexpr int64_t kQuarterParticles = 512 * 16;
 int bond_block(int64_t particles) { return particles <= kQuarterParticles ? 16 : kBondBlock; }
 
-// n: particles per frame, nf: frames of a launch.  allow_tile false: the lane
-// gather even where the tile gather is selected (the fallback when a tile
-// reports an overflow)
-JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nf, bool allow_tile = true)
+// n: particles per frame, nf: frames of a launch, cap: the job's bond slots per
+// particle.  allow_tile false: the lane gather even where the tile gather is
+// selected (the fallback when a tile reports an overflow)
+JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, int nf, int cap,
+                   bool allow_tile = true)
 {
     JobShape j{};
     j.OD = e->prm.dim;
@@ -739,7 +740,7 @@ JobShape job_shape(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t
     j.pl = j.adaptive ? 1 : gather_pl(e->points_per_lane, e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD);
     j.tile = allow_tile && !j.adaptive && n <= kTileMaxParticles && e->ntiles > 0 &&
              (e->gather_mode == 1 ? tile_form(e->prm.cg_kind, (int)e->gl_s.size(), j.D, j.OD, j.fp32)
-                                  : e->gather_mode == -1 && default_tile(e, j, fields));
+                                  : e->gather_mode == -1 && default_tile(e, j, fields, cap));
     if (j.tile) {
         j.block = kTileThreads;
         j.pl = 1;
@@ -814,7 +815,7 @@ int launch_frames(const pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t 
                                          std::max<int64_t>(8, ((int64_t)1 << 21) / per_frame));
     if (f <= 8) return f;
     size_t b[W_NARRAYS], frame = 0;
-    work_bytes(job_shape(e, fields, z_flat, n, f), 1, n, e->G, cap, false, b);
+    work_bytes(job_shape(e, fields, z_flat, n, f, cap), 1, n, e->G, cap, false, b);
     for (size_t x : b) frame += x;
     return (int)std::max<size_t>(8, std::min<size_t>((size_t)f, kLaunchBytes / frame));
 }
@@ -857,7 +858,7 @@ int fit_launch(pgt_ik_engine *e, unsigned fields, bool z_flat, int64_t n, bool a
                JobShape &j, Work &w)
 {
     for (;; fpl = std::max(8, fpl / 2)) {
-        j = job_shape(e, fields, z_flat, n, fpl, allow_tile);
+        j = job_shape(e, fields, z_flat, n, fpl, e->cap, allow_tile);
         const int rc = work_from_engine(e, j, fpl, n, no_alloc, w);
         if (!rc || fpl <= 8 || e->frames_per_launch > 0) return rc;
     }
@@ -1107,7 +1108,7 @@ int run_job(pgt_ik_engine *e, const FrameSet &fs, unsigned fields)
     if ((rc = e->d_maxcount.ensure(2)) || (rc = e->d_stats.ensure(2))) return rc;
     int fpl = fs.nframes, nb = 1;
     bool allow_tile = true, qag_global = false;
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, fpl, e->cap);
     if (j.pairs && e->cap < 1) e->cap = j.D == 3 ? 32 : 16;
     const Deliver dv{e->h_counts, fs.host};
     int mx = 0;
@@ -1807,23 +1808,24 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
     fs.ela = (fields & PGT_FIELD_ELASTIC) ? d_out_elastic : nullptr;
     fs.z_flat = e->grid_z_flat;
     int cap = e->scratch_cap;
-    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, nframes);
+    JobShape j = job_shape(e, fields, fs.z_flat, fs.n, nframes, cap);
     if (j.pairs && cap < 1) cap = j.D == 3 ? 32 : 16;
     if (!j.pairs) cap = 1;
     const int fpl = launch_frames(e, fields, fs.z_flat, n, nframes, cap);
-    j = job_shape(e, fields, fs.z_flat, fs.n, fpl);
+    bool allow_tile = true;
     const Deliver dv{e->h_counts, {}};
     int mx = 0;
     unsigned long long h[2] = {0, 0};
     for (int attempt = 0; attempt < 3; ++attempt) {
         // the most frames per launch whose work arrays fit the scratch array
+        j = job_shape(e, fields, fs.z_flat, fs.n, fpl, cap, allow_tile);
         int nf = fpl;
         while (nf > 0 && work_carve(j, nf, n, e->G, cap, nullptr, nullptr) > kScratchBytes) nf = nf / 2;
         if (nf < 1 && (j.tile || j.bp != kBondBlock)) {
             // the tile gather's counters and those of quarter bond blocks take
             // a few KB more than the lane gather's, which may be the ones that
             // do not fit
-            j = job_shape(e, fields, fs.z_flat, fs.n, 1, false);
+            j = job_shape(e, fields, fs.z_flat, fs.n, 1, cap, false);
             j.bp = kBondBlock;
             nf = work_carve(j, 1, n, e->G, cap, nullptr, nullptr) > kScratchBytes ? 0 : 1;
         }
@@ -1853,7 +1855,7 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
         if (grow && mx > 65535) return fail(PGT_ERR_RANGE, "a particle has more than 65535 interacting neighbours");
         if (flags[1] & 6) {
             if (!j.tile) return fail(PGT_ERR_STATE, "tile overflow reported by a lane gather");
-            j = job_shape(e, fields, fs.z_flat, fs.n, fpl, false);
+            allow_tile = false;
         } else if (!grow) {
             break;
         }

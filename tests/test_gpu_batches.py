@@ -266,3 +266,38 @@ def test_a_sized_engine_takes_more_frames(gpu):
         for k in ref:
             assert np.array_equal(got[k], ref[k][:len(got[k])]), k
     e.release_enqueued()
+
+
+def test_noalloc_of_a_dense_system_runs_once(gpu):
+    """Particles with more than 255 bonds: once the no-allocation entry point
+    has found their capacity, an engine whose gather was not chosen goes to the
+    lane gather at once, as one told to (the shortest of 15 calls within 1.25
+    times the other's; a job that runs with the tile gather first takes 1.5
+    times as long)."""
+    import time
+    import torch
+
+    import oracle
+
+    N, rc = 2500, 10.0
+    s = workload.make_system(N, 2, 19000)
+    pos, diam = _stack([s], "pos"), _stack([s], "diam")
+    took, got = {}, {}
+    for mode in ("lane", None):
+        e = engine.Engine(dim=2, params=oracle.poly12_params(rcut=rc), scaled_rcut=rc, max_rcut=rc * float(s["diam"].max()))
+        if mode:
+            e.set_gather_mode(mode)
+        e.set_box(s["L"], s["periodic"])
+        e.set_grid(_grid("lattice", s["L"][0], 2, 48))
+        out = torch.full((1, e.G, 2, 2), np.nan, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        times = []
+        for _ in range(18):
+            t = time.perf_counter()
+            e.compute_frames_noalloc(1, N, pos, diam, fields=("virial",), d_virial=out)
+            times.append(time.perf_counter() - t)
+        assert e.stats()["max_bonds"] > 255
+        took[mode], got[mode] = min(times[3:]), out.cpu().numpy()
+    print("noalloc, dense: lane %.2f ms, by default %.2f ms" % (1e3 * took["lane"], 1e3 * took[None]), flush=True)
+    assert np.array_equal(got[None], got["lane"])
+    assert took[None] <= 1.25 * took["lane"]
