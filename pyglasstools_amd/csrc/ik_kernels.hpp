@@ -366,11 +366,19 @@ __global__ __launch_bounds__(256) void k_sort_finish(Geom g, int n, int nf, int 
 // Those launches, a few microseconds each whatever their size, were a third
 // of a small frame's time on the GPU: N = 2,000 6 us against 20 in six kernels
 // (and their gaps), N = 4,000 10 us; a driver call on them 147 -> 125 and 194 ->
-// 173 us.  With clear0 and clear1 not null the first workgroup also zeroes
-// the job's counters.
+// 173 us.  The counting is quadratic in a cell's particles (open boxes have
+// cells as long as the box), so a frame with more than kSmallCrowd in one is
+// put in order by a radix sort in LDS instead, which takes up to 25 us longer
+// whatever the cells: sort of an open box of N = 8,192 (one cell) 3,080 us by
+// counting, 18 by this, 15 to 24 by the radix launches; N = 2,000 201 / 11 / 15 to 20;
+// a cluster of N = 8,192 in a periodic box, about 60 in a cell, 48 / 47 / 48 to 65, 90
+// 54 / 45 / 54, 200 80 / 51 / 55, all in one 811 / 52 / 59.  With clear0 and clear1 not
+// null the first workgroup also zeroes the job's counters.
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallParticles = 8192;  // most particles of a frame, eight per thread
 constexpr int kSmallCells = 8192;      // most cells (32 KB of LDS each for cells and particles)
+constexpr int kSmallCrowd = 40;        // most particles of a cell that are counted one against another
+constexpr int kSmallRow = 130;         // counts of a digit, 128 and two that put the digits on other LDS banks
 
 __global__ __launch_bounds__(kSmallBlock) void k_sort_small(Geom g, int n, int ncell, const double *__restrict__ pos,
                                                             int *__restrict__ keys, int *__restrict__ vals,
@@ -378,9 +386,11 @@ __global__ __launch_bounds__(kSmallBlock) void k_sort_small(Geom g, int n, int n
                                                             unsigned long long *__restrict__ clear1)
 {
     constexpr int PER = kSmallParticles / kSmallBlock, CPT = kSmallCells / kSmallBlock;
-    __shared__ int s_cell[kSmallCells];  // counts, then each cell's next slot
+    __shared__ int s_cell[128 * kSmallRow / 2];  // counts, then each cell's next slot
+    unsigned short *const s_count = reinterpret_cast<unsigned short *>(s_cell);  // crowded frames
+    static_assert(128 * kSmallRow / 2 >= kSmallCells, "a slot per cell");
     __shared__ int s_order[kSmallParticles];
-    __shared__ int s_wave[kSmallBlock / 64];
+    __shared__ int s_wave[kSmallBlock / 64], s_most[kSmallBlock / 64];
     const int t = threadIdx.x, f = blockIdx.x;
     const size_t fo = (size_t)f * n;
     pos += fo * 3;
@@ -412,11 +422,12 @@ __global__ __launch_bounds__(kSmallBlock) void k_sort_small(Geom g, int n, int n
     __syncthreads();
     // exclusive scan of the counts, `per` consecutive cells per thread
     const int per = (ncell + kSmallBlock - 1) / kSmallBlock;
-    int own[CPT], sum = 0;
+    int own[CPT], sum = 0, most = 0;
 #pragma unroll
     for (int q = 0; q < CPT; ++q) {
         own[q] = q < per && t * per + q < ncell ? s_cell[t * per + q] : 0;
         sum += own[q];
+        most = max(most, own[q]);
     }
     int v = sum;
 #pragma unroll
@@ -424,15 +435,88 @@ __global__ __launch_bounds__(kSmallBlock) void k_sort_small(Geom g, int n, int n
         const int w = __shfl_up(v, off, 64);
         if ((t & 63) >= off) v += w;
     }
-    if ((t & 63) == 63) s_wave[t >> 6] = v;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
+    if ((t & 63) == 63) {
+        s_wave[t >> 6] = v;
+        s_most[t >> 6] = most;
+    }
     __syncthreads();
     int run = v - sum;
 #pragma unroll
-    for (int w = 0; w < kSmallBlock / 64; ++w) run += w < (t >> 6) ? s_wave[w] : 0;
+    for (int w = 0; w < kSmallBlock / 64; ++w) {
+        run += w < (t >> 6) ? s_wave[w] : 0;
+        most = max(most, s_most[w]);
+    }
 #pragma unroll
     for (int q = 0; q < CPT; ++q) {
         if (q < per && t * per + q < ncell) s_cell[t * per + q] = run;
         run += own[q];
+    }
+    if (most > kSmallCrowd) {
+        // a radix sort of cell << 13 | input index in LDS, digits of 7 bits
+        constexpr int NW = kSmallBlock / 64, NE = PER * NW, ND = 128;  // chunks of 64 items, digits
+        static_assert(NE == 128 && ND * NE == 16 * kSmallBlock && kSmallParticles == 1 << 13, "16 counts a thread");
+        const unsigned long long below = (t & 63) ? (~0ull >> (64 - (t & 63))) : 0ull;  // lanes under this one
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (key[u] >= 0) s_order[u * kSmallBlock + t] = key[u] << 13 | (u * kSmallBlock + t);
+        for (int shift = 13; (ncell - 1) >> (shift - 13); shift += 7) {
+            __syncthreads();
+            int item[PER], rank[PER];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) item[u] = s_order[min(u * kSmallBlock + t, n - 1)];
+            for (int q = t; q < ND * kSmallRow / 2; q += kSmallBlock) s_cell[q] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                if (u * kSmallBlock >= n) continue;
+                const bool valid = u * kSmallBlock + t < n;
+                const int d = item[u] >> shift & (ND - 1);
+                unsigned long long peers = __builtin_amdgcn_ballot_w64(valid);
+#pragma unroll
+                for (int b = 1; b < ND; b <<= 1) {
+                    const unsigned long long m = __builtin_amdgcn_ballot_w64((d & b) != 0);
+                    peers &= (d & b) ? m : ~m;
+                }
+                rank[u] = __popcll(peers & below);
+                if (valid && rank[u] == 0)
+                    s_count[d * kSmallRow + u * NW + (t >> 6)] = (unsigned short)__popcll(peers);
+            }
+            __syncthreads();
+            // the first places: an exclusive scan, a digit's chunks by 8 threads
+            unsigned short *const c = s_count + (t >> 3) * kSmallRow + (t & 7) * 16;
+            int x[16], all = 0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                x[q] = all;
+                all += c[q];
+            }
+            int w = all;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int o = __shfl_up(w, off, 64);
+                if ((t & 63) >= off) w += o;
+            }
+            if ((t & 63) == 63) s_wave[t >> 6] = w;
+            __syncthreads();
+            w -= all;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) w += q < (t >> 6) ? s_wave[q] : 0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) c[q] = (unsigned short)(w + x[q]);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < PER; ++u)
+                if (u * kSmallBlock + t < n)
+                    s_order[s_count[(item[u] >> shift & (ND - 1)) * kSmallRow + u * NW + (t >> 6)] + rank[u]] = item[u];
+        }
+        __syncthreads();
+        for (int k = t; k < n; k += kSmallBlock) {
+            keys[k] = s_order[k] >> 13;
+            vals[k] = s_order[k] & (kSmallParticles - 1);
+        }
+        return;
     }
     __syncthreads();
 #pragma unroll

@@ -301,3 +301,51 @@ def test_noalloc_of_a_dense_system_runs_once(gpu):
     print("noalloc, dense: lane %.2f ms, by default %.2f ms" % (1e3 * took["lane"], 1e3 * took[None]), flush=True)
     assert np.array_equal(got[None], got["lane"])
     assert took[None] <= 1.25 * took["lane"]
+
+
+@pytest.mark.parametrize("dim,N,nf,periodic,squeeze", [
+    (2, 41, 1, (0, 0, 0), 1.0), (2, 1000, 1, (0, 0, 0), 1.0), (2, 8192, 2, (0, 0, 0), 1.0), (2, 8191, 1, (1, 0, 0), 1.0),
+    (2, 8192, 1, (1, 1, 0), 0.25), (2, 3001, 3, (1, 1, 0), 0.02), (3, 8192, 1, (0, 0, 0), 1.0), (3, 8100, 1, (1, 0, 0), 1.0),
+    (3, 8192, 1, (1, 1, 1), 0.1), (3, 1025, 2, (1, 1, 1), 0.3)])
+def test_crowded_small_frames_keep_their_order(gpu, dim, N, nf, periodic, squeeze):
+    """Frames of up to 8,192 particles with crowded cells: boxes of one cell,
+    of a row of cells, of a plane of them, clusters in a periodic box of more
+    than 128 cells.  The lane gather adds the kinetic terms in the order of the
+    cell list: bit for bit those of the same frames with particles far from the
+    grid added until they are sorted by the launches of larger frames.  And in
+    good time (a box of one cell once took 3 ms)."""
+    import time
+    import torch
+
+    frames = _frames(dim, N, nf, 20000)
+    L = np.array([90.0, 90.0, 1.0]) if dim == 2 else np.array([30.0, 30.0, 30.0])
+    rng = np.random.default_rng(5)
+    more = 8193 - N + 100
+    larger = []
+    for s in frames:
+        s["pos"][:, :dim] *= squeeze * 0.4 * L[0] / s["L"][0]
+        far = {"pos": np.zeros((more, 3)), "diam": np.ones(more), "mass": np.ones(more), "vel": rng.normal(size=(more, 3))}
+        far["pos"][:, :dim] = rng.uniform(0.38, 0.42, (more, dim)) * L[:dim]
+        larger.append({k: np.concatenate([s[k], far[k]]) for k in far})
+    grid = _grid("lattice", 0.3 * L[0] * squeeze, dim, 9 if dim == 2 else 5)
+    print("crowded %dD N=%d x %d %s squeeze %.2f" % (dim, N, nf, periodic, squeeze), flush=True)
+    got = []
+    for x in (frames, larger):
+        e = engine.Engine(dim=dim, max_rcut=RMAX)
+        e.set_gather_mode("lane")
+        e.set_box(L, periodic)
+        e.set_grid(grid)
+        got.append((_fields(e, x, ("kinetic",))["kinetic"], e.stats()["n_ball"]))
+        if x is frames:
+            out = torch.empty((nf, e.G, dim, dim), dtype=torch.float64, device="cuda")
+            args = [_stack(x, k) for k in ("pos", "diam", "mass", "vel")]
+            torch.cuda.synchronize()
+            times = []
+            for _ in range(10):
+                t = time.perf_counter()
+                e.compute_frames(nf, N, *args, fields=("kinetic",), d_kinetic=out)
+                times.append(time.perf_counter() - t - 1e-3 * e.stats()["gather_ms"])
+    assert got[0][1] == got[1][1] > 0
+    assert np.isfinite(got[0][0]).all() and np.array_equal(got[0][0], got[1][0])
+    print("  without the gather %.0f us" % (1e6 * min(times)), flush=True)
+    assert min(times) < 8e-4
