@@ -1379,7 +1379,7 @@ void pgt_ik_destroy(pgt_ik_engine *e)
     if (!e) return;
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     DBuf<double> *dbufs[] = {&e->d_pos, &e->d_diam, &e->d_mass, &e->d_vel, &e->d_disp, &e->d_grid,
-                             &e->d_out, &e->d_gl};
+                             &e->d_out, &e->d_gl, &e->d_qag};
     for (auto *b : dbufs) b->release();
     DBuf<int> *ibufs[] = {&e->d_perm, &e->d_tperm, &e->d_maxcount};
     for (auto *b : ibufs) b->release();

@@ -349,3 +349,24 @@ def test_crowded_small_frames_keep_their_order(gpu, dim, N, nf, periodic, squeez
     assert np.isfinite(got[0][0]).all() and np.array_equal(got[0][0], got[1][0])
     print("  without the gather %.0f us" % (1e6 * min(times)), flush=True)
     assert min(times) < 8e-4
+
+
+def test_a_closed_engine_gives_its_interval_tables_back(gpu):
+    """An adaptive job whose integrals outgrow the private tables takes tables
+    of the caller's limit (0.9 GB here) from device memory, which closing the
+    engine gives back."""
+    import torch
+
+    s, grid = workload.config_frame(1, 2)
+    torch.cuda.synchronize()
+    for k in range(2):  # (the first engine loads code and tables of the runtime's)
+        before = torch.cuda.mem_get_info()[0]
+        e = engine.Engine(dim=2, cg="rect", max_rcut=RMAX, adaptive=(900, 0.0, 0.0))
+        e.set_system(s, grid)
+        e.compute(fields=("virial",))
+        took = before - torch.cuda.mem_get_info()[0]
+        e.close()
+        left = before - torch.cuda.mem_get_info()[0]
+        print("interval tables: took %.2f GB, kept %.3f GB" % (took / 2 ** 30, left / 2 ** 30), flush=True)
+    assert took > 5e8
+    assert left < 1e8
