@@ -139,25 +139,7 @@ struct GLRule {
     int n;
     double s[kMaxQArg];
     double w[kMaxQArg];
-    // Octic kernel with 5 nodes (bond_octic5), with q_k = w_k^(1/4): q of
-    // nodes 0, 1, 2 (3 and 4 mirror 1 and 0), s_k q_k, s_k^2 q_k, q_k^2
-    double oct_a[3], oct_b[5], oct_c[5], oct_r[3];
 };
-
-// Fills the oct_ terms of a 5-node rule.
-inline void fold_octic5(GLRule &R)
-{
-    if (R.n != 5) return;
-    for (int k = 0; k < 5; ++k) {
-        const long double q = sqrtl(sqrtl((long double)R.w[k]));
-        R.oct_b[k] = (double)(R.s[k] * q);
-        R.oct_c[k] = (double)(R.s[k] * R.s[k] * q);
-        if (k < 3) {
-            R.oct_a[k] = (double)q;
-            R.oct_r[k] = (double)(q * q);
-        }
-    }
-}
 
 // sum_k w_k shape(t(s_k)), t(s) = A + s B + s^2 C: the bond integral of the
 // unnormalised kernel along the segment, in units of the kernel width.
@@ -182,20 +164,24 @@ __device__ __forceinline__ ER bond_quad(const GLRule &R, const double *__restric
     return acc;
 }
 
-// bond_quad of the Octic kernel's 5-node rule with the weights folded into
-// the nodes: w (1 - t^2)_+^2 = (q^2 - (q t)^2)_+^2, q = w^(1/4), and q t is as
-// many operations as t when q A is at hand (Aq, for nodes 0, 1 and 2).
-__device__ __forceinline__ double bond_octic5(const GLRule &R, const double (&Aq)[3], double B, double C)
+// bond_quad of the Octic kernel's 5-node rule: nodes of one weight are added
+// before they are weighted, 28 operations instead of 30.  Error against long
+// double, 2e7 bonds of a 2D glass, rms (and largest), integrals of 0.5 on
+// average: this 4.5e-17 (2.6e-16), the plain sum 4.9e-17 (2.9e-16).  The fourth
+// root of the weight in the nodes, w (1 - t^2)_+^2 = (q^2 - (q t)^2)_+^2, is 25
+// operations but rounds q, s q and s^2 q: 5.9e-17 (3.6e-16), for 1% of a job of
+// 100 frames of N = 65,536.
+__device__ __forceinline__ double bond_octic5(const GLRule &R, double A, double B, double C)
 {
-    double acc = 0.0;
+    double v[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-        const int h = k < 3 ? k : 4 - k;
-        const double t = fma(R.oct_b[k], B, fma(R.oct_c[k], C, Aq[h]));
-        const double u = fmax(fma(-t, t, R.oct_r[h]), 0.0);
-        acc = fma(u, u, acc);
+        const double s = k == 2 ? 0.5 : R.s[k];
+        const double t = fma(s, fma(s, C, B), A);
+        v[k] = fmax(fma(-t, t, 1.0), 0.0);
     }
-    return acc;
+    const double p0 = fma(v[4], v[4], v[0] * v[0]), p1 = fma(v[3], v[3], v[1] * v[1]);
+    return fma(R.w[0], p0, fma(R.w[1], p1, R.w[2] * (v[2] * v[2])));
 }
 
 // Adaptive quadrature (AdaptiveCGFunc::getBondFunc, CoarseGrainFunction.h:

@@ -1000,7 +1000,6 @@ int run_frames(pgt_ik_engine *e, const JobShape &j, const Work &w, int cap, int 
         c.R.s[k] = e->gl_s[k];
         c.R.w[k] = e->gl_w[k];
     }
-    fold_octic5(c.R);
     c.gld = e->d_gl.p;
     c.cgnorm = cg_norm(e->prm.cg_kind, e->prm.cg_rcut);
     c.cstart = cstart;
@@ -1222,7 +1221,6 @@ GLRule engine_rule(const pgt_ik_engine *e)
         R.s[k] = e->gl_s[k];
         R.w[k] = e->gl_w[k];
     }
-    fold_octic5(R);
     return R;
 }
 

@@ -46,8 +46,8 @@
 // wavefront on the 2D N = 65,536 job with a 256^2 grid, 5,814 VALU
 // instructions.  Here a window particle is loaded once per tile, and an
 // item's entries are shared by its neighbours: 126 loads, 4,501 VALU
-// instructions (5,360 before the product tiles' masks, the folded 5-node rule
-// and the two register sets of the item loop).  Measured (one launch, point
+// instructions (5,360 before the product tiles' masks, fewer operations of the
+// 5-node rule and the two register sets of the item loop).  Measured (one launch, point
 // per lane / particle per lane / with those three): 100 such frames 1.68 /
 // 1.38 / 1.17 ms; 3D N = 131,072 with a 64^3 grid, FP32 form, 20 frames 4.30 /
 // 3.72 / 3.23 ms; 3D FP64 with the kinetic field, N = 20,011, 5 frames 0.43 /
@@ -343,15 +343,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                     ta[0] = (ER)(a[0] * s2);
                     ta[1] = (ER)(a[1] * s2);
                     ta[2] = (ER)(a[2] * s2);
-                    // FP64 with the 5-node Octic rule: nodes with the weights
-                    // folded in (bond_octic5), 35 operations a bond instead
-                    // of 40; the FP32 form keeps its rounding
-                    constexpr bool FOLD = CG == 0 && NQ == 5 && std::is_same<ER, double>::value;
                     const ER Aj = (ER)A;
-                    double Aq[3] = {0.0, 0.0, 0.0};
-                    if constexpr (FOLD)
-#pragma unroll
-                        for (int q = 0; q < 3; ++q) Aq[q] = A * R.oct_a[q];
                     // site: 0 and 1, the loop's even and odd groups; 2, the
                     // last of an odd number of groups
                     auto one = [&](const ER (&Gv)[GV], auto O, auto site) {
@@ -375,7 +367,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                         else B = fma(ta[1], e[1], ta[0] * e[0]);
                         if constexpr (D == 3) B = fma(ta[2], e[2], B);
                         ER wq;
-                        if constexpr (FOLD) wq = bond_octic5(R, Aq, B, C);
+                        if constexpr (CG == 0 && NQ == 5 && std::is_same<ER, double>::value) wq = bond_octic5(R, Aj, B, C);
                         else wq = bond_quad<CG, NQ, ER>(R, gld, R.n, Aj, B, C);
                         if constexpr (VIR) {
                             const ER c = wq * e[LY::OC];
