@@ -263,7 +263,8 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
                 const int first = __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(in)) - 1;
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
-                    const double v = in ? xg[a] : __shfl(xg[a], first, 64);
+                    const double f = __shfl(xg[a], first, 64);  // (with every lane active)
+                    const double v = in ? xg[a] : f;
                     lo[a] = wave_min(v);
                     hi[a] = wave_max(v);
                 }
