@@ -660,10 +660,8 @@ bool default_tile(const pgt_ik_engine *e, const JobShape &j, unsigned fields, in
 // = 4,000, one frame, spacing 1.4 (575, 376) - / 41 / 36; N = 131,072, two, spacing
 // 1.75 (753, 471) - / 169 / 140.  So a unit's window holds at most about 300
 // particles in 2D and 400 in 3D; the step to rows of four, which overlap most,
-// is taken above 500 and 600.  A window that reaches around a periodic axis
-// holds the whole axis, at the minimum image: a smaller unit there too, if that
-// avoids it.  The unit knows nothing of the launch: the sums must not depend on
-// how many frames or systems it holds.
+// is taken above 500 and 600.  The unit knows nothing of the launch: the sums
+// must not depend on how many frames or systems it holds.
 int tile_unit(const pgt_ik_engine *e, const Geom &g, int D, int64_t n)
 {
     int unit = kTilePoints;
@@ -674,13 +672,8 @@ int tile_unit(const pgt_ik_engine *e, const Geom &g, int D, int64_t n)
         const double span[3] = {D == 2 && unit >= 32 ? 7.0 : 3.0,
                                 D == 2 ? (unit == 64 ? 7.0 : 3.0) : (unit >= 32 ? 3.0 : 1.0), unit == 64 ? 3.0 : 1.0};
         double window = density;
-        bool around = false;
-        for (int a = 0; a < D; ++a) {
-            const double reach = span[a] * e->grid_step[a] + 2.0 * g.rc;
-            window *= std::min(g.L[a], reach);
-            around = around || (g.periodic[a] && reach >= 0.99 * g.L[a] && 2.0 * g.rc < 0.99 * g.L[a]);
-        }
-        if (window <= (D == 2 ? (unit > 16 ? 300.0 : 500.0) : (unit > 16 ? 400.0 : 600.0)) && !around) break;
+        for (int a = 0; a < D; ++a) window *= std::min(g.L[a], span[a] * e->grid_step[a] + 2.0 * g.rc);
+        if (window <= (D == 2 ? (unit > 16 ? 300.0 : 500.0) : (unit > 16 ? 400.0 : 600.0))) break;
     }
     return unit;
 }
