@@ -34,10 +34,12 @@
 // Up to four batches go through steps 2 to 4 as one list, each ordered by
 // itself.  Parts scan their unit's cells for it: gather of one frame, their
 // own windows alone / this: 2D N = 2,000, 32^2 grid 12 / 15 us, N = 65,536, 256^2
-// 26 / 30; 3D N = 4,000, 12^3 25 / 41, N = 20,011, 37^3 89 / 106; whole tiles, whose
-// scan is the same, take 0.5 to 2.5% longer.  (Loading a step's candidates
-// during the one before: 2D N = 2,000 15 / 15, 3D N = 20,011 106 / 108; whole
-// tiles of a 2D sweep 2% slower, from the registers.)
+// 26 / 30; 3D N = 4,000, 12^3 25 / 37, N = 20,011, 37^3 89 / 103; whole tiles, whose
+// scan is the same, take as long.  The boxes lie in LDS rather than in
+// registers that the item loop would spill, and a 3D scan loads four steps'
+// candidates together (before / after: N = 20,011 106 / 103, whole tiles of the
+// FP32 form 3,210 / 3,150; 2D N = 2,000 15.4 / 16.2, whole tiles of N = 98,304
+// 129 / 139, where one at a time is kept).
 //
 // Why particles, not points, are spread over the lanes in the scan: scattered
 // loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
@@ -187,7 +189,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     constexpr int GV = LY::GV;    // values per read group
 
     __shared__ double s_pt[64][D];               // the points
-    __shared__ double s_box[2 * D];              // their box: centre, half lengths
+    __shared__ double s_box[2][2 * D];           // centre and half lengths of the unit's box, and of theirs
     __shared__ double s_acc[64][KTA];            // their accumulators
     __shared__ double s_wp[MAXW][D];             // window: positions,
     __shared__ int s_wid[MAXW];                  // particles,
@@ -224,7 +226,6 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     // box and its ball fit in less than a period (near), a particle has one
     // image that can be inside any of the balls, the one nearest to xc.
     const bool part = tp < unit;
-    double xc[D], xh[D];
     int w0[3] = {0, 0, 0}, wn[3] = {1, 1, 1};
     bool near = true;
     {
@@ -277,17 +278,18 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             axis_cells(g, a, lo[a], hi[a], g.rc, w0[a], wn[a]);
             w0[a] = __builtin_amdgcn_readfirstlane(w0[a]);
             wn[a] = __builtin_amdgcn_readfirstlane(wn[a]);
-            xc[a] = uniform(0.5 * (lo[a] + hi[a]));
-            xh[a] = uniform(0.5 * (hi[a] - lo[a]));
-            near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh[a] + g.rc) < 0.999 * g.L[a]);
+            const double xh = 0.5 * (hi[a] - lo[a]);
+            s_box[0][a] = 0.5 * (lo[a] + hi[a]);
+            s_box[0][D + a] = xh;
+            near = near && (g.pinvL[a] == 0.0 || 2.0 * (xh + g.rc) < 0.999 * g.L[a]);
         }
         near = __builtin_amdgcn_ballot_w64(near) != 0ull;  // the same in every lane: a scalar
         if (part && near) {
             box(j0, tp, live, lo, hi);
 #pragma unroll
             for (int a = 0; a < D; ++a) {
-                s_box[a] = 0.5 * (lo[a] + hi[a]);
-                s_box[D + a] = 0.5 * (hi[a] - lo[a]);
+                s_box[1][a] = 0.5 * (lo[a] + hi[a]);
+                s_box[1][D + a] = 0.5 * (hi[a] - lo[a]);
             }
         }
     }
@@ -296,7 +298,7 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
     // itself (or may not be): pairs then take the minimum image, which is the
     // plain difference otherwise
     bool images = !near;
-    auto nearest = [&](double v, int a) { return fma(-g.L[a], rint((v - xc[a]) * g.pinvL[a]), v); };
+    auto nearest = [&](double v, int a) { return fma(-g.L[a], rint((v - s_box[0][a]) * g.pinvL[a]), v); };
 
     unsigned long long nball = 0;     // items (the same in every lane)
     unsigned long long ncontrib = 0;  // bond counts of the items, per lane
@@ -655,61 +657,76 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             s_u.seg.first[l] = v - len;
             s_u.seg.particle[l] = b;
             __syncthreads();
-            for (; c0 < total; c0 += 64) {
-                const int c = min(c0 + l, total - 1);
-                // the last segment that starts at or before candidate c
-                int lo = 0;
-                for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1)
-                    if (lo + h < ns && s_u.seg.first[lo + h] <= c) lo += h;
-                const int id = s_u.seg.particle[lo] + c - s_u.seg.first[lo];
-                double x[D], d2 = 0.0, p2 = 0.0;
+            while (c0 < total && !full) {
+                constexpr int NC = D == 3 ? 4 : 1;  // steps whose candidates are loaded together
+                int ids[NC];
+                double xs[NC][D];
 #pragma unroll
-                for (int a = 0; a < D; ++a) x[a] = sp[(size_t)id * PS + a];
-                bool shift = false;
-                if (near) {
+                for (int q = 0; q < NC; ++q) {
+                    if (c0 + 64 * q >= total) continue;
+                    const int c = min(c0 + 64 * q + l, total - 1);
+                    // the last segment that starts at or before candidate c
+                    int lo = 0;
+                    for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1)
+                        if (lo + h < ns && s_u.seg.first[lo + h] <= c) lo += h;
+                    ids[q] = s_u.seg.particle[lo] + c - s_u.seg.first[lo];
 #pragma unroll
-                    for (int a = 0; a < D; ++a) {
-                        const double y = nearest(x[a], a);
-                        shift = shift || y != x[a];
-                        const double d = fabs(y - xc[a]) - xh[a];
-                        d2 = fma(d > 0.0 ? d : d - d, d > 0.0 ? d : d - d, d2);
-                        if (part) {
-                            const double e = fabs(y - s_box[a]) - s_box[D + a];
-                            p2 = fma(e > 0.0 ? e : e - e, e > 0.0 ? e : e - e, p2);
+                    for (int a = 0; a < D; ++a) xs[q][a] = sp[(size_t)ids[q] * PS + a];
+                }
+#pragma unroll
+                for (int q = 0; q < NC; ++q) {
+                    if (c0 >= total) break;
+                    const int id = ids[q];
+                    double x[D], d2 = 0.0, p2 = 0.0;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) x[a] = xs[q][a];
+                    bool shift = false;
+                    if (near) {
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            const double y = nearest(x[a], a);
+                            shift = shift || y != x[a];
+                            const double d = fabs(y - s_box[0][a]) - s_box[0][D + a];
+                            d2 = fma(d > 0.0 ? d : d - d, d > 0.0 ? d : d - d, d2);
+                            if (part) {
+                                const double e = fabs(y - s_box[1][a]) - s_box[1][D + a];
+                                p2 = fma(e > 0.0 ? e : e - e, e > 0.0 ? e : e - e, p2);
+                            }
                         }
                     }
-                }
-                // not near: any image may matter, so every candidate is kept
-                const bool inu = c0 + l < total && d2 < rr, in = inu && p2 < rr;
-                const int ku = __popcll(__builtin_amdgcn_ballot_w64(inu));
-                const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
-                const int k = __popcll(bm);
-                if (nu + ku > MAXW) {  // these candidates begin the next batch
-                    full = ++nbatch == NBATCH || !part;
-                    if (full) break;
-                    nu = 0;
-                    bs = s0;
-                    bc0 = c0;
-                    bw = nw;
-                }
-                full = nw + k > MAXW;
-                if (full) {  // the batch with the next list
-                    s0 = bs;
-                    c0 = bc0;
-                    nw = bw;
-                    break;
-                }
-                images = images || __builtin_amdgcn_ballot_w64(in && shift) != 0ull;
-                if (in) {
-                    const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
-                                                                      __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
-                    s_wid[w] = id;
-                    s_wnb[w] = (unsigned char)nbatch;
+                    // not near: any image may matter, so every candidate is kept
+                    const bool inu = c0 + l < total && d2 < rr, in = inu && p2 < rr;
+                    const int ku = __popcll(__builtin_amdgcn_ballot_w64(inu));
+                    const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
+                    const int k = __popcll(bm);
+                    if (nu + ku > MAXW) {  // these candidates begin the next batch
+                        full = ++nbatch == NBATCH || !part;
+                        if (full) break;
+                        nu = 0;
+                        bs = s0;
+                        bc0 = c0;
+                        bw = nw;
+                    }
+                    full = nw + k > MAXW;
+                    if (full) {  // the batch with the next list
+                        s0 = bs;
+                        c0 = bc0;
+                        nw = bw;
+                        break;
+                    }
+                    images = images || __builtin_amdgcn_ballot_w64(in && shift) != 0ull;
+                    if (in) {
+                        const int w = nw + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0u));
+                        s_wid[w] = id;
+                        s_wnb[w] = (unsigned char)nbatch;
 #pragma unroll
-                    for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
+                        for (int a = 0; a < D; ++a) s_wp[w][a] = x[a];
+                    }
+                    nw += k;
+                    nu += ku;
+                    c0 += 64;
                 }
-                nw += k;
-                nu += ku;
             }
             if (full) {
                 more = true;
