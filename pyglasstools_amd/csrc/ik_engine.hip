@@ -3,19 +3,22 @@
 //
 // Per batch of frames the engine runs (kernels in ik_kernels.hpp):
 //   1. cell list    stable radix sort of the particles by cell (cells of edge
-//                   >= the largest search radius / reach); inside a cell
-//                   particles keep their input order, so every later sum has
-//                   a fixed order
+//                   >= the largest search radius / reach), in one launch for
+//                   small frames; inside a cell particles keep their input
+//                   order, so every later sum has a fixed order
 //   2. bond list    for every particle i, the neighbours j within max_rcut
 //                   with a nonzero pair force, each stored once with the
 //                   scaled bond vector and the force coefficient: the force is
 //                   evaluated once per ordered pair instead of once per
 //                   (grid point, i, j) triple as in the reference loop
-//   3. field gather one lane per 1, 2 or 4 grid points: the particles inside
-//                   the coarse-graining balls are compacted into a per-lane
-//                   LDS list, then the lane integrates every bond of every
-//                   listed particle (5-node Gauss-Legendre on the Octic kernel
-//                   by default) and accumulates the tensors in FP64
+//   3. field gather by default one wavefront per tile of up to 64 grid points
+//                   or a part of it (ik_gather_tile.hpp): the (point, particle)
+//                   pairs of its balls, ordered by bond count, are dealt to the
+//                   lanes, which integrate the particles' bonds (5-node
+//                   Gauss-Legendre on the Octic kernel by default) and add to
+//                   the points' FP64 sums; or one lane per 1, 2 or 4 points
+//                   (ik_gather.hpp), and the adaptive rule
+//                   (ik_gather_adaptive.hpp)
 // Frames are stacked along blockIdx.y so one launch covers many frames (the
 // cell-list kernels deal whole frames to XCDs, see frame_block).  The learned
 // bond-integral surrogate (ik_surrogate.hpp) has entry points of its own.
@@ -551,10 +554,9 @@ Geom make_geom(const pgt_ik_engine *e, int D)
     g.inv_rc2 = 1.0 / g.rc2;
     for (int a = 0; a < 2; ++a) g.inv_nc[a] = 1.0 / (double)g.nc[a];
     g.mr2 = e->prm.max_rcut * e->prm.max_rcut;
-    // FP32 pre-test bounds for the two search radii (r_cg for the gather,
-    // max_rcut for the bond list): fp32_band, with M the largest coordinate
-    // magnitude of box and grid; every searched axis must be periodic, so
-    // that particle coordinates are wrapped into the box
+    // FP32 pre-test bounds of the lane gather (fp32_band), with M the largest
+    // coordinate magnitude of box and grid; every searched axis must be
+    // periodic, so that particle coordinates are wrapped into the box
     for (int a = 0; a < 3; ++a) {
         g.L32[a] = (float)g.L[a];
         g.invL32[a] = (float)g.invL[a];
@@ -569,7 +571,6 @@ Geom make_geom(const pgt_ik_engine *e, int D)
         Lmin = std::min(Lmin, e->L[a]);
     }
     fp32_band(e->prm.cg_rcut, M, Lm, Lmin, D, ok, g.in32, g.out32);
-    fp32_band(e->prm.max_rcut, M, Lm, Lmin, D, ok, g.bin32, g.bout32);
     return g;
 }
 

@@ -23,14 +23,13 @@ struct Geom {
     double inv_rc2;  // 1/cg_rcut^2
     double mr2;      // max_rcut^2
     double inv_nc[2];  // 1/nc[0], 1/nc[1]
-    // FP32 pre-tests of the 3D candidate scans: with |a|^2 from FP32 copies
-    // of the positions, |a|^2 < in32 means inside the coarse-graining ball
-    // and |a|^2 > out32 outside, whatever the FP64 rounding; in between the
-    // FP64 test decides (in32 < 0 and out32 = inf send every candidate to
-    // it).  bin32 and bout32 do the same for the bond search radius.
+    // FP32 pre-test of the lane gather's 3D candidate scan: with |a|^2 from
+    // FP32 copies of the positions, |a|^2 < in32 means inside the
+    // coarse-graining ball and |a|^2 > out32 outside, whatever the FP64
+    // rounding; in between the FP64 test decides (in32 < 0 and out32 = inf send
+    // every candidate to it).
     float L32[3], invL32[3], pinvL32[3];
     float in32, out32;
-    float bin32, bout32;
 };
 
 // Minimum image with the image index rint(d/L) taken as rint(d * (1/L)).

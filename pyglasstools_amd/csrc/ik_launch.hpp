@@ -35,7 +35,7 @@ struct LaunchCtx {
     const void *bonds;
     GatherOut out;
     int *flags;  // job flags: 1 an adaptive integral ran out of workspace, 2 a tile item had more than 255 bonds
-    int tile;    // 1: item-balanced tile gather (Octic 5-node rule), 0: lane gather
+    int tile;    // 1: item-balanced tile gather (tile_form), 0: lane gather
     int lane_terms;  // tile gather, FP32 entries: terms rounded as the lane gather's (see gather_tile_body)
     hipStream_t stream;
 };

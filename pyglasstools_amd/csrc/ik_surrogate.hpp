@@ -74,9 +74,10 @@ constexpr int kGradRow = (kMlpNParam + 3) / 4 * 4;  // floats of a row: the para
                                                     // (8-byte aligned, in the last two) the loss sum
 static_assert(kGradRow >= ((kMlpNParam + 1) & ~1) + 2, "room for the loss");
 
-// Samples of a chunk: 16 while they leave the GPU's CUs a chunk or less each
-// (64 workgroups for 1,024 samples: 9.4 us a launch; 32 samples each on 32
-// workgroups, with the bias sums in one wavefront, 16.9).
+// Samples of a chunk: 16 spread a batch over more CUs (64 workgroups for 1,024
+// samples: 9.4 us a launch; 32 samples each on 32 workgroups, with the bias sums
+// in one wavefront, 16.9), and would up to 4,096 samples, but only up to 1,177
+// do a row for every 16 fit the workspace that callers allocate.
 inline int grad_chunk(int64_t n) { return n <= 1024 ? 16 : 32; }
 inline int grad_rows(int64_t n)
 {

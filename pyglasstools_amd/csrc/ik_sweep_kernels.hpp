@@ -54,8 +54,8 @@ __global__ __launch_bounds__(kSortBlock) void k_sweep_scatter(const SweepSys *__
                              hist + (size_t)S.h0 + (size_t)f * radix * nchunk, kout + fo, vout + fo);
 }
 
-// skin null: no kinetic field; rec non-null (3D with bonds): the FP32
-// candidate records of the bond kernel and the 3D gather.
+// skin null: no kinetic field; rec non-null (3D with bonds): the FP32 records
+// that the bodies write for the lane gather (a sweep's gather reads none).
 template <int D, int OD>
 __global__ __launch_bounds__(256) void k_sweep_finish(const SweepSys *__restrict__ T, int ns,
                                                       const int *__restrict__ keys, const int *__restrict__ vals,
