@@ -33,13 +33,15 @@
 // order, and a smaller part only leaves out those too far from its own points.
 // Up to four batches go through steps 2 to 4 as one list, each ordered by
 // itself.  Parts scan their unit's cells for it: gather of one frame, their
-// own windows alone / this: 2D N = 2,000, 32^2 grid 12 / 15 us, N = 65,536, 256^2
-// 26 / 30; 3D N = 4,000, 12^3 25 / 37, N = 20,011, 37^3 89 / 103; whole tiles, whose
-// scan is the same, take as long.  The boxes lie in LDS rather than in
-// registers that the item loop would spill, and a 3D scan loads four steps'
-// candidates together (before / after: N = 20,011 106 / 103, whole tiles of the
-// FP32 form 3,210 / 3,150; 2D N = 2,000 15.4 / 16.2, whole tiles of N = 98,304
-// 129 / 139, where one at a time is kept).
+// own windows alone, a step of 64 candidates at a time / this: 2D N = 2,000, 32^2
+// grid 12 / 15 us, N = 65,536, 256^2 26 / 29; 3D N = 4,000, 12^3 25 / 32, N = 20,011,
+// 37^3 89 / 98; whole tiles, whose scan is the same, are no slower (3D FP32 form,
+// 20 frames of N = 131,072, 3,150 / 3,120).  The boxes lie in LDS rather than in
+// registers that the item loop would spill, and four steps' candidates are
+// found and loaded together: a step waited for the six reads of its segment's
+// search and for one load, one after the other (one step at a time / four: the
+// 3D frames 41 / 32 and 106 / 98, 20 frames of N = 20,011, 30^3 616 / 588; 2D N = 8,192,
+// open box, 40 frames 217 / 169).
 //
 // Why particles, not points, are spread over the lanes in the scan: scattered
 // loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
@@ -658,21 +660,27 @@ __device__ __forceinline__ void gather_tile_body(const Geom &g, const double *__
             s_u.seg.particle[l] = b;
             __syncthreads();
             while (c0 < total && !full) {
-                constexpr int NC = D == 3 ? 4 : 1;  // steps whose candidates are loaded together
-                int ids[NC];
+                constexpr int NC = 4;  // steps whose candidates are found and loaded together
+                int ids[NC], lo[NC];
                 double xs[NC][D];
 #pragma unroll
-                for (int q = 0; q < NC; ++q) {
-                    if (c0 + 64 * q >= total) continue;
-                    const int c = min(c0 + 64 * q + l, total - 1);
-                    // the last segment that starts at or before candidate c
-                    int lo = 0;
-                    for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1)
-                        if (lo + h < ns && s_u.seg.first[lo + h] <= c) lo += h;
-                    ids[q] = s_u.seg.particle[lo] + c - s_u.seg.first[lo];
+                for (int q = 0; q < NC; ++q) lo[q] = 0;
+                // the last segment that starts at or before each candidate
+                for (int h = ns > 8 ? 32 : 4; h > 0; h >>= 1) {
+                    int f[NC];
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) f[q] = s_u.seg.first[min(lo[q] + h, 63)];
+#pragma unroll
+                    for (int q = 0; q < NC; ++q)
+                        if (lo[q] + h < ns && f[q] <= min(c0 + 64 * q + l, total - 1)) lo[q] += h;
+                }
+#pragma unroll
+                for (int q = 0; q < NC; ++q)
+                    ids[q] = s_u.seg.particle[lo[q]] + min(c0 + 64 * q + l, total - 1) - s_u.seg.first[lo[q]];
+#pragma unroll
+                for (int q = 0; q < NC; ++q)
 #pragma unroll
                     for (int a = 0; a < D; ++a) xs[q][a] = sp[(size_t)ids[q] * PS + a];
-                }
 #pragma unroll
                 for (int q = 0; q < NC; ++q) {
                     if (c0 >= total) break;
