@@ -190,8 +190,9 @@ int pgt_ik_compute_frames_noalloc(pgt_ik_engine *e, int nframes, int64_t n, cons
  * synchronisation, no device allocation, no memset, no events, so a caller
  * can capture the launches into a HIP graph (hipStreamBeginCapture on the
  * engine's stream, see pgt_ik_set_stream) and replay them.  Needs an earlier
- * pgt_ik_compute_frames on this engine with the same frame count, particle
- * count and fields (it sizes the buffers and the bond-list capacity);
+ * pgt_ik_compute_frames on this engine with the same particle count and fields
+ * and at least as many frames (it sizes the buffers and the bond-list
+ * capacity), or at least eight where the frames per launch were not set;
  * otherwise PGT_ERR_STATE.  Check with pgt_ik_finish.  From then on the
  * engine's device buffers are held for the enqueued (or captured) launches:
  * a later call that would free, grow or replace them (pgt_ik_set_grid, a

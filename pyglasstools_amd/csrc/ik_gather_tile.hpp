@@ -49,7 +49,7 @@
 // own cells and every item fetched its particle from memory: 216 loads a
 // wavefront on the 2D N = 65,536 job with a 256^2 grid, 5,814 VALU
 // instructions.  Here a window particle is loaded once per tile, and an
-// item's entries are shared by its neighbours: 126 loads, 4,501 VALU
+// item's entries are shared by its neighbours: 125 loads, 4,724 VALU
 // instructions (5,360 before the product tiles' masks, fewer operations of the
 // 5-node rule and the two register sets of the item loop).  Measured (one launch, point
 // per lane / particle per lane / with those three): 100 such frames 1.68 /
@@ -57,7 +57,7 @@
 // 3.72 / 3.23 ms; 3D FP64 with the kinetic field, N = 20,011, 5 frames 0.43 /
 // 0.37 / 0.34 ms; 2D FP32 form, N = 30,011, 117^2 grid, 33 frames 0.152 /
 // 0.132 / 0.107 ms; a sweep of eight systems whose grid points are up to 2.4
-// apart (r_cg = 2) 0.80 / 0.65 / 0.58 ms.  VALU issue is now 72% of the time.
+// apart (r_cg = 2) 0.80 / 0.65 / 0.58 ms.  VALU issue is now 73% of the time.
 #pragma once
 #include <hip/hip_runtime.h>
 
