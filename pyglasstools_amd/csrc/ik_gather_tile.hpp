@@ -41,7 +41,10 @@
 // found and loaded together: a step waited for the six reads of its segment's
 // search and for one load, one after the other (one step at a time / four: the
 // 3D frames 41 / 32 and 106 / 98, 20 frames of N = 20,011, 30^3 616 / 588; 2D N = 8,192,
-// open box, 40 frames 217 / 169).
+// open box, 40 frames 217 / 169).  A list of several batches has each batch's
+// bond counts from the largest down, so its steps are less even: what a dear
+// rule pays most for (3D, Mollifier kernel, 10 nodes, N = 8,000, 20^3, one frame
+// 105 / 141).
 //
 // Why particles, not points, are spread over the lanes in the scan: scattered
 // loads pace this kernel (a CU's L1 takes about one lane's 16 bytes a cycle
